@@ -359,7 +359,9 @@ size_t nbla_hip_binary_convolution_workspace_bytes(
  * know).  plan[0] = output positions per block of the form that keeps the input
  * positions under a block in LDS (0: the geometry takes the gathering product),
  * plan[1] = blocks per sample, plan[2] = input positions the LDS of a block
- * holds, plan[3] = LDS bytes per block.  Touches no device. */
+ * holds, plan[3] = LDS bytes per block, all of the form with 32 positions per
+ * block; where a launch has more positions than channels to share out, wider
+ * tiles of the same kernel run instead.  Touches no device. */
 int nbla_hip_binary_convolution_slab_plan(
     int64_t outer, int64_t C, int nd, const int64_t *in_sp, int64_t O,
     const int64_t *kernel, const int64_t *pad, const int64_t *stride,

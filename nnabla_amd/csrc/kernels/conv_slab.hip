@@ -2,7 +2,7 @@
 // unfold_to_patches.cpp:103-194 unfold x into a matrix [positions, channels x taps] and multiply it by the weights;
 // here that matrix is never formed, not even in LDS).
 //
-// A block owns up to 32 consecutive output positions of one sample and 256 output channels.  Every input position
+// A block owns up to 32 WM consecutive output positions of one sample and 64 WN output channels.  Every input position
 // ("pixel") that one of its windows touches lies in one run [lo, hi] of the flattened input map; the block reads that
 // run of all the group's channels once (coalesced along the positions), turns every value into four balanced
 // base-256 int8 digits under ONE power-of-two scale for the whole slab, and keeps the digits in LDS pixel by pixel:
@@ -21,11 +21,23 @@
 // (binary_weight_convolution.cpp:58-69), and its first block writes alpha and the zero count out.  Two launches per
 // group make the whole forward.
 //
-// Numerics: q = rint(x * 2^s) with s chosen so that the slab's largest finite magnitude lands in [2^28, 2^29); the
+// The forms <WN, WM, WK>: WN x WM x WK wavefronts, each with a tile of 64 output channels x 32 windows (two channel
+// fragments x four digits = 128 accumulator registers) and every WK-th k tile.  256 output channels fill <4, 1, 2>; with
+// fewer, wavefronts along the channels would multiply padding, so they are laid along the windows instead, and a slab
+// that serves 128 windows reads and converts far less per window than one for 32 (64 channels at 56 x 56: the three input
+// rows under 32 windows of a 3 x 3 kernel are converted for 32 windows, the four under 112 for 112).  Forms of four
+// wavefronts run two blocks to a CU, so one block's set-up and stores lie under the other's MFMAs.  What bounds the
+// kernel is those serial phases (a block: 5 to 8 thousand cycles until its loads are back, 450 per 64 x 16 values
+// converted, 46 per MFMA of 32, 4 to 8 thousand for the epilogue); slab_form_cost weighs them.  Measured, whole forward
+// with the weights' pass, <4, 1, 2> -> the form taken: [32,64,56,56] x [64,64,3,3] 167 -> 44 us, [64,64,28,28] x
+// [64,64,1,1] 68 -> 18.5, [32,128,28,28] x [128,128,3,3] 71 -> 30, [32,96,27,27] x [48,96,5,5] 94 -> 33;
+// [32,256,14,14] x [256,256,3,3] keeps <4, 1, 2> (28.6 us, 31 in <4, 1, 1>).
+//
+// Numerics: q = rint(x * 2^s) with s chosen so that the slab's largest finite magnitude lands in [2^29, 2^30); the
 // four digit products are accumulated exactly in int32, combined exactly in integers with the windows' sums of q
 // (the bits stand for 0 / 1: sum q * (1 - 2 b) = sum q - 2 sum q b) and rounded once to fp32.  The only error is
-// the rounding of x to a multiple of 2^-s: at most 2^-29 of the slab's largest magnitude per element, i.e. finer than
-// fp32 itself for every window whose own largest value is within 2^-5 of the slab's.  A window that holds a NaN or an
+// the rounding of x to a multiple of 2^-s: at most 2^-30 of the slab's largest magnitude per element, i.e. finer than
+// fp32 itself for every window whose own largest value is within 2^-6 of the slab's.  A window that holds a NaN or an
 // infinity gives NaN in all its outputs; other windows of the slab are not affected (such values are left out of the
 // scale and read as 0).
 #include "common.hpp"
@@ -40,20 +52,22 @@ typedef int i32x4_t __attribute__((ext_vector_type(4)));
 typedef int i32x16_t __attribute__((ext_vector_type(16)));
 typedef uint32_t uint4_t __attribute__((ext_vector_type(4)));
 
-constexpr int kSlabThreads = 512;
-constexpr int kSlabRows = 32;        // windows per block: one MFMA fragment
+constexpr int kSlabRows = 32;        // windows per fragment
 constexpr int kSlabDigits = 4;
 constexpr int kSlabPixPad = 16;      // bytes between two pixels: consecutive pixels start 4 banks apart
 constexpr int kSlabMaxTaps = 64;
-constexpr int kSlabAhead = 4;        // k tiles of packed words a wavefront holds in registers ahead of its MFMAs
-constexpr int kSlabTopBit = 28;      // the slab's largest magnitude lands in [2^28, 2^29): four q add up in 32 bits
-constexpr int kSlabReduceBytes = 8 * 16 * 64 * 4; // one fragment of one digit's accumulators from each wavefront
+constexpr int kSlabAhead = 8;        // k tiles of packed words a wavefront holds in registers ahead of its MFMAs
+constexpr int kSlabTopBit = 29;      // the slab's largest magnitude lands in [2^29, 2^30): two q add up in 32 bits
+constexpr int kSlabReduceBytes = 16 * 64 * 4; // per wavefront: one fragment of one digit's accumulators
+constexpr int kSlabHold = 4;         // work items of the set-up a wavefront keeps in registers between its two steps
 constexpr int kSlabLdsLimit = 156 * 1024;
 constexpr int kPrepThreads = 256;
 
 // Sizes and LDS offsets of one launch (host and device).
 struct SlabPlan {
+  int form;        // index into kSlabForms
   int tile_rows, tiles_per_sample, wide_groups;
+  int col_groups;  // groups of 64 wn output channels
   int ct;          // channel tiles of 32 (channels padded)
   int frags;       // fragments of 32 output channels
   int pix_stride;  // bytes per pixel: 128 per channel tile, and the padding
@@ -100,8 +114,11 @@ __host__ __device__ inline int64_t slab_last_tap(const ConvGeom &g) {
          (int64_t)(g.k[2] - 1) * g.dil[2];
 }
 
-__global__ __launch_bounds__(kSlabThreads, 1) void binary_conv_slab_kernel(ConvSlabArgs a) {
+template <int WN, int WM, int WK>
+__global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(ConvSlabArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)
+  constexpr int kWaves = WN * WM * WK, kThreads = 64 * kWaves, kRows = kSlabRows * WM, kCols = 64 * WN;
+  static_assert(WK == 1 || WK == 2, "the contraction is split at most in two");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const ConvGeom &g = a.g;
   const SlabPlan &P = a.p;
@@ -110,8 +127,9 @@ __global__ __launch_bounds__(kSlabThreads, 1) void binary_conv_slab_kernel(ConvS
   // Blocks go to the eight XCDs round-robin: an XCD takes a contiguous run of tiles, so the tiles of one sample --
   // whose slabs overlap and whose outputs share cache lines -- meet in one L2.
   const int64_t work = xcd_remap(blockIdx.x, gridDim.x);
-  const int wg = (int)(work % P.wide_groups);
-  const int tile_all = (int)(work / P.wide_groups);
+  const int cg = (int)(work % P.col_groups);
+  const int wg = cg * kCols / kWideGroup, frag0 = (cg * kCols % kWideGroup) / 32; // first fragment in its wide group
+  const int tile_all = (int)(work / P.col_groups);
   const int n = tile_all / P.tiles_per_sample, tile = tile_all - n * P.tiles_per_sample;
   const int p0 = tile * P.tile_rows;
   const int rows = min(P.tile_rows, (int)g.out_sp_size - p0);
@@ -121,31 +139,36 @@ __global__ __launch_bounds__(kSlabThreads, 1) void binary_conv_slab_kernel(ConvS
   long long *s_pixsum = reinterpret_cast<long long *>(smem + P.pixsum_off);
   long long *s_rowsum = reinterpret_cast<long long *>(smem + P.rowsum_off);
   uint32_t *s_pixbad = reinterpret_cast<uint32_t *>(smem + P.pixbad_off);
-  uint32_t *s_rowpix = reinterpret_cast<uint32_t *>(smem + P.rowpix_off); // [tap][row]: byte offset inside a plane
-  uint32_t *s_rowidx = reinterpret_cast<uint32_t *>(smem + P.rowidx_off); // [tap][row]: pixel index
+  uint32_t *s_rowpix = reinterpret_cast<uint32_t *>(smem + P.rowpix_off); // [tap][row]: pixel index
   int *s_rowbad = reinterpret_cast<int *>(smem + P.rowbad_off);
-  float *s_alpha = reinterpret_cast<float *>(smem + P.alpha_off), *s_bias = s_alpha + kWideGroup;
+  float *s_alpha = reinterpret_cast<float *>(smem + P.alpha_off), *s_bias = s_alpha + kCols;
   int *s_misc = reinterpret_cast<int *>(smem + P.misc_off); // the wavefronts' maxima
 
-  // ---- 0. the block's rows and the slab's extent.  Every wavefront holds all 32 rows (lane % 32), so each finds the
-  // extent by itself and can start loading the slab before anything goes through LDS.
+  // ---- 0. the block's rows and the slab's extent.  Every wavefront walks all the rows (64 lanes at a time), so each
+  // finds the extent by itself and can start loading the slab before anything goes through LDS.
   const int r = lane & 31, half = lane >> 5;
-  const bool row_in = r < rows;
-  int b0, b1, b2, origin;
-  {
-    int p = row_in ? p0 + r : p0; // rows past the tile repeat its first row
+  const int wm = (wave / WN) % WM, row = wm * kSlabRows + r; // the window of this lane in the product
+  const bool row_in = row < rows;
+  auto decode = [&](int m, int &b0, int &b1, int &b2) __attribute__((always_inline)) {
+    int p = m < rows ? p0 + m : p0; // rows past the tile repeat its first row
     const int o2 = p % g.out_sp[2];
     p /= g.out_sp[2];
     const int o1 = p % g.out_sp[1];
     const int o0 = p / g.out_sp[1];
     b0 = o0 * g.stride[0] - g.pad[0], b1 = o1 * g.stride[1] - g.pad[1], b2 = o2 * g.stride[2] - g.pad[2];
-    origin = (b0 * in1 + b1) * in2 + b2;
-  }
+    return (b0 * in1 + b1) * in2 + b2;
+  };
   int lo, npix;
   {
-    int omin = origin, omax = origin;
+    int omin = 0x7fffffff, omax = -0x7fffffff;
 #pragma unroll
-    for (int off = 16; off >= 1; off >>= 1) {
+    for (int m0 = 0; m0 < kRows; m0 += 64) {
+      int b0, b1, b2;
+      const int origin = decode(m0 + lane, b0, b1, b2);
+      omin = min(omin, origin), omax = max(omax, origin);
+    }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) {
       omin = min(omin, __shfl_xor(omin, off));
       omax = max(omax, __shfl_xor(omax, off));
     }
@@ -155,9 +178,9 @@ __global__ __launch_bounds__(kSlabThreads, 1) void binary_conv_slab_kernel(ConvS
     npix = min(hi - lo + 1, P.cap); // (the host sized the LDS for the exact maximum: the clamp never acts)
   }
   // ---- 1. the slab: largest finite magnitude, then the digits.  A work item is 64 pixels x 16 channels (lanes along
-  // the pixels, sixteen loads per lane); wavefront w takes items w, w + 8, ...  A slab of at most two items per
-  // wavefront (64 pixels x 256 channels, say) is loaded once, all loads in flight together, and kept in registers
-  // between the two steps; a larger one is read twice.
+  // the pixels, sixteen loads per lane); wavefront w takes items w, w + kWaves, ...  A slab of at most kSlabHold items
+  // per wavefront is loaded once, all loads in flight together, and kept in registers between the two steps; a larger
+  // one is read twice.
   const float *xs = a.x + ((int64_t)n * g.C + (int64_t)a.grp * g.Cg) * plane + lo;
   const int groups16 = 2 * CT, items = ((npix + 63) >> 6) * groups16;
   // item -> (first pixel, first channel)
@@ -165,22 +188,31 @@ __global__ __launch_bounds__(kSlabThreads, 1) void binary_conv_slab_kernel(ConvS
     const int pc = item / groups16;
     pix0 = pc * 64, ch0 = (item - pc * groups16) * 16;
   };
+  // Nothing but loads: a select or a branch on their results here would make a wavefront wait for one item's loads
+  // before it issues the next item's.  Channels past the last repeat it, pixels past the slab the first.
   auto load_item = [&](int item, float (&v)[16]) __attribute__((always_inline)) {
     int pix0, ch0;
-    item_of(item < items ? item : 0, pix0, ch0);
+    item_of(item, pix0, ch0);
     const int pix = pix0 + lane;
     const float *src = xs + (pix < npix ? pix : 0);
 #pragma unroll
     for (int c = 0; c < 16; ++c)
-      v[c] = (item < items && ch0 + c < Cg) ? src[(int64_t)(ch0 + c) * plane] : 0.0f;
+      v[c] = src[(int64_t)min(ch0 + c, Cg - 1) * plane];
+  };
+  uint32_t amax = 0u;
+  auto scan_item = [&](int item, float (&v)[16]) __attribute__((always_inline)) {
+    int pix0, ch0;
+    item_of(item, pix0, ch0);
     if (a.in_scale) { // one rounded product per element, before anything else
 #pragma unroll
       for (int c = 0; c < 16; ++c)
-        v[c] = v[c] * ((item < items && ch0 + c < Cg) ? a.in_scale[ch0 + c] : 0.0f);
+        v[c] = v[c] * a.in_scale[min(ch0 + c, Cg - 1)];
     }
-  };
-  uint32_t amax = 0u;
-  auto scan_item = [&](const float (&v)[16]) __attribute__((always_inline)) {
+    if (ch0 + 16 > Cg) { // uniform: only the last channel tile can be padded
+#pragma unroll
+      for (int c = 0; c < 16; ++c)
+        v[c] = ch0 + c < Cg ? v[c] : 0.0f;
+    }
 #pragma unroll
     for (int c = 0; c < 16; ++c) {
       const uint32_t m = __float_as_uint(v[c]) & 0x7fffffffu;
@@ -196,13 +228,13 @@ __global__ __launch_bounds__(kSlabThreads, 1) void binary_conv_slab_kernel(ConvS
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       uint32_t d[4];
-      int part = 0; // four |q| < 2^29
+      int part[2] = {0, 0}; // two |q| < 2^30 each
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
         const bool fin = (__float_as_uint(v[4 * u + c]) & 0x7fffffffu) < 0x7f800000u;
         bad = bad || !fin;
         const int q = fin ? (int)rintf(ldexpf(v[4 * u + c], shift)) : 0;
-        part += q;
+        part[c >> 1] += q;
         // bytes: lowest digit .. top digit (the carries of the balanced form run through the addition)
         d[c] = ((uint32_t)q + 0x808080u) ^ 0x808080u;
       }
@@ -214,11 +246,11 @@ __global__ __launch_bounds__(kSlabThreads, 1) void binary_conv_slab_kernel(ConvS
       w[2][u] = __builtin_amdgcn_perm(t23, t01, 0x07060302u);
       w[1][u] = __builtin_amdgcn_perm(u23, u01, 0x05040100u);
       w[0][u] = __builtin_amdgcn_perm(u23, u01, 0x07060302u); // top digits
-      psum += part;
+      psum += (long long)part[0] + part[1];
     }
     int pix0, ch0;
-    item_of(item < items ? item : 0, pix0, ch0);
-    if (item < items && pix0 + lane < npix) {
+    item_of(item, pix0, ch0);
+    if (pix0 + lane < npix) {
       // channel tile ch0 / 32, half (ch0 / 16) % 2 of its 32 channels: one byte per channel and digit
       unsigned char *dst = smem + (pix0 + lane + 1) * P.pix_stride + (ch0 >> 5) * 128 + (ch0 & 16);
 #pragma unroll
@@ -233,16 +265,18 @@ __global__ __launch_bounds__(kSlabThreads, 1) void binary_conv_slab_kernel(ConvS
         s_pixbad[pix0 + lane + 1] = 1u;
     }
   };
-  const bool hold = items <= 16; // uniform over the block
-  float hv[2][16];
+  const bool hold = items <= kSlabHold * kWaves; // uniform over the block
+  float hv[kSlabHold][16];
   if (hold) {
-    load_item(wave, hv[0]);
-    load_item(wave + 8, hv[1]);
+#pragma unroll
+    for (int h = 0; h < kSlabHold; ++h)
+      if (wave + h * kWaves < items) // uniform
+        load_item(wave + h * kWaves, hv[h]);
   }
   // the partial |W| sums of the block's channels (the first eight channel tiles) and the bias: used in the epilogue
   float av[8], bias_v = -0.0f;
-  const int ogp = P.frags * 32, col = wg * kWideGroup + (tid & (kWideGroup - 1));
-  if (tid < kWideGroup) {
+  const int ogp = P.frags * 32, col = cg * kCols + (tid & (kCols - 1));
+  if (tid < kCols) {
     if (a.wsum) {
       const float *part = a.wsum + (col < ogp ? col : ogp - 1);
 #pragma unroll
@@ -253,39 +287,43 @@ __global__ __launch_bounds__(kSlabThreads, 1) void binary_conv_slab_kernel(ConvS
       bias_v = a.bias[col < g.Og ? col : g.Og - 1];
   }
   // while the loads are in flight: the tables in LDS
-  for (int i = tid; i <= P.cap; i += kSlabThreads) {
+  for (int i = tid; i <= P.cap; i += kThreads) {
     s_pixsum[i] = 0;
     s_pixbad[i] = 0u;
   }
-  if (tid < kSlabRows) {
+  if (tid < kRows) {
     s_rowsum[tid] = 0;
     s_rowbad[tid] = 0;
-    s_rowpix[taps * kSlabRows + tid] = 0u; // the entry of steps past the last k tile: the zero pixel
+    s_rowpix[taps * kRows + tid] = 0u; // the entry of steps past the last k tile: the zero pixel
   }
-  for (int i = tid; i < (P.pix_stride >> 2); i += kSlabThreads) // the zero pixel
+  for (int i = tid; i < (P.pix_stride >> 2); i += kThreads) // the zero pixel
     *reinterpret_cast<uint32_t *>(smem + 4 * i) = 0u;
-  for (int t = tid >> 5; t < taps; t += kSlabThreads / 32) { // tap t of row r: its pixel in the slab, if any
+  const int trow = tid & (kRows - 1);
+  int b0, b1, b2;
+  const int origin = decode(trow, b0, b1, b2);
+  for (int t = tid / kRows; t < taps; t += kThreads / kRows) { // tap t of row trow: its pixel in the slab, if any
     int q = t;
     const int k2 = q % g.k[2];
     q /= g.k[2];
     const int k1 = q % g.k[1], k0 = q / g.k[1];
     const int e0 = k0 * g.dil[0], e1 = k1 * g.dil[1], e2 = k2 * g.dil[2];
     const int i0 = b0 + e0, i1 = b1 + e1, i2 = b2 + e2;
-    const bool ok = row_in && (unsigned)i0 < (unsigned)in0 && (unsigned)i1 < (unsigned)in1 &&
+    const bool ok = trow < rows && (unsigned)i0 < (unsigned)in0 && (unsigned)i1 < (unsigned)in1 &&
                     (unsigned)i2 < (unsigned)in2;
     const int idx = origin + (e0 * in1 + e1) * in2 + e2 - lo + 1;
     const bool held = ok && idx >= 1 && idx <= npix;
-    s_rowidx[t * kSlabRows + r] = held ? (uint32_t)idx : 0u;
-    s_rowpix[t * kSlabRows + r] = held ? (uint32_t)(idx * P.pix_stride) : 0u;
+    s_rowpix[t * kRows + trow] = held ? (uint32_t)idx : 0u;
   }
   if (hold) {
-    scan_item(hv[0]);
-    scan_item(hv[1]);
+#pragma unroll
+    for (int h = 0; h < kSlabHold; ++h)
+      if (wave + h * kWaves < items)
+        scan_item(wave + h * kWaves, hv[h]);
   } else {
-    for (int item = wave; item < items; item += 8) {
+    for (int item = wave; item < items; item += kWaves) {
       float v[16];
       load_item(item, v);
-      scan_item(v);
+      scan_item(item, v);
     }
   }
 #pragma unroll
@@ -297,22 +335,25 @@ __global__ __launch_bounds__(kSlabThreads, 1) void binary_conv_slab_kernel(ConvS
   {
     uint32_t bmax = 0u;
 #pragma unroll
-    for (int w = 0; w < 8; ++w)
+    for (int w = 0; w < kWaves; ++w)
       bmax = max(bmax, (uint32_t)s_misc[w]);
     if (bmax != 0u)
       shift = kSlabTopBit - binade_exponent(binade_of(bmax));
   }
   if (hold) {
-    convert_item(wave, hv[0]);
-    convert_item(wave + 8, hv[1]);
+#pragma unroll
+    for (int h = 0; h < kSlabHold; ++h)
+      if (wave + h * kWaves < items)
+        convert_item(wave + h * kWaves, hv[h]);
   } else {
-    for (int item = wave; item < items; item += 8) {
+    for (int item = wave; item < items; item += kWaves) {
       float v[16];
       load_item(item, v);
+      scan_item(item, v); // (the scale and the padding again; the maximum is not used any more)
       convert_item(item, v);
     }
   }
-  if (tid < kWideGroup) { // alpha = (sum of the partial sums, in channel-tile order: every block forms the same bits) / K
+  if (tid < kCols) { // alpha = (sum of the partial sums, in channel-tile order: every block forms the same bits) / K
     float al = 1.0f;
     if (a.wsum) {
       float acc = 0.0f;
@@ -329,7 +370,7 @@ __global__ __launch_bounds__(kSlabThreads, 1) void binary_conv_slab_kernel(ConvS
     s_alpha[tid] = al;
     s_bias[tid] = bias_v;
   }
-  if (work == 0 && wave == 7 && a.zero_count) {
+  if (work == 0 && wave == kWaves - 1 && a.zero_count) {
     int z = 0;
     for (int i = lane; i < CT * P.wide_groups * 32; i += 64)
       z += a.zeros[i];
@@ -344,20 +385,21 @@ __global__ __launch_bounds__(kSlabThreads, 1) void binary_conv_slab_kernel(ConvS
   {
     long long sum = 0;
     uint32_t bad = 0u;
-    for (int t = tid >> 5; t < taps; t += kSlabThreads / 32) {
-      const uint32_t idx = s_rowidx[t * kSlabRows + r];
+    for (int t = tid / kRows; t < taps; t += kThreads / kRows) {
+      const uint32_t idx = s_rowpix[t * kRows + trow];
       sum += s_pixsum[idx];
       bad |= s_pixbad[idx];
     }
     if (sum != 0)
-      atomicAdd(reinterpret_cast<unsigned long long *>(&s_rowsum[r]), (unsigned long long)sum);
+      atomicAdd(reinterpret_cast<unsigned long long *>(&s_rowsum[trow]), (unsigned long long)sum);
     if (bad)
-      s_rowbad[r] = 1;
+      s_rowbad[trow] = 1;
   }
 
-  // ---- 2. the product.  Wavefront (wn, wk): channel fragments 2 wn, 2 wn + 1 of the wide group, k tiles wk, wk + 2, ...
-  const int wn = wave & 3, wk = wave >> 2;
-  const int nk = (P.k_tiles - wk + 1) / 2;
+  // ---- 2. the product.  Wavefront (wn, wm, wk): channel fragments 2 wn, 2 wn + 1 of the block's, window fragment wm,
+  // k tiles wk, wk + WK, ...
+  const int wn = wave % WN, wk = wave / (WN * WM);
+  const int nk = (P.k_tiles - wk + WK - 1) / WK;
   i32x16_t acc[kSlabDigits][2];
 #pragma unroll
   for (int d = 0; d < kSlabDigits; ++d)
@@ -369,13 +411,13 @@ __global__ __launch_bounds__(kSlabThreads, 1) void binary_conv_slab_kernel(ConvS
   uint32_t frag_mask[2];
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
-    frag_mask[j] = 0x01010101u << (2 * wn + j);
+    frag_mask[j] = 0x01010101u << (frag0 + 2 * wn + j);
     asm volatile("" : "+s"(frag_mask[j]));
   }
   if (nk > 0) {
     // the words of step i sit at wnext[lane] when they are loaded: a uniform pointer that stops at the last step
     const uint4_t *wnext = a.bits + ((int64_t)wk * P.wide_groups + wg) * 64;
-    const int64_t wstep = (int64_t)2 * P.wide_groups * 64;
+    const int64_t wstep = (int64_t)WK * P.wide_groups * 64;
     int wleft = nk - 1; // steps the pointer may still advance
     uint4_t words[kSlabAhead];
 #pragma unroll
@@ -384,24 +426,25 @@ __global__ __launch_bounds__(kSlabThreads, 1) void binary_conv_slab_kernel(ConvS
       wnext += wleft > 0 ? wstep : 0;
       --wleft;
     }
-    // position (tap, channel tile) of the k tile two steps ahead, advanced by two k tiles per step
+    // position (tap, channel tile) of the k tile two steps ahead, advanced by WK k tiles per step
     int tap2 = 0, ct2 = wk;
     auto normalise = [&]() __attribute__((always_inline)) {
       if (ct2 >= CT) {
         ct2 -= CT, ++tap2;
-        if (ct2 >= CT)
+        if (WK == 2 && ct2 >= CT)
           ct2 -= CT, ++tap2;
       }
     };
     normalise();
     const uint32_t lane_off = (uint32_t)(half * 16);
-    const uint32_t *my_rowpix = s_rowpix + r;
+    const uint32_t *my_rowpix = s_rowpix + row;
     // LDS offset of the lane's sixteen bytes of step (tap2, ct2); past the last k tile: inside the zero pixel
     auto row_off = [&]() __attribute__((always_inline)) {
-      return my_rowpix[(tap2 < taps ? tap2 : taps) * kSlabRows] + (uint32_t)(ct2 * 128) + lane_off;
+      return __umul24(my_rowpix[(tap2 < taps ? tap2 : taps) * kRows], (uint32_t)P.pix_stride) +
+             (uint32_t)(ct2 * 128) + lane_off;
     };
     auto advance = [&]() __attribute__((always_inline)) {
-      ct2 += 2;
+      ct2 += WK;
       normalise();
     };
     auto read_a = [&](uint32_t off, uint4_t (&af)[kSlabDigits]) __attribute__((always_inline)) {
@@ -435,6 +478,8 @@ __global__ __launch_bounds__(kSlabThreads, 1) void binary_conv_slab_kernel(ConvS
     for (int i0 = 0; i0 < nk; i0 += kSlabAhead) {
 #pragma unroll
       for (int u = 0; u < kSlabAhead; ++u) {
+        if (i0 + u >= nk)
+          break;
         const uint32_t off_c = row_off(); // step i + 2
         advance();
         read_a(off_b, af[(u + 1) & 1]); // step i + 1
@@ -456,17 +501,17 @@ __global__ __launch_bounds__(kSlabThreads, 1) void binary_conv_slab_kernel(ConvS
     }
   }
 
-  // ---- 3. the two k groups' accumulators added exactly through LDS (the planes are free once every wavefront has
-  // left the loop), one digit at a time, in two alternating areas: wavefront (wn, wk) hands the fragment it does not
-  // finish (1 - wk) to its partner (wn, 1 - wk) and adds the partner's copy of fragment wk to its own.
+  // ---- 3. (WK == 2) the two k groups' accumulators added exactly through LDS (the planes are free once every
+  // wavefront has left the loop), one digit at a time, in two alternating areas: a wavefront hands the fragment it does
+  // not finish (1 - wk) to its partner in the other k group and adds the partner's copy of fragment wk to its own.
   i32x16_t fin[kSlabDigits];
-  {
+  if constexpr (WK == 2) {
     uint4_t *red = reinterpret_cast<uint4_t *>(smem);
-    const int mine = wave * 4 * 64 + lane, theirs = (wave ^ 4) * 4 * 64 + lane;
+    const int mine = wave * 4 * 64 + lane, theirs = (wave ^ (WN * WM)) * 4 * 64 + lane;
     __syncthreads();
 #pragma unroll
     for (int d = 0; d < kSlabDigits; ++d) {
-      uint4_t *area = red + (d & 1) * (kSlabReduceBytes / 16);
+      uint4_t *area = red + (d & 1) * (kWaves * kSlabReduceBytes / 16);
       const i32x16_t give = wk ? acc[d][0] : acc[d][1];
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
@@ -493,22 +538,32 @@ __global__ __launch_bounds__(kSlabThreads, 1) void binary_conv_slab_kernel(ConvS
   // while |A| < 2^24 (sums below 2^40), else twice (2^-24 of the sum).
   if (!row_in)
     return;
-  const long long rowsum = s_rowsum[r];
-  const bool rowbad = s_rowbad[r] != 0;
+  const long long rowsum = s_rowsum[row];
+  const bool rowbad = s_rowbad[row] != 0;
   const int s_hi = (int)(rowsum >> 16), s_lo = (int)(rowsum & 0xffff);
-  const int F = 2 * wn + wk;
+  const int osz = (int)g.out_sp_size;
+#pragma unroll
+  for (int jj = 0; jj < 3 - WK; ++jj) { // the fragments this wavefront finishes: both, or the one of its k group
+  const int jf = WK == 2 ? wk : jj, fb = 2 * wn + jf;
+  if constexpr (WK == 1) {
+#pragma unroll
+    for (int d = 0; d < kSlabDigits; ++d)
+      fin[d] = acc[d][jj];
+  }
+  const int F = frag0 + fb; // the fragment's place in its wide group: the scale of its accumulators
   const bool negate = F == 7;
   // channel of register q: c0 + 8 (q / 4) + q % 4; everything an output needs besides its accumulators is fetched
   // before the stores (the compiler does not move a load across them)
-  const int c0 = F * 32 + 4 * half, og_left = (int)g.Og - wg * kWideGroup - c0; // channels from c0 to the group's last
-  const int osz = (int)g.out_sp_size;
+  const int c0 = fb * 32 + 4 * half, og_left = (int)g.Og - cg * kCols - c0; // channels from c0 to the group's last
+  if (og_left <= 0)
+    break;
   float al[16], bi[16];
 #pragma unroll
   for (int q = 0; q < 16; ++q) {
     al[q] = s_alpha[c0 + 8 * (q >> 2) + (q & 3)];
     bi[q] = s_bias[c0 + 8 * (q >> 2) + (q & 3)];
   }
-  float *ybase = a.y + (((int64_t)n * g.O + (int64_t)a.grp * g.Og + (int64_t)wg * kWideGroup + c0) * g.out_sp_size + p0 + r);
+  float *ybase = a.y + (((int64_t)n * g.O + (int64_t)a.grp * g.Og + (int64_t)cg * kCols + c0) * g.out_sp_size + p0 + row);
   float prev[16];
   if (a.accumulate) {
 #pragma unroll
@@ -537,18 +592,15 @@ __global__ __launch_bounds__(kSlabThreads, 1) void binary_conv_slab_kernel(ConvS
   // Ws = Wb * alpha, then + b: Inf * w = +-Inf, Inf - Inf = NaN), so the lane recomputes its sixteen outputs as plain
   // fp32 dot products over the materialised signs and replaces the NaN stored above.
   if (rowbad && a.redo_w) {
-    int p = p0 + r;
-    const int o2 = p % g.out_sp[2];
-    p /= g.out_sp[2];
-    const int o1 = p % g.out_sp[1], o0 = p / g.out_sp[1];
-    const int w0 = o0 * g.stride[0] - g.pad[0], w1 = o1 * g.stride[1] - g.pad[1], w2 = o2 * g.stride[2] - g.pad[2];
+    int w0, w1, w2;
+    decode(row, w0, w1, w2);
     const float *xn = a.x + ((int64_t)n * g.C + (int64_t)a.grp * g.Cg) * plane;
 #pragma unroll 1
     for (int q = 0; q < 16; ++q) {
       const int cq = 8 * (q >> 2) + (q & 3);
       if (cq >= og_left)
         continue;
-      const float *wrow = a.redo_w + ((int64_t)wg * kWideGroup + c0 + cq) * ((int64_t)Cg * taps);
+      const float *wrow = a.redo_w + ((int64_t)cg * kCols + c0 + cq) * ((int64_t)Cg * taps);
       const float scale = s_alpha[c0 + cq];
       float acc = 0.0f;
 #pragma unroll 1
@@ -566,33 +618,44 @@ __global__ __launch_bounds__(kSlabThreads, 1) void binary_conv_slab_kernel(ConvS
       ybase[cq * osz] = acc + s_bias[c0 + cq];
     }
   }
+  }
 #endif
 }
+
+// Division of a small non-negative number (below 2^21) by a constant of the launch: the quotient of the number plus one
+// half is at least 1 / (2 d) away from a whole number, more than the rounding of the two fp32 operations for
+// d <= 2048 (kSlabMaxTaps * 32).
+struct SmallDivide {
+  float inv;
+  __device__ __forceinline__ explicit SmallDivide(int d) : inv(1.0f / (float)d) {}
+  __device__ __forceinline__ int operator()(int v) const { return (int)(((float)v + 0.5f) * inv); }
+};
 
 // One pass over the weights W [Og, Cg, taps] of a group: Wb = Sign(W) (sign.hpp:48-50), the packed bits of the product
 // above in the order k' = tap * (32 ct) + channel, and per channel tile the sums of |W| and the counts of weights that
 // are neither negative nor positive.  Block (wide group, channel tile ct, r): the eight output channels
 // 256 wg + 32 F + r, F = 0..7 -- the ones whose bits share the packed words of lanes r and r + 32 -- and the 32 input
-// channels of the tile: a contiguous run of 32 * taps floats per row.  The signs go to LDS as bytes, from where
-// thread (tap, half) assembles its packed word; |w| goes through LDS so that a row's sum is formed by one wavefront in
-// a fixed order.
+// channels of the tile: a contiguous run of 32 * taps floats per row.  A negative weight sets its bit of the packed
+// words in LDS with an atomic OR (nothing waits for it; assembling a word from 32 bytes in LDS afterwards took as long
+// as the rest of the kernel: 8.4 -> 6.0 us for 256 x 256 x 9 weights); |w| goes through LDS so that a row's sum is formed
+// by one wavefront in a fixed order.
 __global__ __launch_bounds__(kPrepThreads) void conv_taps_prepare(const float *__restrict__ W, float *__restrict__ Wb,
                                                                   uint4_t *__restrict__ bits, float *__restrict__ wsum,
                                                                   int *__restrict__ zeros, int Og, int Cg, int taps,
                                                                   int ct_count, int frags, int wide_groups,
                                                                   float zero_to) {
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  // [8 rows][32 * taps]: |w| as floats, then the "negative" flags as bytes
+  // [8 rows][32 * taps] |w|, then the packed words of the block's k tiles: [tap][half][4]
+  extern __shared__ __attribute__((aligned(16))) float s_abs[];
   const int seg_full = 32 * taps;
-  float *s_abs = reinterpret_cast<float *>(smem);
-  unsigned char *s_neg = smem + (size_t)8 * seg_full * 4;
+  uint32_t *s_words = reinterpret_cast<uint32_t *>(s_abs + 8 * seg_full);
   __shared__ int s_zero[kPrepThreads / 64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wg = blockIdx.x / 32, r = blockIdx.x % 32, ct = blockIdx.y;
   const int c0 = ct * 32, cn = min(32, Cg - c0), seg = cn * taps, elems = 8 * seg;
   const int64_t Kg = (int64_t)Cg * taps;
-  for (int i = tid; i < 8 * seg_full / 4; i += kPrepThreads)
-    reinterpret_cast<uint32_t *>(s_neg)[i] = 0u; // rows and channels past the end: bit clear (their digits are 0)
+  const SmallDivide by_seg(seg), by_taps(taps);
+  for (int i = tid; i < 8 * taps; i += kPrepThreads)
+    s_words[i] = 0u; // rows and channels past the end: bit clear (their digits are 0)
   __syncthreads();
   int nzero = 0;
   for (int base = 0; base < elems; base += 12 * kPrepThreads) {
@@ -601,16 +664,16 @@ __global__ __launch_bounds__(kPrepThreads) void conv_taps_prepare(const float *_
 #pragma unroll
     for (int m = 0; m < 12; ++m) {
       const int idx = base + tid + kPrepThreads * m;
-      const int f = idx / seg, kl = idx - f * seg;
+      const int f = by_seg(idx), kl = idx - f * seg;
       const int n = wg * kWideGroup + 32 * f + r;
       const bool in = idx < elems && n < Og;
       at[m] = in ? (int64_t)n * Kg + (int64_t)c0 * taps + kl : -1;
-      w[m] = in ? W[at[m]] : 1.0f;
+      w[m] = W[in ? at[m] : 0];
     }
 #pragma unroll
     for (int m = 0; m < 12; ++m) {
       const int idx = base + tid + kPrepThreads * m;
-      const int f = idx / seg, kl = idx - f * seg;
+      const int f = by_seg(idx), kl = idx - f * seg;
       if (idx < elems)
         s_abs[f * seg_full + kl] = at[m] >= 0 ? fabsf(w[m]) : 0.0f;
       if (at[m] >= 0) {
@@ -618,12 +681,28 @@ __global__ __launch_bounds__(kPrepThreads) void conv_taps_prepare(const float *_
         const bool neg = (w[m] < 0.0f) || (is_zero && zero_to < 0.0f);
         if (Wb)
           Wb[at[m]] = (w[m] > 0.0f) ? 1.0f : ((w[m] < 0.0f) ? -1.0f : zero_to);
-        s_neg[f * seg_full + kl] = neg ? 1 : 0;
+        const int ch = by_taps(kl), t = kl - ch * taps;
+        if (neg)
+          atomicOr(&s_words[8 * t + (ch >> 2)], 1u << (f + 8 * (ch & 3)));
         nzero += is_zero ? 1 : 0;
       }
     }
   }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1)
+    nzero += __shfl_xor(nzero, off);
+  if (lane == 0)
+    s_zero[wave] = nzero;
   __syncthreads();
+  // the packed words of lanes r and r + 32 of the block's k tiles (tap, ct): word i, byte c, bit F <- row F, channel
+  // c0 + 16 half + 4 i + c
+  for (int item = tid; item < 2 * taps; item += kPrepThreads) {
+    const int t = item >> 1, g16 = item & 1;
+    bits[((int64_t)(t * ct_count + ct) * wide_groups + wg) * 64 + g16 * 32 + r] =
+        reinterpret_cast<const uint4_t *>(s_words)[item];
+  }
+  if (tid == 0)
+    zeros[(ct * wide_groups + wg) * 32 + r] = s_zero[0] + s_zero[1] + s_zero[2] + s_zero[3];
   for (int f = wave; f < 8; f += kPrepThreads / 64) {
     float asum = 0.0f;
     for (int kl = lane; kl < seg; kl += 64)
@@ -634,30 +713,6 @@ __global__ __launch_bounds__(kPrepThreads) void conv_taps_prepare(const float *_
     const int n = wg * kWideGroup + 32 * f + r;
     if (lane == 0 && n < frags * 32)
       wsum[(int64_t)ct * frags * 32 + n] = asum; // rows past Og: zero
-  }
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1)
-    nzero += __shfl_xor(nzero, off);
-  if (lane == 0)
-    s_zero[wave] = nzero;
-  __syncthreads();
-  if (tid == 0)
-    zeros[(ct * wide_groups + wg) * 32 + r] = s_zero[0] + s_zero[1] + s_zero[2] + s_zero[3];
-  // the packed words of lanes r and r + 32 of the block's k tiles (tap, ct): word i, byte c, bit F <- row F, channel
-  // c0 + 16 half + 4 i + c
-  for (int item = tid; item < 2 * taps; item += kPrepThreads) {
-    const int t = item >> 1, g16 = item & 1;
-    uint32_t o[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-    for (int f = 0; f < 8; ++f) {
-      const unsigned char *src = s_neg + f * seg_full + (g16 * 16) * taps + t;
-#pragma unroll
-      for (int j = 0; j < 16; ++j)
-        o[j >> 2] |= (uint32_t)src[j * taps] << (8 * (j & 3) + f);
-    }
-    uint4_t v;
-    v.x = o[0], v.y = o[1], v.z = o[2], v.w = o[3];
-    bits[((int64_t)(t * ct_count + ct) * wide_groups + wg) * 64 + g16 * 32 + r] = v;
   }
 }
 
@@ -670,37 +725,40 @@ __global__ __launch_bounds__(kPrepThreads) void conv_taps_prepare_transposed(con
                                                                              uint4_t *__restrict__ bits, int Og, int Cg,
                                                                              int taps, int ct_count, int wide_groups,
                                                                              float zero_to) {
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  extern __shared__ __attribute__((aligned(16))) uint32_t s_words[]; // [tap, flipped][half][4]
   const int seg_full = 32 * taps;
-  unsigned char *s_neg = smem; // [8 rows c][32 channels o][tap, flipped]
+  const SmallDivide by_taps(taps);
   const int tid = threadIdx.x;
   const int wg = blockIdx.x / 32, r = blockIdx.x % 32, ct = blockIdx.y;
   const int o0 = ct * 32;
-  for (int idx = tid; idx < 8 * seg_full; idx += kPrepThreads) {
-    const int f = idx / seg_full, rem = idx - f * seg_full, ol = rem / taps, t = rem - ol * taps;
-    const int c = wg * kWideGroup + 32 * f + r, o = o0 + ol;
-    unsigned char neg = 0;
-    if (c < Cg && o < Og) {
-      const float w = W[((int64_t)o * Cg + c) * taps + t];
-      const bool is_zero = !(w > 0.0f) && !(w < 0.0f);
-      neg = ((w < 0.0f) || (is_zero && zero_to < 0.0f)) ? 1 : 0;
+  for (int i = tid; i < 8 * taps; i += kPrepThreads)
+    s_words[i] = 0u;
+  __syncthreads();
+  // one output channel o after the other: its rows c = 256 wg + 32 f + r are runs of `taps` floats 32 * taps apart
+  for (int base = 0; base < 8 * seg_full; base += 8 * kPrepThreads) {
+    float w[8];
+    int at[8]; // word * 32 + bit; -1: outside
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+      const int idx = base + tid + kPrepThreads * m;
+      const int rest = by_taps(idx), t = idx - rest * taps, f = rest & 7, ol = rest >> 3;
+      const int c = wg * kWideGroup + 32 * f + r, o = o0 + ol;
+      const bool in = idx < 8 * seg_full && c < Cg && o < Og;
+      at[m] = in ? (8 * (taps - 1 - t) + (ol >> 2)) * 32 + f + 8 * (ol & 3) : -1;
+      w[m] = W[in ? ((int64_t)o * Cg + c) * taps + t : 0];
     }
-    s_neg[f * seg_full + ol * taps + (taps - 1 - t)] = neg;
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+      const bool is_zero = !(w[m] > 0.0f) && !(w[m] < 0.0f);
+      if (at[m] >= 0 && ((w[m] < 0.0f) || (is_zero && zero_to < 0.0f)))
+        atomicOr(&s_words[at[m] >> 5], 1u << (at[m] & 31));
+    }
   }
   __syncthreads();
   for (int item = tid; item < 2 * taps; item += kPrepThreads) {
     const int t = item >> 1, g16 = item & 1;
-    uint32_t o[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-    for (int f = 0; f < 8; ++f) {
-      const unsigned char *src = s_neg + f * seg_full + (g16 * 16) * taps + t;
-#pragma unroll
-      for (int j = 0; j < 16; ++j)
-        o[j >> 2] |= (uint32_t)src[j * taps] << (8 * (j & 3) + f);
-    }
-    uint4_t v;
-    v.x = o[0], v.y = o[1], v.z = o[2], v.w = o[3];
-    bits[((int64_t)(t * ct_count + ct) * wide_groups + wg) * 64 + g16 * 32 + r] = v;
+    bits[((int64_t)(t * ct_count + ct) * wide_groups + wg) * 64 + g16 * 32 + r] =
+        reinterpret_cast<const uint4_t *>(s_words)[item];
   }
 }
 
@@ -730,11 +788,11 @@ int64_t slab_longest_run(const ConvGeom &g, int tile_rows, int tiles_per_sample)
   return longest;
 }
 
-bool compute_slab_plan(const ConvGeom &g, SlabPlan &p);
+bool compute_slab_plan(const ConvGeom &g, SlabPlan &narrow, SlabPlan &p);
 
 // The plan of a geometry is asked for several times per call (does it apply, how much workspace, the launches) and
 // sizing the slab walks the tiles of a sample: the last few answers are kept per thread.
-bool make_slab_plan(const ConvGeom &g, SlabPlan &p) {
+bool make_slab_plan(const ConvGeom &g, SlabPlan &p, bool narrow = false) {
   struct Key {
     int64_t outer, C, O, group;
     int in_sp[kMaxSpatial], k[kMaxSpatial], pad[kMaxSpatial], stride[kMaxSpatial], dil[kMaxSpatial];
@@ -749,7 +807,7 @@ bool make_slab_plan(const ConvGeom &g, SlabPlan &p) {
   constexpr int kKept = 4; // a forward and a backward geometry alternate in training
   static thread_local bool have[kKept] = {false, false, false, false}, kept_ok[kKept];
   static thread_local Key kept_key[kKept];
-  static thread_local SlabPlan kept_plan[kKept];
+  static thread_local SlabPlan kept_plan[kKept][2]; // the narrowest form and the one that runs
   static thread_local int next = 0;
   Key key;
   key.outer = g.outer, key.C = g.C, key.O = g.O, key.group = g.group;
@@ -758,40 +816,45 @@ bool make_slab_plan(const ConvGeom &g, SlabPlan &p) {
     key.dil[i] = g.dil[i];
   for (int e = 0; e < kKept; ++e)
     if (have[e] && key == kept_key[e]) {
-      p = kept_plan[e];
+      p = kept_plan[e][narrow ? 0 : 1];
       return kept_ok[e];
     }
   const int e = next;
   next = (next + 1) % kKept;
-  kept_ok[e] = compute_slab_plan(g, kept_plan[e]);
+  kept_ok[e] = compute_slab_plan(g, kept_plan[e][0], kept_plan[e][1]);
   kept_key[e] = key;
   have[e] = true;
-  p = kept_plan[e];
+  p = kept_plan[e][narrow ? 0 : 1];
   return kept_ok[e];
 }
 
-bool compute_slab_plan(const ConvGeom &g, SlabPlan &p) {
-  if (g.k_size > kSlabMaxTaps || g.Cg < 24 || g.in_sp_size >= ((int64_t)1 << 30) ||
-      g.out_sp_size >= ((int64_t)1 << 30) || g.Og >= ((int64_t)1 << 24) ||
-      (g.Og + kWideGroup) * g.out_sp_size >= ((int64_t)1 << 31))
-    return false;
+// The forms of the product: WN x WM x WK wavefronts, each with a tile of 64 output channels x 32 windows.
+struct SlabForm {
+  int wn, wm, wk;
+};
+constexpr SlabForm kSlabForms[] = {{4, 1, 2}, {4, 2, 1}, {4, 1, 1}, {2, 2, 1}, {1, 4, 2}, {1, 4, 1}};
+constexpr int kSlabFormCount = (int)(sizeof(kSlabForms) / sizeof(kSlabForms[0]));
+
+// The plan of one form; false when its slab does not fit the LDS.
+bool compute_slab_form(const ConvGeom &g, int form, SlabPlan &p) {
+  const SlabForm &f = kSlabForms[form];
+  const int waves = f.wn * f.wm * f.wk, rows = kSlabRows * f.wm;
+  p.form = form;
   const int64_t cgp = ceil_div(g.Cg, 32) * 32;
-  // padded channels cost as much as real ones; the epilogue's 32-bit steps hold kChunkK terms
-  if (cgp * 3 > g.Cg * 4 || g.k_size * cgp > kChunkK)
-    return false;
   const int64_t ow = g.out_sp[2], map_rows = g.out_sp_size / ow;
-  if (ow <= kSlabRows) { // whole rows of the output map, evenly
-    const int64_t per = kSlabRows / ow, tiles = ceil_div(map_rows, per);
+  if (ow <= rows) { // whole rows of the output map, evenly
+    const int64_t per = rows / ow, tiles = ceil_div(map_rows, per);
     p.tile_rows = (int)(ceil_div(map_rows, tiles) * ow);
   } else {
-    p.tile_rows = (int)ceil_div(g.out_sp_size, ceil_div(g.out_sp_size, kSlabRows));
+    p.tile_rows = (int)ceil_div(g.out_sp_size, ceil_div(g.out_sp_size, rows));
   }
   const int64_t tiles = ceil_div(g.out_sp_size, p.tile_rows);
   if (tiles > 16384) // the host walks them to size the slab
     return false;
   p.tiles_per_sample = (int)tiles;
   p.wide_groups = (int)bits_wide_groups(g.Og);
-  if (g.outer * tiles * p.wide_groups >= ((int64_t)1 << 31))
+  p.col_groups = (int)ceil_div(g.Og, 64 * f.wn);
+  if (g.outer * tiles * p.col_groups >= ((int64_t)1 << 31))
     return false;
   p.ct = (int)(cgp / 32);
   p.frags = (int)ceil_div(g.Og, 32);
@@ -804,16 +867,16 @@ bool compute_slab_plan(const ConvGeom &g, SlabPlan &p) {
   p.slab_bytes = (int)slab_bytes;
   p.k_tiles = (int)(g.k_size * p.ct);
   int64_t off = slab_bytes;
-  if (off < 2 * kSlabReduceBytes) // two areas for the exchange between the k groups
-    off = 2 * kSlabReduceBytes;
+  if (f.wk == 2 && off < 2 * waves * kSlabReduceBytes) // two areas for the exchange between the k groups
+    off = 2 * waves * kSlabReduceBytes;
+  off = (int64_t)round_up((size_t)off, 16);
   p.pixsum_off = (int)off, off += 8 * (cap + 1);
-  p.rowsum_off = (int)off, off += 8 * kSlabRows;
+  p.rowsum_off = (int)off, off += 8 * rows;
   off = (int64_t)round_up((size_t)off, 16);
   p.pixbad_off = (int)off, off += 4 * (cap + 1);
-  p.rowpix_off = (int)off, off += 4 * kSlabRows * (g.k_size + 1);
-  p.rowidx_off = (int)off, off += 4 * kSlabRows * g.k_size;
-  p.rowbad_off = (int)off, off += 4 * kSlabRows;
-  p.alpha_off = (int)off, off += 2 * 4 * kWideGroup;
+  p.rowpix_off = (int)off, off += 4 * rows * (g.k_size + 1);
+  p.rowbad_off = (int)off, off += 4 * rows;
+  p.alpha_off = (int)off, off += 2 * 4 * 64 * f.wn;
   p.misc_off = (int)off, off += 64;
   p.total = (int)off;
   p.bits_bytes = (size_t)p.k_tiles * p.wide_groups * kFragBytes;
@@ -821,6 +884,64 @@ bool compute_slab_plan(const ConvGeom &g, SlabPlan &p) {
   p.zeros_off = p.wsum_off + round_up((size_t)p.ct * p.frags * 32 * sizeof(float), 256);
   p.prep_bytes = p.zeros_off + round_up((size_t)p.ct * p.wide_groups * 32 * sizeof(int), 256);
   return off <= kSlabLdsLimit;
+}
+
+// Cycles of the launch, roughly: what the phases of a block measured (time stamps in blocks of 64, 256 and 512 input
+// channels).  A block starts and waits for its first loads for about 7500 cycles, a work item of the set-up costs
+// about 450 (half as much again when the slab is read twice), an MFMA 46 of which 32 are its own, and the epilogue
+// about 2800 per fragment of a wavefront.  Two blocks of four wavefronts share a CU where the LDS holds both slabs:
+// each then takes 1.13 times as long, or what their MFMAs and vector instructions add up to.
+double slab_form_cost(const ConvGeom &g, const SlabPlan &p) {
+  const SlabForm &f = kSlabForms[p.form];
+  const int waves = f.wn * f.wm * f.wk;
+  const double items = (double)ceil_div(p.cap, 64) * 2 * p.ct;
+  const double load = items * (items > kSlabHold * waves ? 700.0 : 450.0);
+  const double mma = 46.0 * p.k_tiles * 8 * f.wn * f.wm / 4;
+  const double out = 1500.0 + 2800.0 * (f.wk == 2 ? 1 : 2) * (waves == 8 && f.wk == 1 ? 1.3 : 1.0);
+  const double one = 7500.0 + load + mma + out;
+  const double pair = one * 1.13 > 2 * mma * 0.92 + load + out ? one * 1.13 : 2 * mma * 0.92 + load + out;
+  const int64_t blocks = g.outer * p.tiles_per_sample * p.col_groups;
+  if (waves == 8 || p.total > 79 * 1024)
+    return (double)ceil_div(blocks, 256) * one;
+  const int64_t rest = blocks % 512;
+  return (double)(blocks / 512) * pair + (rest > 256 ? pair : rest > 0 ? one : 0.0);
+}
+
+bool compute_slab_plan(const ConvGeom &g, SlabPlan &narrow, SlabPlan &p) {
+  if (g.k_size > kSlabMaxTaps || g.Cg < 24 || g.in_sp_size >= ((int64_t)1 << 30) ||
+      g.out_sp_size >= ((int64_t)1 << 30) || g.Og >= ((int64_t)1 << 24) ||
+      (g.Og + kWideGroup) * g.out_sp_size >= ((int64_t)1 << 31))
+    return false;
+  const int64_t cgp = ceil_div(g.Cg, 32) * 32;
+  // padded channels cost as much as real ones; the epilogue's 32-bit steps hold kChunkK terms
+  if (cgp * 3 > g.Cg * 4 || g.k_size * cgp > kChunkK)
+    return false;
+  if (!compute_slab_form(g, 0, narrow))
+    return false;
+  p = narrow;
+  double best = slab_form_cost(g, p);
+  for (int form = 1; form < kSlabFormCount; ++form) {
+    SlabPlan q;
+    if (!compute_slab_form(g, form, q))
+      continue;
+    const double cost = slab_form_cost(g, q);
+    if (cost < best)
+      p = q, best = cost;
+  }
+  return true;
+}
+
+template <int kForm> int run_slab_form(const ConvSlabArgs &a, unsigned blocks, hipStream_t stream) {
+  constexpr SlabForm f = kSlabForms[kForm];
+  static std::atomic<uint64_t> configured{0};
+  const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(binary_conv_slab_kernel<f.wn, f.wm, f.wk>),
+                                   kSlabLdsLimit, configured, "hipFuncSetAttribute(binary_conv_slab LDS size)");
+  if (rc)
+    return rc;
+  hipLaunchKernelGGL((binary_conv_slab_kernel<f.wn, f.wm, f.wk>), dim3(blocks), dim3(64 * f.wn * f.wm * f.wk),
+                     (size_t)a.p.total, stream, a);
+  NBLA_HIP_LAUNCH_CHECK("binary_conv_slab");
+  return NBLA_HIP_OK;
 }
 
 } // namespace
@@ -832,7 +953,7 @@ bool conv_slab_applies(const ConvGeom &g) {
 
 bool conv_slab_plan_summary(const ConvGeom &g, int32_t out[4]) {
   SlabPlan p;
-  if (!make_slab_plan(g, p))
+  if (!make_slab_plan(g, p, true))
     return false;
   out[0] = p.tile_rows, out[1] = p.tiles_per_sample, out[2] = p.cap, out[3] = p.total;
   return true;
@@ -850,9 +971,9 @@ int launch_conv_slab_prepare(const float *Wg, float *Wbg, void *prepared, const 
     return fail(NBLA_HIP_ERR_NOT_IMPLEMENTED, "the slab convolution does not cover this geometry.");
   if (!aligned16(prepared))
     return fail(NBLA_HIP_ERR_MEMORY, "prepared-weight buffer must be 16-byte aligned.");
-  const size_t lds = (size_t)8 * 32 * g.k_size * 5; // |w| as floats and the sign flags as bytes
+  const size_t lds = (size_t)(8 * 32 + 8) * g.k_size * 4; // |w| and the packed words
   static std::atomic<uint64_t> configured{0};
-  const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(conv_taps_prepare), 8 * 32 * kSlabMaxTaps * 5,
+  const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(conv_taps_prepare), (8 * 32 + 8) * kSlabMaxTaps * 4,
                                    configured, "hipFuncSetAttribute(conv_taps_prepare LDS size)");
   if (rc)
     return rc;
@@ -895,13 +1016,7 @@ int launch_conv_slab_prepare_transposed(const float *Wg, void *prepared, const C
     return fail(NBLA_HIP_ERR_NOT_IMPLEMENTED, "the slab convolution does not cover this input gradient.");
   if (!aligned16(prepared))
     return fail(NBLA_HIP_ERR_MEMORY, "prepared-weight buffer must be 16-byte aligned.");
-  const size_t lds = (size_t)8 * 32 * g.k_size;
-  static std::atomic<uint64_t> configured{0};
-  const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(conv_taps_prepare_transposed),
-                                   8 * 32 * kSlabMaxTaps, configured,
-                                   "hipFuncSetAttribute(conv_taps_prepare_transposed LDS size)");
-  if (rc)
-    return rc;
+  const size_t lds = (size_t)8 * g.k_size * sizeof(uint32_t);
   hipLaunchKernelGGL(conv_taps_prepare_transposed, dim3((unsigned)p.wide_groups * 32, (unsigned)p.ct),
                      dim3(kPrepThreads), lds, stream, Wg, static_cast<uint4_t *>(prepared), (int)g.Og, (int)g.Cg,
                      (int)g.k_size, p.ct, p.wide_groups, zero_to);
@@ -920,11 +1035,6 @@ int launch_conv_slab(const float *x, const ConvGeom &g, int64_t grp, const void 
   int rc = ensure_init();
   if (rc)
     return rc;
-  static std::atomic<uint64_t> configured{0};
-  rc = allow_dynamic_lds(reinterpret_cast<const void *>(binary_conv_slab_kernel), kSlabLdsLimit, configured,
-                         "hipFuncSetAttribute(binary_conv_slab LDS size)");
-  if (rc)
-    return rc;
   const char *base = static_cast<const char *>(prepared);
   a.x = x;
   a.bits = reinterpret_cast<const uint4_t *>(base);
@@ -940,10 +1050,21 @@ int launch_conv_slab(const float *x, const ConvGeom &g, int64_t grp, const void 
   a.g = g;
   a.grp = (int)grp;
   a.inv_k = (float)1 / g.Kg;
-  const unsigned blocks = (unsigned)(g.outer * a.p.tiles_per_sample * a.p.wide_groups);
-  hipLaunchKernelGGL(binary_conv_slab_kernel, dim3(blocks), dim3(kSlabThreads), (size_t)a.p.total, stream, a);
-  NBLA_HIP_LAUNCH_CHECK("binary_conv_slab");
-  return NBLA_HIP_OK;
+  const unsigned blocks = (unsigned)(g.outer * a.p.tiles_per_sample * a.p.col_groups);
+  switch (a.p.form) {
+  case 0:
+    return run_slab_form<0>(a, blocks, stream);
+  case 1:
+    return run_slab_form<1>(a, blocks, stream);
+  case 2:
+    return run_slab_form<2>(a, blocks, stream);
+  case 3:
+    return run_slab_form<3>(a, blocks, stream);
+  case 4:
+    return run_slab_form<4>(a, blocks, stream);
+  default:
+    return run_slab_form<5>(a, blocks, stream);
+  }
 }
 
 } // namespace nbla_hip

@@ -73,7 +73,7 @@ int launch_conv_direct_backward(const float *dy, const float *x, const float *w,
 // positive to *zero_count when that is not null.  alpha_out and bias belong to the group; y is the whole output.
 bool conv_slab_applies(const ConvGeom &g);
 size_t conv_slab_prepared_bytes(const ConvGeom &g);
-// The plan's figures for a geometry it covers: windows per block, blocks per sample, the input positions its LDS
+// The figures of the form with 32 windows per block for a geometry it covers: windows per block, blocks per sample, the input positions its LDS
 // holds per block, LDS bytes.  Host only.
 bool conv_slab_plan_summary(const ConvGeom &g, int32_t out[4]);
 int launch_conv_slab_prepare(const float *Wg, float *Wbg, void *prepared, const ConvGeom &g, float zero_to,

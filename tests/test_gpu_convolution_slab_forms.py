@@ -1,0 +1,64 @@
+"""The forms of the binary convolution that keeps input positions in LDS (csrc/kernels/conv_slab.hip): sizes at the
+edges of their tiles -- output channels one short of, at and past 64, 128 and 256, maps whose rows do and do not fit a
+tile of 32 or 128 windows, a last tile of few windows, channel tiles with padding, one tap -- against float64.
+
+Bound: x is rounded to a multiple of 2^-30 of the largest magnitude under a block's windows, so an output of K terms is
+off by at most K * 2^-30 * max|x|, and by the roundings of its conversion to fp32 (two, 2^-24 of the result each).
+"""
+import numpy as np
+import pytest
+import torch
+
+from nnabla_amd import kernels
+
+pytestmark = pytest.mark.gpu
+
+# (x shape, output channels, kernel, pad, stride, group)
+CASES = [
+    ((2, 64, 56, 56), 64, (3, 3), (1, 1), (1, 1), 1),
+    ((1, 64, 55, 57), 63, (3, 3), (1, 1), (1, 1), 1),
+    ((3, 32, 13, 150), 32, (3, 3), (1, 1), (1, 1), 1),    # rows of the map longer than a tile
+    ((40, 32, 28, 28), 1, (1, 1), (0, 0), (1, 1), 1),
+    ((9, 128, 28, 28), 128, (3, 3), (1, 1), (1, 1), 1),
+    ((4, 96, 27, 27), 65, (5, 5), (2, 2), (1, 1), 1),
+    ((2, 48, 31, 17), 127, (3, 3), (1, 1), (2, 2), 1),
+    ((1, 96, 9, 9), 129, (3, 3), (0, 2), (1, 1), 1),
+    ((2, 256, 14, 14), 257, (1, 1), (0, 0), (1, 1), 1),
+    ((40, 64, 14, 14), 512, (1, 1), (0, 0), (1, 1), 1),
+    ((64, 96, 28, 28), 128, (3, 3), (1, 1), (1, 1), 2),
+    ((1, 30, 5, 5), 40, (3, 3), (1, 1), (1, 1), 1),       # two channels of padding
+]
+
+
+@pytest.mark.parametrize("xs,O,k,pad,stride,group", CASES)
+def test_forward_and_input_gradient_against_float64(xs, O, k, pad, stride, group):
+    rng = np.random.RandomState(20)
+    dev = torch.device("cuda:0")
+    kernels.init(0)
+    x = torch.from_numpy(rng.randn(*xs).astype(np.float32))
+    W = torch.from_numpy(rng.randn(O, xs[1] // group, *k).astype(np.float32))
+    s64 = torch.where(W < 0, -1.0, 1.0).double()
+    x64 = x.double().requires_grad_()
+    y64 = torch.nn.functional.conv2d(x64, s64, None, stride, pad, 1, group)
+    y, Wb = kernels.binary_connect_convolution(x.to(dev), W.to(dev), None, pad, stride, (1, 1), group)
+    assert torch.equal(Wb.cpu().double(), s64)
+    K = s64[0].numel()
+    bound = K * 2.0 ** -30 * float(x.abs().max()) + 2.0 ** -23 * y64.abs()
+    assert bool(((y.cpu().double() - y64).abs() <= bound).all())
+    # unit strides: the input gradient is the same product on dy, here added to a gradient that is there already
+    dy = torch.from_numpy(rng.randn(*y64.shape).astype(np.float32))
+    y64.backward(dy.double())
+    dx0 = torch.from_numpy(rng.randn(*xs).astype(np.float32))
+    dx, _, _ = kernels.binary_convolution_backward(dy.to(dev), x.to(dev), W.to(dev), Wb, None, pad, stride, (1, 1), group,
+                                                   dx=dx0.to(dev), want=(True, False, False))
+    K, taps, most = (O // group) * k[0] * k[1], k[0] * k[1], float(dy.abs().max())
+    want = x64.grad + dx0.double()
+    flip = [k[i] - 1 - pad[i] for i in (0, 1)]
+    slab = stride == (1, 1) and kernels.binary_convolution_slab_plan(
+        xs[0], O, y64.shape[2:], xs[1], k, flip, (1, 1), (1, 1), group) is not None
+    bound = 2.0 ** -22 * (want.abs() + x64.grad.abs())
+    if slab:
+        bound = bound + K * 2.0 ** -30 * most
+    else:  # unfolded: three digits, 2^-23 of a row's largest; every tap's product and every addition rounded to fp32
+        bound = bound + K * most * (2.0 ** -23 + 2 * taps * 2.0 ** -24)
+    assert bool(((dx.cpu().double() - want).abs() <= bound).all())
