@@ -5,7 +5,8 @@
 // samples at once, with m = (sample, output position) as the long dimension:
 //   dyt [M, Og]          the output gradient of the group, transposed so that m is the row index
 //   colg[n][kk][l]       = sum over o of dyt[m, o] * w[o, kk]   (then folded into dx by a gather)
-//   dW  [Og, Kg]         = dyt^T . col(x)                        (col(x) [M, Kg] is the unfolded input; digit x digit)
+//   dW  [Og, Kg]         = dyt^T . col(x)                        (col(x) [M, Kg] is the unfolded input; digit x digit,
+//                          or without the unfolded matrix in conv_dw.hip)
 //   db  [O]              = sums of dy over samples and positions, straight from dy
 #include "common.hpp"
 #include "conv_geom.hpp"
@@ -145,7 +146,7 @@ __global__ __launch_bounds__(256) void col2im_gather_unit(const float *__restric
 
 struct ConvBackwardPlan {
   size_t dyt_off, col_off, a_planes_off, b_planes_off, digits_off, bits_off, prep_off, count_off,
-      flag_off, sums_off, slab_off, total;
+      flag_off, sums_off, slab_off, dw_off, total;
 };
 
 size_t larger(size_t a, size_t b) { return a > b ? a : b; }
@@ -181,6 +182,8 @@ ConvBackwardPlan plan_conv_backward(const ConvGeom &g) {
     if (conv_slab_transposed_geom(g, t))
       off += round_up(conv_slab_prepared_bytes(t), 256);
   }
+  p.dw_off = off; // maxima, scales and partial results of the weight gradient on the fp16 matrix cores
+  off += round_up(conv_dw_workspace_bytes(g), 256);
   p.total = off;
   return p;
 }
@@ -254,9 +257,10 @@ int conv_backward(const float *dy, const float *x, const float *W, const float *
       return rc;
     dx = nullptr, dx_slab = false;
   }
-  // few weights under many windows: the weight gradient in fp32 straight from dy and x, all groups at once (its
+  // few weights under many windows of a geometry that the matrix-core product below does not cover (it is two to four
+  // times as fast where both apply): the weight gradient in fp32 straight from dy and x, all groups at once (its
   // partial results lie in the unfolded gradient's buffer, so it runs before the loop that fills that buffer)
-  if (dW && conv_direct_dw_applies(g)) {
+  if (dW && !conv_dw_applies(g) && conv_direct_dw_applies(g)) {
     rc = launch_conv_direct_dw(dy, x, dW, g, accum_w, col, (size_t)g.M * g.Kg * sizeof(float), stream);
     if (rc)
       return rc;
@@ -270,7 +274,15 @@ int conv_backward(const float *dy, const float *x, const float *W, const float *
       return rc;
     db = nullptr;
   }
-  for (int64_t grp = 0; grp < g.group; ++grp) {
+  if (dW && conv_dw_applies(g)) { // kernels of width 1, 3, 5 with half their width of padding: no unfolded matrix
+    for (int64_t grp = 0; grp < g.group; ++grp) {
+      rc = launch_conv_dw(dy, x, dW, g, grp, accum_w, base + p.dw_off, conv_dw_workspace_bytes(g), stream);
+      if (rc)
+        return rc;
+    }
+    dW = nullptr;
+  }
+  for (int64_t grp = 0; grp < g.group && (dx || dW); ++grp) {
     const float *Wg = W + grp * g.Og * g.Kg;
     const float *ag = alpha ? alpha + grp * g.Og : nullptr;
     if ((dx && !dx_slab) || dW) {

@@ -1,0 +1,618 @@
+// Weight gradient of a two-dimensional convolution on the fp16 matrix cores, without an unfolded matrix:
+//     dW[o, c, ky, kx] = sum over (n, oy, ox) of dy[n, o, oy, ox] * x[n, c, oy s - p + ky, ox s - p + kx]
+// (convolution.cpp:199-283 unfolds x per sample and multiplies; the contraction here is the same sum over positions).
+//
+// Arithmetic.  Every fp32 value, scaled by a power of two that puts its channel's largest finite magnitude into
+// [2^14, 2^15), is the sum of two fp16 numbers, hi = fp16(v) and lo = fp16(v - hi), exactly or to one unit of its last
+// fp32 place (v - hi has at most 12 bits and a sign) for every value within 2^-18 of the channel's largest; below that to
+// 2^-39 of the largest.  Three products (hi hi, hi lo, lo hi) accumulate in fp32 inside the matrix instruction; the
+// fourth is below 2^-22 of the product.  A block's sums (a few hundred positions) go to memory as fp32 and are added in a
+// fixed order in double.  Against float64 the gradient of [32,64,56,56] x [64,64,3,3] is off by 2.5e-7 of its norm
+// (1.4e-6 with the products of 24-bit digits of the unfolded matrix, 9.4e-7 for fp32 sums in order).  A NaN or an
+// infinity makes NaN of every gradient it reaches (v - hi is then NaN).
+//
+// Layout.  A tile is R output rows of one sample (or NS whole samples of a small map), its positions in groups of eight
+// along the rows: dy as [group][hi / lo][64 output channels][8 fp16], x as [input row][column phase][group][hi / lo]
+// [channel][8 fp16].  A lane's eight k-slots of v_mfma_f32_32x32x16_f16 are one group of one channel, sixteen bytes.
+// Under the tap (ky, kx) the positions of a dy group meet the x group of row oy s + ky shifted by floor((kx - p) / s)
+// positions inside the column phase (kx - p) mod s: the wavefront reads the x group and a word of either neighbour once
+// per (step, ky) and forms the operands of the kx by shifting registers, under the MFMAs.  A group of zeros in front of
+// every row is also the end of the row before.  16 bytes of padding behind each group keep writes (lanes along the
+// groups) and reads (lanes along the channels) apart in the banks.  Widths 1, 3 and 5 with padding k / 2, strides 1 and 2:
+// the shifts are constants of the kernel, and the output row has as many groups as a phase of the input row.
+//
+// Four wavefronts: two fragments of 32 output channels x two halves of the steps; each holds NKY x KW x NC fragments
+// of 32 input channels (nine for 3 x 3: 144 accumulator registers).  Two blocks share a CU (LDS below 80 KB), one
+// converting the rows it loaded into registers a tile ahead while the other multiplies.
+//
+// What bounds it: at 64 channels a tile of 112 positions takes two blocks 12200 cycles, of which their MFMAs are 6000
+// and the conversions of either 4000; the maxima of the channels (8.4 us for 51 MB) and the sum over the splits
+// (6.4 us) come on top.  The whole weight gradient, in place of unfolding x into a digit matrix chunk by chunk:
+// [32,64,56,56] x [64,64,3,3] 400 -> 54 us, [32,256,14,14] x [256,256,3,3] 95 -> 56, [16,128,28,28] x [256,128,3,3]
+// stride 2 62 -> 34; and against fp32 sums on the vector units (few weights, many positions): [32,32,56,56] x
+// [32,32,3,3] 154 -> 38, [64,64,28,28] x [64,64,1,1] 117 -> 28, [64,8,28,28] x [32,8,3,3] 50 -> 26.
+#include "common.hpp"
+#include "conv_geom.hpp"
+#include "gemm_layout.hpp"
+#include "internal.hpp"
+
+namespace nbla_hip {
+namespace {
+
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef uint32_t uint4_t __attribute__((ext_vector_type(4)));
+
+constexpr int kDwThreads = 256;
+constexpr int kDwO = 64;                    // output channels per block
+constexpr int kDwLds = 78 * 1024;           // two blocks to a CU
+constexpr int kDwTopBit = 14;               // a channel's largest magnitude lands in [2^14, 2^15)
+constexpr int kDwMaxSlices = 16;            // partial maxima per channel
+constexpr int kDwQStride = 2 * kDwO * 16 + 16;
+constexpr uint32_t kDwOutside = 0x80000000u; // a byte offset past the end of any tensor: such loads give zeros
+
+// The kernel's parameters for a kernel width and stride: rows of taps per wavefront, fragments of input channels per
+// wavefront, the items of eight positions a thread holds of x and of dy.
+template <int KW, int S> struct DwShape {
+  static constexpr int nky = KW == 3 ? 3 : 1, nc = KW == 1 ? 4 : 1;
+  static constexpr int phases = KW == 1 ? 1 : S;
+  static constexpr int mx = KW == 1 ? (S == 1 ? 6 : 4) : (S == 1 ? 4 : 3);
+  static constexpr int my = KW == 1 ? 3 : (S == 1 ? 4 : 2);
+  static constexpr int row_step = nky == 1 ? 1 : S;      // x rows kept per output row
+  static constexpr int lead = KW > 1 ? 1 : 0;            // the group of zeros in front of a row
+  static constexpr int rg_stride = 2 * 32 * nc * 16 + 16;
+  static constexpr int phase(int kx) { return ((kx - KW / 2) % S + S) % S; }
+  static constexpr int shift(int kx) { return (kx - KW / 2 - phase(kx)) / S; }
+  // whether a tap of this phase shifts to the left (dir < 0) or to the right
+  static constexpr bool shifts(int ph, int dir) {
+    for (int kx = 0; kx < KW; ++kx)
+      if (phase(kx) == ph && shift(kx) * dir > 0)
+        return true;
+    return false;
+  }
+};
+
+// Division of a small non-negative number by a constant of the launch (v < 2^20, d < 2^12: v + 1/2 is at least 1 / (2 d)
+// away from a multiple of d, more than the roundings).
+struct DwDivide {
+  float inv; // (from the host: kept in a scalar register)
+  int d;
+  void set(int d_) { d = d_, inv = 1.0f / (float)d_; }
+  __device__ __forceinline__ int operator()(int v, int &rest) const {
+    const int q = (int)(((float)v + 0.5f) * inv);
+    rest = v - q * d;
+    return q;
+  }
+};
+
+struct DwPlan {
+  int KH, KW, S, nky, nc;
+  int G, Gx, R, NS, rows_x, Q, steps, row_tiles; // (G groups per output row; Gx = G and the zeros in front)
+  int ot, ct, kg, splits, tiles, per_split;
+  int dy_off, tab_off, misc_off, lds;
+  int slices;
+  DwDivide by_xc, by_rows_x, by_q, by_g, by_r;
+  size_t max_off, shift_off, partial_off, total;
+};
+
+struct DwArgs {
+  const float *dy, *x;       // first channel of the group
+  const uint32_t *maxima;    // [slice][Cg + Og]
+  int32_t *shifts;           // [Cg + Og], written by the first blocks for the last pass
+  float *partial;            // [split][tap][Og][Cg]
+  int N, C, O, Cg, Og, IH, IW, OH, OW, pad_h;
+  uint32_t x_bytes, dy_bytes, partial_bytes; // from the pointers above to the end of the tensors
+  DwPlan p;
+};
+
+// Largest finite magnitude of every channel of x and dy over slices of the samples: block (slice, channel).
+__global__ __launch_bounds__(256) void conv_dw_maxima(const float *__restrict__ x, const float *__restrict__ dy,
+                                                      uint32_t *__restrict__ maxima, int N, int C, int O, int Cg, int Og,
+                                                      int xplane, int yplane) {
+  __shared__ uint32_t s_max[4];
+  const int ch = blockIdx.y, slice = blockIdx.x, tid = threadIdx.x;
+  const bool is_x = ch < Cg;
+  const int plane = is_x ? xplane : yplane;
+  const float *src = is_x ? x + (int64_t)ch * xplane : dy + (int64_t)(ch - Cg) * yplane;
+  const int64_t sample = is_x ? (int64_t)C * xplane : (int64_t)O * yplane;
+  const int per = (N + (int)gridDim.x - 1) / (int)gridDim.x, n0 = slice * per, n1 = min(N, n0 + per);
+  uint32_t amax = 0u;
+  auto take = [&](float v) __attribute__((always_inline)) {
+    const uint32_t m = __float_as_uint(v) & 0x7fffffffu;
+    amax = max(amax, m < 0x7f800000u ? m : 0u);
+  };
+  if (plane >= 256) {
+    for (int n = n0; n < n1; ++n) {
+      const float *p = src + n * sample;
+      for (int i = tid; i < plane; i += 1024) {
+        float v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          v[j] = p[min(i + 256 * j, plane - 1)];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          take(v[j]);
+      }
+    }
+  } else { // several samples' planes side by side
+    const int total = (n1 - n0) * plane;
+    for (int i = tid; i < total; i += 1024) {
+      float v[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int at = min(i + 256 * j, total - 1), n = at / plane;
+        v[j] = src[(n0 + n) * sample + (at - n * plane)];
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        take(v[j]);
+    }
+  }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1)
+    amax = max(amax, (uint32_t)__shfl_xor((int)amax, off));
+  if ((tid & 63) == 0)
+    s_max[tid >> 6] = amax;
+  __syncthreads();
+  if (tid == 0)
+    maxima[slice * (Cg + Og) + ch] = max(max(s_max[0], s_max[1]), max(s_max[2], s_max[3]));
+}
+
+#if defined(__HIP_DEVICE_COMPILE__)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t dw_rsrc(const float *p, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p), 0, (int)bytes, 0x00020000);
+}
+__device__ __forceinline__ f32x4_t dw_load4(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+  return __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0));
+}
+#endif
+
+template <int KW, int S>
+__global__ __launch_bounds__(kDwThreads, 2) void conv_dw_kernel(DwArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  using T = DwShape<KW, S>;
+  constexpr int kNky = T::nky, kNc = T::nc, kPhases = T::phases, kMx = T::mx, kMy = T::my, kRowStep = T::row_step;
+  constexpr int kRg = T::rg_stride, kUnits = kNky * KW * kNc, kC = 32 * kNc;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const DwPlan &P = a.p;
+  const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, half = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wo = wave & 1, wk = wave >> 1;
+  // neighbouring blocks share a run of tiles: the channels' tiles fastest
+  int work = (int)xcd_remap(blockIdx.x, gridDim.x);
+  const int cells = P.ot * P.ct * P.kg, split = work / cells;
+  work -= split * cells;
+  const int kg = work / (P.ot * P.ct);
+  work -= kg * (P.ot * P.ct);
+  const int ot = work / P.ct, ct = work - ot * P.ct;
+  const int o0 = ot * kDwO, c0 = ct * kC, ky0 = kg * kNky;
+  unsigned char *s_dy = smem + P.dy_off;
+  uint32_t *s_tab = reinterpret_cast<uint32_t *>(smem + P.tab_off); // x group of every dy group, bytes
+  int *s_shift = reinterpret_cast<int *>(smem + P.misc_off);        // [kC] of x, [kDwO] of dy
+
+  // ---- set-up: the channels' scales, the table of groups, zeros where no load ever writes
+  for (int i = tid; i < kC + kDwO; i += kDwThreads) {
+    const bool is_x = i < kC;
+    const int ch = is_x ? c0 + i : o0 + (i - kC);
+    int shift = 0;
+    if (ch < (is_x ? a.Cg : a.Og)) {
+      const int at = is_x ? ch : a.Cg + ch;
+      uint32_t m = 0u, part[kDwMaxSlices];
+#pragma unroll
+      for (int s = 0; s < kDwMaxSlices; ++s)
+        part[s] = a.maxima[min(s, P.slices - 1) * (a.Cg + a.Og) + at];
+#pragma unroll
+      for (int s = 0; s < kDwMaxSlices; ++s)
+        m = max(m, part[s]);
+      shift = m ? kDwTopBit - binade_exponent(binade_of(m)) : 0;
+      if (split == 0 && kg == 0 && (is_x ? ot : ct) == 0)
+        a.shifts[at] = shift;
+    }
+    s_shift[i] = shift;
+  }
+  for (int q = tid; q <= P.Q; q += kDwThreads) {
+    const int row = q / P.G, g = q - row * P.G, ns = row / P.R, rr = row - ns * P.R;
+    s_tab[q] = q < P.Q ? (uint32_t)(((ns * P.rows_x + rr * kRowStep) * (kPhases * P.Gx) + T::lead + g) * kRg)
+                       : (uint32_t)(T::lead * kRg);
+  }
+  for (int i = tid * 16; i < kDwQStride; i += kDwThreads * 16) // the group that fills up the last step
+    *reinterpret_cast<uint4_t *>(s_dy + P.Q * kDwQStride + i) = uint4_t{0u, 0u, 0u, 0u};
+  if (T::lead) {
+    const int rows = P.NS * P.rows_x * kPhases, words = kRg / 16;
+    for (int i = tid; i < (rows + 1) * words; i += kDwThreads) {
+      const int row = i / words;
+      *reinterpret_cast<uint4_t *>(smem + row * P.Gx * kRg + (i - row * words) * 16) = uint4_t{0u, 0u, 0u, 0u};
+    }
+  }
+  __syncthreads();
+
+  const __amdgpu_buffer_rsrc_t xr = dw_rsrc(a.x, a.x_bytes), yr = dw_rsrc(a.dy, a.dy_bytes);
+  const int x_rows = P.NS * P.rows_x, x_items = kC * x_rows * P.G, y_items = kDwO * P.Q;
+  f32x4_t xv[kMx][2 * S], yv[kMy][2];
+  // item -> (channel, row inside the tile, group): groups and rows fastest, as they lie in memory.  Computed anew for
+  // every tile: kept over the tiles the offsets would spill, and a reload waits for the loads issued before it.
+  auto x_item = [&](int m, int &c, int &nsr, int &g) __attribute__((always_inline)) {
+    int rest, item = tid + kDwThreads * m;
+    asm volatile("" : "+v"(item));
+    c = P.by_xc(item, rest);
+    nsr = P.by_g(rest, g);
+    return item < x_items;
+  };
+  auto y_item = [&](int m, int &o, int &row, int &g) __attribute__((always_inline)) {
+    int rest, item = tid + kDwThreads * m;
+    asm volatile("" : "+v"(item));
+    o = P.by_q(item, rest);
+    row = P.by_g(rest, g);
+    return item < y_items;
+  };
+  auto load_tile = [&](int tile) __attribute__((always_inline)) {
+    const int n_part = P.NS > 1 ? tile : tile / P.row_tiles;
+    const int n0 = n_part * P.NS, oy0 = P.NS > 1 ? 0 : (tile - n_part * P.row_tiles) * P.R;
+#pragma unroll
+    for (int m = 0; m < kMx; ++m) {
+      int c, nsr, g, rr;
+      const bool have = x_item(m, c, nsr, g);
+      const int ns = P.by_rows_x(nsr, rr);
+      const int iy = kRowStep == 1 && S > 1 ? (oy0 + rr) * S + ky0 - a.pad_h : oy0 * S + rr + ky0 - a.pad_h;
+      const bool ok = have && c0 + c < a.Cg && n0 + ns < a.N && (unsigned)iy < (unsigned)a.IH;
+      const uint32_t off = (uint32_t)(((((n0 + ns) * a.C + c0 + c) * a.IH + iy) * a.IW + 8 * S * g) * 4);
+#pragma unroll
+      for (int j = 0; j < 2 * S; ++j)
+        xv[m][j] = dw_load4(xr, ok ? off + 16 * j : kDwOutside);
+      __builtin_amdgcn_sched_barrier(0); // one item's address arithmetic at a time
+    }
+#pragma unroll
+    for (int m = 0; m < kMy; ++m) {
+      int o, row, g, rr;
+      const bool have = y_item(m, o, row, g);
+      const int ns = P.by_r(row, rr);
+      const bool ok = have && o0 + o < a.Og && n0 + ns < a.N && oy0 + rr < a.OH;
+      const uint32_t off = (uint32_t)(((((n0 + ns) * a.O + o0 + o) * a.OH + oy0 + rr) * a.OW + 8 * g) * 4);
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        yv[m][j] = dw_load4(yr, ok ? off + 16 * j : kDwOutside);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  // eight values -> their hi and lo halves; values outside the row (columns before first or from end on) are zeros
+  auto split8 = [&](const float (&v)[8], int shift, uint4_t &hi, uint4_t &lo) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      f32x2_t t;
+      t.x = ldexpf(v[2 * j], shift), t.y = ldexpf(v[2 * j + 1], shift);
+      const half2_t h = __builtin_convertvector(t, half2_t);
+      const f32x2_t back = __builtin_convertvector(h, f32x2_t);
+      f32x2_t rest;
+      rest.x = t.x - back.x, rest.y = t.y - back.y;
+      const half2_t l = __builtin_convertvector(rest, half2_t);
+      hi[j] = __builtin_bit_cast(uint32_t, h);
+      lo[j] = __builtin_bit_cast(uint32_t, l);
+    }
+  };
+  auto store_tile = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int m = 0; m < kMx; ++m) {
+      __builtin_amdgcn_sched_barrier(0);
+      int c, nsr, g;
+      if (x_item(m, c, nsr, g)) {
+        const int shift = s_shift[c];
+#pragma unroll
+        for (int ph = 0; ph < kPhases; ++ph) {
+          float v[8];
+#pragma unroll
+          for (int j = 0; j < 8; ++j)
+            v[j] = 8 * S * g + S * j + ph < a.IW ? xv[m][(S * j + ph) >> 2][(S * j + ph) & 3] : 0.0f;
+          uint4_t hi, lo;
+          split8(v, shift, hi, lo);
+          unsigned char *dst = smem + ((nsr * kPhases + ph) * P.Gx + T::lead + g) * kRg + c * 16;
+          *reinterpret_cast<uint4_t *>(dst) = hi;
+          *reinterpret_cast<uint4_t *>(dst + kC * 16) = lo;
+        }
+      }
+    }
+#pragma unroll
+    for (int m = 0; m < kMy; ++m) {
+      __builtin_amdgcn_sched_barrier(0);
+      int o, row, g;
+      if (y_item(m, o, row, g)) {
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          v[j] = 8 * g + j < a.OW ? yv[m][j >> 2][j & 3] : 0.0f;
+        uint4_t hi, lo;
+        split8(v, s_shift[kC + o], hi, lo);
+        unsigned char *dst = s_dy + (row * P.G + g) * kDwQStride + o * 16;
+        *reinterpret_cast<uint4_t *>(dst) = hi;
+        *reinterpret_cast<uint4_t *>(dst + kDwO * 16) = lo;
+      }
+    }
+  };
+
+  f32x16_t acc[kUnits];
+#pragma unroll
+  for (int u = 0; u < kUnits; ++u)
+#pragma unroll
+    for (int q = 0; q < 16; ++q)
+      acc[u][q] = 0.0f;
+  const int ky_stride = kPhases * P.Gx * kRg, ph_stride = P.Gx * kRg;
+  auto multiply_step = [&](int t) __attribute__((always_inline)) {
+    const int q = 2 * t + half;
+    const unsigned char *ap = s_dy + (q < P.Q ? q : P.Q) * kDwQStride + (wo * 32 + r) * 16;
+    const half8_t ah = *reinterpret_cast<const half8_t *>(ap), al = *reinterpret_cast<const half8_t *>(ap + kDwO * 16);
+    const unsigned char *bp = smem + s_tab[q < P.Q ? q : P.Q] + r * 16;
+#pragma unroll
+    for (int ky = 0; ky < kNky; ++ky) {
+      uint32_t w[kPhases][kNc][2][6]; // the last word of the group before, the group, the first word of the next
+#pragma unroll
+      for (int ph = 0; ph < kPhases; ++ph)
+#pragma unroll
+        for (int nc = 0; nc < kNc; ++nc)
+#pragma unroll
+          for (int hl = 0; hl < 2; ++hl) {
+            const unsigned char *src = bp + ky * ky_stride + ph * ph_stride + hl * (kC * 16) + nc * 512;
+            const uint4_t v = *reinterpret_cast<const uint4_t *>(src);
+            w[ph][nc][hl][1] = v.x, w[ph][nc][hl][2] = v.y, w[ph][nc][hl][3] = v.z, w[ph][nc][hl][4] = v.w;
+            w[ph][nc][hl][0] = T::shifts(ph, -1) ? *reinterpret_cast<const uint32_t *>(src - kRg + 12) : 0u;
+            w[ph][nc][hl][5] = T::shifts(ph, 1) ? *reinterpret_cast<const uint32_t *>(src + kRg) : 0u;
+          }
+#pragma unroll
+      for (int kx = 0; kx < KW; ++kx)
+#pragma unroll
+        for (int nc = 0; nc < kNc; ++nc) {
+          const int ph = T::phase(kx), sh = T::shift(kx);
+          uint4_t b[2];
+#pragma unroll
+          for (int hl = 0; hl < 2; ++hl)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) // positions sh + 2 j and sh + 2 j + 1 of the group
+              b[hl][j] = sh == -1  ? __builtin_amdgcn_alignbit(w[ph][nc][hl][j + 1], w[ph][nc][hl][j], 16)
+                         : sh == 1 ? __builtin_amdgcn_alignbit(w[ph][nc][hl][j + 2], w[ph][nc][hl][j + 1], 16)
+                                   : w[ph][nc][hl][j + 1 + sh / 2];
+          const half8_t bh = __builtin_bit_cast(half8_t, b[0]), bl = __builtin_bit_cast(half8_t, b[1]);
+          f32x16_t &d = acc[(ky * KW + kx) * kNc + nc];
+          d = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bh, d, 0, 0, 0);
+          d = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bl, d, 0, 0, 0);
+          d = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, bh, d, 0, 0, 0);
+        }
+    }
+  };
+
+  // ---- the tiles of this block: a tile's values wait in registers while the one before is multiplied
+  const int first = split * P.per_split, last = min(first + P.per_split, P.tiles);
+  load_tile(first);
+  for (int tile = first; tile < last; ++tile) {
+    store_tile();
+    __syncthreads();
+    if (tile + 1 < last)
+      load_tile(tile + 1);
+    for (int t = wk; t < P.steps; t += 2)
+      multiply_step(t);
+    __syncthreads();
+  }
+
+  // ---- the two halves of the steps added through LDS: a wavefront finishes the first units (wk = 0) or the rest, and
+  // hands its sums of the others to its partner.  Stores outside the channels fall past the buffer's end.
+  constexpr int kFirst = (kUnits + 1) / 2;
+  float *red = reinterpret_cast<float *>(smem) + wo * (kUnits * 16 * 64) + lane;
+#pragma unroll
+  for (int u = 0; u < kUnits; ++u)
+    if ((u < kFirst) == (wk == 1)) {
+#pragma unroll
+      for (int q = 0; q < 16; ++q)
+        red[(u * 16 + q) * 64] = acc[u][q];
+    }
+  __syncthreads();
+  const int taps = P.KH * KW;
+  const __amdgpu_buffer_rsrc_t pr = dw_rsrc(a.partial, a.partial_bytes);
+#pragma unroll
+  for (int u = 0; u < kUnits; ++u)
+    if ((u < kFirst) == (wk == 0)) {
+      const int nc = u % kNc, kx = u / kNc % KW, ky = ky0 + u / (kNc * KW);
+      const int c = c0 + nc * 32 + r, o = o0 + wo * 32 + 4 * half;
+      const uint32_t base = (uint32_t)((((split * taps + ky * KW + kx) * a.Og + o) * a.Cg + c) * 4);
+      const bool ok = ky < P.KH && c < a.Cg;
+#pragma unroll
+      for (int q = 0; q < 16; ++q) {
+        const int oq = 8 * (q >> 2) + (q & 3);
+        const float v = acc[u][q] + red[(u * 16 + q) * 64];
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), pr,
+                                              (int)(ok && o + oq < a.Og ? base + (uint32_t)(oq * a.Cg * 4) : kDwOutside),
+                                              0, 0);
+      }
+    }
+#endif
+}
+
+// dW[o, c, tap] (+)= 2^-(shifts) * the splits' sums added in double: 32 outputs along c x 8 runs of the splits per block.
+__global__ __launch_bounds__(256) void conv_dw_sum(const float *__restrict__ partial, const int32_t *__restrict__ shifts,
+                                                   float *__restrict__ dW, int Og, int Cg, int taps, int splits,
+                                                   int accumulate) {
+  __shared__ double s_sum[8][32];
+  const int lane = threadIdx.x & 31, run = threadIdx.x >> 5;
+  const int64_t outs = (int64_t)taps * Og * Cg, at = (int64_t)blockIdx.x * 32 + lane;
+  double sum = 0.0;
+  if (at < outs) {
+    int s = run;
+    for (; s + 24 < splits; s += 32) {
+      float v[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        v[j] = partial[(int64_t)(s + 8 * j) * outs + at];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        sum += (double)v[j];
+    }
+    for (; s < splits; s += 8)
+      sum += (double)partial[(int64_t)s * outs + at];
+  }
+  s_sum[run][lane] = sum;
+  __syncthreads();
+  if (run == 0 && at < outs) {
+#pragma unroll
+    for (int j = 1; j < 8; ++j)
+      sum += s_sum[j][lane];
+    const int64_t tap = at / ((int64_t)Og * Cg), oc = at - tap * ((int64_t)Og * Cg);
+    const int o = (int)(oc / Cg), c = (int)(oc - (int64_t)o * Cg);
+    const float v = (float)ldexp(sum, -(shifts[c] + shifts[Cg + o]));
+    float *dst = dW + oc * taps + tap;
+    *dst = accumulate ? *dst + v : v;
+  }
+}
+
+template <int KW, int S> void plan_shape(DwPlan &p, int &mx, int &my, int &row_step, int &phases, int &rg, int &lead) {
+  using T = DwShape<KW, S>;
+  p.nky = T::nky, p.nc = T::nc;
+  mx = T::mx, my = T::my, row_step = T::row_step, phases = T::phases, rg = T::rg_stride, lead = T::lead;
+}
+
+bool make_dw_plan(const ConvGeom &g, DwPlan &p) {
+  for (int i = 0; i < kMaxSpatial; ++i)
+    if (g.dil[i] != 1 && g.k[i] != 1)
+      return false;
+  if (g.k[0] != 1 || g.in_sp[0] != 1 || g.out_sp[0] != 1 || g.pad[0] != 0)
+    return false;
+  p.KH = g.k[1], p.KW = g.k[2], p.S = g.stride[2];
+  if (g.stride[1] != g.stride[2] || p.KH > 16 || g.pad[2] != p.KW / 2)
+    return false;
+  int mx, my, row_step, phases, rg, lead;
+  switch (p.KW * 4 + p.S) {
+  case 1 * 4 + 1: plan_shape<1, 1>(p, mx, my, row_step, phases, rg, lead); break;
+  case 1 * 4 + 2: plan_shape<1, 2>(p, mx, my, row_step, phases, rg, lead); break;
+  case 3 * 4 + 1: plan_shape<3, 1>(p, mx, my, row_step, phases, rg, lead); break;
+  case 3 * 4 + 2: plan_shape<3, 2>(p, mx, my, row_step, phases, rg, lead); break;
+  case 5 * 4 + 1: plan_shape<5, 1>(p, mx, my, row_step, phases, rg, lead); break;
+  case 5 * 4 + 2: plan_shape<5, 2>(p, mx, my, row_step, phases, rg, lead); break;
+  default: return false;
+  }
+  // a tile of 64 output channels x 32 (1 x 1: 128) input channels should not be mostly padding, and offsets are 32 bits
+  if (g.Og < 16 || g.Cg < (p.nc > 1 ? 32 : 8) || g.outer * g.C * g.in_sp_size * 4 >= ((int64_t)1 << 31) ||
+      g.outer * g.O * g.out_sp_size * 4 >= ((int64_t)1 << 31) || g.Og * g.Kg >= ((int64_t)1 << 28) || g.Cg + g.Og > 65535)
+    return false;
+  const int OH = g.out_sp[1], OW = g.out_sp[2], C = 32 * p.nc;
+  if (OW > 512)
+    return false;
+  p.G = (int)ceil_div(OW, 8);
+  p.Gx = p.G + lead;
+  auto sizes = [&](int R, int NS) {
+    p.R = R, p.NS = NS, p.rows_x = (R - 1) * row_step + p.nky, p.Q = R * NS * p.G;
+    p.dy_off = (NS * p.rows_x * phases * p.Gx + lead) * rg;
+    p.tab_off = p.dy_off + (p.Q + 1) * kDwQStride;
+    p.misc_off = (int)round_up((size_t)p.tab_off + 4 * (p.Q + 1), 16);
+    p.lds = p.misc_off + 4 * (C + kDwO);
+    const int reduce = 2 * p.nky * p.KW * p.nc * 16 * 64 * 4; // the sums two wavefronts exchange
+    if (p.lds < reduce)
+      p.lds = reduce;
+    return C * NS * p.rows_x * p.G <= mx * kDwThreads && kDwO * p.Q <= my * kDwThreads && p.lds <= kDwLds;
+  };
+  if (!sizes(1, 1))
+    return false;
+  int R = 1, NS = 1;
+  while (R < OH && sizes(R + 1, 1))
+    ++R;
+  if (R == OH)
+    while (NS < g.outer && sizes(OH, NS + 1))
+      ++NS;
+  p.row_tiles = (int)ceil_div(OH, R);
+  R = (int)ceil_div(OH, p.row_tiles); // as even as possible
+  sizes(R, NS);
+  p.steps = (p.Q + 1) / 2;
+  p.by_xc.set(NS * p.rows_x * p.G), p.by_rows_x.set(p.rows_x), p.by_q.set(p.Q), p.by_g.set(p.G), p.by_r.set(p.R);
+  p.ot = (int)ceil_div(g.Og, kDwO), p.ct = (int)ceil_div(g.Cg, C), p.kg = (int)ceil_div(p.KH, p.nky);
+  const int64_t tiles = NS > 1 ? ceil_div(g.outer, NS) : g.outer * p.row_tiles;
+  if (tiles >= ((int64_t)1 << 30))
+    return false;
+  p.tiles = (int)tiles;
+  // two blocks per CU: as many splits as fill 512 places once, each with the same number of tiles (the last fewer)
+  const int64_t cells = (int64_t)p.ot * p.ct * p.kg;
+  int64_t splits = 512 / cells;
+  if (splits < 1)
+    splits = 1;
+  if (splits > tiles)
+    splits = tiles;
+  p.per_split = (int)ceil_div(tiles, splits);
+  p.splits = (int)ceil_div(tiles, p.per_split);
+  if (cells * p.splits >= ((int64_t)1 << 30) || p.splits * g.Og * g.Kg * 4 >= ((int64_t)1 << 31))
+    return false;
+  const int64_t channels = g.Cg + g.Og;
+  int64_t slices = ceil_div(2048, channels);
+  if (slices > g.outer)
+    slices = g.outer;
+  if (slices > kDwMaxSlices)
+    slices = kDwMaxSlices;
+  p.slices = (int)ceil_div(g.outer, ceil_div(g.outer, slices));
+  p.max_off = 0;
+  p.shift_off = round_up((size_t)p.slices * channels * sizeof(uint32_t), 256);
+  p.partial_off = p.shift_off + round_up((size_t)channels * sizeof(int32_t), 256);
+  p.total = p.partial_off + round_up((size_t)p.splits * g.Og * g.Kg * sizeof(float), 256);
+  return true;
+}
+
+template <int KW, int S> int run_conv_dw(const DwArgs &a, hipStream_t stream) {
+  static std::atomic<uint64_t> configured{0};
+  const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(conv_dw_kernel<KW, S>), kDwLds, configured,
+                                   "hipFuncSetAttribute(conv_dw LDS size)");
+  if (rc)
+    return rc;
+  const unsigned blocks = (unsigned)(a.p.ot * a.p.ct * a.p.kg * a.p.splits);
+  hipLaunchKernelGGL((conv_dw_kernel<KW, S>), dim3(blocks), dim3(kDwThreads), (size_t)a.p.lds, stream, a);
+  NBLA_HIP_LAUNCH_CHECK("conv_dw");
+  return NBLA_HIP_OK;
+}
+
+} // namespace
+
+bool conv_dw_applies(const ConvGeom &g) {
+  DwPlan p;
+  return make_dw_plan(g, p);
+}
+
+size_t conv_dw_workspace_bytes(const ConvGeom &g) {
+  DwPlan p;
+  return make_dw_plan(g, p) ? p.total : 0;
+}
+
+int launch_conv_dw(const float *dy, const float *x, float *dW, const ConvGeom &g, int64_t grp, bool accumulate,
+                   void *workspace, size_t workspace_bytes, hipStream_t stream) {
+  DwArgs a;
+  if (!make_dw_plan(g, a.p))
+    return fail(NBLA_HIP_ERR_NOT_IMPLEMENTED, "the weight gradient product does not cover this geometry.");
+  if (workspace_bytes < a.p.total || !aligned256(workspace))
+    return fail(NBLA_HIP_ERR_MEMORY, "weight gradient workspace too small (%zu < %zu) or misaligned.", workspace_bytes,
+                a.p.total);
+  char *base = static_cast<char *>(workspace);
+  uint32_t *maxima = reinterpret_cast<uint32_t *>(base + a.p.max_off);
+  const int64_t x_first = grp * g.Cg * g.in_sp_size, dy_first = grp * g.Og * g.out_sp_size;
+  a.x = x + x_first, a.dy = dy + dy_first;
+  a.maxima = maxima;
+  a.shifts = reinterpret_cast<int32_t *>(base + a.p.shift_off);
+  a.partial = reinterpret_cast<float *>(base + a.p.partial_off);
+  a.N = (int)g.outer, a.C = (int)g.C, a.O = (int)g.O, a.Cg = (int)g.Cg, a.Og = (int)g.Og;
+  a.IH = g.in_sp[1], a.IW = g.in_sp[2], a.OH = g.out_sp[1], a.OW = g.out_sp[2];
+  a.pad_h = g.pad[1];
+  a.x_bytes = (uint32_t)((g.outer * g.C * g.in_sp_size - x_first) * 4);
+  a.partial_bytes = (uint32_t)(a.p.splits * g.Og * g.Kg * 4);
+  a.dy_bytes = (uint32_t)((g.outer * g.O * g.out_sp_size - dy_first) * 4);
+  hipLaunchKernelGGL(conv_dw_maxima, dim3((unsigned)a.p.slices, (unsigned)(g.Cg + g.Og)), dim3(256), 0, stream, a.x,
+                     a.dy, maxima, a.N, a.C, a.O, a.Cg, a.Og, (int)g.in_sp_size, (int)g.out_sp_size);
+  NBLA_HIP_LAUNCH_CHECK("conv_dw_maxima");
+  int rc;
+  switch (a.p.KW * 4 + a.p.S) {
+  case 1 * 4 + 1: rc = run_conv_dw<1, 1>(a, stream); break;
+  case 1 * 4 + 2: rc = run_conv_dw<1, 2>(a, stream); break;
+  case 3 * 4 + 1: rc = run_conv_dw<3, 1>(a, stream); break;
+  case 3 * 4 + 2: rc = run_conv_dw<3, 2>(a, stream); break;
+  case 5 * 4 + 1: rc = run_conv_dw<5, 1>(a, stream); break;
+  default: rc = run_conv_dw<5, 2>(a, stream); break;
+  }
+  if (rc)
+    return rc;
+  const int64_t outs = g.Og * g.Kg;
+  hipLaunchKernelGGL(conv_dw_sum, dim3((unsigned)ceil_div(outs, 32)), dim3(256), 0, stream, a.partial, a.shifts,
+                     dW + grp * g.Og * g.Kg, a.Og, a.Cg, (int)g.k_size, a.p.splits, accumulate ? 1 : 0);
+  NBLA_HIP_LAUNCH_CHECK("conv_dw_sum");
+  return NBLA_HIP_OK;
+}
+
+} // namespace nbla_hip

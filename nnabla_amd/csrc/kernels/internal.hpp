@@ -65,6 +65,13 @@ int launch_conv_direct_backward(const float *dy, const float *x, const float *w,
                                 float *dW, float *db, const ConvGeom &g, bool accum_x, bool accum_w, bool accum_b,
                                 bool take_sign, float zero_to, float *scratch, size_t scratch_bytes,
                                 hipStream_t stream);
+// The weight gradient of one group on the fp16 matrix cores without an unfolded matrix (conv_dw.hip): dW (+)= the sum
+// over positions of dy x, for two-dimensional kernels of width 1, 3 or 5 padded by half their width, strides 1 and 2.
+// x, dy and dW are the whole tensors; workspace: conv_dw_workspace_bytes(g), 256-byte aligned.
+bool conv_dw_applies(const ConvGeom &g);
+size_t conv_dw_workspace_bytes(const ConvGeom &g);
+int launch_conv_dw(const float *dy, const float *x, float *dW, const ConvGeom &g, int64_t grp, bool accumulate,
+                   void *workspace, size_t workspace_bytes, hipStream_t stream);
 // The binary convolution forward with the unfold done by LDS addressing (conv_slab.hip), two launches per group:
 // launch_conv_slab_prepare reads the group's weights [Og, Cg, taps] once and writes Wb = Sign(W) (may be null) and,
 // into `prepared` (conv_slab_prepared_bytes, 16-byte aligned), the packed bits in (tap, channel) order with the

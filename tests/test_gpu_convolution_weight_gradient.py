@@ -1,0 +1,82 @@
+"""The weight gradient on the fp16 matrix cores (csrc/kernels/conv_dw.hip) against float64, at the sizes where its tiles,
+groups of eight positions, phases and splits have their edges, alone and added to a gradient that is there already.
+
+A value is held as two fp16 numbers (22 bits at least: 2^-22 of a product per factor, and 2^-22 for the product of the
+two remainders) and sums are fp32: an element is off by at most (3 * 2^-22 + n * 2^-24) * sum |x dy|, n the roundings of
+the longest chain of sums (three per sixteen positions of a block).  The errors of the products are independent of each
+other, so the norm of the error is far below that: 2^-23 for the products and 2^-25 * sqrt(3 n / 2) for the sums of random
+terms, under 1e-6 of the norm of the gradient for n up to a few thousand.
+"""
+import numpy as np
+import pytest
+import torch
+
+from nnabla_amd import kernels
+
+pytestmark = pytest.mark.gpu
+
+# (x shape, output channels, kernel, pad, stride, group)
+CASES = [
+    ((2, 64, 56, 56), 64, (3, 3), (1, 1), 1, 1),
+    ((3, 33, 55, 57), 65, (3, 3), (1, 1), 1, 1),     # channels one past a tile, rows of 57 = 7 groups and one position
+    ((5, 8, 7, 7), 16, (3, 3), (1, 1), 1, 1),        # the fewest channels; whole samples of a small map per tile
+    ((37, 40, 7, 7), 24, (3, 3), (1, 1), 1, 1),      # a last tile of fewer samples
+    ((1, 96, 9, 8), 63, (5, 3), (2, 1), 1, 1),       # rows of taps in two passes, the second of two rows
+    ((2, 32, 13, 17), 32, (1, 3), (0, 1), 1, 1),     # one row of taps
+    ((2, 40, 28, 28), 48, (3, 3), (1, 1), 2, 1),
+    ((2, 31, 27, 29), 130, (3, 3), (0, 1), 2, 1),    # no padding above and below, odd extents, two strides
+    ((2, 48, 27, 27), 33, (5, 5), (2, 2), 1, 1),
+    ((3, 17, 14, 15), 64, (5, 5), (2, 2), 2, 1),
+    ((4, 129, 14, 14), 65, (1, 1), (0, 0), 1, 1),    # 128 input channels and one
+    ((3, 64, 13, 13), 48, (1, 1), (0, 0), 2, 1),
+    ((2, 64, 14, 14), 64, (3, 3), (1, 1), 1, 2),     # groups
+    ((70, 32, 5, 3), 32, (3, 3), (1, 1), 1, 1),      # rows shorter than a group of positions
+    ((2, 16, 3, 80), 32, (3, 3), (1, 1), 1, 1),      # the longest rows
+]
+
+
+@pytest.mark.parametrize("xs,O,k,pad,stride,group", CASES)
+def test_against_float64(xs, O, k, pad, stride, group):
+    rng = np.random.RandomState(7)
+    dev = torch.device("cuda:0")
+    kernels.init(0)
+    scale = (10.0 ** rng.uniform(-3, 3, (1, xs[1], 1, 1)))   # channels of very different magnitudes
+    x = torch.from_numpy((rng.randn(*xs) * scale).astype(np.float32))
+    W = torch.from_numpy(rng.randn(O, xs[1] // group, *k).astype(np.float32))
+
+    def gradient(x64, dy64):
+        w = W.double().requires_grad_()
+        torch.nn.functional.conv2d(x64, w, None, stride, pad, 1, group).backward(dy64)
+        return w.grad
+    oh = [(xs[2 + i] + 2 * pad[i] - k[i]) // stride + 1 for i in (0, 1)]
+    dy = torch.from_numpy((rng.randn(xs[0], O, *oh) * 1e-2).astype(np.float32))
+    ref, most = gradient(x.double(), dy.double()), gradient(x.double().abs(), dy.double().abs())
+    n = 3 * (xs[0] * oh[0] * (-(-oh[1] // 8) * 8) / 16 + 16)
+    bound = (3 * 2.0 ** -22 + n * 2.0 ** -24) * most
+    s = (stride, stride)
+    _, dW, _ = kernels.convolution_backward(dy.to(dev), x.to(dev), W.to(dev), pad, s, (1, 1), group,
+                                            want=(False, True, False))
+    err = (dW.cpu().double() - ref).abs()
+    assert bool((err <= bound).all())
+    per_channel = (err ** 2).sum((0, 2, 3)).sqrt() / (ref ** 2).sum((0, 2, 3)).sqrt()
+    assert float(per_channel.max()) <= 1e-6
+    dW0 = torch.from_numpy(rng.randn(*W.shape).astype(np.float32)) * ref.float().abs().mean()
+    _, acc, _ = kernels.binary_convolution_backward(dy.to(dev), x.to(dev), W.to(dev), None, None, pad, s, (1, 1), group,
+                                                    dW=dW0.to(dev), want=(False, True, False))
+    assert torch.equal(acc, dW0.to(dev) + dW)
+
+
+def test_a_non_finite_value_reaches_its_channel_only():
+    rng = np.random.RandomState(8)
+    dev = torch.device("cuda:0")
+    x = torch.from_numpy(rng.randn(2, 32, 9, 9).astype(np.float32)).to(dev)
+    dy = torch.from_numpy(rng.randn(2, 40, 9, 9).astype(np.float32)).to(dev)
+    W = torch.zeros(40, 32, 3, 3, device=dev)
+    _, clean, _ = kernels.convolution_backward(dy, x, W, (1, 1), (1, 1), (1, 1), 1, want=(False, True, False))
+    x[1, 5, 4, 4] = float("inf")
+    dy[0, 7, 0, 0] = float("nan")
+    _, dW, _ = kernels.convolution_backward(dy, x, W, (1, 1), (1, 1), (1, 1), 1, want=(False, True, False))
+    hit = torch.zeros_like(dW, dtype=torch.bool)
+    hit[:, 5] = True
+    hit[7] = True
+    assert bool(dW[hit].isnan().all()) and torch.equal(dW[~hit], clean[~hit])
