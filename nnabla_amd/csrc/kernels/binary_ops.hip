@@ -97,6 +97,10 @@ int binary_affine_forward(const float *x, const float *W, float *Wb, float *alph
   hipStream_t stream = as_stream(stream_);
   int rc;
 
+  if (!one_walk && fused_affine_applies(W, Wb, M, K, N, zero_to)) {
+    rc = ensure_init();
+    return rc ? rc : launch_fused_affine(x, W, Wb, alpha, bias, y, M, K, N, zero_to, stream);
+  }
   if (one_walk || (rows_affine_covers(W, Wb, alpha, bias, y, M, K, N) && rows_affine_pays(M, K, N))) {
     // one walk over W: signs, column sums and the product together
     if (!representable && (rc = launch_clear_words(count, 1, stream)))

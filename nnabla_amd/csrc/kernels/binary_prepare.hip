@@ -11,6 +11,7 @@ namespace nbla_hip {
 namespace {
 
 typedef float float4_t __attribute__((ext_vector_type(4)));
+typedef float float4_u __attribute__((ext_vector_type(4), aligned(4))); // one 128-bit access at any multiple of four bytes
 typedef uint32_t uint4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kPrepBlock = 256;
@@ -139,58 +140,61 @@ __global__ __launch_bounds__(kPrepBlock) void binarize_kn(const float *__restric
 
 // W stored [K, N], N % 4 == 0, 16-byte aligned: the streaming path.  A block of four wavefronts covers 256 rows of one
 // 256-column group, wavefront w rows 64 w .. 64 w + 63 (two k tiles); a lane owns four consecutive columns, so every
-// load and store instruction of a wavefront moves 1 KiB of one row.  Four rows are in flight while four are consumed
-// (128 registers per lane: sixteen wavefronts per CU).
+// load and store instruction of a wavefront moves 1 KiB of one row.  kBatch rows are in flight while as many are
+// consumed: four (128 registers per lane, sixteen wavefronts per CU), or sixteen -- a whole k tile -- for matrices of so
+// few blocks that a wavefront's 32 rows one batch after the other are the launch's time.
 // Per element: Sign -> Wb (nontemporal store), |w| into the lane's column sums, the sign bit shifted into a 32-bit
 // word per column (bit k = row k of the k tile).  After 32 rows the wavefront transposes those words through LDS into
 // the packed operand's own layout (lane l: columns F * 32 + l % 32, k slots (l / 32) * 16 + j; bit F + 8 c of word i
 // for k slot 4 i + c) and writes the k tile's 1 KiB straight into the packed operand.  No intermediate pair words and
 // no relayout pass.  Column sums: lanes in row order, then the block's four wavefronts through LDS in wavefront order.
-constexpr int kWideBatch = 4;
-constexpr int kWideTileBatches = kTileK / kWideBatch; // batches per k tile
-// kAligned: N a multiple of four and 16-byte aligned W / Wb, a lane's four columns are one 128-bit access; otherwise
-// four 32-bit ones, each column clamped and masked on its own (a row of W then starts at any multiple of four bytes).
-template <int kWideWaveRows, bool kFull, bool kCountZeros, bool kAligned>
+// kAligned: N a multiple of four and 16-byte aligned W / Wb.  Otherwise a row of W starts at any multiple of four bytes:
+// still one 128-bit access per lane (the forward of 300 rows under 4095 x 11007: 124 us with four 32-bit ones, 113 with
+// these, 134 with ordinary instead of nontemporal stores), except that the lane
+// whose columns end past N loads the last four and takes its own from among them, and stores them one by one.
+template <int kWideWaveRows, int kBatch, bool kFull, bool kCountZeros, bool kAligned>
 __device__ __forceinline__ void binarize_wide_walk(const float *__restrict__ W, float *__restrict__ Wb,
                                                    uint4_t *__restrict__ bits_out, int64_t tile_stride, uint32_t *s_x,
                                                    int64_t K, int64_t N, int64_t k_wave, int64_t n0, int lane,
                                                    float zero_to,
                                                    float (&cs)[4], int &nzero) {
   const bool col_ok = kFull || n0 < N;
-  const int64_t n_ld = col_ok ? n0 : N - 4; // loads are unconditional: a clamped address, masked afterwards
+  // loads are unconditional: a clamped address, masked afterwards
+  const int64_t n_ld = kFull || n0 + 4 <= N ? n0 : N - 4;
+  const int ahead = kFull || kAligned ? 0 : (int)(n0 - n_ld); // columns that the clamped address starts before the lane's
   const uint32_t lane_bytes = (uint32_t)(n_ld * 4);
-  uint32_t col_bytes[4];
   bool col_in[4];
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
+  for (int c = 0; c < 4; ++c)
     col_in[c] = kFull || n0 + c < N;
-    col_bytes[c] = (uint32_t)((col_in[c] ? n0 + c : N - 1) * 4);
-  }
-  float4_t va[kWideBatch], vb[kWideBatch];
+  float4_t va[kBatch], vb[kBatch];
   uint32_t word[4] = {0u, 0u, 0u, 0u};
-  auto load_batch = [&](int b, float4_t (&dst)[kWideBatch]) {
+  auto load_batch = [&](int b, float4_t (&dst)[kBatch]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < kWideBatch; ++j) {
-      int64_t k = k_wave + b * kWideBatch + j;
+    for (int j = 0; j < kBatch; ++j) {
+      int64_t k = k_wave + b * kBatch + j;
       if (!kFull && k >= K)
         k = K - 1;
       const char *row = reinterpret_cast<const char *>(W + k * N); // uniform base + 32-bit lane offset
-      if (kAligned) {
+      if (kAligned)
         dst[j] = *reinterpret_cast<const float4_t *>(row + lane_bytes);
-      } else {
-        dst[j].x = *reinterpret_cast<const float *>(row + col_bytes[0]);
-        dst[j].y = *reinterpret_cast<const float *>(row + col_bytes[1]);
-        dst[j].z = *reinterpret_cast<const float *>(row + col_bytes[2]);
-        dst[j].w = *reinterpret_cast<const float *>(row + col_bytes[3]);
-      }
+      else
+        dst[j] = *reinterpret_cast<const float4_u *>(row + lane_bytes);
     }
   };
-  auto consume_batch = [&](int b, const float4_t (&src)[kWideBatch]) {
+  auto consume_batch = [&](int b, const float4_t (&src)[kBatch]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < kWideBatch; ++j) {
-      const int64_t k = k_wave + b * kWideBatch + j;
+    for (int j = 0; j < kBatch; ++j) {
+      const int64_t k = k_wave + b * kBatch + j;
       const bool row_in = kFull || k < K;
-      const float w[4] = {src[j].x, src[j].y, src[j].z, src[j].w};
+      float w[4] = {src[j].x, src[j].y, src[j].z, src[j].w};
+      if (!kFull && !kAligned) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+          for (int s = 1; s + c < 4; ++s)
+            w[c] = ahead == s ? src[j][c + s] : w[c];
+      }
       float sg[4];
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
@@ -206,23 +210,25 @@ __device__ __forceinline__ void binarize_wide_walk(const float *__restrict__ W, 
         if (kCountZeros)
           nzero += (in && !nonzero) ? 1 : 0;
       }
-      if (Wb && kAligned && (kFull || (col_ok && row_in))) {
+      if (Wb && row_in && (kFull || (kAligned ? col_ok : col_in[3]))) {
         float4_t o;
         o.x = sg[0], o.y = sg[1], o.z = sg[2], o.w = sg[3];
         char *row = reinterpret_cast<char *>(Wb + k * N);
-        __builtin_nontemporal_store(o, reinterpret_cast<float4_t *>(row + lane_bytes));
+        if (kAligned)
+          __builtin_nontemporal_store(o, reinterpret_cast<float4_t *>(row + lane_bytes));
+        else
+          __builtin_nontemporal_store(o, reinterpret_cast<float4_u *>(row + lane_bytes));
       }
-      if (Wb && !kAligned && row_in) {
-        char *row = reinterpret_cast<char *>(Wb + k * N);
+      if (!kFull && !kAligned && Wb && row_in && col_ok && !col_in[3]) {
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
+        for (int c = 0; c < 3; ++c)
           if (col_in[c])
-            __builtin_nontemporal_store(sg[c], reinterpret_cast<float *>(row + col_bytes[c]));
+            Wb[k * N + n0 + c] = sg[c];
       }
     }
   };
   // 32 rows are in `word`: transpose them into the packed layout and write the k tile
-  auto emit_tile = [&](int t) {
+  auto emit_tile = [&](int t) __attribute__((always_inline)) {
     uint4_t mine;
     mine.x = word[0], mine.y = word[1], mine.z = word[2], mine.w = word[3];
     *reinterpret_cast<uint4_t *>(s_x + 4 * lane) = mine;
@@ -245,7 +251,7 @@ __device__ __forceinline__ void binarize_wide_walk(const float *__restrict__ W, 
     o.x = out[0], o.y = out[1], o.z = out[2], o.w = out[3];
     bits_out[(size_t)t * tile_stride] = o; // bits_out: this lane's slot in the wavefront's first k tile
   };
-  constexpr int kBatches = kWideWaveRows / kWideBatch;
+  constexpr int kBatches = kWideWaveRows / kBatch, kTileBatches = kTileK / kBatch;
   load_batch(0, va);
 #pragma clang loop unroll(disable)
   for (int b = 0; b < kBatches; b += 2) {
@@ -254,8 +260,8 @@ __device__ __forceinline__ void binarize_wide_walk(const float *__restrict__ W, 
     if (b + 2 < kBatches)
       load_batch(b + 2, va);
     consume_batch(b + 1, vb);
-    if ((b + 2) % kWideTileBatches == 0) {
-      emit_tile(b / kWideTileBatches);
+    if ((b + 2) % kTileBatches == 0) {
+      emit_tile(b / kTileBatches);
 #pragma unroll
       for (int c = 0; c < 4; ++c)
         word[c] = 0u;
@@ -264,8 +270,8 @@ __device__ __forceinline__ void binarize_wide_walk(const float *__restrict__ W, 
 }
 
 // kWideWaveRows: 64 (two k tiles per wavefront), or 32 for matrices that would otherwise give the CUs too few blocks.
-template <int kWideWaveRows, bool kCountZeros, bool kAligned>
-__global__ __launch_bounds__(kPrepBlock, 4) void binarize_kn_wide(const float *__restrict__ W, float *__restrict__ Wb,
+template <int kWideWaveRows, int kBatch, bool kCountZeros, bool kAligned>
+__global__ __launch_bounds__(kPrepBlock, kBatch > 4 ? 1 : 4) void binarize_kn_wide(const float *__restrict__ W, float *__restrict__ Wb,
                                                                  uint4_t *__restrict__ bits, float *__restrict__ sums,
                                                                  int *__restrict__ zeros, int64_t K, int64_t N,
                                                                  int64_t wide_groups, int64_t Npw, float zero_to) {
@@ -284,10 +290,10 @@ __global__ __launch_bounds__(kPrepBlock, 4) void binarize_kn_wide(const float *_
   const int64_t tile_stride = wide_groups * 64;
   const bool full = k_wave + kWideWaveRows <= K && (wg + 1) * kWideGroup <= N;
   if (full)
-    binarize_wide_walk<kWideWaveRows, true, kCountZeros, kAligned>(W, Wb, tile0, tile_stride, s_x[wave], K, N, k_wave, n0,
+    binarize_wide_walk<kWideWaveRows, kBatch, true, kCountZeros, kAligned>(W, Wb, tile0, tile_stride, s_x[wave], K, N, k_wave, n0,
                                                                    lane, zero_to, cs, nzero);
   else
-    binarize_wide_walk<kWideWaveRows, false, kCountZeros, kAligned>(W, Wb, tile0, tile_stride, s_x[wave], K, N, k_wave, n0,
+    binarize_wide_walk<kWideWaveRows, kBatch, false, kCountZeros, kAligned>(W, Wb, tile0, tile_stride, s_x[wave], K, N, k_wave, n0,
                                                                     lane, zero_to, cs, nzero);
   // column sums of the block's 256 rows, wavefronts in order
   *reinterpret_cast<float4_t *>(&s_sum[wave][4 * lane]) = float4_t{cs[0], cs[1], cs[2], cs[3]};
@@ -1128,7 +1134,7 @@ int nbla_hip_binarize_weights_f32(const float *W, float *Wb, float *alpha, uint3
   uint32_t *pairs = reinterpret_cast<uint32_t *>(static_cast<char *>(workspace) + P.sums_bytes + P.zeros_bytes);
   int64_t slices = P.slices;
   if (!transposed) {
-    if (P.slabs <= 65535 && (uint64_t)N * 4 < (1ull << 32)) {
+    if (P.slabs <= 65535 && (uint64_t)N * 4 < (1ull << 32) && N >= 4) {
       // a lane's four columns as one 128-bit access where the rows allow it (a null Wb -- no fp32 signs wanted --
       // counts as aligned), else as four 32-bit ones
       const bool aligned = N % 4 == 0 && N >= 4 && aligned16(W) && aligned16(Wb);
@@ -1138,23 +1144,30 @@ int nbla_hip_binarize_weights_f32(const float *W, float *Wb, float *alpha, uint3
       const int64_t slabs = fine ? 2 * P.slabs : P.slabs;
       const dim3 grid((unsigned)P.wide_groups, (unsigned)slabs);
       uint4_t *packed = reinterpret_cast<uint4_t *>(bits);
-#define NBLA_BINARIZE_WIDE(ROWS, COUNT)                                                                                \
+      // blocks for half of the CUs at most: all rows of a wavefront in flight at once (1500 rows under 2048 x 2048, 128
+      // blocks: forward 45.2 -> 43.4 us; under 2048 x 4096, 256 blocks, four rows at a time are the faster: 59.2, 61.6)
+      const bool deep = fine && P.wide_groups * slabs <= 128;
+#define NBLA_BINARIZE_WIDE(ROWS, BATCH, COUNT)                                                                         \
   do {                                                                                                                 \
     if (aligned)                                                                                                       \
-      hipLaunchKernelGGL((binarize_kn_wide<ROWS, COUNT, true>), grid, dim3(kPrepBlock), 0, stream, W, Wb, packed, sums,  \
-                         zeros, K, N, P.wide_groups, P.Npw, quantize_zero_to);                                         \
+      hipLaunchKernelGGL((binarize_kn_wide<ROWS, BATCH, COUNT, true>), grid, dim3(kPrepBlock), 0, stream, W, Wb, packed, \
+                         sums, zeros, K, N, P.wide_groups, P.Npw, quantize_zero_to);                                   \
     else                                                                                                               \
-      hipLaunchKernelGGL((binarize_kn_wide<ROWS, COUNT, false>), grid, dim3(kPrepBlock), 0, stream, W, Wb, packed, sums, \
-                         zeros, K, N, P.wide_groups, P.Npw, quantize_zero_to);                                         \
+      hipLaunchKernelGGL((binarize_kn_wide<ROWS, BATCH, COUNT, false>), grid, dim3(kPrepBlock), 0, stream, W, Wb,      \
+                         packed, sums, zeros, K, N, P.wide_groups, P.Npw, quantize_zero_to);                           \
   } while (0)
-      if (fine && zero_count)
-        NBLA_BINARIZE_WIDE(32, true);
+      if (deep && zero_count)
+        NBLA_BINARIZE_WIDE(32, 16, true);
+      else if (deep)
+        NBLA_BINARIZE_WIDE(32, 16, false);
+      else if (fine && zero_count)
+        NBLA_BINARIZE_WIDE(32, 4, true);
       else if (fine)
-        NBLA_BINARIZE_WIDE(32, false);
+        NBLA_BINARIZE_WIDE(32, 4, false);
       else if (zero_count)
-        NBLA_BINARIZE_WIDE(64, true);
+        NBLA_BINARIZE_WIDE(64, 4, true);
       else
-        NBLA_BINARIZE_WIDE(64, false);
+        NBLA_BINARIZE_WIDE(64, 4, false);
 #undef NBLA_BINARIZE_WIDE
       NBLA_HIP_LAUNCH_CHECK("binarize_kn_wide");
       if (alpha || zero_count) {

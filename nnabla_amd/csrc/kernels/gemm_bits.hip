@@ -1141,10 +1141,9 @@ int launch_tile(const GemmBitsArgs &args, hipStream_t stream, unsigned splits = 
   a.blocks_m = ceil_div(a.M, BM);
   a.blocks_n = ceil_div(a.n_end - a.n_begin, BN);
   const dim3 grid((unsigned)(a.blocks_m * a.blocks_n), splits);
-  if (t_timer.used < t_timer.start.size()) {
-    hipExtLaunchKernelGGL((NBLA_GEMM_BITS_KERNEL), grid, dim3(kThreads), kSmem, stream, t_timer.start[t_timer.used],
-                          t_timer.stop[t_timer.used], 0, a);
-    ++t_timer.used;
+  hipEvent_t start, stop;
+  if (product_timer_next(&start, &stop)) {
+    hipExtLaunchKernelGGL((NBLA_GEMM_BITS_KERNEL), grid, dim3(kThreads), kSmem, stream, start, stop, 0, a);
   } else {
     hipLaunchKernelGGL((NBLA_GEMM_BITS_KERNEL), grid, dim3(kThreads), kSmem, stream, a);
   }
@@ -1387,6 +1386,14 @@ extern "C" int nbla_hip_gemm_bits_f32(const void *xdigits, const uint32_t *bits,
   // m-contiguous outputs (n_stride != 1) store from the transposed accumulator tile
   return launch_gemm_bits(xdigits, bits, alpha, bias, y, M, K, N, inner, outer_stride, n_stride, n_stride != 1,
                           as_stream(stream), false, workspace, workspace_bytes);
+}
+
+bool nbla_hip::product_timer_next(hipEvent_t *start, hipEvent_t *stop) {
+  if (t_timer.used >= t_timer.start.size())
+    return false;
+  *start = t_timer.start[t_timer.used], *stop = t_timer.stop[t_timer.used];
+  ++t_timer.used;
+  return true;
 }
 
 extern "C" int nbla_hip_gemm_bits_timer_arm(int launches) {

@@ -28,6 +28,9 @@ int launch_gemm_bits(const void *xsplit, const uint32_t *bits, const float *alph
                      int64_t M, int64_t K, int64_t N, int64_t inner, int64_t outer_stride, int64_t n_stride,
                      bool swap_out, hipStream_t stream, bool accumulate = false, void *split_ws = nullptr,
                      size_t split_ws_bytes = 0, bool keep_bad_rows = false, const int *skip_if = nullptr);
+// While the calling thread's product timer (nbla_hip_gemm_bits_timer_arm) is armed: the events that its next launch of
+// the product is to carry.
+bool product_timer_next(hipEvent_t *start, hipEvent_t *stop);
 // The same product for a convolution with the unfold fused in: the rows are the unfolded windows of x (group `grp`),
 // converted to digits inside the kernel; y is [sample, O, output position].  gemm_bits_unfold_applies tells whether
 // the geometry is covered (otherwise: launch_im2col_digits + launch_gemm_bits).  row_shift (may be null): M words that
@@ -165,6 +168,12 @@ size_t rows_affine_workspace_bytes(int64_t M, int64_t K, int64_t N);
 int launch_rows_affine(const void *xdigits, const float *W, float *Wb, float *alpha, const float *bias, float *y,
                        int64_t M, int64_t K, int64_t N, float zero_to, int *zero_flag, void *workspace,
                        size_t workspace_bytes, hipStream_t stream);
+
+// The same forward in one launch for small layers of any alignment (binary_fused.hip): a block computes 32 rows x 64
+// columns from x and W themselves.
+bool fused_affine_applies(const float *W, const float *Wb, int64_t M, int64_t K, int64_t N, float zero_to);
+int launch_fused_affine(const float *x, const float *W, float *Wb, float *alpha, const float *bias, float *y, int64_t M,
+                        int64_t K, int64_t N, float zero_to, hipStream_t stream);
 
 // db[n] (+)= sum over m of dy[m, n]; `partial` holds ceil(M / 256) * N floats.
 size_t column_sums_workspace_bytes(int64_t M, int64_t N);
