@@ -70,7 +70,10 @@ struct SlabPlan {
   int col_groups;  // groups of 64 wn output channels
   int ct;          // channel tiles of 32 (channels padded)
   int frags;       // fragments of 32 output channels
-  int pix_stride;  // bytes per pixel: 128 per channel tile, and the padding
+  int ct_chunk;    // channel tiles that the slab holds at a time
+  int chunks;      // fills of the slab
+  bool fits_once;  // some form holds all channels at a time
+  int pix_stride;  // bytes per pixel: 128 per channel tile held, and the padding
   int cap;         // pixels a slab may hold (the zero pixel not counted)
   int slab_bytes;
   int k_tiles;     // taps * ct
@@ -114,7 +117,7 @@ __host__ __device__ inline int64_t slab_last_tap(const ConvGeom &g) {
          (int64_t)(g.k[2] - 1) * g.dil[2];
 }
 
-template <int WN, int WM, int WK>
+template <int WN, int WM, int WK, bool kChunked>
 __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(ConvSlabArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int kWaves = WN * WM * WK, kThreads = 64 * kWaves, kRows = kSlabRows * WM, kCols = 64 * WN;
@@ -182,11 +185,19 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
   // per wavefront is loaded once, all loads in flight together, and kept in registers between the two steps; a larger
   // one is read twice.
   const float *xs = a.x + ((int64_t)n * g.C + (int64_t)a.grp * g.Cg) * plane + lo;
-  const int groups16 = 2 * CT, items = ((npix + 63) >> 6) * groups16;
+  // Where all channels of the slab do not fit the LDS, it is filled a chunk of channel tiles at a time, the accumulators
+  // staying in their registers; the scale is that of all channels, found before the first chunk is converted.
+  const int pixel_runs = (npix + 63) >> 6;
+  int groups16 = 2 * CT, ch_first = 0, items = pixel_runs * groups16; // the items that are walked: all channels, or a chunk
   // item -> (first pixel, first channel)
   auto item_of = [&](int item, int &pix0, int &ch0) __attribute__((always_inline)) {
     const int pc = item / groups16;
-    pix0 = pc * 64, ch0 = (item - pc * groups16) * 16;
+    pix0 = pc * 64, ch0 = ch_first + (item - pc * groups16) * 16;
+  };
+  auto take_chunk = [&](int chunk) __attribute__((always_inline)) {
+    ch_first = chunk * P.ct_chunk * 32;
+    groups16 = 2 * min(P.ct_chunk, CT - chunk * P.ct_chunk);
+    items = pixel_runs * groups16;
   };
   // Nothing but loads: a select or a branch on their results here would make a wavefront wait for one item's loads
   // before it issues the next item's.  Channels past the last repeat it, pixels past the slab the first.
@@ -251,8 +262,8 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
     int pix0, ch0;
     item_of(item, pix0, ch0);
     if (pix0 + lane < npix) {
-      // channel tile ch0 / 32, half (ch0 / 16) % 2 of its 32 channels: one byte per channel and digit
-      unsigned char *dst = smem + (pix0 + lane + 1) * P.pix_stride + (ch0 >> 5) * 128 + (ch0 & 16);
+      // channel tile ch0 / 32 of the chunk, half (ch0 / 16) % 2 of its 32 channels: one byte per channel and digit
+      unsigned char *dst = smem + (pix0 + lane + 1) * P.pix_stride + ((ch0 - ch_first) >> 5) * 128 + (ch0 & 16);
 #pragma unroll
       for (int dg = 0; dg < kSlabDigits; ++dg) {
         uint4_t o;
@@ -265,7 +276,7 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
         s_pixbad[pix0 + lane + 1] = 1u;
     }
   };
-  const bool hold = items <= kSlabHold * kWaves; // uniform over the block
+  const bool hold = !kChunked && items <= kSlabHold * kWaves; // uniform over the block
   float hv[kSlabHold][16];
   if (hold) {
 #pragma unroll
@@ -340,18 +351,23 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
     if (bmax != 0u)
       shift = kSlabTopBit - binade_exponent(binade_of(bmax));
   }
-  if (hold) {
-#pragma unroll
-    for (int h = 0; h < kSlabHold; ++h)
-      if (wave + h * kWaves < items)
-        convert_item(wave + h * kWaves, hv[h]);
-  } else {
+  auto convert_chunk = [&]() __attribute__((always_inline)) {
     for (int item = wave; item < items; item += kWaves) {
       float v[16];
       load_item(item, v);
       scan_item(item, v); // (the scale and the padding again; the maximum is not used any more)
       convert_item(item, v);
     }
+  };
+  if (kChunked)
+    take_chunk(0);
+  if (hold) {
+#pragma unroll
+    for (int h = 0; h < kSlabHold; ++h)
+      if (wave + h * kWaves < items)
+        convert_item(wave + h * kWaves, hv[h]);
+  } else {
+    convert_chunk();
   }
   if (tid < kCols) { // alpha = (sum of the partial sums, in channel-tile order: every block forms the same bits) / K
     float al = 1.0f;
@@ -382,7 +398,7 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
   }
   __syncthreads();
   // the windows' sums of q and whether they hold a non-finite value (read again only after the product)
-  {
+  auto sum_windows = [&]() __attribute__((always_inline)) {
     long long sum = 0;
     uint32_t bad = 0u;
     for (int t = tid / kRows; t < taps; t += kThreads / kRows) {
@@ -394,12 +410,11 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
       atomicAdd(reinterpret_cast<unsigned long long *>(&s_rowsum[trow]), (unsigned long long)sum);
     if (bad)
       s_rowbad[trow] = 1;
-  }
+  };
 
   // ---- 2. the product.  Wavefront (wn, wm, wk): channel fragments 2 wn, 2 wn + 1 of the block's, window fragment wm,
   // k tiles wk, wk + WK, ...
   const int wn = wave % WN, wk = wave / (WN * WM);
-  const int nk = (P.k_tiles - wk + WK - 1) / WK;
   i32x16_t acc[kSlabDigits][2];
 #pragma unroll
   for (int d = 0; d < kSlabDigits; ++d)
@@ -414,28 +429,59 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
     frag_mask[j] = 0x01010101u << (frag0 + 2 * wn + j);
     asm volatile("" : "+s"(frag_mask[j]));
   }
-  if (nk > 0) {
-    // the words of step i sit at wnext[lane] when they are loaded: a uniform pointer that stops at the last step
-    const uint4_t *wnext = a.bits + ((int64_t)wk * P.wide_groups + wg) * 64;
-    const int64_t wstep = (int64_t)WK * P.wide_groups * 64;
-    int wleft = nk - 1; // steps the pointer may still advance
-    uint4_t words[kSlabAhead];
-#pragma unroll
-    for (int u = 0; u < kSlabAhead; ++u) {
-      words[u] = wnext[lane];
-      wnext += wleft > 0 ? wstep : 0;
-      --wleft;
+  const int chunks = kChunked ? P.chunks : 1;
+  for (int chunk = 0; chunk < chunks; ++chunk) {
+    if (chunk > 0) {
+      __syncthreads(); // every wavefront is through with the chunk before
+      take_chunk(chunk);
+      convert_chunk();
+      __syncthreads();
     }
-    // position (tap, channel tile) of the k tile two steps ahead, advanced by WK k tiles per step
-    int tap2 = 0, ct2 = wk;
-    auto normalise = [&]() __attribute__((always_inline)) {
-      if (ct2 >= CT) {
-        ct2 -= CT, ++tap2;
-        if (WK == 2 && ct2 >= CT)
-          ct2 -= CT, ++tap2;
+    if (chunk == chunks - 1)
+      sum_windows();
+    const int ctn = kChunked ? groups16 >> 1 : CT; // channel tiles of the chunk
+    const int nk = (taps * ctn - wk + WK - 1) / WK;
+    if (nk <= 0)
+      continue;
+    // (tap, channel tile of the chunk), advanced by WK k tiles per step
+    auto normalise = [&](int &tap, int &ct) __attribute__((always_inline)) {
+      if (ct >= ctn) {
+        ct -= ctn, ++tap;
+        if (WK == 2 && ct >= ctn)
+          ct -= ctn, ++tap;
       }
     };
-    normalise();
+    // the words of the next step to load: a uniform pointer that stops at the last step (the k tiles of all channels
+    // follow each other; those of a chunk are found by their tap and channel tile)
+    int tapw = 0, ctw = wk;
+    if (kChunked)
+      normalise(tapw, ctw);
+    int wleft = nk - 1; // steps the position may still advance
+    const uint4_t *wnext = a.bits + ((int64_t)(kChunked ? chunk * P.ct_chunk : wk) * P.wide_groups + wg) * 64;
+    const int64_t wstep = (int64_t)WK * P.wide_groups * 64;
+    auto load_words = [&]() __attribute__((always_inline)) {
+      if constexpr (kChunked) {
+        const uint4_t w = wnext[(int64_t)(tapw * CT + ctw) * P.wide_groups * 64 + lane];
+        if (wleft > 0) {
+          ctw += WK;
+          normalise(tapw, ctw);
+        }
+        --wleft;
+        return w;
+      } else {
+        const uint4_t w = wnext[lane];
+        wnext += wleft > 0 ? wstep : 0;
+        --wleft;
+        return w;
+      }
+    };
+    uint4_t words[kSlabAhead];
+#pragma unroll
+    for (int u = 0; u < kSlabAhead; ++u)
+      words[u] = load_words();
+    // position of the k tile two steps ahead
+    int tap2 = 0, ct2 = wk;
+    normalise(tap2, ct2);
     const uint32_t lane_off = (uint32_t)(half * 16);
     const uint32_t *my_rowpix = s_rowpix + row;
     // LDS offset of the lane's sixteen bytes of step (tap2, ct2); past the last k tile: inside the zero pixel
@@ -445,7 +491,7 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
     };
     auto advance = [&]() __attribute__((always_inline)) {
       ct2 += WK;
-      normalise();
+      normalise(tap2, ct2);
     };
     auto read_a = [&](uint32_t off, uint4_t (&af)[kSlabDigits]) __attribute__((always_inline)) {
 #pragma unroll
@@ -484,9 +530,7 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
         advance();
         read_a(off_b, af[(u + 1) & 1]); // step i + 1
         mma(af[u & 1], words[u]);
-        words[u] = wnext[lane];
-        wnext += wleft > 0 ? wstep : 0;
-        --wleft;
+        words[u] = load_words();
 #pragma unroll
         for (int q = 0; q < kSlabDigits + 1; ++q) {
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -835,8 +879,8 @@ struct SlabForm {
 constexpr SlabForm kSlabForms[] = {{4, 1, 2}, {4, 2, 1}, {4, 1, 1}, {2, 2, 1}, {1, 4, 2}, {1, 4, 1}};
 constexpr int kSlabFormCount = (int)(sizeof(kSlabForms) / sizeof(kSlabForms[0]));
 
-// The plan of one form; false when its slab does not fit the LDS.
-bool compute_slab_form(const ConvGeom &g, int form, SlabPlan &p) {
+// The plan of one form that fills its slab `chunks` times; false when it does not fit the LDS.
+bool compute_slab_form(const ConvGeom &g, int form, int chunks, SlabPlan &p) {
   const SlabForm &f = kSlabForms[form];
   const int waves = f.wn * f.wm * f.wk, rows = kSlabRows * f.wm;
   p.form = form;
@@ -858,7 +902,9 @@ bool compute_slab_form(const ConvGeom &g, int form, SlabPlan &p) {
     return false;
   p.ct = (int)(cgp / 32);
   p.frags = (int)ceil_div(g.Og, 32);
-  p.pix_stride = kSlabDigits * (int)cgp + kSlabPixPad;
+  p.ct_chunk = (int)ceil_div(p.ct, chunks);
+  p.chunks = (int)ceil_div(p.ct, p.ct_chunk);
+  p.pix_stride = kSlabDigits * 32 * p.ct_chunk + kSlabPixPad;
   const int64_t cap = slab_longest_run(g, p.tile_rows, p.tiles_per_sample);
   const int64_t slab_bytes = (cap + 1) * p.pix_stride;
   if (slab_bytes > kSlabLdsLimit)
@@ -888,57 +934,88 @@ bool compute_slab_form(const ConvGeom &g, int form, SlabPlan &p) {
 
 // Cycles of the launch, roughly: what the phases of a block measured (time stamps in blocks of 64, 256 and 512 input
 // channels).  A block starts and waits for its first loads for about 7500 cycles, a work item of the set-up costs
-// about 450 (half as much again when the slab is read twice), an MFMA 46 of which 32 are its own, and the epilogue
+// about 450 (half as much again when the slab is read twice, and 5000 in all for each further fill), an MFMA 46 of which 32 are its own, and the epilogue
 // about 2800 per fragment of a wavefront.  Two blocks of four wavefronts share a CU where the LDS holds both slabs:
-// each then takes 1.13 times as long, or what their MFMAs and vector instructions add up to.
+// each then takes 1.13 times as long, or what their MFMAs and vector instructions add up to, and a third more where all
+// CUs do so (memory); tiles one column group wide take a quarter more than this, their loads being the most.
 double slab_form_cost(const ConvGeom &g, const SlabPlan &p) {
   const SlabForm &f = kSlabForms[p.form];
   const int waves = f.wn * f.wm * f.wk;
   const double items = (double)ceil_div(p.cap, 64) * 2 * p.ct;
-  const double load = items * (items > kSlabHold * waves ? 700.0 : 450.0);
+  const double load = items * (p.chunks > 1 || items > kSlabHold * waves ? 700.0 : 450.0) + 5000.0 * (p.chunks - 1);
   const double mma = 46.0 * p.k_tiles * 8 * f.wn * f.wm / 4;
   const double out = 1500.0 + 2800.0 * (f.wk == 2 ? 1 : 2) * (waves == 8 && f.wk == 1 ? 1.3 : 1.0);
   const double one = 7500.0 + load + mma + out;
-  const double pair = one * 1.13 > 2 * mma * 0.92 + load + out ? one * 1.13 : 2 * mma * 0.92 + load + out;
+  const double both = 2 * mma * 0.92 + load + out, pair = 1.3 * (one * 1.13 > both ? one * 1.13 : both);
   const int64_t blocks = g.outer * p.tiles_per_sample * p.col_groups;
   if (waves == 8 || p.total > 79 * 1024)
-    return (double)ceil_div(blocks, 256) * one;
+    return (double)ceil_div(blocks, 256) * one * (waves == 8 && f.wn == 1 ? 1.25 : 1.0);
   const int64_t rest = blocks % 512;
   return (double)(blocks / 512) * pair + (rest > 256 ? pair : rest > 0 ? one : 0.0);
 }
 
 bool compute_slab_plan(const ConvGeom &g, SlabPlan &narrow, SlabPlan &p) {
-  if (g.k_size > kSlabMaxTaps || g.Cg < 24 || g.in_sp_size >= ((int64_t)1 << 30) ||
+  if (g.k_size > kSlabMaxTaps || g.Cg < 16 || g.in_sp_size >= ((int64_t)1 << 30) ||
       g.out_sp_size >= ((int64_t)1 << 30) || g.Og >= ((int64_t)1 << 24) ||
       (g.Og + kWideGroup) * g.out_sp_size >= ((int64_t)1 << 31))
     return false;
   const int64_t cgp = ceil_div(g.Cg, 32) * 32;
-  // padded channels cost as much as real ones; the epilogue's 32-bit steps hold kChunkK terms
-  if (cgp * 3 > g.Cg * 4 || g.k_size * cgp > kChunkK)
+  if (g.k_size * cgp > kChunkK) // the epilogue's 32-bit steps hold kChunkK terms
     return false;
-  if (!compute_slab_form(g, 0, narrow))
-    return false;
-  p = narrow;
-  double best = slab_form_cost(g, p);
+  // <4, 1, 2> with the slab filled once is for geometries of little padding (padded channels cost as much as real ones)
+  narrow.form = -1;
+  double best = 0.0;
+  bool any = false;
+  if (cgp * 3 <= g.Cg * 4 && compute_slab_form(g, 0, 1, p)) {
+    narrow = p;
+    best = slab_form_cost(g, p);
+    any = true;
+  } else {
+    narrow.form = -1;
+  }
   for (int form = 1; form < kSlabFormCount; ++form) {
     SlabPlan q;
-    if (!compute_slab_form(g, form, q))
+    if (!compute_slab_form(g, form, 1, q))
       continue;
     const double cost = slab_form_cost(g, q);
-    if (cost < best)
-      p = q, best = cost;
+    if (!any || cost < best)
+      p = q, best = cost, any = true;
   }
-  return true;
+  // The slab filled several times: against the forms that hold all channels at once, or where none does against the
+  // product that gathers its operands window by window (912 cycles per k tile of 32 windows x 256 channels), if clearly
+  // cheaper by these estimates: [4,512,28,28] x [512,512,3,3] 64 us there and 69 here, [16,512,28,28] x [256,512,3,3]
+  // 111 and 76; [8,256,56,56] x [128,256,3,3] 107 filled once and 61 filled several times, [8,200,28,28] x [300,200,5,5]
+  // 99 and 120.
+  p.fits_once = any;
+  best /= 1.3;
+  if (!any) {
+    const double tiles = (double)ceil_div(ceil_div(g.M, kSlabRows) * bits_wide_groups(g.Og), 256);
+    best = tiles * (10000.0 + 912.0 * (double)ceil_div(g.Kg, kTileK)) / 1.3;
+  }
+  for (int form : {1, 2, 3, 5})
+    for (int chunks = 2; chunks <= (int)(cgp / 32); ++chunks) {
+      SlabPlan q;
+      if (!compute_slab_form(g, form, chunks, q))
+        continue;
+      const double cost = slab_form_cost(g, q);
+      if (cost < best) {
+        q.fits_once = p.fits_once;
+        p = q, best = cost, any = true;
+      }
+      if (q.total <= 79 * 1024) // more fills only cost
+        break;
+    }
+  return any;
 }
 
-template <int kForm> int run_slab_form(const ConvSlabArgs &a, unsigned blocks, hipStream_t stream) {
+template <int kForm, bool kChunked = false> int run_slab_form(const ConvSlabArgs &a, unsigned blocks, hipStream_t stream) {
   constexpr SlabForm f = kSlabForms[kForm];
   static std::atomic<uint64_t> configured{0};
-  const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(binary_conv_slab_kernel<f.wn, f.wm, f.wk>),
+  const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(binary_conv_slab_kernel<f.wn, f.wm, f.wk, kChunked>),
                                    kSlabLdsLimit, configured, "hipFuncSetAttribute(binary_conv_slab LDS size)");
   if (rc)
     return rc;
-  hipLaunchKernelGGL((binary_conv_slab_kernel<f.wn, f.wm, f.wk>), dim3(blocks), dim3(64 * f.wn * f.wm * f.wk),
+  hipLaunchKernelGGL((binary_conv_slab_kernel<f.wn, f.wm, f.wk, kChunked>), dim3(blocks), dim3(64 * f.wn * f.wm * f.wk),
                      (size_t)a.p.total, stream, a);
   NBLA_HIP_LAUNCH_CHECK("binary_conv_slab");
   return NBLA_HIP_OK;
@@ -953,7 +1030,7 @@ bool conv_slab_applies(const ConvGeom &g) {
 
 bool conv_slab_plan_summary(const ConvGeom &g, int32_t out[4]) {
   SlabPlan p;
-  if (!make_slab_plan(g, p, true))
+  if (!make_slab_plan(g, p, true) || p.form < 0)
     return false;
   out[0] = p.tile_rows, out[1] = p.tiles_per_sample, out[2] = p.cap, out[3] = p.total;
   return true;
@@ -1004,8 +1081,8 @@ bool conv_slab_transposed_geom(const ConvGeom &g, ConvGeom &t) {
   t.in_sp_size = g.out_sp_size, t.out_sp_size = g.in_sp_size;
   t.Kg = t.Cg * g.k_size;
   t.M = g.outer * t.out_sp_size;
-  SlabPlan p;
-  return make_slab_plan(t, p);
+  SlabPlan p; // (a slab that has to be filled several times loses to the unfolded gradient)
+  return make_slab_plan(t, p) && p.fits_once;
 }
 
 int launch_conv_slab_prepare_transposed(const float *Wg, void *prepared, const ConvGeom &g, float zero_to,
@@ -1051,6 +1128,11 @@ int launch_conv_slab(const float *x, const ConvGeom &g, int64_t grp, const void 
   a.grp = (int)grp;
   a.inv_k = (float)1 / g.Kg;
   const unsigned blocks = (unsigned)(g.outer * a.p.tiles_per_sample * a.p.col_groups);
+  if (a.p.chunks > 1)
+    return a.p.form == 1   ? run_slab_form<1, true>(a, blocks, stream)
+           : a.p.form == 2 ? run_slab_form<2, true>(a, blocks, stream)
+           : a.p.form == 3 ? run_slab_form<3, true>(a, blocks, stream)
+                           : run_slab_form<5, true>(a, blocks, stream);
   switch (a.p.form) {
   case 0:
     return run_slab_form<0>(a, blocks, stream);
