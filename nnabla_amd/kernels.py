@@ -98,15 +98,33 @@ def _i64(v):
     return ctypes.c_int64(int(v))
 
 
+_SHAPE_TYPES = {n: ctypes.c_int64 * n for n in range(9)}
+
+
 def _shape(seq):
-    return (ctypes.c_int64 * len(seq))(*[int(s) for s in seq])
+    n = len(seq)
+    return (_SHAPE_TYPES.get(n) or ctypes.c_int64 * n)(*[int(s) for s in seq])
+
+
+_raw_stream = None   # () -> handle of torch's current stream
+
+
+def _find_raw_stream():
+    """torch.cuda.current_stream() builds a Stream object, 2.8 us of an 8.5 us call; the handle alone takes 0.2."""
+    import torch
+    raw, device = getattr(torch._C, "_cuda_getCurrentRawStream", None), getattr(torch._C, "_cuda_getDevice", None)
+    if raw is None or device is None:
+        return lambda: torch.cuda.current_stream().cuda_stream
+    return lambda: raw(device())
 
 
 def _stream(stream):
-    if stream is None:
-        import torch
-        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-    return ctypes.c_void_p(int(stream))
+    if stream is not None:
+        return ctypes.c_void_p(int(stream))
+    global _raw_stream
+    if _raw_stream is None:
+        _raw_stream = _find_raw_stream()
+    return ctypes.c_void_p(_raw_stream())
 
 
 def _workspace(nbytes, like):
