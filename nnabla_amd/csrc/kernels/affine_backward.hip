@@ -87,6 +87,8 @@ BackwardPlan plan_backward(int64_t M, int64_t K, int64_t N) {
 // columns of x and of dy, the contraction runs over the M samples.
 int grad_weights(const float *x, const float *dy, float *dW, int64_t M, int64_t K, int64_t N, bool accumulate,
                  char *base, const BackwardPlan &p, hipStream_t stream) {
+  if (gemm_small_applies(K, M, N, kSmallGradWeights))
+    return launch_gemm_small(x, true, dy, true, nullptr, dW, K, M, N, accumulate, stream);
   int rc = launch_split_digits_columns(x, K, base + p.a_planes_off, M, K, false, stream);
   if (rc)
     return rc;
@@ -101,6 +103,8 @@ int grad_weights(const float *x, const float *dy, float *dW, int64_t M, int64_t 
 // row-scaled (rows m of dy', rows k of W, contraction over n)
 int grad_input_planes(const float *dyp, const float *W, float *dx, int64_t M, int64_t K, int64_t N, bool accumulate,
                       char *base, const BackwardPlan &p, hipStream_t stream) {
+  if (gemm_small_applies(M, N, K, kSmallGradInput))
+    return launch_gemm_small(dyp, false, W, false, nullptr, dx, M, N, K, accumulate, stream);
   int rc = nbla_hip_split_digits_f32(dyp, N, base + p.a_planes_off, M, N, stream);
   if (rc)
     return rc;
@@ -247,6 +251,8 @@ int nbla_hip_affine_digits_f32(const float *x, const float *W, const float *bias
   // a handful of rows: one fp32 pass over W instead of its conversion to digit operands
   if (affine_few_rows_applies(x, W, y, M, K, N) && workspace_bytes >= affine_few_rows_workspace_bytes(M, K, N))
     return launch_affine_few_rows(x, W, bias, y, M, K, N, workspace, workspace_bytes, stream);
+  if (gemm_small_applies(M, K, N, kSmallForward))
+    return launch_gemm_small(x, false, W, true, bias, y, M, K, N, false, stream);
   char *xd = static_cast<char *>(workspace);
   char *wd = xd + round_up(nbla_hip_digit_operand_bytes(M, K), 256);
   rc = nbla_hip_split_digits_f32(x, K, xd, M, K, stream_);

@@ -776,10 +776,11 @@ int nbla_hip_inq_affine_f32(const float *x, float *W, int32_t *I, float *old_W, 
   // integer in one digit and three exact digit products give the result; otherwise six (weights still being learnt).
   // The weight update's last pass gathers the column statistics of that operand on the way.
   bool cols_done = false;
+  const bool small = gemm_small_applies(M, K, N, kSmallForward); // neither needs an operand nor its statistics
   if (step >= 0) {
     const ColumnScratch cols = column_scratch(base + p.planes_off, K, N);
     rc = update_weights(W, I, old_W, old_I, K * N, num_bits, step, draw, draw_ctx, nullptr, base + p.update_off,
-                        p.split_off - p.update_off, stream, &cols, N, &cols_done);
+                        p.split_off - p.update_off, stream, small ? nullptr : &cols, N, &cols_done);
     if (rc)
       return rc;
   } else {
@@ -792,6 +793,8 @@ int nbla_hip_inq_affine_f32(const float *x, float *W, int32_t *I, float *old_W, 
   if (affine_few_rows_applies(x, W, y, M, K, N) &&
       p.flag_off - p.split_off >= affine_few_rows_workspace_bytes(M, K, N))
     return launch_affine_few_rows(x, W, bias, y, M, K, N, base + p.split_off, p.flag_off - p.split_off, stream);
+  if (small)
+    return launch_gemm_small(x, false, W, true, bias, y, M, K, N, false, stream);
   rc = nbla_hip_split_digits_f32(x, K, base + p.split_off, M, K, stream_);
   if (rc)
     return rc;
