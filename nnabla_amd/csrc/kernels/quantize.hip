@@ -25,6 +25,19 @@ __device__ __forceinline__ float4_t load4(const float *p) { return *reinterpret_
 __device__ __forceinline__ void store4(float *p, float4_t v) {
   __builtin_nontemporal_store(v, reinterpret_cast<float4_t *>(p));
 }
+typedef float float4_u __attribute__((ext_vector_type(4), aligned(4)));
+// the same at any multiple of four bytes; the store goes through the caches, which put its partial lines together
+template <bool kAligned> __device__ __forceinline__ float4_t load4_as(const float *p) {
+  if (kAligned)
+    return load4(p);
+  return *reinterpret_cast<const float4_u *>(p);
+}
+template <bool kAligned> __device__ __forceinline__ void store4_as(float *p, float4_t v) {
+  if (kAligned)
+    store4(p, v);
+  else
+    *reinterpret_cast<float4_u *>(p) = v;
+}
 
 // Generic driver: applies `op` (a functor float -> float) to `size` elements.
 // The vector body covers size/4 float4s; the tail (size % 4) is done by block 0.
@@ -700,24 +713,43 @@ __global__ __launch_bounds__(kBlock) void minmax_apply_flat(const float *__restr
   }
 }
 
-// Stage 3b: per-channel rows of R1 contiguous elements (R1 % 4 == 0, aligned):
-// blockIdx.x = row (r0 * K + k), blockIdx.y = tile along the row.
-__global__ __launch_bounds__(kBlock) void minmax_apply_rows(const float *__restrict__ x, float *__restrict__ y, int64_t K,
-                                                            int64_t R1, const float4_t *__restrict__ params) {
-  const int64_t row = blockIdx.x;
+// Stage 3b: per-channel rows of R1 contiguous elements.  kLanes == kBlock: blockIdx.x = row (r0 * K + k), blockIdx.y =
+// tile along the row; kLanes == 64: a wavefront per row, four rows to a block.  kAligned: R1 % 4 == 0 and 16-byte
+// aligned; otherwise 128-bit accesses at any multiple of four bytes, the row's last R1 % 4 elements by themselves
+// (element by element [64,256,27,27] took 27 us, this way 19).
+template <int kLanes, bool kAligned>
+__global__ __launch_bounds__(kBlock) void minmax_apply_rows(const float *__restrict__ x, float *__restrict__ y, int64_t rows,
+                                                            int64_t K, int64_t R1, const float4_t *__restrict__ params) {
+  const int lane = threadIdx.x & (kLanes - 1);
+  const int64_t row =
+      (int64_t)blockIdx.x * (kBlock / kLanes) + __builtin_amdgcn_readfirstlane((int)threadIdx.x / kLanes);
+  if (row >= rows)
+    return;
   const float4_t pr = params[row % K];
   const int64_t n4 = R1 / 4;
   const float *xr = x + row * R1;
   float *yr = y + row * R1;
-  for (int64_t i = (int64_t)blockIdx.y * kBlock + threadIdx.x; i < n4; i += (int64_t)gridDim.y * kBlock) {
-    const float4_t v = load4(xr + 4 * i);
-    float4_t r;
-    r.x = minmax_apply(v.x, pr.x, pr.y, pr.z);
-    r.y = minmax_apply(v.y, pr.x, pr.y, pr.z);
-    r.z = minmax_apply(v.z, pr.x, pr.y, pr.z);
-    r.w = minmax_apply(v.w, pr.x, pr.y, pr.z);
-    store4(yr + 4 * i, r);
+  const int64_t step = (int64_t)gridDim.y * kLanes;
+  for (int64_t i0 = (int64_t)blockIdx.y * kLanes + lane; i0 < n4; i0 += 4 * step) {
+    float4_t v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (i0 + j * step < n4)
+        v[j] = load4_as<kAligned>(xr + 4 * (i0 + j * step));
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (i0 + j * step < n4) {
+        float4_t r;
+        r.x = minmax_apply(v[j].x, pr.x, pr.y, pr.z);
+        r.y = minmax_apply(v[j].y, pr.x, pr.y, pr.z);
+        r.z = minmax_apply(v[j].z, pr.x, pr.y, pr.z);
+        r.w = minmax_apply(v[j].w, pr.x, pr.y, pr.z);
+        store4_as<kAligned>(yr + 4 * (i0 + j * step), r);
+      }
+    }
   }
+  if (!kAligned && blockIdx.y == 0 && 4 * n4 + lane < R1)
+    yr[4 * n4 + lane] = minmax_apply(xr[4 * n4 + lane], pr.x, pr.y, pr.z);
 }
 
 // Stage 3c: any layout / alignment, one element per step.
@@ -1132,12 +1164,24 @@ int min_max_quantize_forward(const float *x, float *y, const int64_t *xshape, in
     const size_t blocks = n4 ? (n4 + kTile - 1) / kTile : 1;
     hipLaunchKernelGGL(minmax_apply_flat, dim3((unsigned)blocks), dim3(kBlock), 0, stream, x, y, n4, (size_t)L.total,
                        params);
-  } else if (aligned16(x) && aligned16(y) && L.R1 % 4 == 0 && L.R1 >= 256 && L.R0 * L.K < 0x7fffffffll) {
+  } else if (L.R1 >= 256 && L.R0 * L.K < 0x7fffffffll && (L.K > 1 || (aligned16(x) && aligned16(y) && L.R1 % 4 == 0))) {
+    const bool quads = aligned16(x) && aligned16(y) && L.R1 % 4 == 0, waves = L.R1 < kWaveRowsBelow;
+    const int64_t rows = L.R0 * L.K;
     int64_t ytiles = (L.R1 / 4 + kBlock - 1) / kBlock;
     if (ytiles > 64)
       ytiles = 64;
-    hipLaunchKernelGGL(minmax_apply_rows, dim3((unsigned)(L.R0 * L.K), (unsigned)ytiles), dim3(kBlock), 0, stream, x,
-                       y, L.K, L.R1, params);
+    const dim3 grid((unsigned)(waves ? (rows + 3) / 4 : rows), (unsigned)(waves ? 1 : ytiles));
+#define NBLA_APPLY_ROWS(W, A)                                                                                          \
+  hipLaunchKernelGGL((minmax_apply_rows<W, A>), grid, dim3(kBlock), 0, stream, x, y, rows, L.K, L.R1, params)
+    if (waves && quads)
+      NBLA_APPLY_ROWS(64, true);
+    else if (waves)
+      NBLA_APPLY_ROWS(64, false);
+    else if (quads)
+      NBLA_APPLY_ROWS(kBlock, true);
+    else
+      NBLA_APPLY_ROWS(kBlock, false);
+#undef NBLA_APPLY_ROWS
   } else {
     int64_t blocks = (L.total + kBlock - 1) / kBlock;
     if (blocks > 65536)

@@ -17,6 +17,19 @@ __device__ __forceinline__ float4_t load4(const float *p) { return *reinterpret_
 __device__ __forceinline__ void store4(float *p, float4_t v) {
   __builtin_nontemporal_store(v, reinterpret_cast<float4_t *>(p));
 }
+typedef float float4_u __attribute__((ext_vector_type(4), aligned(4)));
+// the same at any multiple of four bytes; the store goes through the caches, which put its partial lines together
+template <bool kAligned> __device__ __forceinline__ float4_t load4_as(const float *p) {
+  if (kAligned)
+    return load4(p);
+  return *reinterpret_cast<const float4_u *>(p);
+}
+template <bool kAligned> __device__ __forceinline__ void store4_as(float *p, float4_t v) {
+  if (kAligned)
+    store4(p, v);
+  else
+    *reinterpret_cast<float4_u *>(p) = v;
+}
 
 // dx[i] = op(dy[i], x[i], i) (+ dx[i] when kAccum).  `op` returns the gradient contribution; kUseX tells whether x is
 // read at all.
@@ -328,7 +341,9 @@ struct RangeInputs {
 };
 
 // kN float4s per thread, all loads issued before the first store (the compiler does not move a load across a store)
-template <int kN>
+// kAligned: 16-byte aligned addresses; otherwise 4-byte aligned ones (the same 128-bit accesses, which may straddle
+// cache lines)
+template <int kN, bool kAligned = true>
 __device__ __forceinline__ void minmax_grad4(const float *__restrict__ dy, const float *__restrict__ x,
                                              float *__restrict__ dx, const int64_t (&at)[kN], const bool (&in)[kN],
                                              const float2 &b, const GradMode &m, float &lo, float &hi) {
@@ -336,9 +351,9 @@ __device__ __forceinline__ void minmax_grad4(const float *__restrict__ dy, const
   float4_t g[kN], v[kN], o[kN];
 #pragma unroll
   for (int j = 0; j < kN; ++j) {
-    g[j] = in[j] ? load4(dy + at[j]) : zero;
-    v[j] = (in[j] && (m.dx_mode == 2 || m.sums)) ? load4(x + at[j]) : zero;
-    o[j] = (in[j] && m.dx_mode && m.accum) ? load4(dx + at[j]) : zero;
+    g[j] = in[j] ? load4_as<kAligned>(dy + at[j]) : zero;
+    v[j] = (in[j] && (m.dx_mode == 2 || m.sums)) ? load4_as<kAligned>(x + at[j]) : zero;
+    o[j] = (in[j] && m.dx_mode && m.accum) ? load4_as<kAligned>(dx + at[j]) : zero;
   }
 #pragma unroll
   for (int j = 0; j < kN; ++j) {
@@ -348,7 +363,7 @@ __device__ __forceinline__ void minmax_grad4(const float *__restrict__ dy, const
       float4_t r;
       r.x = minmax_dx(g[j].x, v[j].x, o[j].x, b, m), r.y = minmax_dx(g[j].y, v[j].y, o[j].y, b, m);
       r.z = minmax_dx(g[j].z, v[j].z, o[j].z, b, m), r.w = minmax_dx(g[j].w, v[j].w, o[j].w, b, m);
-      store4(dx + at[j], r);
+      store4_as<kAligned>(dx + at[j], r);
     }
     if (m.sums) {
       minmax_sums(g[j].x, v[j].x, b, lo, hi), minmax_sums(g[j].y, v[j].y, b, lo, hi);
@@ -389,28 +404,59 @@ __global__ __launch_bounds__(kBlock) void minmax_grad_flat(const float *__restri
     block_sums(lo, hi, partial + blockIdx.x);
 }
 
-// Ranges per channel, rows of R1 contiguous elements (R1 % 4 == 0, 16-byte aligned): blockIdx.x = row (r0 * K + k),
-// blockIdx.y = part of the row; the sums go to partial[k * nchunks + r0 * gridDim.y + blockIdx.y], nchunks =
-// R0 * gridDim.y.
+// Ranges per channel, rows of R1 contiguous elements, row (r0 * K + k).  kLanes == kBlock: blockIdx.x = row, blockIdx.y =
+// part of the row; kLanes == 64: a wavefront per row, four rows to a block (gridDim.y = 1).  The sums go to
+// partial[k * nchunks + r0 * gridDim.y + blockIdx.y], nchunks = R0 * gridDim.y.  kAligned: R1 % 4 == 0 and 16-byte
+// aligned; otherwise rows start at any multiple of four bytes and up to three elements follow a row's last float4.
+//
+// Bound by memory: dy and x are read once and dx is written.  Rows of odd length went through an element-wise pass for
+// dx and a second one, by scalar loads, for the sums: [64,256,27,27] with both range gradients 28 + 24 us and the
+// bounds' launch 5, now 26.
+template <int kLanes, bool kAligned>
 __global__ __launch_bounds__(kBlock) void minmax_grad_rows(const float *__restrict__ dy, const float *__restrict__ x,
-                                                           float *__restrict__ dx, int64_t K, int64_t R1,
+                                                           float *__restrict__ dx, int64_t rows, int64_t K, int64_t R1,
                                                            RangeInputs q, float2 *__restrict__ partial,
                                                            int64_t nchunks, GradMode m) {
-  const int64_t row = blockIdx.x, r0 = row / K, k = row - r0 * K;
+  const int lane = threadIdx.x & (kLanes - 1);
+  const int64_t row =
+      (int64_t)blockIdx.x * (kBlock / kLanes) + __builtin_amdgcn_readfirstlane((int)threadIdx.x / kLanes);
+  if (kLanes == 64 && row >= rows) // (no barrier follows in that form)
+    return;
+  const int64_t r0 = row / K, k = row - r0 * K;
   const float2 b = q.bounds(k);
   const int64_t n4 = R1 / 4, at0 = row * R1;
   float lo = 0.0f, hi = 0.0f;
-  const int64_t step = (int64_t)gridDim.y * kBlock;
-  for (int64_t i0 = (int64_t)blockIdx.y * kBlock + threadIdx.x; i0 < n4; i0 += 4 * step) {
+  const int64_t step = (int64_t)gridDim.y * kLanes;
+  for (int64_t i0 = (int64_t)blockIdx.y * kLanes + lane; i0 < n4; i0 += 4 * step) {
     int64_t at[4];
     bool in[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       in[j] = i0 + j * step < n4, at[j] = at0 + 4 * (i0 + j * step);
-    minmax_grad4<4>(dy, x, dx, at, in, b, m, lo, hi);
+    minmax_grad4<4, kAligned>(dy, x, dx, at, in, b, m, lo, hi);
   }
-  if (m.sums)
-    block_sums(lo, hi, partial + k * nchunks + r0 * gridDim.y + blockIdx.y);
+  if (!kAligned && blockIdx.y == 0 && 4 * n4 + lane < R1) {
+    const int64_t i = at0 + 4 * n4 + lane;
+    const float g = dy[i], xv = x[i];
+    if (m.dx_mode)
+      dx[i] = minmax_dx(g, xv, m.accum ? dx[i] : 0.0f, b, m);
+    if (m.sums)
+      minmax_sums(g, xv, b, lo, hi);
+  }
+  if (!m.sums)
+    return;
+  float2 *dst = partial + k * nchunks + r0 * gridDim.y + blockIdx.y;
+  if (kLanes == kBlock) {
+    block_sums(lo, hi, dst);
+    return;
+  }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    lo += __shfl_xor(lo, off);
+    hi += __shfl_xor(hi, off);
+  }
+  if (lane == 0)
+    *dst = float2{lo, hi};
 }
 
 // The inner-kept form (MinMaxInner: lanes along the kept innermost axis), block (ko, chunk) as in the forward's
@@ -620,7 +666,7 @@ struct RangeGradPlan {
   MinMaxRows R;
   int row_form_chunks;
   int64_t flat_chunks;  // K == 1
-  int64_t row_parts;    // rows form (R1 % 4 == 0, R1 >= 256): blocks along a row; partial sums per range = R0 * row_parts
+  int64_t row_parts;    // rows form (R1 >= 256): blocks along a row; partial sums per range = R0 * row_parts
   size_t bounds_bytes, partial_bytes;
 };
 
@@ -667,15 +713,15 @@ RangeGradPlan make_range_plan(const int64_t *xshape, int ndim, const int64_t *qs
     most = most > P.flat_chunks ? most : P.flat_chunks;
   }
   P.row_parts = 0;
-  if (P.L.ok && P.L.K > 1 && P.L.R1 % 4 == 0 && P.L.R1 >= 256 && P.L.R0 * P.L.K <= 0x7fffffffll) {
-    // about 4096 blocks; a block takes at least one float4 per thread
+  if (P.L.ok && P.L.K > 1 && P.L.R1 >= 256 && P.L.R0 * P.L.K <= 0x7fffffffll) {
+    // about 4096 blocks; a block takes at least one float4 per thread (or four rows, one per wavefront)
     int64_t parts = (4096 + P.L.R0 * P.L.K - 1) / (P.L.R0 * P.L.K);
     const int64_t longest = (P.L.R1 / 4 + kBlock - 1) / kBlock;
     if (parts > longest)
       parts = longest;
     if (parts > 64)
       parts = 64;
-    P.row_parts = parts < 1 ? 1 : parts;
+    P.row_parts = parts < 1 || P.L.R1 < kWaveRowsBelow ? 1 : parts;
     most = most > P.L.R0 * P.row_parts ? most : P.L.R0 * P.row_parts;
   }
   P.bounds_bytes = round_up((size_t)P.L.K * sizeof(float2), 256);
@@ -788,7 +834,7 @@ int nbla_hip_min_max_quantize_backward_f32(const float *dy, const float *x, floa
   const GradMode mode{dx ? (ste_fine_grained ? 2 : 1) : 0, accum_x, range_grads ? 1 : 0};
   const bool wanted = range_grads || (mode.dx_mode == 2 && P.L.K > 1);
   const bool vec = aligned16(dy) && aligned16(x) && (!dx || aligned16(dx));
-  const bool one_range_per_block = wanted && !P.inner && !P.rows && vec && (P.flat_chunks || P.row_parts);
+  const bool one_range_per_block = wanted && !P.inner && !P.rows && ((P.flat_chunks && vec) || P.row_parts);
   if (((dx && ste_fine_grained) || range_grads) && !one_range_per_block) {
     hipLaunchKernelGGL(minmax_bounds, dim3((unsigned)((P.L.K + 63) / 64)), dim3(64), 0, stream, qr_min, ql_min, ql_max,
                        scale, bounds, P.L.K);
@@ -843,10 +889,22 @@ int nbla_hip_min_max_quantize_backward_f32(const float *dy, const float *x, floa
     NBLA_HIP_LAUNCH_CHECK("min_max_quantize backward range gradients");
     return NBLA_HIP_OK;
   }
-  if (wanted && P.row_parts && vec) {
-    const int64_t chunks = P.L.R0 * P.row_parts;
-    hipLaunchKernelGGL(minmax_grad_rows, dim3((unsigned)(P.L.R0 * P.L.K), (unsigned)P.row_parts), dim3(kBlock), 0,
-                       stream, dy, x, dx, P.L.K, P.L.R1, ranges, partial, chunks, mode);
+  if (wanted && P.row_parts) {
+    const int64_t chunks = P.L.R0 * P.row_parts, rows = P.L.R0 * P.L.K;
+    const bool quads = vec && P.L.R1 % 4 == 0, waves = P.L.R1 < kWaveRowsBelow;
+    const dim3 grid((unsigned)(waves ? (rows + 3) / 4 : rows), (unsigned)P.row_parts);
+#define NBLA_GRAD_ROWS(W, A)                                                                                           \
+  hipLaunchKernelGGL((minmax_grad_rows<W, A>), grid, dim3(kBlock), 0, stream, dy, x, dx, rows, P.L.K, P.L.R1, ranges,  \
+                     partial, chunks, mode)
+    if (waves && quads)
+      NBLA_GRAD_ROWS(64, true);
+    else if (waves)
+      NBLA_GRAD_ROWS(64, false);
+    else if (quads)
+      NBLA_GRAD_ROWS(kBlock, true);
+    else
+      NBLA_GRAD_ROWS(kBlock, false);
+#undef NBLA_GRAD_ROWS
     NBLA_HIP_LAUNCH_CHECK("min_max_quantize backward");
     if (range_grads) {
       launch_range_final(partial, chunks, g_qr_min, g_qr_max, accum_min, accum_max, P.L.K, stream);

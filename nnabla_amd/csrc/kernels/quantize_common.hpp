@@ -218,6 +218,9 @@ inline int64_t row_chunks(const MinMaxRows &R) {
   return want < 1 ? 1 : want;
 }
 // Short runs per channel (q shape (1, C, 1, 1) over rows of fewer than 256 elements) take this form as well.
+// Below this many elements a wavefront takes a whole row in at most eight 128-bit accesses per lane; a block per row
+// would leave a quarter of its lanes idle at 27 x 27 and have one access in flight per lane.
+constexpr int64_t kWaveRowsBelow = 2048;
 inline bool short_rows(const MinMaxLayout &L) { return L.ok && L.K > 1 && L.R1 > 1 && L.R1 < 256; }
 struct RowWalk {
   int64_t ro_begin, ro_end;
