@@ -146,7 +146,7 @@ __global__ __launch_bounds__(256) void col2im_gather_unit(const float *__restric
 
 struct ConvBackwardPlan {
   size_t dyt_off, col_off, a_planes_off, b_planes_off, digits_off, bits_off, prep_off, count_off,
-      flag_off, sums_off, slab_off, dw_off, total;
+      flag_off, sums_off, slab_off, dw_off, real_off, total;
 };
 
 size_t larger(size_t a, size_t b) { return a > b ? a : b; }
@@ -184,6 +184,8 @@ ConvBackwardPlan plan_conv_backward(const ConvGeom &g) {
   }
   p.dw_off = off; // maxima, scales and partial results of the weight gradient on the fp16 matrix cores
   off += round_up(conv_dw_workspace_bytes(g), 256);
+  p.real_off = off; // prepared weights of the input gradient on the bf16 matrix cores
+  off += round_up(conv_real_workspace_bytes(g, true), 256);
   p.total = off;
   return p;
 }
@@ -281,6 +283,16 @@ int conv_backward(const float *dy, const float *x, const float *W, const float *
         return rc;
     }
     dW = nullptr;
+  }
+  if (dx && !dx_slab && conv_real_applies(g, true, binary) && (!binary || Wb || representable)) { // no unfolded gradient
+    for (int64_t grp = 0; grp < g.group; ++grp) {
+      rc = launch_conv_real(dy, ((binary && Wb) ? Wb : W) + grp * g.Og * g.Kg, nullptr, dx, g, true, grp, accum_x,
+                            binary && alpha ? alpha + grp * g.Og : nullptr, binary && !Wb, zero_to, base + p.real_off,
+                            conv_real_workspace_bytes(g, true), stream);
+      if (rc)
+        return rc;
+    }
+    dx = nullptr;
   }
   for (int64_t grp = 0; grp < g.group && (dx || dW); ++grp) {
     const float *Wg = W + grp * g.Og * g.Kg;

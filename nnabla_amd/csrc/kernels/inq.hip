@@ -732,7 +732,9 @@ size_t conv_channel_max_bytes(const ConvGeom &g) {
   return round_up((size_t)16 * g.outer * g.in_sp_size * sizeof(uint32_t), 256);
 }
 size_t conv_product_extra(const ConvGeom &g) {
-  return conv_channel_max_bytes(g) + gemm_digits_split_bytes(g.M, g.Kg, g.Og);
+  const size_t digits = conv_channel_max_bytes(g) + gemm_digits_split_bytes(g.M, g.Kg, g.Og);
+  const size_t real = conv_real_workspace_bytes(g, false); // (the prepared weights of the other form)
+  return digits > real ? digits : real;
 }
 
 } // namespace
@@ -848,6 +850,15 @@ int nbla_hip_inq_convolution_f32(const float *x, float *W, int32_t *I, float *ol
   }
   if (conv_direct_forward_applies(g)) // many small groups: all of them in one fp32 launch
     return launch_conv_direct_forward(x, W, nullptr, bias, y, g, stream);
+  if (conv_real_applies(g, false, false)) { // two dimensions, no dilation: no unfolded matrix
+    for (int64_t grp = 0; grp < g.group; ++grp) {
+      rc = launch_conv_real(x, W + grp * g.Og * g.Kg, bias ? bias + grp * g.Og : nullptr, y, g, false, grp, false, nullptr,
+                            false, 0.0f, base + p.extra_off, conv_product_extra(g), stream);
+      if (rc)
+        return rc;
+    }
+    return NBLA_HIP_OK;
+  }
   // The product runs on the int8 digit kernels: the unfolded input goes straight into a row-scaled digit operand
   // (rows = output positions), the weights [Og, Kg] into another (rows = output channels); six exact digit products.
   const int64_t hw = g.out_sp_size;

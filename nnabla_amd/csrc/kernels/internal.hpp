@@ -78,6 +78,14 @@ int launch_conv_direct_backward(const float *dy, const float *x, const float *w,
                                 float *dW, float *db, const ConvGeom &g, bool accum_x, bool accum_w, bool accum_b,
                                 bool take_sign, float zero_to, float *scratch, size_t scratch_bytes,
                                 hipStream_t stream);
+// Two-dimensional convolution of real-valued weights on the bf16 matrix cores (conv_real.hip), group `grp` of the whole
+// tensors: the forward, or (transposed) the input gradient, dx (+)= from dy.  W: the group's weights, alpha (may be null)
+// scales them per output channel; signs: Sign(W) stands for them.  bias: the group's, forward only.
+bool conv_real_applies(const ConvGeom &g, bool transposed, bool binary); // and is the faster form
+size_t conv_real_workspace_bytes(const ConvGeom &g, bool transposed);
+int launch_conv_real(const float *in, const float *W, const float *bias, float *out, const ConvGeom &g, bool transposed,
+                     int64_t grp, bool accumulate, const float *alpha, bool signs, float zero_to, void *workspace,
+                     size_t workspace_bytes, hipStream_t stream);
 // The weight gradient of one group on the fp16 matrix cores without an unfolded matrix (conv_dw.hip): dW (+)= the sum
 // over positions of dy x, for two-dimensional kernels of width 1, 3 or 5 padded by half their width, strides 1 and 2.
 // x, dy and dW are the whole tensors; workspace: conv_dw_workspace_bytes(g), 256-byte aligned.
