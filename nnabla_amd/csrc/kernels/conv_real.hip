@@ -87,14 +87,18 @@ __device__ __forceinline__ void split3_pair(float a, float b, uint32_t &hi, uint
   lo = __builtin_amdgcn_perm(l[1], l[0], 0x07060302u);
 }
 
-__device__ __forceinline__ float real_weight(const float *w, int64_t at, int64_t k, const float *alpha, int signs,
-                                             float zero_to) {
-  float v = w[at];
+// A weight as it takes part: itself or its sign, times alpha.
+__device__ __forceinline__ float weight_value(float v, bool scaled, float alpha, int signs, float zero_to) {
   if (signs)
     v = v < 0.0f ? -1.0f : (v > 0.0f ? 1.0f : zero_to);
-  return alpha ? v * alpha[k] : v;
+  return scaled ? v * alpha : v;
+}
+__device__ __forceinline__ float real_weight(const float *w, int64_t at, int64_t k, const float *alpha, int signs,
+                                             float zero_to) {
+  return weight_value(w[at], alpha != nullptr, alpha ? alpha[k] : 1.0f, signs, zero_to);
 }
 
+constexpr int kFlight = 10; // loads of a row a thread has in flight
 // Block = one row r: its largest magnitude, then the three planes in the lanes' order,
 // [tap][16 channels][plane][32 rows][lane (half, row)][8 bf16]; rows and channels past the ends are zeros.
 __global__ __launch_bounds__(kThreads) void conv_real_weights(const float *__restrict__ W, unsigned char *__restrict__ dst,
@@ -106,11 +110,23 @@ __global__ __launch_bounds__(kThreads) void conv_real_weights(const float *__res
   const int r = blockIdx.x, tid = threadIdx.x, n = Kc * taps;
   uint32_t amax = 0u;
   if (r < R)
-    for (int i = tid; i < n; i += kThreads) {
-      const int k = i / taps, t = i - k * taps;
-      const float v = real_weight(W, r * w_row + k * w_k + t, k, alpha, signs, zero_to);
-      s_row[i] = v;
-      amax = max(amax, __float_as_uint(v) & 0x7fffffffu);
+    for (int i0 = tid; i0 < n; i0 += kFlight * kThreads) { // (a load a time is a round trip each: 8.4 us, this way 7.1)
+      float v[kFlight], sc[kFlight];
+#pragma unroll
+      for (int j = 0; j < kFlight; ++j) {
+        const int i = min(i0 + j * kThreads, n - 1), k = i / taps, t = i - k * taps;
+        v[j] = W[r * w_row + k * w_k + t];
+        sc[j] = alpha ? alpha[k] : 1.0f;
+      }
+#pragma unroll
+      for (int j = 0; j < kFlight; ++j) {
+        const int i = i0 + j * kThreads;
+        if (i >= n)
+          break;
+        const float q = weight_value(v[j], alpha != nullptr, sc[j], signs, zero_to);
+        s_row[i] = q;
+        amax = max(amax, __float_as_uint(q) & 0x7fffffffu);
+      }
     }
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1)
