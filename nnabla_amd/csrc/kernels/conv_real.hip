@@ -110,7 +110,7 @@ __global__ __launch_bounds__(kThreads) void conv_real_weights(const float *__res
   const int r = blockIdx.x, tid = threadIdx.x, n = Kc * taps;
   uint32_t amax = 0u;
   if (r < R)
-    for (int i0 = tid; i0 < n; i0 += kFlight * kThreads) { // (a load a time is a round trip each: 8.4 us, this way 7.1)
+    for (int i0 = tid; i0 < n; i0 += kFlight * kThreads) { // (a load a time is a round trip each: 8.4 us, this way 6.2)
       float v[kFlight], sc[kFlight];
 #pragma unroll
       for (int j = 0; j < kFlight; ++j) {
@@ -121,11 +121,11 @@ __global__ __launch_bounds__(kThreads) void conv_real_weights(const float *__res
 #pragma unroll
       for (int j = 0; j < kFlight; ++j) {
         const int i = i0 + j * kThreads;
-        if (i >= n)
-          break;
         const float q = weight_value(v[j], alpha != nullptr, sc[j], signs, zero_to);
-        s_row[i] = q;
-        amax = max(amax, __float_as_uint(q) & 0x7fffffffu);
+        if (i < n) {
+          s_row[i] = q;
+          amax = max(amax, __float_as_uint(q) & 0x7fffffffu);
+        }
       }
     }
 #pragma unroll
