@@ -77,7 +77,7 @@ struct SlabPlan {
   int cap;         // pixels a slab may hold (the zero pixel not counted)
   int slab_bytes;
   int k_tiles;     // taps * ct
-  int pixsum_off, rowsum_off, pixbad_off, rowpix_off, rowidx_off, rowbad_off, alpha_off, misc_off, total;
+  int pixsum_off, pixbad_off, rowpix_off, alpha_off, misc_off, total;
   // the prepared weights of one group: packed bits [k tile][wide group][lane], partial |W| sums [ct][frags * 32],
   // partial zero counts [ct][wide groups * 32]
   size_t bits_bytes, wsum_off, zeros_off, prep_bytes;
@@ -140,10 +140,8 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
   const int in0 = g.in_sp[0], in1 = g.in_sp[1], in2 = g.in_sp[2];
 
   long long *s_pixsum = reinterpret_cast<long long *>(smem + P.pixsum_off);
-  long long *s_rowsum = reinterpret_cast<long long *>(smem + P.rowsum_off);
   uint32_t *s_pixbad = reinterpret_cast<uint32_t *>(smem + P.pixbad_off);
   uint32_t *s_rowpix = reinterpret_cast<uint32_t *>(smem + P.rowpix_off); // [tap][row]: pixel index
-  int *s_rowbad = reinterpret_cast<int *>(smem + P.rowbad_off);
   float *s_alpha = reinterpret_cast<float *>(smem + P.alpha_off), *s_bias = s_alpha + kCols;
   int *s_misc = reinterpret_cast<int *>(smem + P.misc_off); // the wavefronts' maxima
 
@@ -302,11 +300,8 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
     s_pixsum[i] = 0;
     s_pixbad[i] = 0u;
   }
-  if (tid < kRows) {
-    s_rowsum[tid] = 0;
-    s_rowbad[tid] = 0;
+  if (tid < kRows)
     s_rowpix[taps * kRows + tid] = 0u; // the entry of steps past the last k tile: the zero pixel
-  }
   for (int i = tid; i < (P.pix_stride >> 2); i += kThreads) // the zero pixel
     *reinterpret_cast<uint32_t *>(smem + 4 * i) = 0u;
   const int trow = tid & (kRows - 1);
@@ -397,21 +392,6 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
       *a.zero_count = z;
   }
   __syncthreads();
-  // the windows' sums of q and whether they hold a non-finite value (read again only after the product)
-  auto sum_windows = [&]() __attribute__((always_inline)) {
-    long long sum = 0;
-    uint32_t bad = 0u;
-    for (int t = tid / kRows; t < taps; t += kThreads / kRows) {
-      const uint32_t idx = s_rowpix[t * kRows + trow];
-      sum += s_pixsum[idx];
-      bad |= s_pixbad[idx];
-    }
-    if (sum != 0)
-      atomicAdd(reinterpret_cast<unsigned long long *>(&s_rowsum[trow]), (unsigned long long)sum);
-    if (bad)
-      s_rowbad[trow] = 1;
-  };
-
   // ---- 2. the product.  Wavefront (wn, wm, wk): channel fragments 2 wn, 2 wn + 1 of the block's, window fragment wm,
   // k tiles wk, wk + WK, ...
   const int wn = wave % WN, wk = wave / (WN * WM);
@@ -437,8 +417,6 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
       convert_chunk();
       __syncthreads();
     }
-    if (chunk == chunks - 1)
-      sum_windows();
     const int ctn = kChunked ? groups16 >> 1 : CT; // channel tiles of the chunk
     const int nk = (taps * ctn - wk + WK - 1) / WK;
     if (nk <= 0)
@@ -574,6 +552,25 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
     }
   }
 
+  // The sum of q over the lane's window and whether it holds a non-finite value: every wavefront adds up the windows it
+  // finishes from the pixels' sums, which are complete since the barrier in front of the (last) product; its lanes
+  // l and l + 32 share a window and take every second tap each, five reads in flight at a time.
+  long long rowsum = 0;
+  uint32_t rowmark = 0u;
+  for (int t0 = half; t0 < taps; t0 += 10) {
+    uint32_t idx[5];
+#pragma unroll
+    for (int j = 0; j < 5; ++j) // (past the last tap: the zero pixel)
+      idx[j] = t0 + 2 * j < taps ? s_rowpix[(t0 + 2 * j) * kRows + row] : 0u;
+#pragma unroll
+    for (int j = 0; j < 5; ++j) {
+      rowsum += s_pixsum[idx[j]];
+      rowmark |= s_pixbad[idx[j]];
+    }
+  }
+  rowsum += __shfl_xor(rowsum, 32);
+  rowmark |= (uint32_t)__shfl_xor((int)rowmark, 32);
+
   // ---- 4. epilogue.  Accumulator register q of lane l: channel 8 (q / 4) + 4 (l / 32) + q % 4 of the fragment,
   // window l % 32.  dot = rowsum - 2 * sum(q * bit); the accumulators carry the factor 2^F of the fragment's byte
   // (-128 for F = 7).  With m_d = acc_d / 2^F:  sum(q * bit) = hi * 2^16 + lo, hi = m_0 * 256 + m_1,
@@ -582,8 +579,7 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
   // while |A| < 2^24 (sums below 2^40), else twice (2^-24 of the sum).
   if (!row_in)
     return;
-  const long long rowsum = s_rowsum[row];
-  const bool rowbad = s_rowbad[row] != 0;
+  const bool rowbad = rowmark != 0u;
   const int s_hi = (int)(rowsum >> 16), s_lo = (int)(rowsum & 0xffff);
   const int osz = (int)g.out_sp_size;
 #pragma unroll
@@ -917,11 +913,9 @@ bool compute_slab_form(const ConvGeom &g, int form, int chunks, SlabPlan &p) {
     off = 2 * waves * kSlabReduceBytes;
   off = (int64_t)round_up((size_t)off, 16);
   p.pixsum_off = (int)off, off += 8 * (cap + 1);
-  p.rowsum_off = (int)off, off += 8 * rows;
   off = (int64_t)round_up((size_t)off, 16);
   p.pixbad_off = (int)off, off += 4 * (cap + 1);
   p.rowpix_off = (int)off, off += 4 * rows * (g.k_size + 1);
-  p.rowbad_off = (int)off, off += 4 * rows;
   p.alpha_off = (int)off, off += 2 * 4 * 64 * f.wn;
   p.misc_off = (int)off, off += 64;
   p.total = (int)off;

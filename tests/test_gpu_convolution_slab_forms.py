@@ -64,3 +64,30 @@ def test_forward_and_input_gradient_against_float64(xs, O, k, pad, stride, group
     else:  # unfolded: three digits, 2^-23 of a row's largest; every tap's product and every addition rounded to fp32
         bound = bound + K * most * (2.0 ** -23 + 2 * taps * 2.0 ** -24)
     assert bool(((dx.cpu().double() - want).abs() <= bound).all())
+
+
+# contractions of one or two k tiles: hardly anything lies between a block's conversion of its inputs and its epilogue
+SHORT = [((64, 16, 28, 28), 64, 1), ((64, 32, 28, 28), 64, 1), ((32, 32, 28, 28), 128, 1), ((32, 32, 28, 28), 256, 1),
+         ((64, 64, 14, 14), 64, 1), ((64, 32, 27, 27), 33, 1), ((64, 32, 14, 14), 64, 3)]
+
+
+@pytest.mark.parametrize("xs,O,k", SHORT)
+def test_short_contractions(xs, O, k):
+    """The windows' sums and their marks of a value that is not finite come from what other wavefronts converted: exact
+    results (whole numbers times Sign(W)) in every one of several runs, and one marked window in each run of 32."""
+    rng = np.random.RandomState(3)
+    kernels.init(0)
+    x = torch.from_numpy(rng.randint(-99, 100, xs).astype(np.float32))
+    W = torch.from_numpy(rng.randn(O, xs[1], k, k).astype(np.float32))
+    s64 = torch.where(W < 0, -1.0, 1.0).double()
+    y64 = torch.nn.functional.conv2d(x.double(), s64, None, 1, k // 2)
+    xd, Wd = x.cuda(), W.cuda()
+    geo = ((k // 2,) * 2, (1, 1), (1, 1), 1)
+    for _ in range(5):
+        assert torch.equal(kernels.binary_connect_convolution(xd, Wd, None, *geo)[0].cpu().double(), y64)
+    xn = x.flatten(2).clone()
+    xn[:, 0, 5::32] = float("nan")
+    y64 = torch.nn.functional.conv2d(xn.view(xs).double(), s64, None, 1, k // 2)
+    for _ in range(5):
+        y = kernels.binary_connect_convolution(xn.view(xs).cuda(), Wd, None, *geo)[0].cpu().double()
+        assert torch.equal(y.isnan(), y64.isnan()) and torch.equal(y.nan_to_num(), y64.nan_to_num())
