@@ -5,7 +5,7 @@
 // A block owns up to 32 WM consecutive output positions of one sample and 64 WN output channels.  Every input position
 // ("pixel") that one of its windows touches lies in one run [lo, hi] of the flattened input map; the block reads that
 // run of all the group's channels once (coalesced along the positions), turns every value into four balanced
-// base-256 int8 digits under ONE power-of-two scale for the whole slab, and keeps the digits in LDS pixel by pixel:
+// base-256 int8 digits under one power-of-two scale for the whole slab, and keeps the digits in LDS pixel by pixel:
 //     slab[pixel 0..npix][channel tile of 32][digit 0..3][32 channels]   (pixel 0 is all zeros: the taps that fall
 //                                                                         outside the input)
 // The contraction runs over k' = (tap, channel) instead of the reference's (channel, tap): exact integer sums do not
@@ -36,14 +36,21 @@
 // Numerics: q = rint(x * 2^s) with s chosen so that the slab's largest finite magnitude lands in [2^29, 2^30); the
 // four digit products are accumulated exactly in int32, combined exactly in integers with the windows' sums of q
 // (the bits stand for 0 / 1: sum q * (1 - 2 b) = sum q - 2 sum q b) and rounded once to fp32.  The only error is
-// the rounding of x to a multiple of 2^-s: at most 2^-30 of the slab's largest magnitude per element, i.e. finer than
-// fp32 itself for every window whose own largest value is within 2^-6 of the slab's.  A window that holds a NaN or an
+// the rounding of x to a multiple of 2^-s: at most 2^-30 of the slab's largest magnitude per element.  Windows whose own
+// largest value is more than kSlabLevel binades below that are finished by further rounds of the block, each under the
+// scale of the largest of the windows left: so an element is off by at most 2^-27 of the largest value of its own window,
+// whatever else lies in the slab.  (On inputs of one magnitude no block has a second round, and the window maxima, the test
+// for windows left and the second copy of the product cost 2 to 4 %: [32,64,56,56] x [64,64,3,3] 47.7 -> 49.1 us with the
+// host's call, [32,256,14,14] x [256,256,3,3] 29.3 -> 29.9.  One loop around a single copy of the product costs 8 to 11 %:
+// the loop's values crowd the product's registers.)  A window that holds a NaN or an
 // infinity gives NaN in all its outputs; other windows of the slab are not affected (such values are left out of the
 // scale and read as 0).
 #include "common.hpp"
 #include "conv_geom.hpp"
 #include "gemm_layout.hpp"
 #include "internal.hpp"
+
+#include <type_traits>
 
 namespace nbla_hip {
 namespace {
@@ -58,6 +65,7 @@ constexpr int kSlabPixPad = 16;      // bytes between two pixels: consecutive pi
 constexpr int kSlabMaxTaps = 64;
 constexpr int kSlabAhead = 8;        // k tiles of packed words a wavefront holds in registers ahead of its MFMAs
 constexpr int kSlabTopBit = 29;      // the slab's largest magnitude lands in [2^29, 2^30): two q add up in 32 bits
+constexpr int kSlabLevel = 3;        // windows smaller by more binades than this take a scale of their own
 constexpr int kSlabReduceBytes = 16 * 64 * 4; // per wavefront: one fragment of one digit's accumulators
 constexpr int kSlabHold = 4;         // work items of the set-up a wavefront keeps in registers between its two steps
 constexpr int kSlabLdsLimit = 156 * 1024;
@@ -77,7 +85,7 @@ struct SlabPlan {
   int cap;         // pixels a slab may hold (the zero pixel not counted)
   int slab_bytes;
   int k_tiles;     // taps * ct
-  int pixsum_off, pixbad_off, rowpix_off, alpha_off, misc_off, total;
+  int pixsum_off, pixmax_off, rowpix_off, alpha_off, misc_off, total;
   // the prepared weights of one group: packed bits [k tile][wide group][lane], partial |W| sums [ct][frags * 32],
   // partial zero counts [ct][wide groups * 32]
   size_t bits_bytes, wsum_off, zeros_off, prep_bytes;
@@ -125,7 +133,7 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const ConvGeom &g = a.g;
   const SlabPlan &P = a.p;
-  const int tid = threadIdx.x, lane = tid & 63;
+  int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // Blocks go to the eight XCDs round-robin: an XCD takes a contiguous run of tiles, so the tiles of one sample --
   // whose slabs overlap and whose outputs share cache lines -- meet in one L2.
@@ -140,15 +148,15 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
   const int in0 = g.in_sp[0], in1 = g.in_sp[1], in2 = g.in_sp[2];
 
   long long *s_pixsum = reinterpret_cast<long long *>(smem + P.pixsum_off);
-  uint32_t *s_pixbad = reinterpret_cast<uint32_t *>(smem + P.pixbad_off);
+  uint32_t *s_pixmax = reinterpret_cast<uint32_t *>(smem + P.pixmax_off); // largest magnitude, as bits
   uint32_t *s_rowpix = reinterpret_cast<uint32_t *>(smem + P.rowpix_off); // [tap][row]: pixel index
   float *s_alpha = reinterpret_cast<float *>(smem + P.alpha_off), *s_bias = s_alpha + kCols;
-  int *s_misc = reinterpret_cast<int *>(smem + P.misc_off); // the wavefronts' maxima
+  int *s_misc = reinterpret_cast<int *>(smem + P.misc_off); // the wavefronts' maxima, of the slab and of windows left
 
   // ---- 0. the block's rows and the slab's extent.  Every wavefront walks all the rows (64 lanes at a time), so each
   // finds the extent by itself and can start loading the slab before anything goes through LDS.
-  const int r = lane & 31, half = lane >> 5;
-  const int wm = (wave / WN) % WM, row = wm * kSlabRows + r; // the window of this lane in the product
+  int half = lane >> 5;
+  int row = (wave / WN) % WM * kSlabRows + (lane & 31); // the window of this lane in the product
   const bool row_in = row < rows;
   auto decode = [&](int m, int &b0, int &b1, int &b2) __attribute__((always_inline)) {
     int p = m < rows ? p0 + m : p0; // rows past the tile repeat its first row
@@ -229,20 +237,21 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
     }
   };
   int shift = 0;
+  uint32_t limit = 0u; // magnitudes above it (non-finite ones always) are converted to zeros
   // the item's digits -> LDS: sixteen consecutive channels of a pixel are sixteen consecutive bytes of each digit
   auto convert_item = [&](int item, const float (&v)[16]) __attribute__((always_inline)) {
     uint32_t w[kSlabDigits][4];
     long long psum = 0;
-    bool bad = false;
+    uint32_t pmax = 0u;
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       uint32_t d[4];
       int part[2] = {0, 0}; // two |q| < 2^30 each
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        const bool fin = (__float_as_uint(v[4 * u + c]) & 0x7fffffffu) < 0x7f800000u;
-        bad = bad || !fin;
-        const int q = fin ? (int)rintf(ldexpf(v[4 * u + c], shift)) : 0;
+        const uint32_t m = __float_as_uint(v[4 * u + c]) & 0x7fffffffu;
+        pmax = max(pmax, m);
+        const int q = m <= limit ? (int)rintf(ldexpf(v[4 * u + c], shift)) : 0;
         part[c >> 1] += q;
         // bytes: lowest digit .. top digit (the carries of the balanced form run through the addition)
         d[c] = ((uint32_t)q + 0x808080u) ^ 0x808080u;
@@ -270,8 +279,8 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
       }
       if (psum != 0)
         atomicAdd(reinterpret_cast<unsigned long long *>(&s_pixsum[pix0 + lane + 1]), (unsigned long long)psum);
-      if (bad)
-        s_pixbad[pix0 + lane + 1] = 1u;
+      if (pmax != 0u)
+        atomicMax(&s_pixmax[pix0 + lane + 1], pmax);
     }
   };
   const bool hold = !kChunked && items <= kSlabHold * kWaves; // uniform over the block
@@ -298,7 +307,7 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
   // while the loads are in flight: the tables in LDS
   for (int i = tid; i <= P.cap; i += kThreads) {
     s_pixsum[i] = 0;
-    s_pixbad[i] = 0u;
+    s_pixmax[i] = 0u;
   }
   if (tid < kRows)
     s_rowpix[taps * kRows + tid] = 0u; // the entry of steps past the last k tile: the zero pixel
@@ -345,6 +354,7 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
       bmax = max(bmax, (uint32_t)s_misc[w]);
     if (bmax != 0u)
       shift = kSlabTopBit - binade_exponent(binade_of(bmax));
+    limit = bmax;
   }
   auto convert_chunk = [&]() __attribute__((always_inline)) {
     for (int item = wave; item < items; item += kWaves) {
@@ -395,6 +405,19 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
   // ---- 2. the product.  Wavefront (wn, wm, wk): channel fragments 2 wn, 2 wn + 1 of the block's, window fragment wm,
   // k tiles wk, wk + WK, ...
   const int wn = wave % WN, wk = wave / (WN * WM);
+  uint32_t frag_mask[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    frag_mask[j] = 0x01010101u << (frag0 + 2 * wn + j);
+    asm volatile("" : "+s"(frag_mask[j]));
+  }
+  const int chunks = kChunked ? P.chunks : 1;
+  // One round finishes the windows whose largest magnitude is within 2^-kSlabLevel of the slab's scale -- all of them,
+  // for inputs of one magnitude.  Windows much smaller than their slab's largest value are finished by a further round,
+  // whose scale is that of the largest among them: it converts the slab again, with zeros for whatever is larger still
+  // (no window left holds any of it).  A round finishes the largest window left at least, so the rounds end.
+  // Returns the largest magnitude of the windows left, 0 when there is none (the same in every wavefront).
+  auto round = [&](auto again) __attribute__((always_inline)) -> uint32_t {
   i32x16_t acc[kSlabDigits][2];
 #pragma unroll
   for (int d = 0; d < kSlabDigits; ++d)
@@ -403,17 +426,11 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
 #pragma unroll
       for (int q = 0; q < 16; ++q)
         acc[d][j][q] = 0;
-  uint32_t frag_mask[2];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    frag_mask[j] = 0x01010101u << (frag0 + 2 * wn + j);
-    asm volatile("" : "+s"(frag_mask[j]));
-  }
-  const int chunks = kChunked ? P.chunks : 1;
   for (int chunk = 0; chunk < chunks; ++chunk) {
-    if (chunk > 0) {
+    if (chunk > 0 || again.value) {
       __syncthreads(); // every wavefront is through with the chunk before
-      take_chunk(chunk);
+      if (kChunked)
+        take_chunk(chunk);
       convert_chunk();
       __syncthreads();
     }
@@ -523,6 +540,41 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
     }
   }
 
+  // The sum of q over the lane's window and its largest magnitude: every wavefront adds up the windows it
+  // finishes from the pixels' sums, which are complete since the barrier in front of the (last) product; its lanes
+  // l and l + 32 share a window and take every second tap each, five reads in flight at a time.
+  long long rowsum = 0;
+  uint32_t rowmax = 0u;
+  for (int t0 = half; t0 < taps; t0 += 10) {
+    uint32_t idx[5];
+#pragma unroll
+    for (int j = 0; j < 5; ++j) // (past the last tap: the zero pixel)
+      idx[j] = t0 + 2 * j < taps ? s_rowpix[(t0 + 2 * j) * kRows + row] : 0u;
+#pragma unroll
+    for (int j = 0; j < 5; ++j) {
+      rowsum += s_pixsum[idx[j]];
+      rowmax = max(rowmax, s_pixmax[idx[j]]);
+    }
+  }
+  rowsum += __shfl_xor(rowsum, 32);
+  rowmax = max(rowmax, (uint32_t)__shfl_xor((int)rowmax, 32));
+  const bool rowbad = rowmax >= 0x7f800000u; // a NaN or an infinity
+  // (a window all zero is finished by any scale)
+  const bool todo = row_in && (!again.value || (rowmax != 0u && rowmax <= limit)); // (larger ones are finished)
+  const bool finish = todo && (rowbad || rowmax == 0u ||
+                               binade_exponent(binade_of(rowmax)) + kSlabLevel >= binade_exponent(binade_of(limit)));
+  {
+    uint32_t left = todo && !finish ? rowmax : 0u;
+    if (__ballot(left != 0u) != 0) {
+#pragma unroll
+      for (int off = 16; off >= 1; off >>= 1)
+        left = max(left, (uint32_t)__shfl_xor((int)left, off));
+    }
+    if (lane == 0)
+      s_misc[8 + wave] = (int)left;
+  }
+  __syncthreads(); // (and every wavefront has left the product)
+
   // ---- 3. (WK == 2) the two k groups' accumulators added exactly through LDS (the planes are free once every
   // wavefront has left the loop), one digit at a time, in two alternating areas: a wavefront hands the fragment it does
   // not finish (1 - wk) to its partner in the other k group and adds the partner's copy of fragment wk to its own.
@@ -530,7 +582,6 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
   if constexpr (WK == 2) {
     uint4_t *red = reinterpret_cast<uint4_t *>(smem);
     const int mine = wave * 4 * 64 + lane, theirs = (wave ^ (WN * WM)) * 4 * 64 + lane;
-    __syncthreads();
 #pragma unroll
     for (int d = 0; d < kSlabDigits; ++d) {
       uint4_t *area = red + (d & 1) * (kWaves * kSlabReduceBytes / 16);
@@ -552,34 +603,13 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
     }
   }
 
-  // The sum of q over the lane's window and whether it holds a non-finite value: every wavefront adds up the windows it
-  // finishes from the pixels' sums, which are complete since the barrier in front of the (last) product; its lanes
-  // l and l + 32 share a window and take every second tap each, five reads in flight at a time.
-  long long rowsum = 0;
-  uint32_t rowmark = 0u;
-  for (int t0 = half; t0 < taps; t0 += 10) {
-    uint32_t idx[5];
-#pragma unroll
-    for (int j = 0; j < 5; ++j) // (past the last tap: the zero pixel)
-      idx[j] = t0 + 2 * j < taps ? s_rowpix[(t0 + 2 * j) * kRows + row] : 0u;
-#pragma unroll
-    for (int j = 0; j < 5; ++j) {
-      rowsum += s_pixsum[idx[j]];
-      rowmark |= s_pixbad[idx[j]];
-    }
-  }
-  rowsum += __shfl_xor(rowsum, 32);
-  rowmark |= (uint32_t)__shfl_xor((int)rowmark, 32);
-
   // ---- 4. epilogue.  Accumulator register q of lane l: channel 8 (q / 4) + 4 (l / 32) + q % 4 of the fragment,
   // window l % 32.  dot = rowsum - 2 * sum(q * bit); the accumulators carry the factor 2^F of the fragment's byte
   // (-128 for F = 7).  With m_d = acc_d / 2^F:  sum(q * bit) = hi * 2^16 + lo, hi = m_0 * 256 + m_1,
   // lo = m_2 * 256 + m_3 (|m_d| <= 2^21 for the k the host admits), and with rowsum = s_hi * 2^16 + s_lo the result is
   // (s_hi -+ 2 hi) * 2^16 + (s_lo -+ 2 lo) = A * 2^16 + B with 0 <= B < 2^16: one fused multiply-add, rounded once
   // while |A| < 2^24 (sums below 2^40), else twice (2^-24 of the sum).
-  if (!row_in)
-    return;
-  const bool rowbad = rowmark != 0u;
+  if (finish) {
   const int s_hi = (int)(rowsum >> 16), s_lo = (int)(rowsum & 0xffff);
   const int osz = (int)g.out_sp_size;
 #pragma unroll
@@ -658,6 +688,27 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
       ybase[cq * osz] = acc + s_bias[c0 + cq];
     }
   }
+  }
+  }
+  // ---- 5. windows left?
+  uint32_t left = 0u;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w)
+    left = max(left, (uint32_t)s_misc[8 + w]);
+  return left;
+  };
+  uint32_t left = round(std::false_type{});
+  while (left != 0u) {
+    // (opaque: nothing derived from these is kept in registers from one round to the next)
+    asm volatile("" : "+v"(tid), "+v"(row));
+    tid &= kThreads - 1, row &= kRows - 1, lane = tid & 63, half = lane >> 5; // (the compiler knows their ranges again)
+    limit = left;
+    shift = kSlabTopBit - binade_exponent(binade_of(left));
+    for (int i = tid; i <= P.cap; i += kThreads)
+      s_pixsum[i] = 0;
+    for (int i = tid; i < (P.pix_stride >> 2); i += kThreads) // the zero pixel: the exchange lies over it
+      *reinterpret_cast<uint32_t *>(smem + 4 * i) = 0u;
+    left = round(std::true_type{});
   }
 #endif
 }
@@ -914,7 +965,7 @@ bool compute_slab_form(const ConvGeom &g, int form, int chunks, SlabPlan &p) {
   off = (int64_t)round_up((size_t)off, 16);
   p.pixsum_off = (int)off, off += 8 * (cap + 1);
   off = (int64_t)round_up((size_t)off, 16);
-  p.pixbad_off = (int)off, off += 4 * (cap + 1);
+  p.pixmax_off = (int)off, off += 4 * (cap + 1);
   p.rowpix_off = (int)off, off += 4 * rows * (g.k_size + 1);
   p.alpha_off = (int)off, off += 2 * 4 * 64 * f.wn;
   p.misc_off = (int)off, off += 64;

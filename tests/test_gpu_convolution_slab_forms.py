@@ -4,6 +4,8 @@ tile of 32 or 128 windows, a last tile of few windows, channel tiles with paddin
 
 Bound: x is rounded to a multiple of 2^-30 of the largest magnitude under a block's windows, so an output of K terms is
 off by at most K * 2^-30 * max|x|, and by the roundings of its conversion to fp32 (two, 2^-24 of the result each).
+Windows more than three binades below that largest magnitude have a scale of their own: whatever else lies in their block,
+they are off by at most K * 2^-27 of their own largest value.
 """
 import numpy as np
 import pytest
@@ -91,3 +93,41 @@ def test_short_contractions(xs, O, k):
     for _ in range(5):
         y = kernels.binary_connect_convolution(xn.view(xs).cuda(), Wd, None, *geo)[0].cpu().double()
         assert torch.equal(y.isnan(), y64.isnan()) and torch.equal(y.nan_to_num(), y64.nan_to_num())
+
+
+def _window_max(v, k, pad, stride):
+    m = v.abs().amax(1, keepdim=True)
+    return torch.nn.functional.max_pool2d(torch.nn.functional.pad(m, (pad[1], pad[1], pad[0], pad[0])), k, stride)
+
+
+@pytest.mark.parametrize("xs,O,k,pad,stride,group", [c for c in CASES if c[-1] == 1])
+def test_windows_of_different_magnitudes(xs, O, k, pad, stride, group):
+    """Patches of the map 2^0 to 2^-70 in size: every output is as good as its own window allows."""
+    rng = np.random.RandomState(21)
+    kernels.init(0)
+
+    def patches(B, C, H, W):
+        e = rng.choice([0, 0, -2, -5, -12, -22, -70], (B, 1, -(-H // 5), -(-W // 6))).repeat(5, 2).repeat(6, 3)
+        return torch.from_numpy((rng.randn(B, C, H, W) * 2.0 ** e[:, :, :H, :W]).astype(np.float32))
+    x = patches(*xs)
+    W = torch.from_numpy(rng.randn(O, xs[1], *k).astype(np.float32))
+    s64 = torch.where(W < 0, -1.0, 1.0).double()
+    y64 = torch.nn.functional.conv2d(x.double(), s64, None, stride, pad)
+    y, Wb = kernels.binary_connect_convolution(x.cuda(), W.cuda(), None, pad, stride, (1, 1), 1)
+    bound = s64[0].numel() * 2.0 ** -27 * _window_max(x, k, pad, stride) + 2.0 ** -23 * y64.abs()
+    assert bool(((y.cpu().double() - y64).abs() <= bound).all())
+    if stride != (1, 1) or O < 16:
+        return
+    # the input gradient: windows of dy * alpha, the padding that of the transposed convolution
+    dy, alpha = patches(*y64.shape), torch.from_numpy(rng.rand(O).astype(np.float32) + 0.5)
+    scaled = dy * alpha[None, :, None, None]
+    want = torch.nn.grad.conv2d_input(xs, s64, scaled.double(), stride, pad)
+    old = torch.zeros(xs)
+    old[:, :, ::2] = 2.0 ** -30
+    dx, _, _ = kernels.binary_convolution_backward(dy.cuda(), x.cuda(), W.cuda(), Wb, alpha.cuda(), pad, stride, (1, 1), 1,
+                                                   dx=old.cuda(), want=(True, False, False))
+    n, taps = O * k[0] * k[1], k[0] * k[1]
+    most = _window_max(scaled, k, (k[0] - 1 - pad[0], k[1] - 1 - pad[1]), (1, 1))
+    # (where the geometry is unfolded instead: three digits of every position's largest, and every addition rounded)
+    bound = n * most * (2.0 ** -23 + 2 * taps * 2.0 ** -24) + 2.0 ** -22 * (want.abs() + old)
+    assert bool(((dx.cpu().double() - (want + old)).abs() <= bound).all())
