@@ -9,7 +9,9 @@
 // fourth is below 2^-22 of the product.  A block's sums (a few hundred positions) go to memory as fp32 and are added in a
 // fixed order in double.  Against float64 the gradient of [32,64,56,56] x [64,64,3,3] is off by 2.5e-7 of its norm
 // (1.4e-6 with the products of 24-bit digits of the unfolded matrix, 9.4e-7 for fp32 sums in order).  A NaN or an
-// infinity makes NaN of every gradient it reaches (v - hi is then NaN).
+// infinity makes NaN of every sum it meets (v - hi is then NaN), those included where it only meets the zeros that fill up
+// a row, a tile or a step; the sums that are NaN are therefore formed once more, one by one, in the order and with the
+// zeros of the reference (convolution.cpp:199-283).
 //
 // Layout.  A tile is R output rows of one sample (or NS whole samples of a small map), its positions in groups of eight
 // along the rows: dy as [group][hi / lo][64 output channels][8 fp16], x as [input row][column phase][group][hi / lo]
@@ -426,10 +428,14 @@ __global__ __launch_bounds__(kDwThreads, 2) void conv_dw_kernel(DwArgs a) {
 }
 
 // dW[o, c, tap] (+)= 2^-(shifts) * the splits' sums added in double: 32 outputs along c x 8 runs of the splits per block.
+// Sums that are not finite are formed anew from dy and the unfolded input, by the whole block each (the values of a
+// finite x and dy never overflow here).
 __global__ __launch_bounds__(256) void conv_dw_sum(const float *__restrict__ partial, const int32_t *__restrict__ shifts,
                                                    float *__restrict__ dW, int Og, int Cg, int taps, int splits,
-                                                   int accumulate) {
+                                                   int accumulate, const float *__restrict__ x,
+                                                   const float *__restrict__ dy, ConvGeom g, int64_t grp) {
   __shared__ double s_sum[8][32];
+  __shared__ int s_redo[32];
   const int lane = threadIdx.x & 31, run = threadIdx.x >> 5;
   const int64_t outs = (int64_t)taps * Og * Cg, at = (int64_t)blockIdx.x * 32 + lane;
   double sum = 0.0;
@@ -449,15 +455,51 @@ __global__ __launch_bounds__(256) void conv_dw_sum(const float *__restrict__ par
   }
   s_sum[run][lane] = sum;
   __syncthreads();
+  int redo = 0;
   if (run == 0 && at < outs) {
 #pragma unroll
     for (int j = 1; j < 8; ++j)
       sum += s_sum[j][lane];
+    redo = !__builtin_isfinite(sum);
+  }
+  if (run == 0 && at < outs && !redo) {
     const int64_t tap = at / ((int64_t)Og * Cg), oc = at - tap * ((int64_t)Og * Cg);
     const int o = (int)(oc / Cg), c = (int)(oc - (int64_t)o * Cg);
     const float v = (float)ldexp(sum, -(shifts[c] + shifts[Cg + o]));
     float *dst = dW + oc * taps + tap;
     *dst = accumulate ? *dst + v : v;
+  }
+  if (run == 0)
+    s_redo[lane] = redo;
+  if (!__syncthreads_or(redo))
+    return;
+  for (int j = 0; j < 32; ++j) {
+    if (!s_redo[j]) // uniform over the block
+      continue;
+    const int64_t out = (int64_t)blockIdx.x * 32 + j, tap = out / ((int64_t)Og * Cg), oc = out - tap * ((int64_t)Og * Cg);
+    const int64_t o = oc / Cg, c = oc - o * Cg, L = g.out_sp_size;
+    double part = 0.0;
+    for (int64_t m0 = 0; m0 < g.M; m0 += 16 * 256) {
+      for (int64_t m = m0 + threadIdx.x; m < g.M && m < m0 + 16 * 256; m += 256) {
+        const int64_t n = m / L, l = m - n * L;
+        part += (double)dy[(n * g.O + grp * g.Og + o) * L + l] * (double)col_value(x, g, grp, m, c * taps + tap);
+      }
+      if (__syncthreads_or(__builtin_isnan(part))) // nothing brings a NaN back
+        break;
+    }
+    __syncthreads(); // (the sums of the output before have been read)
+    double *s_part = &s_sum[0][0];
+    s_part[threadIdx.x] = part;
+    __syncthreads();
+    for (int half = 128; half >= 1; half >>= 1) {
+      if ((int)threadIdx.x < half)
+        s_part[threadIdx.x] += s_part[threadIdx.x + half];
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+      float *dst = dW + oc * taps + tap;
+      *dst = accumulate ? *dst + (float)s_part[0] : (float)s_part[0];
+    }
   }
 }
 
@@ -610,7 +652,7 @@ int launch_conv_dw(const float *dy, const float *x, float *dW, const ConvGeom &g
     return rc;
   const int64_t outs = g.Og * g.Kg;
   hipLaunchKernelGGL(conv_dw_sum, dim3((unsigned)ceil_div(outs, 32)), dim3(256), 0, stream, a.partial, a.shifts,
-                     dW + grp * g.Og * g.Kg, a.Og, a.Cg, (int)g.k_size, a.p.splits, accumulate ? 1 : 0);
+                     dW + grp * g.Og * g.Kg, a.Og, a.Cg, (int)g.k_size, a.p.splits, accumulate ? 1 : 0, x, dy, g, grp);
   NBLA_HIP_LAUNCH_CHECK("conv_dw_sum");
   return NBLA_HIP_OK;
 }

@@ -66,17 +66,50 @@ def test_against_float64(xs, O, k, pad, stride, group):
     assert torch.equal(acc, dW0.to(dev) + dW)
 
 
-def test_a_non_finite_value_reaches_its_channel_only():
+# places where a value only meets the zeros that fill up a row, a map, a tile or the last step, besides ordinary ones
+@pytest.mark.parametrize("xs,k,s,at", [((2, 32, 9, 9), 3, 1, [(4, 4)]), ((2, 32, 9, 9), 3, 1, [(0, 8), (8, 0), (8, 8)]),
+                                       ((3, 40, 7, 11), 3, 2, [(6, 10), (0, 0), (5, 9)]), ((2, 16, 14, 13), 5, 1, [(13, 12)]),
+                                       ((5, 24, 5, 5), 3, 1, [(0, 0), (4, 4)]), ((3, 130, 13, 7), 1, 1, [(12, 6)]),
+                                       ((2, 32, 10, 12), 1, 2, [(9, 11), (8, 10)]), ((1, 20, 11, 9), 5, 2, [(10, 8), (0, 7)])])
+def test_non_finite_values(xs, k, s, at):
+    """As the unfolded product gives it: an infinity where it stands against a finite gradient, NaN against a zero or the
+    padding or another one of the other sign, and nothing in the weights that it does not meet."""
     rng = np.random.RandomState(8)
-    dev = torch.device("cuda:0")
-    x = torch.from_numpy(rng.randn(2, 32, 9, 9).astype(np.float32)).to(dev)
-    dy = torch.from_numpy(rng.randn(2, 40, 9, 9).astype(np.float32)).to(dev)
-    W = torch.zeros(40, 32, 3, 3, device=dev)
-    _, clean, _ = kernels.convolution_backward(dy, x, W, (1, 1), (1, 1), (1, 1), 1, want=(False, True, False))
-    x[1, 5, 4, 4] = float("inf")
-    dy[0, 7, 0, 0] = float("nan")
-    _, dW, _ = kernels.convolution_backward(dy, x, W, (1, 1), (1, 1), (1, 1), 1, want=(False, True, False))
-    hit = torch.zeros_like(dW, dtype=torch.bool)
-    hit[:, 5] = True
-    hit[7] = True
-    assert bool(dW[hit].isnan().all()) and torch.equal(dW[~hit], clean[~hit])
+    kernels.init(0)
+    B, C, H, W_ = xs
+    p, O = k // 2, 40
+    x = torch.from_numpy(rng.randn(*xs).astype(np.float32))
+    oh, ow = (H + 2 * p - k) // s + 1, (W_ + 2 * p - k) // s + 1
+    dy = torch.from_numpy(rng.randn(B, O, oh, ow).astype(np.float32))
+    run = lambda: kernels.convolution_backward(dy.cuda(), x.cuda(), torch.zeros(O, C, k, k, device="cuda"), (p, p), (s, s),
+                                               (1, 1), 1, want=(False, True, False))[1].cpu()
+    for i, (y_, x_) in enumerate(at):
+        x[i % B, 5 + i, y_, x_] = 0.0
+    dy[0, 7, 0, 0], dy[B - 1, 9, oh - 1, ow - 1], dy[0, 3] = 0.0, 0.0, 0.0
+    clean = run()
+    for i, (y_, x_) in enumerate(at):
+        x[i % B, 5 + i, y_, x_] = float("inf") if i != 1 else float("nan")
+    dy[0, 7, 0, 0] = float("-inf")
+    dy[B - 1, 9, oh - 1, ow - 1] = float("nan")
+    cols = torch.nn.functional.unfold(x.double(), k, padding=p, stride=s)
+    want = sum(torch.nan_to_num(d, 0, 0, 0) @ torch.nan_to_num(u, 0, 0, 0).t() for d, u in zip(dy.double().flatten(2), cols))
+    # which outputs, term by term: 0 * Inf and Inf - Inf are NaN
+    nan, plus, minus = (torch.zeros(O, C * k * k, dtype=torch.bool) for _ in range(3))
+    for d, u in zip(dy.double().flatten(2), cols):
+        for m in range(oh * ow):
+            if d[:, m].isfinite().all() and u[:, m].isfinite().all():
+                continue
+            t = d[:, m, None] * u[None, :, m]
+            nan |= t.isnan()
+            plus |= t == float("inf")
+            minus |= t == float("-inf")
+    nan |= plus & minus
+    got = run().flatten(1)
+    assert torch.equal(got.isnan(), nan)
+    assert torch.equal(got == float("inf"), plus & ~nan) and torch.equal(got == float("-inf"), minus & ~nan)
+    fin = ~(nan | plus | minus)
+    assert float((got.double() - want)[fin].abs().max()) <= 1e-5 * float(want.abs().max())
+    got, clean = got.view(O, C, -1), clean.view(O, C, -1)
+    rows = [o for o in range(O) if o not in (7, 9)]
+    channels = [c for c in range(C) if not 5 <= c < 5 + len(at)]
+    assert torch.equal(got[rows][:, channels], clean[rows][:, channels])
