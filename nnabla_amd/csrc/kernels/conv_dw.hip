@@ -427,78 +427,68 @@ __global__ __launch_bounds__(kDwThreads, 2) void conv_dw_kernel(DwArgs a) {
 #endif
 }
 
-// dW[o, c, tap] (+)= 2^-(shifts) * the splits' sums added in double: 32 outputs along c x 8 runs of the splits per block.
-// Sums that are not finite are formed anew from dy and the unfolded input, by the whole block each (the values of a
-// finite x and dy never overflow here).
+// dW[o, c, tap] (+)= 2^-(shifts) * the splits' sums added in double: a thread adds every kRuns-th split of an output,
+// 256 / kRuns outputs along c to a block (the launch takes as many runs as give every CU eight blocks: with more, the
+// blocks' starts are the time).  Sums that are not finite are formed anew from dy and the unfolded input, by the wavefront
+// (the values of a finite x and dy never overflow here).
+template <int kRuns>
 __global__ __launch_bounds__(256) void conv_dw_sum(const float *__restrict__ partial, const int32_t *__restrict__ shifts,
                                                    float *__restrict__ dW, int Og, int Cg, int taps, int splits,
                                                    int accumulate, const float *__restrict__ x,
                                                    const float *__restrict__ dy, ConvGeom g, int64_t grp) {
-  __shared__ double s_sum[8][32];
-  __shared__ int s_redo[32];
-  const int lane = threadIdx.x & 31, run = threadIdx.x >> 5;
-  const int64_t outs = (int64_t)taps * Og * Cg, at = (int64_t)blockIdx.x * 32 + lane;
+  constexpr int kOuts = 256 / kRuns;
+  __shared__ double s_sum[kRuns][kOuts];
+  const int col = threadIdx.x % kOuts, run = threadIdx.x / kOuts;
+  const int64_t outs = (int64_t)taps * Og * Cg, at = (int64_t)blockIdx.x * kOuts + col;
   double sum = 0.0;
   if (at < outs) {
     int s = run;
-    for (; s + 24 < splits; s += 32) {
+    for (; s + 3 * kRuns < splits; s += 4 * kRuns) {
       float v[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        v[j] = partial[(int64_t)(s + 8 * j) * outs + at];
+        v[j] = partial[(int64_t)(s + kRuns * j) * outs + at];
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         sum += (double)v[j];
     }
-    for (; s < splits; s += 8)
+    for (; s < splits; s += kRuns)
       sum += (double)partial[(int64_t)s * outs + at];
   }
-  s_sum[run][lane] = sum;
-  __syncthreads();
-  int redo = 0;
+  if (kRuns > 1) {
+    s_sum[run][col] = sum;
+    __syncthreads();
+    if ((int)threadIdx.x >= (kOuts > 64 ? kOuts : 64)) // whole wavefronts
+      return;
+  }
+  bool redo = false;
   if (run == 0 && at < outs) {
 #pragma unroll
-    for (int j = 1; j < 8; ++j)
-      sum += s_sum[j][lane];
+    for (int j = 1; j < kRuns; ++j)
+      sum += s_sum[j][col];
     redo = !__builtin_isfinite(sum);
-  }
-  if (run == 0 && at < outs && !redo) {
     const int64_t tap = at / ((int64_t)Og * Cg), oc = at - tap * ((int64_t)Og * Cg);
     const int o = (int)(oc / Cg), c = (int)(oc - (int64_t)o * Cg);
     const float v = (float)ldexp(sum, -(shifts[c] + shifts[Cg + o]));
     float *dst = dW + oc * taps + tap;
-    *dst = accumulate ? *dst + v : v;
+    if (!redo)
+      *dst = accumulate ? *dst + v : v;
   }
-  if (run == 0)
-    s_redo[lane] = redo;
-  if (!__syncthreads_or(redo))
-    return;
-  for (int j = 0; j < 32; ++j) {
-    if (!s_redo[j]) // uniform over the block
-      continue;
-    const int64_t out = (int64_t)blockIdx.x * 32 + j, tap = out / ((int64_t)Og * Cg), oc = out - tap * ((int64_t)Og * Cg);
-    const int64_t o = oc / Cg, c = oc - o * Cg, L = g.out_sp_size;
+  for (uint64_t left = __ballot(redo); left; left &= left - 1) {
+    const int64_t out = (int64_t)blockIdx.x * kOuts + (threadIdx.x & ~63u) + __builtin_ctzll(left), tap = out / ((int64_t)Og * Cg);
+    const int64_t oc = out - tap * ((int64_t)Og * Cg), o = oc / Cg, c = oc - o * Cg, L = g.out_sp_size;
     double part = 0.0;
-    for (int64_t m0 = 0; m0 < g.M; m0 += 16 * 256) {
-      for (int64_t m = m0 + threadIdx.x; m < g.M && m < m0 + 16 * 256; m += 256) {
+    for (int64_t m0 = 0; m0 < g.M && !__ballot(__builtin_isnan(part)); m0 += 16 * 64) // (nothing brings a NaN back)
+      for (int64_t m = m0 + (threadIdx.x & 63); m < g.M && m < m0 + 16 * 64; m += 64) {
         const int64_t n = m / L, l = m - n * L;
         part += (double)dy[(n * g.O + grp * g.Og + o) * L + l] * (double)col_value(x, g, grp, m, c * taps + tap);
       }
-      if (__syncthreads_or(__builtin_isnan(part))) // nothing brings a NaN back
-        break;
-    }
-    __syncthreads(); // (the sums of the output before have been read)
-    double *s_part = &s_sum[0][0];
-    s_part[threadIdx.x] = part;
-    __syncthreads();
-    for (int half = 128; half >= 1; half >>= 1) {
-      if ((int)threadIdx.x < half)
-        s_part[threadIdx.x] += s_part[threadIdx.x + half];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) {
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1)
+      part += __shfl_xor(part, off);
+    if ((threadIdx.x & 63) == 0) {
       float *dst = dW + oc * taps + tap;
-      *dst = accumulate ? *dst + (float)s_part[0] : (float)s_part[0];
+      *dst = accumulate ? *dst + (float)part : (float)part;
     }
   }
 }
@@ -651,8 +641,19 @@ int launch_conv_dw(const float *dy, const float *x, float *dW, const ConvGeom &g
   if (rc)
     return rc;
   const int64_t outs = g.Og * g.Kg;
-  hipLaunchKernelGGL(conv_dw_sum, dim3((unsigned)ceil_div(outs, 32)), dim3(256), 0, stream, a.partial, a.shifts,
-                     dW + grp * g.Og * g.Kg, a.Og, a.Cg, (int)g.k_size, a.p.splits, accumulate ? 1 : 0, x, dy, g, grp);
+#define NBLA_DW_SUM(RUNS)                                                                                              \
+  hipLaunchKernelGGL(conv_dw_sum<RUNS>, dim3((unsigned)ceil_div(outs * RUNS, 256)), dim3(256), 0, stream, a.partial,   \
+                     a.shifts, dW + grp * g.Og * g.Kg, a.Og, a.Cg, (int)g.k_size, a.p.splits, accumulate ? 1 : 0, x,   \
+                     dy, g, grp)
+  if (outs >= 2048 * 256)
+    NBLA_DW_SUM(1);
+  else if (outs >= 1024 * 256)
+    NBLA_DW_SUM(2);
+  else if (outs >= 512 * 256)
+    NBLA_DW_SUM(4);
+  else
+    NBLA_DW_SUM(8);
+#undef NBLA_DW_SUM
   NBLA_HIP_LAUNCH_CHECK("conv_dw_sum");
   return NBLA_HIP_OK;
 }
