@@ -32,6 +32,11 @@ CASES = [
     ((2, 64, 14, 14), 64, (3, 3), (1, 1), 1, 2),     # groups
     ((70, 32, 5, 3), 32, (3, 3), (1, 1), 1, 1),      # rows shorter than a group of positions
     ((2, 16, 3, 80), 32, (3, 3), (1, 1), 1, 1),      # the longest rows
+    # blocks of several tiles, the last one of fewer
+    ((41, 512, 7, 7), 512, (3, 3), (1, 1), 1, 1),
+    ((9, 256, 14, 14), 512, (3, 3), (1, 1), 2, 1),
+    ((9, 512, 14, 14), 1024, (1, 1), (0, 0), 1, 1),
+    ((7, 128, 14, 14), 256, (5, 5), (2, 2), 1, 1),
 ]
 
 
@@ -113,3 +118,24 @@ def test_non_finite_values(xs, k, s, at):
     rows = [o for o in range(O) if o not in (7, 9)]
     channels = [c for c in range(C) if not 5 <= c < 5 + len(at)]
     assert torch.equal(got[rows][:, channels], clean[rows][:, channels])
+
+
+@pytest.mark.parametrize("sign,limit", [(False, 6e-7), (True, 1e-7)])
+def test_many_positions_under_many_weights(sign, limit):
+    """A wavefront adds up at most 512 positions in fp32 (four roundings in each of three products per sixteen: 384), the
+    rest is added in double: terms of random signs are off by 0.29 * 2^-23.5 * sqrt(384 * 384 / 2) / sqrt(384) of the norm
+    for a chain and for the whole (3e-7), besides 1e-7 for the products; terms of one sign by
+    0.29 * 2^-23.5 * sqrt(384 / 3) for a chain and a tenth of it for the mean of 98 (3e-8), besides the result's rounding.
+    Chains of 6272 positions are off by 1.0e-6 and 3.3e-7."""
+    kernels.init(0)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(5)
+    x = torch.randn(64, 512, 28, 28, device="cuda", generator=gen).clamp_(min=0)
+    dy = torch.randn(64, 512, 28, 28, device="cuda", generator=gen) * 1e-2
+    dy = dy.abs() if sign else dy
+    dW = kernels.convolution_backward(dy, x, torch.zeros(512, 512, 3, 3, device="cuda"), (1, 1), (1, 1), (1, 1), 1,
+                                      want=(False, True, False))[1]
+    want = torch.zeros(512, 512 * 9, dtype=torch.float64, device="cuda")
+    for n in range(64):
+        want += dy[n].double().flatten(1) @ torch.nn.functional.unfold(x[n:n + 1].double(), 3, padding=1)[0].t().contiguous()
+    assert float((dW.double().flatten(1) - want).norm() / want.norm()) <= limit
