@@ -259,11 +259,16 @@ int conv_backward(const float *dy, const float *x, const float *W, const float *
       return rc;
     dx = nullptr, dx_slab = false;
   }
-  // few weights under many windows of a geometry that the matrix-core product below does not cover (it is two to four
-  // times as fast where both apply): the weight gradient in fp32 straight from dy and x, all groups at once (its
-  // partial results lie in the unfolded gradient's buffer, so it runs before the loop that fills that buffer)
-  if (dW && !conv_dw_applies(g) && conv_direct_dw_applies(g)) {
-    rc = launch_conv_direct_dw(dy, x, dW, g, accum_w, col, (size_t)g.M * g.Kg * sizeof(float), stream);
+  // few weights under many windows: the weight gradient in fp32 straight from dy and x, all groups at once (its
+  // partial results lie in the unfolded gradient's buffer, so it runs before the loop that fills that buffer).  Of the
+  // geometries that the product on the matrix cores below covers, only those whose sums lie in short chains here are: the
+  // products of two fp16 numbers each are 1.1e-7 off before any sum, so there they would lose bits ([32,32,56,56] x
+  // [32,32,3,3] 1.4e-7 off float64 here in 168 us, 2.1e-7 there in 41; [64,64,28,28] x [64,64,1,1], whose chains are long
+  // here, 3.4e-7 in 121 us and 1.8e-7 in 30).
+  const size_t col_bytes = (size_t)g.M * g.Kg * sizeof(float);
+  const bool dw_product = conv_dw_applies(g) && !conv_direct_dw_by_pairs(g, col_bytes);
+  if (dW && !dw_product && conv_direct_dw_applies(g)) {
+    rc = launch_conv_direct_dw(dy, x, dW, g, accum_w, col, col_bytes, stream);
     if (rc)
       return rc;
     dW = nullptr;
@@ -276,7 +281,7 @@ int conv_backward(const float *dy, const float *x, const float *W, const float *
       return rc;
     db = nullptr;
   }
-  if (dW && conv_dw_applies(g)) { // kernels of width 1, 3, 5 with half their width of padding: no unfolded matrix
+  if (dW && dw_product) { // kernels of width 1, 3, 5 with half their width of padding: no unfolded matrix
     for (int64_t grp = 0; grp < g.group; ++grp) {
       rc = launch_conv_dw(dy, x, dW, g, grp, accum_w, base + p.dw_off, conv_dw_workspace_bytes(g), stream);
       if (rc)

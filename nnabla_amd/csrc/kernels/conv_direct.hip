@@ -803,16 +803,23 @@ static int dw_chunks(const ConvGeom &g) {
     chunks = g.M / g.O;
   return (int)(chunks < 1 ? 1 : chunks);
 }
+// Very few weights (a first layer of 3 x 3 taps, 16 or 32 channels): a tile of 64 x 64 would be mostly empty, the kernel
+// that keeps (channel pair, taps) sums per thread loads less (rough counts of loads per window).
+static bool takes_pairs(const ConvGeom &g, const PairsPlan &pairs) {
+  return pairs.fits &&
+         pairs.loads_per_window() < ceil_div(g.Kg, kDwTile) * ceil_div(g.Og, kDwTile) * g.group * 1024;
+}
+bool conv_direct_dw_by_pairs(const ConvGeom &g, size_t scratch_bytes) {
+  return conv_direct_dw_applies(g) && takes_pairs(g, plan_dw_pairs(g, scratch_bytes));
+}
 int launch_conv_direct_dw(const float *dy, const float *x, float *dW, const ConvGeom &g, bool accum, void *scratch,
                           size_t scratch_bytes, hipStream_t stream) {
   const int chunks = dw_chunks(g);
   if (scratch_bytes < (size_t)chunks * g.O * g.Kg * sizeof(float) || !aligned16(scratch))
     return fail(NBLA_HIP_ERR_MEMORY, "weight gradient: scratch too small or misaligned.");
   const int64_t ktiles = ceil_div(g.Kg, kDwTile), otiles = ceil_div(g.Og, kDwTile);
-  // very few weights (a first layer of 3 x 3 taps, 16 or 32 channels): a tile of 64 x 64 would be mostly empty, the
-  // kernel that keeps (channel pair, taps) sums per thread loads less (rough counts of loads per window)
   const PairsPlan pairs = plan_dw_pairs(g, scratch_bytes);
-  if (pairs.fits && pairs.loads_per_window() < ktiles * otiles * g.group * 1024)
+  if (takes_pairs(g, pairs))
     return launch_dw_pairs(dy, x, dW, g, accum, static_cast<float *>(scratch), pairs, stream);
   float *partial = static_cast<float *>(scratch);
   hipLaunchKernelGGL(conv_direct_dw_tile, dim3((unsigned)(ktiles * otiles * g.group), (unsigned)chunks),

@@ -34,8 +34,8 @@
 // and the conversions of either 4000; the maxima of the channels (8.4 us for 51 MB) and the sum over the splits
 // (6.4 us) come on top.  The whole weight gradient, in place of unfolding x into a digit matrix chunk by chunk:
 // [32,64,56,56] x [64,64,3,3] 400 -> 54 us, [32,256,14,14] x [256,256,3,3] 95 -> 56, [16,128,28,28] x [256,128,3,3]
-// stride 2 62 -> 34; and against fp32 sums on the vector units (few weights, many positions): [32,32,56,56] x
-// [32,32,3,3] 154 -> 38, [64,64,28,28] x [64,64,1,1] 117 -> 28, [64,8,28,28] x [32,8,3,3] 50 -> 26.
+// stride 2 62 -> 34; and against tiles of fp32 sums on the vector units (few weights, many positions): [64,64,28,28] x
+// [64,64,1,1] 117 -> 28, [64,16,28,28] x [64,16,3,3] 125 -> 32.
 #include "common.hpp"
 #include "conv_geom.hpp"
 #include "gemm_layout.hpp"

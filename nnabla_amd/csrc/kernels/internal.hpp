@@ -63,6 +63,9 @@ bool conv_direct_applies(const ConvGeom &g);
 bool conv_direct_forward_applies(const ConvGeom &g); // (also a single group of very few input channels, many taps)
 // The weight gradient of few weights under many windows in fp32 (all groups); scratch: M * Kg floats are enough.
 bool conv_direct_dw_applies(const ConvGeom &g);
+// Whether it then keeps the sums of every (channel pair, tap) in threads, in this much scratch memory: short chains of
+// fp32 products, off float64 by 1.0e-7 to 1.9e-7 of the norm.
+bool conv_direct_dw_by_pairs(const ConvGeom &g, size_t scratch_bytes);
 int launch_conv_direct_dw(const float *dy, const float *x, float *dW, const ConvGeom &g, bool accum, void *scratch,
                           size_t scratch_bytes, hipStream_t stream);
 int launch_conv_direct_binarize(const float *W, float *Wb, float *alpha, const ConvGeom &g, float zero_to,
