@@ -96,6 +96,7 @@ struct DwDivide {
 
 struct DwPlan {
   int KH, KW, S, nky, nc;
+  int items; // runs of eight values that a thread converts per tile
   int G, Gx, R, NS, rows_x, Q, steps, row_tiles; // (G groups per output row; Gx = G and the zeros in front)
   int ot, ct, kg, splits, tiles, per_split;
   int dy_off, tab_off, misc_off, lds;
@@ -540,6 +541,7 @@ bool make_dw_plan(const ConvGeom &g, DwPlan &p) {
     const int reduce = 2 * p.nky * p.KW * p.nc * 16 * 64 * 4; // the sums two wavefronts exchange
     if (p.lds < reduce)
       p.lds = reduce;
+    p.items = (int)(ceil_div(C * NS * p.rows_x * p.G, kDwThreads) * p.S + ceil_div(kDwO * p.Q, kDwThreads));
     return C * NS * p.rows_x * p.G <= mx * kDwThreads && kDwO * p.Q <= my * kDwThreads && p.lds <= kDwLds;
   };
   if (!sizes(1, 1))
@@ -602,14 +604,31 @@ template <int KW, int S> int run_conv_dw(const DwArgs &a, hipStream_t stream) {
 
 } // namespace
 
+// Where the geometry is covered, by an estimate of both forms in microseconds, fitted to 110 geometries measured on both
+// (1 to 4096 samples of 1 x 1 to 56 x 56 positions, 16 to 512 channels; off by 15 % at the median).  Here: a wavefront's
+// MFMAs of a tile at 1.46 times their 32 cycles, 490 cycles for each run of eight values that a thread converts, twice as
+// long where blocks share a CU, and the splits' partial sums through memory.  The product of digit operands: x unfolded
+// and converted, dy transposed and converted, tiles of 128 x 128 weights.  It wins where a kernel of five rows, whose taps
+// take a pass over x for each row, meets many channels on both sides: [32,512,14,14] x [512,512,5,5] 306 us against 530
+// here; [64,512,14,14] x [512,512,3,3] 302 against 309, [64,512,2,2] 47 against 48.  A tie goes to this form, the more
+// precise one.
 bool conv_dw_applies(const ConvGeom &g) {
   DwPlan p;
-  return make_dw_plan(g, p);
+  if (!make_dw_plan(g, p))
+    return false;
+  const int64_t blocks = (int64_t)p.ot * p.ct * p.kg * p.splits;
+  const double rounds = (double)ceil_div(blocks, 512) * (blocks > 256 ? 2.0 : 1.0);
+  const double mfma = 32.0 * 3 * ceil_div(p.steps, 2) * p.nky * p.KW * p.nc, M = (double)g.M;
+  const double here = 20.0 + rounds * p.per_split * (1.46 * mfma + 490.0 * p.items) / 2400.0 +
+                      1.5e-6 * (double)p.splits * (double)g.Og * (double)g.Kg;
+  const double digits = 45.0 + 2.3e-6 * M * (double)g.Kg + 11.5e-6 * M * (double)g.Og +
+                        1.2e-9 * M * (double)(ceil_div(g.Kg, 128) * ceil_div(g.Og, 128) * 128 * 128);
+  return here <= 1.15 * digits;
 }
 
 size_t conv_dw_workspace_bytes(const ConvGeom &g) {
   DwPlan p;
-  return make_dw_plan(g, p) ? p.total : 0;
+  return conv_dw_applies(g) && make_dw_plan(g, p) ? p.total : 0;
 }
 
 int launch_conv_dw(const float *dy, const float *x, float *dW, const ConvGeom &g, int64_t grp, bool accumulate,

@@ -37,6 +37,7 @@ CASES = [
     ((9, 256, 14, 14), 512, (3, 3), (1, 1), 2, 1),
     ((9, 512, 14, 14), 1024, (1, 1), (0, 0), 1, 1),
     ((7, 128, 14, 14), 256, (5, 5), (2, 2), 1, 1),
+    ((4, 512, 14, 14), 512, (5, 5), (2, 2), 1, 1),   # left to the product of digit operands
 ]
 
 
