@@ -510,6 +510,8 @@ bool make_dw_plan(const ConvGeom &g, DwPlan &p) {
       return false;
   if (g.k[0] != 1 || g.in_sp[0] != 1 || g.out_sp[0] != 1 || g.pad[0] != 0)
     return false;
+  if (g.outer > 65535) // the unfolded form refuses such calls, with whatever other gradient they want
+    return false;
   p.KH = g.k[1], p.KW = g.k[2], p.S = g.stride[2];
   if (g.stride[1] != g.stride[2] || p.KH > 16 || g.pad[2] != p.KW / 2)
     return false;

@@ -447,6 +447,8 @@ int64_t class_slots(int64_t QH, int64_t QW, int64_t IH, int64_t IW, int64_t N, i
 bool plan_real(const ConvGeom &g, bool transposed, RealArgs &a) {
   if (g.in_sp[0] != 1 || g.k[0] != 1 || g.pad[0] != 0 || g.dil[1] != 1 || g.dil[2] != 1)
     return false;
+  if (transposed && g.outer > 65535) // (refused, as the unfolded gradient does)
+    return false;
   const int s = g.stride[1], KH = g.k[1], KW = g.k[2];
   if (g.stride[2] != s || s < 1 || s > 3 || KH * KW > kMaxTaps || KH > 25 || KW > 25 || g.pad[1] > 12 || g.pad[2] > 12 ||
       g.pad[1] >= KH || g.pad[2] >= KW)

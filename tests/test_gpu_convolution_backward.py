@@ -177,3 +177,13 @@ def test_config4_backward(dev):
     assert max_rel_err(to_np(gdx), tx.grad.numpy()) <= TIGHT
     assert max_rel_err(to_np(gdw), Ws.grad.numpy()) <= TIGHT
     assert max_rel_err(to_np(gdb), dy.astype(np.float64).sum((0, 2, 3))) <= TIGHT
+
+
+@pytest.mark.parametrize("want", [(False, True, False), (True, False, False), (True, True, True)])
+def test_more_samples_than_a_call_takes_are_refused(want):
+    kernels.init(0)
+    x = torch.ones(65536, 32, 1, 1, device="cuda")
+    dy = torch.ones(65536, 520, 1, 1, device="cuda")
+    W = torch.ones(520, 32, 1, 1, device="cuda")
+    with pytest.raises(Exception, match="65535 samples"):
+        kernels.convolution_backward(dy, x, W, (0, 0), (1, 1), (1, 1), 1, want=want)
