@@ -253,7 +253,7 @@ template <int kItems> __global__ __launch_bounds__(kThreads, 2) void conv_real_k
 #pragma unroll
       for (int q = 0; q < 16; ++q)
         acc[i][f][q] = 0.0f;
-  uint32_t amax = 0u;
+  uint32_t amax = 0u, amin = ~0u; // the largest magnitude of the run; the smallest one that is not zero, less one
   const int row_frags = a.row_tiles * 2, sub_shift = a.chunk == 32 ? 1 : 0;
   const int steps = C.taps << sub_shift;
   const uint4_t *wbase = reinterpret_cast<const uint4_t *>(a.w) + (int64_t)(row_tile * 2) * 64 + lane;
@@ -314,7 +314,9 @@ template <int kItems> __global__ __launch_bounds__(kThreads, 2) void conv_real_k
       uint4_t p[3];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        amax = max(amax, max(__float_as_uint(xv[i][2 * j]) & 0x7fffffffu, __float_as_uint(xv[i][2 * j + 1]) & 0x7fffffffu));
+        const uint32_t m0 = __float_as_uint(xv[i][2 * j]) & 0x7fffffffu, m1 = __float_as_uint(xv[i][2 * j + 1]) & 0x7fffffffu;
+        amax = max(amax, max(m0, m1));
+        amin = min(amin, min(m0 - 1u, m1 - 1u));
         uint32_t hi, mid, lo;
         split3_pair(xv[i][2 * j], xv[i][2 * j + 1], hi, mid, lo);
         p[0][j] = hi, p[1][j] = mid, p[2][j] = lo;
@@ -344,14 +346,16 @@ template <int kItems> __global__ __launch_bounds__(kThreads, 2) void conv_real_k
     load_w(next, wave + 2 * kWaves, w2);
   }
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1)
+  for (int off = 32; off >= 1; off >>= 1) {
     amax = max(amax, (uint32_t)__shfl_xor((int)amax, off));
+    amin = min(amin, (uint32_t)__shfl_xor((int)amin, off));
+  }
   if (lane == 0)
-    s_max[0][wave] = amax;
+    s_max[0][wave] = amax, s_max[1][wave] = amin;
   __syncthreads();
 #pragma unroll
   for (int w = 0; w < kWaves; ++w)
-    amax = max(amax, s_max[0][w]);
+    amax = max(amax, s_max[0][w]), amin = min(amin, s_max[1][w]);
   // ---- the wavefronts' sums: each finishes sixteen of the rows
   float *s_red = reinterpret_cast<float *>(smem); // [wave][row][position]
 #pragma unroll
@@ -370,7 +374,7 @@ template <int kItems> __global__ __launch_bounds__(kThreads, 2) void conv_real_k
   const int out_plane = a.OH * a.OW;
   float *out = a.out + (int64_t)n * a.CD * out_plane + (qy * a.ds + C.cy) * a.OW + (qx * a.ds + C.cx);
   // a window to be recomputed: only blocks whose run holds something out of range look for them
-  const bool suspect = amax >= kMost || (amax != 0u && amax < kLeast);
+  const bool suspect = amax >= kMost || amin < kLeast - 1u;
   int any_bad = 0;
   if (suspect) {
     uint32_t big = 0u;

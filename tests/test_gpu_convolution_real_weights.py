@@ -52,7 +52,7 @@ def _grad64(case, w, dy):
 def _bound(terms, n):
     # a term is good to 2^-23 (the products left out), n terms summed by 16 with six roundings of the running sum each;
     # the digit and fp32 paths, which some of the sizes take, are within it too (24 bits of a row's largest)
-    return terms * 2.0 ** -24 * (6 * n / 64.0 + 24) + 1e-30
+    return terms * 2.0 ** -24 * (6 * n / 64.0 + 24)
 
 
 @pytest.mark.parametrize("case", CASES)
@@ -109,3 +109,20 @@ def test_values_out_of_range():
     y, _ = _run(case, x, w, None, dy)
     ref, terms = _conv64(case, x, w), _conv64(case, np.abs(x), np.abs(w))
     assert (np.abs(y - ref) <= _bound(terms, 288) + 2.0 ** -149).all()
+
+
+@pytest.mark.parametrize("case", [(4, 32, 28, 28, 72, (3, 3), (1, 1), 2, 1), (2, 40, 27, 27, 70, (3, 3), (1, 1), 1, 1)])
+@pytest.mark.parametrize("size", [1e-28, 1e-33, 1e-36, 1e-40])
+def test_windows_of_tiny_values_beside_ordinary_ones(case, size):
+    """A corner of every map (inputs and output gradients) far below the range of the bf16 parts: what only it reaches is
+    as good as anywhere else, down to the last place of the smallest numbers."""
+    kernels.init(0)
+    x, w, b, dy = _data(case)
+    x[:, :, :12, :11] *= np.float32(size)
+    dy[:, :, :6, :7] *= np.float32(size)
+    y, dx = _run(case, x, w, None, dy)
+    ref, n = _conv64(case, x, w), 9 * case[1]
+    assert (np.abs(y - ref) <= _bound(_conv64(case, np.abs(x), np.abs(w)), n) + 2.0 ** -23 * np.abs(ref) + 2.0 ** -149).all()
+    ref = _grad64(case, w, dy)
+    bound = _bound(_grad64(case, np.abs(w), np.abs(dy)), 9 * case[4]) + 2.0 ** -23 * np.abs(ref) + 2.0 ** -149
+    assert (np.abs(dx - ref) <= bound).all()
