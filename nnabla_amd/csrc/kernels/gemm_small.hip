@@ -10,8 +10,8 @@
 // cost it no roundings.  The wavefronts walk every kWaves-th tile, two tiles in registers and two in flight, and their
 // sums are added in double and rounded once.
 //
-// bf16 products lose bits below 2^-126 and sums overflow near 2^128: rows of A and columns of B whose largest magnitude
-// is outside 2^-50 .. 2^60, or that hold a NaN or an infinity, are marked, and the block recomputes the marked ones'
+// bf16 products lose bits below 2^-126 and sums overflow at 2^128 (up to 2^13 products, of either sign one after the
+// other): rows of A and columns of B whose largest magnitude is outside 2^-50 .. 2^56, or that hold a NaN or an infinity, are marked, and the block recomputes the marked ones'
 // outputs one by one in double (affine.cpp:87-95 propagates NaN and Inf output by output).
 //
 // What bounds it: the splitting, ten vector operations per value (a value of A is split by every column block), and for
@@ -34,7 +34,7 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 constexpr int kWavesPerBlock = 8; // one block to a CU, two wavefronts to a SIMD
 constexpr int kRows = 32, kCols = 64, kTile = 32; // a tile of the contraction: two MFMA steps
 constexpr uint32_t kOutside = 0x80000000u;        // a byte offset past the end of any buffer here
-constexpr uint32_t kLeast = (127u - 50u) << 23, kMost = (127u + 60u) << 23; // magnitudes, as bits
+constexpr uint32_t kLeast = (127u - 50u) << 23, kMost = (127u + 56u) << 23; // magnitudes, as bits
 
 struct SmallArgs {
   const float *a, *b;
@@ -276,7 +276,7 @@ template <int kWaves, bool kAAcross, bool kBAcross> int run_small(const SmallArg
 // x . W, 512 x 2048 x 2048 (two of eight) 46, 4096 x 256 x 1024 (eight of one) 53, past the line: the digits take 43.  `limit` is where
 // the digit path's chain takes the same: see the callers.
 bool gemm_small_applies(int64_t M, int64_t K, int64_t N, int64_t limit) {
-  if (M <= 0 || K <= 0 || N <= 0 || K > (1 << 20) || M > (1 << 24) || N > (1 << 24))
+  if (M <= 0 || K <= 0 || N <= 0 || K > (1 << 13) || M > (1 << 24) || N > (1 << 24))
     return false;
   // 32-bit offsets, the rows of the tiles past the ends included
   if ((K + 64) * N * 4 >= (1ll << 31) || (M + kRows) * (K + 64) * 4 >= (1ll << 31) || (K + 64) * M * 4 >= (1ll << 31) ||

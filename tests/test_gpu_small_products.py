@@ -88,3 +88,16 @@ def test_non_finite_values():
         assert np.array_equal(f(y), f(ref))
     rows, cols = np.isfinite(x).all(1), np.isfinite(W).all(0)
     assert np.array_equal(y[rows][:, cols], clean[rows][:, cols])
+
+
+@pytest.mark.parametrize("size", [2.0 ** 56, 2.0 ** 57, 2.0 ** 60])
+def test_sums_that_cancel_do_not_overflow_on_the_way(size):
+    kernels.init(0)
+    x = torch.full((20, 4096), size, device="cuda")
+    x[:, 2048:] = -size
+    x[7, 5] = 0.0
+    W, b = torch.full((4096, 64), size, device="cuda"), torch.ones(64, device="cuda")
+    y = kernels.affine_digits(x, W, b)
+    want = torch.ones(20, 64, device="cuda")
+    want[7] = -size * size
+    assert torch.equal(y, want)
