@@ -357,11 +357,12 @@ size_t nbla_hip_binary_convolution_workspace_bytes(
  * the host from the shapes alone (no counterpart in nnabla, whose one
  * forward_impl serves every geometry; for tests and for callers that want to
  * know).  plan[0] = output positions per block of the form that keeps the input
- * positions under a block in LDS (0: the geometry takes the gathering product),
- * plan[1] = blocks per sample, plan[2] = input positions the LDS of a block
- * holds, plan[3] = LDS bytes per block, all of the form with 32 positions per
- * block; where a launch has more positions than channels to share out, wider
- * tiles of the same kernel run instead.  Touches no device. */
+ * positions under a block in LDS (0: the geometry takes another form -- the
+ * gathering product, or plain fp32 for many small groups and few channels),
+ * plan[1] = blocks per sample and tile of channels, plan[2] = input positions the
+ * LDS of a block holds, plan[3] = LDS bytes per block, of the tile that the launch
+ * takes (32, 64 or 128 positions at most; all channels at a time, or some of
+ * them after the other where they do not fit).  Touches no device. */
 int nbla_hip_binary_convolution_slab_plan(
     int64_t outer, int64_t C, int nd, const int64_t *in_sp, int64_t O,
     const int64_t *kernel, const int64_t *pad, const int64_t *stride,

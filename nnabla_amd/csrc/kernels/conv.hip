@@ -893,7 +893,8 @@ int nbla_hip_binary_convolution_slab_plan(int64_t outer, int64_t C, int nd, cons
   if (rc)
     return rc;
   plan[0] = plan[1] = plan[2] = plan[3] = 0;
-  conv_slab_plan_summary(g, plan);
+  if (!conv_direct_forward_applies(g))
+    conv_slab_plan_summary(g, plan);
   return NBLA_HIP_OK;
 }
 

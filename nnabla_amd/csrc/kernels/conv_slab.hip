@@ -879,11 +879,11 @@ int64_t slab_longest_run(const ConvGeom &g, int tile_rows, int tiles_per_sample)
   return longest;
 }
 
-bool compute_slab_plan(const ConvGeom &g, SlabPlan &narrow, SlabPlan &p);
+bool compute_slab_plan(const ConvGeom &g, SlabPlan &p);
 
 // The plan of a geometry is asked for several times per call (does it apply, how much workspace, the launches) and
 // sizing the slab walks the tiles of a sample: the last few answers are kept per thread.
-bool make_slab_plan(const ConvGeom &g, SlabPlan &p, bool narrow = false) {
+bool make_slab_plan(const ConvGeom &g, SlabPlan &p) {
   struct Key {
     int64_t outer, C, O, group;
     int in_sp[kMaxSpatial], k[kMaxSpatial], pad[kMaxSpatial], stride[kMaxSpatial], dil[kMaxSpatial];
@@ -898,7 +898,7 @@ bool make_slab_plan(const ConvGeom &g, SlabPlan &p, bool narrow = false) {
   constexpr int kKept = 4; // a forward and a backward geometry alternate in training
   static thread_local bool have[kKept] = {false, false, false, false}, kept_ok[kKept];
   static thread_local Key kept_key[kKept];
-  static thread_local SlabPlan kept_plan[kKept][2]; // the narrowest form and the one that runs
+  static thread_local SlabPlan kept_plan[kKept];
   static thread_local int next = 0;
   Key key;
   key.outer = g.outer, key.C = g.C, key.O = g.O, key.group = g.group;
@@ -907,15 +907,15 @@ bool make_slab_plan(const ConvGeom &g, SlabPlan &p, bool narrow = false) {
     key.dil[i] = g.dil[i];
   for (int e = 0; e < kKept; ++e)
     if (have[e] && key == kept_key[e]) {
-      p = kept_plan[e][narrow ? 0 : 1];
+      p = kept_plan[e];
       return kept_ok[e];
     }
   const int e = next;
   next = (next + 1) % kKept;
-  kept_ok[e] = compute_slab_plan(g, kept_plan[e][0], kept_plan[e][1]);
+  kept_ok[e] = compute_slab_plan(g, kept_plan[e]);
   kept_key[e] = key;
   have[e] = true;
-  p = kept_plan[e][narrow ? 0 : 1];
+  p = kept_plan[e];
   return kept_ok[e];
 }
 
@@ -999,7 +999,7 @@ double slab_form_cost(const ConvGeom &g, const SlabPlan &p) {
   return (double)(blocks / 512) * pair + (rest > 256 ? pair : rest > 0 ? one : 0.0);
 }
 
-bool compute_slab_plan(const ConvGeom &g, SlabPlan &narrow, SlabPlan &p) {
+bool compute_slab_plan(const ConvGeom &g, SlabPlan &p) {
   if (g.k_size > kSlabMaxTaps || g.Cg < 16 || g.in_sp_size >= ((int64_t)1 << 30) ||
       g.out_sp_size >= ((int64_t)1 << 30) || g.Og >= ((int64_t)1 << 24) ||
       (g.Og + kWideGroup) * g.out_sp_size >= ((int64_t)1 << 31))
@@ -1008,15 +1008,11 @@ bool compute_slab_plan(const ConvGeom &g, SlabPlan &narrow, SlabPlan &p) {
   if (g.k_size * cgp > kChunkK) // the epilogue's 32-bit steps hold kChunkK terms
     return false;
   // <4, 1, 2> with the slab filled once is for geometries of little padding (padded channels cost as much as real ones)
-  narrow.form = -1;
   double best = 0.0;
   bool any = false;
   if (cgp * 3 <= g.Cg * 4 && compute_slab_form(g, 0, 1, p)) {
-    narrow = p;
     best = slab_form_cost(g, p);
     any = true;
-  } else {
-    narrow.form = -1;
   }
   for (int form = 1; form < kSlabFormCount; ++form) {
     SlabPlan q;
@@ -1075,7 +1071,7 @@ bool conv_slab_applies(const ConvGeom &g) {
 
 bool conv_slab_plan_summary(const ConvGeom &g, int32_t out[4]) {
   SlabPlan p;
-  if (!make_slab_plan(g, p, true) || p.form < 0)
+  if (!make_slab_plan(g, p))
     return false;
   out[0] = p.tile_rows, out[1] = p.tiles_per_sample, out[2] = p.cap, out[3] = p.total;
   return true;

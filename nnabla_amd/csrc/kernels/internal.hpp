@@ -104,8 +104,8 @@ int launch_conv_dw(const float *dy, const float *x, float *dW, const ConvGeom &g
 // positive to *zero_count when that is not null.  alpha_out and bias belong to the group; y is the whole output.
 bool conv_slab_applies(const ConvGeom &g);
 size_t conv_slab_prepared_bytes(const ConvGeom &g);
-// The figures of the form with 32 windows per block for a geometry it covers: windows per block, blocks per sample, the input positions its LDS
-// holds per block, LDS bytes.  Host only.
+// The figures of the form that a geometry takes, where the kernel covers it: windows per block, blocks per sample (and
+// tile of channels), the input positions its LDS holds per block, LDS bytes.  Host only.
 bool conv_slab_plan_summary(const ConvGeom &g, int32_t out[4]);
 int launch_conv_slab_prepare(const float *Wg, float *Wbg, void *prepared, const ConvGeom &g, float zero_to,
                              hipStream_t stream);

@@ -438,7 +438,7 @@ def binary_weight_convolution(x, W, bias=None, pad=None, stride=None, dilation=N
 def binary_convolution_slab_plan(outer, C, in_sp, O, kernel, pad, stride, dilation, group=1):
     """The host's plan for a binary convolution that keeps a block's input positions in LDS: a dict with the output
     positions per block, blocks per sample, input positions held and LDS bytes, or None where the geometry takes
-    the gathering product.  Shapes only; touches no device."""
+    another form.  Shapes only; touches no device."""
     plan = (ctypes.c_int32 * 4)()
     check(lib().nbla_hip_binary_convolution_slab_plan(
         _i64(outer), _i64(C), ctypes.c_int(len(in_sp)), _shape(in_sp), _i64(O), _shape(kernel), _shape(pad),
