@@ -882,7 +882,8 @@ int64_t slab_longest_run(const ConvGeom &g, int tile_rows, int tiles_per_sample)
 bool compute_slab_plan(const ConvGeom &g, SlabPlan &p);
 
 // The plan of a geometry is asked for several times per call (does it apply, how much workspace, the launches) and
-// sizing the slab walks the tiles of a sample: the last few answers are kept per thread.
+// sizing the slab walks the tiles of a sample once per width of a tile (5 us at 56 x 56, 60 at 224 x 224): the last answers
+// are kept per thread, as many as the layers of a large network have geometries, forward and backward.
 bool make_slab_plan(const ConvGeom &g, SlabPlan &p) {
   struct Key {
     int64_t outer, C, O, group;
@@ -895,26 +896,30 @@ bool make_slab_plan(const ConvGeom &g, SlabPlan &p) {
       return same;
     }
   };
-  constexpr int kKept = 4; // a forward and a backward geometry alternate in training
-  static thread_local bool have[kKept] = {false, false, false, false}, kept_ok[kKept];
+  constexpr int kKept = 64;
+  static thread_local bool kept_ok[kKept];
   static thread_local Key kept_key[kKept];
   static thread_local SlabPlan kept_plan[kKept];
-  static thread_local int next = 0;
+  static thread_local int count = 0, next = 0, last = 0;
   Key key;
   key.outer = g.outer, key.C = g.C, key.O = g.O, key.group = g.group;
   for (int i = 0; i < kMaxSpatial; ++i)
     key.in_sp[i] = g.in_sp[i], key.k[i] = g.k[i], key.pad[i] = g.pad[i], key.stride[i] = g.stride[i],
     key.dil[i] = g.dil[i];
-  for (int e = 0; e < kKept; ++e)
-    if (have[e] && key == kept_key[e]) {
+  for (int i = 0; i < count; ++i) { // from the last answer on: a call asks for the same geometry again and again
+    const int e = (last + i) % count;
+    if (key == kept_key[e]) {
+      last = e;
       p = kept_plan[e];
       return kept_ok[e];
     }
+  }
   const int e = next;
   next = (next + 1) % kKept;
   kept_ok[e] = compute_slab_plan(g, kept_plan[e]);
   kept_key[e] = key;
-  have[e] = true;
+  count = count < kKept ? count + 1 : kKept;
+  last = e;
   p = kept_plan[e];
   return kept_ok[e];
 }
@@ -926,8 +931,21 @@ struct SlabForm {
 constexpr SlabForm kSlabForms[] = {{4, 1, 2}, {4, 2, 1}, {4, 1, 1}, {2, 2, 1}, {1, 4, 2}, {1, 4, 1}};
 constexpr int kSlabFormCount = (int)(sizeof(kSlabForms) / sizeof(kSlabForms[0]));
 
+// The longest run of input positions under a tile, by the tile's windows: the forms share a few widths.
+struct SlabRuns {
+  int tile_rows[3], found = 0;
+  int64_t longest[3];
+  int64_t operator()(const ConvGeom &g, int rows, int tiles_per_sample) {
+    for (int i = 0; i < found; ++i)
+      if (tile_rows[i] == rows)
+        return longest[i];
+    tile_rows[found] = rows;
+    return longest[found++] = slab_longest_run(g, rows, tiles_per_sample);
+  }
+};
+
 // The plan of one form that fills its slab `chunks` times; false when it does not fit the LDS.
-bool compute_slab_form(const ConvGeom &g, int form, int chunks, SlabPlan &p) {
+bool compute_slab_form(const ConvGeom &g, int form, int chunks, SlabRuns &runs, SlabPlan &p) {
   const SlabForm &f = kSlabForms[form];
   const int waves = f.wn * f.wm * f.wk, rows = kSlabRows * f.wm;
   p.form = form;
@@ -952,7 +970,7 @@ bool compute_slab_form(const ConvGeom &g, int form, int chunks, SlabPlan &p) {
   p.ct_chunk = (int)ceil_div(p.ct, chunks);
   p.chunks = (int)ceil_div(p.ct, p.ct_chunk);
   p.pix_stride = kSlabDigits * 32 * p.ct_chunk + kSlabPixPad;
-  const int64_t cap = slab_longest_run(g, p.tile_rows, p.tiles_per_sample);
+  const int64_t cap = runs(g, p.tile_rows, p.tiles_per_sample);
   const int64_t slab_bytes = (cap + 1) * p.pix_stride;
   if (slab_bytes > kSlabLdsLimit)
     return false;
@@ -1008,15 +1026,16 @@ bool compute_slab_plan(const ConvGeom &g, SlabPlan &p) {
   if (g.k_size * cgp > kChunkK) // the epilogue's 32-bit steps hold kChunkK terms
     return false;
   // <4, 1, 2> with the slab filled once is for geometries of little padding (padded channels cost as much as real ones)
+  SlabRuns runs;
   double best = 0.0;
   bool any = false;
-  if (cgp * 3 <= g.Cg * 4 && compute_slab_form(g, 0, 1, p)) {
+  if (cgp * 3 <= g.Cg * 4 && compute_slab_form(g, 0, 1, runs, p)) {
     best = slab_form_cost(g, p);
     any = true;
   }
   for (int form = 1; form < kSlabFormCount; ++form) {
     SlabPlan q;
-    if (!compute_slab_form(g, form, 1, q))
+    if (!compute_slab_form(g, form, 1, runs, q))
       continue;
     const double cost = slab_form_cost(g, q);
     if (!any || cost < best)
@@ -1036,7 +1055,7 @@ bool compute_slab_plan(const ConvGeom &g, SlabPlan &p) {
   for (int form : {1, 2, 3, 5})
     for (int chunks = 2; chunks <= (int)(cgp / 32); ++chunks) {
       SlabPlan q;
-      if (!compute_slab_form(g, form, chunks, q))
+      if (!compute_slab_form(g, form, chunks, runs, q))
         continue;
       const double cost = slab_form_cost(g, q);
       if (cost < best) {

@@ -116,3 +116,18 @@ def test_whole_rows_of_the_output_map_per_block():
     # the run: two output rows' windows span four input rows, plus the position before the first row's first window
     # (origin one column to the left) and the one after the last window's last tap
     assert plan["cap"] == 4 * 14 + 2
+
+
+def test_the_layers_of_a_network_do_not_plan_anew_on_every_call():
+    """Forty geometries one after the other, as a training step asks for them: from the second round on an answer is a
+    look-up (planning one of these anew takes 50 us and more)."""
+    import time
+    geometries = [(1, 64, (224, 224), 64 + 8 * i, (3, 3), (1, 1), (1, 1), (1, 1), 1) for i in range(40)]
+    answers = [kernels.binary_convolution_slab_plan(*g) for g in geometries]
+    best = 1.0
+    for _ in range(5):
+        t = time.perf_counter()
+        again = [kernels.binary_convolution_slab_plan(*g) for g in geometries]
+        best = min(best, (time.perf_counter() - t) / len(geometries))
+        assert again == answers
+    assert best < 30e-6
