@@ -145,21 +145,49 @@ __global__ __launch_bounds__(256) void col2im_gather_unit(const float *__restric
 }
 
 struct ConvBackwardPlan {
-  size_t dyt_off, col_off, a_planes_off, b_planes_off, digits_off, bits_off, prep_off, count_off,
-      flag_off, sums_off, slab_off, dw_off, real_off, total;
+  size_t dyt_off, col_off, a_planes_off, b_planes_off, digits_off, bits_off, prep_off, count_off, slab_off, total;
+  bool direct_dx;  // the input gradient as a gather
+  bool direct_dw;  // the weight gradient in fp32 on the vector units
+  bool product_dw; // on the fp16 matrix cores without an unfolded matrix
 };
 
 size_t larger(size_t a, size_t b) { return a > b ? a : b; }
 
-// One layout for both entry points; every region is reused group after group.
+// One layout for both entry points; every region is reused group after group.  The forms run one after the other in the
+// stream, so each starts at the beginning of the workspace: only the slab convolution's weights are laid out beside the
+// regions of the unfolded forms, whose loop it runs in.  Those are asked for where some call of the geometry unfolds.
 ConvBackwardPlan plan_conv_backward(const ConvGeom &g) {
   ConvBackwardPlan p;
+  const size_t col_bytes = round_up((size_t)g.M * g.Kg * sizeof(float), 256);
+  const bool small_groups = conv_direct_applies(g); // (takes as much scratch memory as there is)
+  p.direct_dx = conv_direct_dx_applies(g);
+  // Few weights under many windows go to the vector units.  Of the geometries that the product on the matrix cores covers
+  // as well only those whose sums lie in short chains there do: the products of two fp16 numbers each are 1.1e-7 off before
+  // any sum, so those would lose bits ([32,32,56,56] x [32,32,3,3] 1.4e-7 off float64 on the vector units in 168 us,
+  // 2.1e-7 on the matrix cores in 41; [64,64,28,28] x [64,64,1,1], whose chains are long there, 3.4e-7 in 121 us and
+  // 1.8e-7 in 30).
+  p.product_dw = conv_dw_applies(g) && !conv_direct_dw_by_pairs(g, (size_t)g.M * g.Kg * sizeof(float));
+  p.direct_dw = !p.product_dw && conv_direct_dw_applies(g);
+  const bool unfolded = small_groups || !(p.product_dw || p.direct_dw) ||
+                        !(p.direct_dx || (conv_real_applies(g, true, false) && conv_real_applies(g, true, true)));
+  ConvGeom t;
+  const size_t slab_bytes = conv_slab_transposed_geom(g, t) ? round_up(conv_slab_prepared_bytes(t), 256) : 0;
+  p.total = larger(conv_dw_workspace_bytes(g), conv_real_workspace_bytes(g, true));
+  // the partial sums of the bias gradient; the scratch memory of the direct forms is the unfolded matrix's
+  p.total = larger(p.total, p.direct_dx || p.direct_dw || col_bytes < 4 * (4096 + (size_t)g.O) ? col_bytes
+                                                                                           : 4 * (4096 + (size_t)g.O));
+  if (!unfolded) {
+    p.dyt_off = p.col_off = p.a_planes_off = p.b_planes_off = p.digits_off = p.bits_off = p.prep_off = p.count_off = 0;
+    p.slab_off = 0;
+    p.total = round_up(larger(p.total, slab_bytes), 256);
+    return p;
+  }
   size_t off = 0;
   const size_t dyt_bytes = round_up((size_t)g.M * g.Og * sizeof(float), 256);
   p.dyt_off = off;
   off += dyt_bytes;
   p.col_off = off; // unfolded input [M, Kg], and the unfolded gradient [outer][Kg][L]
-  off += round_up((size_t)g.M * g.Kg * sizeof(float), 256);
+  off += col_bytes;
   p.a_planes_off = off; // dyt^T for dW (rows o, contraction m) or dyt for dx (rows m, contraction o)
   off += round_up(larger(nbla_hip_digit_operand_bytes(g.M, g.Og), nbla_hip_digit_operand_bytes(g.Og, g.M)), 256);
   p.b_planes_off = off; // col(x) (columns kk, contraction m) or w (columns kk, contraction o)
@@ -172,21 +200,9 @@ ConvBackwardPlan plan_conv_backward(const ConvGeom &g) {
   off += round_up(nbla_hip_binarize_workspace_bytes(g.Og, g.Kg), 256);
   p.count_off = off;
   off += 256;
-  p.flag_off = off;
-  off += 256;
-  p.sums_off = off;
-  off += round_up(column_sums_workspace_bytes(g.M, g.Og), 256);
   p.slab_off = off; // packed bits of the transposed convolution, when the input gradient takes that form
-  {
-    ConvGeom t;
-    if (conv_slab_transposed_geom(g, t))
-      off += round_up(conv_slab_prepared_bytes(t), 256);
-  }
-  p.dw_off = off; // maxima, scales and partial results of the weight gradient on the fp16 matrix cores
-  off += round_up(conv_dw_workspace_bytes(g), 256);
-  p.real_off = off; // prepared weights of the input gradient on the bf16 matrix cores
-  off += round_up(conv_real_workspace_bytes(g, true), 256);
-  p.total = off;
+  off += slab_bytes;
+  p.total = round_up(larger(p.total, off), 256);
   return p;
 }
 
@@ -231,9 +247,10 @@ int conv_backward(const float *dy, const float *x, const float *W, const float *
   if (rc)
     return rc;
   hipStream_t stream = as_stream(stream_);
+  const bool representable = (zero_to == 1.0f || zero_to == -1.0f);
   if (conv_direct_applies(g)) { // many small groups: all of them in one launch per gradient
     // the forward multiplied with Wb = Sign(W) (* alpha): the signs passed in, or taken from W on the way
-    if (binary && !Wb && !(zero_to == 1.0f || zero_to == -1.0f))
+    if (binary && !Wb && !representable)
       return fail(NBLA_HIP_ERR_VALUE, "the binarised weights are needed when Sign(0) is neither +1 nor -1.");
     return launch_conv_direct_backward(dy, x, (binary && Wb) ? Wb : W, binary ? alpha : nullptr, dx, dW, db, g, accum_x,
                                        accum_w, accum_b, binary && !Wb, zero_to, static_cast<float *>(workspace),
@@ -244,30 +261,26 @@ int conv_backward(const float *dy, const float *x, const float *W, const float *
   float *col = reinterpret_cast<float *>(base + p.col_off);
   int *count = reinterpret_cast<int *>(base + p.count_off);
   uint32_t *bits = reinterpret_cast<uint32_t *>(base + p.bits_off);
-  const bool representable = (zero_to == 1.0f || zero_to == -1.0f);
   const int64_t L = g.out_sp_size;
+  if (dx && binary && !Wb && !representable)
+    return fail(NBLA_HIP_ERR_VALUE, "the binarised weights are needed when Sign(0) is neither +1 nor -1.");
   // The input gradient of a binary convolution of unit stride is itself a binary convolution (dy in the place of x,
   // channels' roles exchanged, taps flipped): it takes the product that keeps input positions in LDS.
   ConvGeom gt;
   bool dx_slab = dx && binary && representable && conv_slab_transposed_geom(g, gt);
   // a first layer's input gradient (few input channels, little work) as a gather; its scratch memory is the unfolded
   // gradient's buffer, used by the next launches only afterwards in the stream
-  if (dx && conv_direct_dx_applies(g) && (!binary || Wb || representable)) {
+  if (dx && p.direct_dx) {
     rc = launch_conv_direct_dx(dy, (binary && Wb) ? Wb : W, binary ? alpha : nullptr, dx, g, accum_x, binary && !Wb,
                                zero_to, col, (size_t)g.M * g.Kg * sizeof(float), stream);
     if (rc)
       return rc;
     dx = nullptr, dx_slab = false;
   }
-  // few weights under many windows: the weight gradient in fp32 straight from dy and x, all groups at once (its
-  // partial results lie in the unfolded gradient's buffer, so it runs before the loop that fills that buffer).  Of the
-  // geometries that the product on the matrix cores below covers, only those whose sums lie in short chains here are: the
-  // products of two fp16 numbers each are 1.1e-7 off before any sum, so there they would lose bits ([32,32,56,56] x
-  // [32,32,3,3] 1.4e-7 off float64 here in 168 us, 2.1e-7 there in 41; [64,64,28,28] x [64,64,1,1], whose chains are long
-  // here, 3.4e-7 in 121 us and 1.8e-7 in 30).
+  // few weights under many windows: the weight gradient in fp32 straight from dy and x, all groups at once (its partial
+  // results lie in the unfolded gradient's buffer, so it runs before the loop that fills that buffer)
   const size_t col_bytes = (size_t)g.M * g.Kg * sizeof(float);
-  const bool dw_product = conv_dw_applies(g) && !conv_direct_dw_by_pairs(g, col_bytes);
-  if (dW && !dw_product && conv_direct_dw_applies(g)) {
+  if (dW && p.direct_dw) {
     rc = launch_conv_direct_dw(dy, x, dW, g, accum_w, col, col_bytes, stream);
     if (rc)
       return rc;
@@ -276,23 +289,23 @@ int conv_backward(const float *dy, const float *x, const float *W, const float *
   // the bias gradient straight from dy, every group at once (partial sums in the same buffer, after the weight
   // gradient's in the stream)
   if (db) {
-    rc = launch_conv_direct_db(dy, db, g, accum_b, col, (size_t)g.M * g.Kg * sizeof(float), stream);
+    rc = launch_conv_direct_db(dy, db, g, accum_b, col, col_bytes, stream);
     if (rc)
       return rc;
     db = nullptr;
   }
-  if (dW && dw_product) { // kernels of width 1, 3, 5 with half their width of padding: no unfolded matrix
+  if (dW && p.product_dw) { // kernels of width 1, 3, 5 with half their width of padding: no unfolded matrix
     for (int64_t grp = 0; grp < g.group; ++grp) {
-      rc = launch_conv_dw(dy, x, dW, g, grp, accum_w, base + p.dw_off, conv_dw_workspace_bytes(g), stream);
+      rc = launch_conv_dw(dy, x, dW, g, grp, accum_w, base, conv_dw_workspace_bytes(g), stream);
       if (rc)
         return rc;
     }
     dW = nullptr;
   }
-  if (dx && !dx_slab && conv_real_applies(g, true, binary) && (!binary || Wb || representable)) { // no unfolded gradient
+  if (dx && !dx_slab && conv_real_applies(g, true, binary)) { // no unfolded gradient
     for (int64_t grp = 0; grp < g.group; ++grp) {
       rc = launch_conv_real(dy, ((binary && Wb) ? Wb : W) + grp * g.Og * g.Kg, nullptr, dx, g, true, grp, accum_x,
-                            binary && alpha ? alpha + grp * g.Og : nullptr, binary && !Wb, zero_to, base + p.real_off,
+                            binary && alpha ? alpha + grp * g.Og : nullptr, binary && !Wb, zero_to, base,
                             conv_real_workspace_bytes(g, true), stream);
       if (rc)
         return rc;
@@ -334,8 +347,6 @@ int conv_backward(const float *dy, const float *x, const float *W, const float *
           // on the device by the pass above) the unfolded gradient is recomputed in fp32 from the forward's signs,
           //   col[m, kk] = sum_o (dyt[m, o] alpha[o]) Wb[o, kk],
           // by a launch that leaves at once otherwise.  The host never reads the count.
-          if (!Wb)
-            return fail(NBLA_HIP_ERR_VALUE, "the binarised weights are needed when Sign(0) is neither +1 nor -1.");
           rc = launch_gemm_f32_mapped(dyt, Wb + grp * g.Og * g.Kg, false, nullptr, nullptr, col, g.M, g.Og, g.Kg, L,
                                       g.Kg * L, L, stream, count, ag, false);
         }
