@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
 # batch, channels, height, width, maps, kernel, pad, stride, group
 CASES = [(1, 16, 7, 7, 16, (3, 3), (1, 1), 1, 1), (3, 17, 9, 5, 65, (3, 3), (1, 1), 2, 1), (2, 33, 14, 14, 70, (1, 1), (0, 0), 2, 1),
          (5, 48, 4, 6, 64, (5, 5), (2, 2), 1, 1), (2, 24, 13, 27, 31, (5, 5), (2, 2), 2, 1), (2, 32, 12, 11, 40, (2, 3), (1, 0), 3, 1),
-         (9, 20, 3, 3, 33, (3, 3), (0, 0), 1, 1), (2, 64, 20, 56, 48, (3, 3), (1, 1), 2, 2), (1, 40, 1, 50, 24, (1, 5), (0, 2), 1, 1)]
+         (9, 20, 3, 3, 33, (3, 3), (0, 0), 1, 1), (2, 64, 20, 56, 48, (3, 3), (1, 1), 2, 2), (1, 40, 1, 50, 24, (1, 5), (0, 2), 1, 1),
+         (8, 128, 56, 56, 64, (5, 5), (2, 2), 2, 1)]  # the longest runs of input a block stages
 
 
 def _data(case):
