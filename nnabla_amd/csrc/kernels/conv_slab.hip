@@ -40,8 +40,8 @@
 // largest value is more than kSlabLevel binades below that are finished by further rounds of the block, each under the
 // scale of the largest of the windows left: so an element is off by at most 2^-27 of the largest value of its own window,
 // whatever else lies in the slab.  (On inputs of one magnitude no block has a second round, and the window maxima, the test
-// for windows left and the second copy of the product cost 2 to 4 %: [32,64,56,56] x [64,64,3,3] 47.7 -> 49.1 us with the
-// host's call, [32,256,14,14] x [256,256,3,3] 29.3 -> 29.9.  One loop around a single copy of the product costs 8 to 11 %:
+// for windows left and the second copy of the product cost 2 to 3 %: [32,64,56,56] x [64,64,3,3] 46.8 -> 48.0 us with the
+// host's call, [32,256,14,14] x [256,256,3,3] 29.3 -> 29.8; 49.1 and 29.9 with the windows summed behind the product.  One loop around a single copy of the product costs 8 to 11 %:
 // the loop's values crowd the product's registers.)  A window that holds a NaN or an
 // infinity gives NaN in all its outputs; other windows of the slab are not affected (such values are left out of the
 // scale and read as 0).
@@ -426,6 +426,9 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
 #pragma unroll
       for (int q = 0; q < 16; ++q)
         acc[d][j][q] = 0;
+  long long rowsum = 0; // the sum of q over the lane's window
+  uint32_t left = 0u;
+  bool rowbad = false, finish = false; // the window holds a NaN or an infinity; is finished by this round
   for (int chunk = 0; chunk < chunks; ++chunk) {
     if (chunk > 0 || again.value) {
       __syncthreads(); // every wavefront is through with the chunk before
@@ -433,6 +436,42 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
         take_chunk(chunk);
       convert_chunk();
       __syncthreads();
+    }
+    if (chunk == chunks - 1) {
+      // Every wavefront adds up the windows it finishes from the pixels' sums, which are complete since the barrier just
+      // passed; its lanes l and l + 32 share a window and take every second tap each, five reads in flight at a time.
+      uint32_t rowmax = 0u;
+      for (int t0 = half; t0 < taps; t0 += 10) {
+        uint32_t idx[5];
+#pragma unroll
+        for (int j = 0; j < 5; ++j) // (past the last tap: the zero pixel)
+          idx[j] = t0 + 2 * j < taps ? s_rowpix[(t0 + 2 * j) * kRows + row] : 0u;
+#pragma unroll
+        for (int j = 0; j < 5; ++j) {
+          rowsum += s_pixsum[idx[j]];
+          rowmax = max(rowmax, s_pixmax[idx[j]]);
+        }
+      }
+      rowsum += __shfl_xor(rowsum, 32);
+      rowmax = max(rowmax, (uint32_t)__shfl_xor((int)rowmax, 32));
+      rowbad = rowmax >= 0x7f800000u;
+      const bool todo = row_in && (!again.value || (rowmax != 0u && rowmax <= limit)); // (larger ones are finished)
+      // (a window all zero is finished by any scale)
+      finish = todo && (rowbad || rowmax == 0u ||
+                        binade_exponent(binade_of(rowmax)) + kSlabLevel >= binade_exponent(binade_of(limit)));
+      uint32_t mine = todo && !finish ? rowmax : 0u;
+      if (__ballot(mine != 0u) != 0) {
+#pragma unroll
+        for (int off = 16; off >= 1; off >>= 1)
+          mine = max(mine, (uint32_t)__shfl_xor((int)mine, off));
+      }
+      if (lane == 0)
+        s_misc[8 + wave] = (int)mine;
+      __syncthreads();
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w)
+        left = max(left, (uint32_t)s_misc[8 + w]);
+      left = __builtin_amdgcn_readfirstlane(left);
     }
     const int ctn = kChunked ? groups16 >> 1 : CT; // channel tiles of the chunk
     const int nk = (taps * ctn - wk + WK - 1) / WK;
@@ -540,41 +579,6 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
     }
   }
 
-  // The sum of q over the lane's window and its largest magnitude: every wavefront adds up the windows it
-  // finishes from the pixels' sums, which are complete since the barrier in front of the (last) product; its lanes
-  // l and l + 32 share a window and take every second tap each, five reads in flight at a time.
-  long long rowsum = 0;
-  uint32_t rowmax = 0u;
-  for (int t0 = half; t0 < taps; t0 += 10) {
-    uint32_t idx[5];
-#pragma unroll
-    for (int j = 0; j < 5; ++j) // (past the last tap: the zero pixel)
-      idx[j] = t0 + 2 * j < taps ? s_rowpix[(t0 + 2 * j) * kRows + row] : 0u;
-#pragma unroll
-    for (int j = 0; j < 5; ++j) {
-      rowsum += s_pixsum[idx[j]];
-      rowmax = max(rowmax, s_pixmax[idx[j]]);
-    }
-  }
-  rowsum += __shfl_xor(rowsum, 32);
-  rowmax = max(rowmax, (uint32_t)__shfl_xor((int)rowmax, 32));
-  const bool rowbad = rowmax >= 0x7f800000u; // a NaN or an infinity
-  // (a window all zero is finished by any scale)
-  const bool todo = row_in && (!again.value || (rowmax != 0u && rowmax <= limit)); // (larger ones are finished)
-  const bool finish = todo && (rowbad || rowmax == 0u ||
-                               binade_exponent(binade_of(rowmax)) + kSlabLevel >= binade_exponent(binade_of(limit)));
-  {
-    uint32_t left = todo && !finish ? rowmax : 0u;
-    if (__ballot(left != 0u) != 0) {
-#pragma unroll
-      for (int off = 16; off >= 1; off >>= 1)
-        left = max(left, (uint32_t)__shfl_xor((int)left, off));
-    }
-    if (lane == 0)
-      s_misc[8 + wave] = (int)left;
-  }
-  __syncthreads(); // (and every wavefront has left the product)
-
   // ---- 3. (WK == 2) the two k groups' accumulators added exactly through LDS (the planes are free once every
   // wavefront has left the loop), one digit at a time, in two alternating areas: a wavefront hands the fragment it does
   // not finish (1 - wk) to its partner in the other k group and adds the partner's copy of fragment wk to its own.
@@ -582,6 +586,7 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
   if constexpr (WK == 2) {
     uint4_t *red = reinterpret_cast<uint4_t *>(smem);
     const int mine = wave * 4 * 64 + lane, theirs = (wave ^ (WN * WM)) * 4 * 64 + lane;
+    __syncthreads();
 #pragma unroll
     for (int d = 0; d < kSlabDigits; ++d) {
       uint4_t *area = red + (d & 1) * (kWaves * kSlabReduceBytes / 16);
@@ -690,11 +695,6 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
   }
   }
   }
-  // ---- 5. windows left?
-  uint32_t left = 0u;
-#pragma unroll
-  for (int w = 0; w < kWaves; ++w)
-    left = max(left, (uint32_t)s_misc[8 + w]);
   return left;
   };
   uint32_t left = round(std::false_type{});
