@@ -6,8 +6,8 @@
 // [2^14, 2^15), is the sum of two fp16 numbers, hi = fp16(v) and lo = fp16(v - hi), exactly or to one unit of its last
 // fp32 place (v - hi has at most 12 bits and a sign) for every value within 2^-18 of the channel's largest; below that to
 // 2^-39 of the largest.  Three products (hi hi, hi lo, lo hi) accumulate in fp32 inside the matrix instruction; the
-// fourth is below 2^-22 of the product.  A block's sums (at most kDwChain positions, half of them in each of two
-// wavefronts) go to memory as fp32 and are added in a fixed order in double, so the error does not grow with the batch.
+// fourth is below 2^-22 of the product.  A block's sums (kDwChain positions at most unless their partial sums would pass
+// 2 GiB; half of them in each of two wavefronts) go to memory as fp32 and are added in a fixed order in double, so the error does not grow with the batch.
 // With chains as long as 512 places for blocks made them (12544 positions at [64,512,28,28] x [512,512,3,3]) that gradient
 // was 1.0e-6 off float64 for random signs and 3.3e-7 for terms of one sign; now 2.9e-7 and 3.8e-8, at 860 -> 970 us.
 // Against float64 the gradient of [32,64,56,56] x [64,64,3,3] is off by 2.5e-7 of its norm
@@ -565,11 +565,14 @@ bool make_dw_plan(const ConvGeom &g, DwPlan &p) {
     return false;
   p.tiles = (int)tiles;
   // two blocks per CU: as many splits as fill 512 places once -- or several times, where a block would otherwise sum more
-  // than kDwChain positions -- each with the same number of tiles (the last fewer)
+  // than kDwChain positions (and the splits' sums stay below 2 GiB) -- each with the same number of tiles (the last fewer)
   const int64_t cells = (int64_t)p.ot * p.ct * p.kg;
   const int64_t most = p.Q * 8 < kDwChain ? kDwChain / (p.Q * 8) : 1; // tiles of a block
   const int64_t rounds = ceil_div(cells * ceil_div(tiles, most), 512);
   int64_t splits = 512 * rounds / cells;
+  const int64_t room = (((int64_t)1 << 31) - 1) / (4 * g.Og * g.Kg);
+  if (splits > room)
+    splits = room;
   if (splits < 1)
     splits = 1;
   if (splits > tiles)

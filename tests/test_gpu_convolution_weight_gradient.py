@@ -160,3 +160,20 @@ def test_few_weights_keep_their_fp32_products(xs, O, k):
         cols = torch.nn.functional.unfold(x[n:n + 1].double(), k, padding=k // 2)[0]
         want += dy[n].double().flatten(1) @ cols.t().contiguous()
     assert float((dW.double().flatten(1) - want).norm() / want.norm()) <= 2.0e-7
+
+
+def test_partial_sums_up_to_2_gib():
+    """Blocks of 1024 positions would write 3.7 GB: 227 splits of 1792 positions instead (1e-7 for the products and
+    0.29 * 2^-23.5 * sqrt(672 / 2) for the chains: 4.6e-7; digit operands are 1.3e-6 off)."""
+    kernels.init(0)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(9)
+    x = torch.randn(128, 512, 56, 56, device="cuda", generator=gen)
+    dy = torch.randn(128, 512, 56, 56, device="cuda", generator=gen)
+    W = torch.empty(512, 512, 3, 3, device="cuda")
+    dW = kernels.convolution_backward(dy, x, W, (1, 1), (1, 1), (1, 1), 1, want=(False, True, False))[1]
+    want = torch.zeros(8, 18, dtype=torch.float64, device="cuda")
+    for n in range(128):
+        cols = torch.nn.functional.unfold(x[n:n + 1, ::256].double(), 3, padding=1)[0]
+        want += dy[n, ::64].flatten(1).double() @ cols.t().contiguous()
+    assert float((dW[::64, ::256].reshape(8, -1).double() - want).norm() / want.norm()) <= 8e-7
