@@ -26,6 +26,7 @@
 //
 // Positions whose input window holds a NaN, an infinity, a magnitude of 2^100 or more or nothing above 2^-90, and rows of
 // weights with a NaN or an infinity, are recomputed one by one in double.
+#include "bf16_parts.hpp"
 #include "common.hpp"
 #include "conv_geom.hpp"
 #include "gemm_layout.hpp"
@@ -71,21 +72,6 @@ struct RealArgs {
   RealClass cls[kMaxClasses];
   signed char ty[kMaxTaps], tx[kMaxTaps], tap[kMaxTaps];
 };
-
-__device__ __forceinline__ void split3_pair(float a, float b, uint32_t &hi, uint32_t &mid, uint32_t &lo) {
-  uint32_t h[2], m[2], l[2];
-  const float v[2] = {a, b};
-#pragma unroll
-  for (int c = 0; c < 2; ++c) { // v = hi + mid + lo exactly, eight bits each
-    h[c] = (__float_as_uint(v[c]) + 0x8000u) & 0xffff0000u;
-    const float r = v[c] - __uint_as_float(h[c]);
-    m[c] = (__float_as_uint(r) + 0x8000u) & 0xffff0000u;
-    l[c] = __float_as_uint(r - __uint_as_float(m[c]));
-  }
-  hi = __builtin_amdgcn_perm(h[1], h[0], 0x07060302u);
-  mid = __builtin_amdgcn_perm(m[1], m[0], 0x07060302u);
-  lo = __builtin_amdgcn_perm(l[1], l[0], 0x07060302u);
-}
 
 // A weight as it takes part: itself or its sign, times alpha.
 __device__ __forceinline__ float weight_value(float v, bool scaled, float alpha, int signs, float zero_to) {

@@ -19,6 +19,7 @@
 // 35.2 -> 7.5 us, 512^3 40.6 -> 9.5, 200 x 1000 x 1000 43.7 -> 14.8, 1024^3 53 -> 29, 128 x 4096 x 4096 88 -> 45; weight
 // gradient at 200 x 1000 x 1000 36.4 -> 13.3, input gradient 31.9 -> 15.3.  Off float64 (relative, 2-norm): 3e-8 to 1.0e-7
 // where the digits are 1.6e-7 to 8.6e-7 off.
+#include "bf16_parts.hpp"
 #include "common.hpp"
 #include "gemm_layout.hpp"
 #include "internal.hpp"
@@ -72,22 +73,13 @@ __device__ __forceinline__ void load_tile(const __amdgpu_buffer_rsrc_t rsrc, int
   }
 }
 
-// v = hi + mid + lo exactly, eight bits each (hi and mid rounded half up in magnitude)
+// eight of the sixteen values (s: which) as bf16 operands
 __device__ __forceinline__ void split3(const float (&v)[16], int s, uint4_t &hi, uint4_t &mid, uint4_t &lo) {
 #pragma unroll
   for (int p = 0; p < 4; ++p) {
-    uint32_t h[2], m[2], l[2];
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const float w = v[8 * s + 2 * p + c];
-      h[c] = (__float_as_uint(w) + 0x8000u) & 0xffff0000u;
-      const float r = w - __uint_as_float(h[c]);
-      m[c] = (__float_as_uint(r) + 0x8000u) & 0xffff0000u;
-      l[c] = __float_as_uint(r - __uint_as_float(m[c]));
-    }
-    hi[p] = __builtin_amdgcn_perm(h[1], h[0], 0x07060302u);
-    mid[p] = __builtin_amdgcn_perm(m[1], m[0], 0x07060302u);
-    lo[p] = __builtin_amdgcn_perm(l[1], l[0], 0x07060302u);
+    uint32_t h, m, l;
+    split3_pair(v[8 * s + 2 * p], v[8 * s + 2 * p + 1], h, m, l);
+    hi[p] = h, mid[p] = m, lo[p] = l;
   }
 }
 

@@ -21,24 +21,6 @@ constexpr int kTile = kBlock * kUnroll; // float4 per block at full unroll
 
 // Streaming access pattern that measured best on MI355X for a read-once/write-once map: ordinary 128-bit loads,
 // nontemporal 128-bit stores.
-__device__ __forceinline__ float4_t load4(const float *p) { return *reinterpret_cast<const float4_t *>(p); }
-__device__ __forceinline__ void store4(float *p, float4_t v) {
-  __builtin_nontemporal_store(v, reinterpret_cast<float4_t *>(p));
-}
-typedef float float4_u __attribute__((ext_vector_type(4), aligned(4)));
-// the same at any multiple of four bytes; the store goes through the caches, which put its partial lines together
-template <bool kAligned> __device__ __forceinline__ float4_t load4_as(const float *p) {
-  if (kAligned)
-    return load4(p);
-  return *reinterpret_cast<const float4_u *>(p);
-}
-template <bool kAligned> __device__ __forceinline__ void store4_as(float *p, float4_t v) {
-  if (kAligned)
-    store4(p, v);
-  else
-    *reinterpret_cast<float4_u *>(p) = v;
-}
-
 // Generic driver: applies `op` (a functor float -> float) to `size` elements.
 // The vector body covers size/4 float4s; the tail (size % 4) is done by block 0.
 template <typename Op, int kUnroll> __global__ __launch_bounds__(kBlock) void map_vec4(const float *__restrict__ x, float *__restrict__ y, size_t n4, size_t size, Op op) {

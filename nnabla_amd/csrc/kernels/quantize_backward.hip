@@ -13,24 +13,6 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kUnroll = 4;
 
-__device__ __forceinline__ float4_t load4(const float *p) { return *reinterpret_cast<const float4_t *>(p); }
-__device__ __forceinline__ void store4(float *p, float4_t v) {
-  __builtin_nontemporal_store(v, reinterpret_cast<float4_t *>(p));
-}
-typedef float float4_u __attribute__((ext_vector_type(4), aligned(4)));
-// the same at any multiple of four bytes; the store goes through the caches, which put its partial lines together
-template <bool kAligned> __device__ __forceinline__ float4_t load4_as(const float *p) {
-  if (kAligned)
-    return load4(p);
-  return *reinterpret_cast<const float4_u *>(p);
-}
-template <bool kAligned> __device__ __forceinline__ void store4_as(float *p, float4_t v) {
-  if (kAligned)
-    store4(p, v);
-  else
-    *reinterpret_cast<float4_u *>(p) = v;
-}
-
 // dx[i] = op(dy[i], x[i], i) (+ dx[i] when kAccum).  `op` returns the gradient contribution; kUseX tells whether x is
 // read at all.
 template <typename Op, bool kAccum, bool kUseX>

@@ -6,6 +6,25 @@ namespace nbla_hip {
 
 typedef float float4_t __attribute__((ext_vector_type(4)));
 
+// Four elements at a 16-byte aligned address, and stored past the caches.
+__device__ __forceinline__ float4_t load4(const float *p) { return *reinterpret_cast<const float4_t *>(p); }
+__device__ __forceinline__ void store4(float *p, float4_t v) {
+  __builtin_nontemporal_store(v, reinterpret_cast<float4_t *>(p));
+}
+typedef float float4_u __attribute__((ext_vector_type(4), aligned(4)));
+// the same at any multiple of four bytes; the store goes through the caches, which put its partial lines together
+template <bool kAligned> __device__ __forceinline__ float4_t load4_as(const float *p) {
+  if (kAligned)
+    return load4(p);
+  return *reinterpret_cast<const float4_u *>(p);
+}
+template <bool kAligned> __device__ __forceinline__ void store4_as(float *p, float4_t v) {
+  if (kAligned)
+    store4(p, v);
+  else
+    *reinterpret_cast<float4_u *>(p) = v;
+}
+
 // (x shape, q shape) collapsed to element index = (r0 * K + k) * R1 + r1 with k
 // the kept (per-channel) index and r0, r1 the reduced ones.
 struct MinMaxLayout {
