@@ -7,8 +7,12 @@
 // sums in integer arithmetic, converts once and applies the two scales, so the result does not depend on the order
 // of summation.  Used for the weight gradients (x^T . dy), where neither factor is a sign matrix.
 //
-// Tiling: 128 x 128 outputs per block of four wavefronts (2 x 2, 64 x 64 each: 2 x 2 fragments x 3 accumulators =
-// 192 registers), k in tiles of 32 (one v_mfma_i32_32x32x32_i8 fragment).
+// Tiling: 128 x 128 outputs per block of four wavefronts (2 x 2, 64 x 64 each: 4 x 4 tiles of
+// v_mfma_i32_16x16x64_i8 x 3 accumulators = 192 registers), k in steps of 64 (two k tiles of the operands).  Why the
+// 16 x 16 instruction: on large products the part runs at its power limit, and a loop of nothing but these
+// instructions sustains 3.9 POP/s on random digits where the 32 x 32 x 32 form, which moves twice the accumulator bytes
+// per operation, sustains 3.2 to 3.4.  The weight gradient of 4096 x 4096 x 11008: 870 us with the 32 x 32 x 32 form in
+// the same tiles (2.55 POP/s), 760 with this one; 1024 x 4096 x 4096 against one-digit rows: 28.0 and 24.1.
 #include "common.hpp"
 #include "copy_pipeline.hpp"
 #include "gemm_layout.hpp"
@@ -20,7 +24,8 @@ namespace nbla_hip {
 namespace {
 
 typedef int i32x4_t __attribute__((ext_vector_type(4)));
-typedef int i32x16_t __attribute__((ext_vector_type(16)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x2_u __attribute__((ext_vector_type(2), aligned(4))); // a 64-bit access at any multiple of four bytes
 typedef uint32_t uint4_t __attribute__((ext_vector_type(4)));
 
 struct GemmDigitsArgs {
@@ -38,31 +43,21 @@ struct GemmDigitsArgs {
 };
 
 constexpr int kBM = 128, kBN = 128, kThreads = 256, kWaves = 4;
-constexpr int kSegs = 4;               // 32-row fragments per tile side
-constexpr int kSegVec = kDigits * 64;  // uint4 per fragment and k step
-constexpr int kSideVec = kSegs * kSegVec;
-constexpr int kStageBytes = 2 * kSideVec * 16; // 24 KiB: the A and B fragments of one k tile
-constexpr int kChunks = 2 * kSegs * kDigits;   // 1 KiB copies per k tile
-constexpr int kPerWave = kChunks / kWaves;     // 6
-// Three LDS stages when two blocks share a CU; six (the whole LDS) when the output has so few tiles that a CU holds
-// one block anyway: with one wavefront per SIMD a k tile is multiplied in a few hundred cycles and the copies need
-// the longer head start to cover the memory latency.
-constexpr int kStagesShared = 3, kStagesAlone = 6;
+constexpr int kSegs = 4;              // 32-row fragments per tile side
+constexpr int kSegVec = kDigits * 64; // uint4 per fragment and k tile
+// A k step is multiplied in phases, each of which needs two parts: one digit of one side (four row blocks x two k
+// tiles, 8 KiB).  A phase's two parts lie in one LDS buffer; kStages buffers, so the copies of a phase are issued
+// three phases before it (the phases of two k tiles of all digits: 4096 cycles of the matrix pipe with two blocks per
+// CU).  64 KiB of LDS per block, two blocks per CU (or two k groups in one).
+constexpr int kStages = 4;
+constexpr int kPartBytes = kSegs * 2 * kFragBytes, kStageBytes = 2 * kPartBytes;
+constexpr int kCopies = kStageBytes / kFragBytes / kWaves; // 1 KiB copies per wavefront and phase
 
-// Which of a wavefront's kPerWave copy slots a call of copy_next issues (the list of a k tile is ordered so that
-// every form of the product needs a prefix of each wavefront's share), and how many that makes: the unit in which the
-// loop's wait counts copies in flight.
-constexpr bool copy_slot_used(int p, bool one_a, bool narrow, int groups) {
-  const int all_waves = kWaves * groups, per_tile = kChunks / all_waves;
-  return one_a ? p < (2 * kSegs / all_waves) * groups
-               : !(narrow && p % per_tile >= (kSegs * kDigits + kSegs) / all_waves);
-}
-constexpr int copies_per_call(bool one_a, bool narrow, int groups) {
-  int n = 0;
-  for (int p = 0; p < kPerWave; ++p)
-    n += copy_slot_used(p, one_a, narrow, groups) ? 1 : 0;
-  return n;
-}
+// Phases per k step: all nine digit pairs' leading six: {a0 b0} {a0 b2, a0 b1} {a1 b0, a1 b1, a2 b0}; one-digit B:
+// {a0 b} {a1 b, a2 b}; both one-digit: {a b}.
+constexpr int phases_per_step(bool one_a, bool narrow) { return one_a ? 1 : (narrow ? 2 : 3); }
+// Copies that a wavefront issues per phase, whatever the form: the unit in which the loop's wait counts.
+constexpr int copies_per_call(bool /*one_a*/, bool /*narrow*/, int /*groups*/) { return kCopies; }
 
 // Workgroup barrier without the memory fence of __syncthreads() (which would wait for every global -> LDS copy in
 // flight, including those of later k tiles); the waits that matter are explicit.
@@ -75,10 +70,15 @@ constexpr int copies_per_call(bool one_a, bool narrow, int groups) {
 // vmcnt(n) with the other counters left alone (gfx9 encoding: vmcnt in bits 3:0 and 15:14).
 #define NBLA_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xf) | (((n) >> 4) << 14) | (0x7 << 4) | (0xf << 8))
 
-// Staging: global -> LDS copies bypass the registers (one wavefront instruction moves one 1 KiB fragment); kStages
-// LDS buffers hold consecutive k tiles and the copy of tile t + kStages - 1 is issued while tile t is multiplied.  Two blocks
-// share a CU (256 registers per lane: 192 accumulators + the 12 operand quads of a tile), so one block's LDS reads
-// and barrier waits are covered by the other's MFMAs.
+// Staging: global -> LDS copies bypass the registers (one wavefront instruction moves one 1 KiB fragment of the
+// operand).  Two blocks share a CU (256 registers per lane: 192 accumulators, at most 13 operand quads), so one
+// block's LDS reads and barrier waits are covered by the other's MFMAs.
+//
+// A 16 x 64 fragment is put together from the operands' 32 x 32 ones by the LDS address alone: lane l reads row
+// l % 16 of half h of a row block, k slots (l / 16) % 2 of k tile l / 32 of the step -- the same 64 k for A and B,
+// in an order of their own.  The copy of B sends row 2 r + h of a row block to where half h's row r is read, so a
+// lane's accumulators of the two halves are neighbouring columns and are stored as one 64-bit word.
+//
 // kNarrow: the B operand holds every value in its lowest digit alone (a small integer): three products
 // a_t x b2 -> accumulator t, nothing dropped, and only the lowest-digit fragments of B are copied.
 // kTopB (a form of kNarrow): every row of the tile's B row blocks is a one-digit row of a row-scaled operand (its value
@@ -86,21 +86,19 @@ constexpr int copies_per_call(bool one_a, bool narrow, int groups) {
 // b2, and the factor 2^16 of the top digit in the epilogue.
 // kOneA (only with kNarrow): every row of the tile's A row blocks is a one-digit row (gemm_layout.hpp: its value sits
 // in the top digit): a single product a0 x b2 -> accumulator 0, and only the top-digit fragments of A and the
-// lowest-digit fragments of B are copied (eight per k tile, dealt evenly over the wavefronts).  Same bits as the other
-// forms: the other digits are zero.
+// lowest-digit fragments of B are copied.  Same bits as the other forms: the other digits are zero.
 // kGroups = 2 (outputs of at most one tile per CU): eight wavefronts, two groups of four; group g multiplies the k
-// tiles g, g + 2, ... of the same output tile (a stage then holds two consecutive k tiles), so every SIMD has a second
-// wavefront to issue from while the first waits.  At the end the groups swap halves of their int32 accumulators
-// through LDS (exactly) and group g finishes row fragment g of each wavefront tile.
-template <bool kNarrow, bool kOneA, int kStages, int kGroups, bool kTopB = false>
+// steps g, g + 2, ... of the same output tile from stages of its own, so every SIMD has a second wavefront to issue
+// from while the first waits.  At the end the groups swap halves of their int32 accumulators through LDS (exactly)
+// and group g finishes row block g of each wavefront tile.
+template <bool kNarrow, bool kOneA, int kGroups, bool kTopB = false>
 __device__ __forceinline__ void gemm_digits_tile(const GemmDigitsArgs &a, unsigned char *smem) {
 #if defined(__HIP_DEVICE_COMPILE__) // the host pass only needs the launch stub; the body uses LDS address-space pointers
   static_assert(kGroups == 1 || kGroups == 2, "k groups per block");
   static_assert(!kOneA || kNarrow, "the one-digit A form is implemented for one-digit B operands");
   static_assert(!kTopB || kNarrow, "the top-digit B form is a narrow form");
-  constexpr int kBDigit = kTopB ? 0 : kDigits - 1; // the one digit of B a narrow form multiplies
-  constexpr int kAllWaves = kWaves * kGroups;
-  constexpr int kGroupStageBytes = kGroups * kStageBytes;
+  constexpr int kBDigit = !kNarrow || kTopB ? 0 : kDigits - 1; // the digit of B that the first phase multiplies
+  constexpr int kPhases = phases_per_step(kOneA, kNarrow);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int group = wave_all / kWaves, wave = wave_all % kWaves;
@@ -108,232 +106,286 @@ __device__ __forceinline__ void gemm_digits_tile(const GemmDigitsArgs &a, unsign
   int64_t bm, bn;
   band_tile<8>(blockIdx.x, a.blocks_m, a.blocks_n, bm, bn); // two blocks per CU: 64 resident tiles per XCD = 8 x 8
 
-  // This wavefront's copies.  The 24 fragments of a k tile are numbered u: [0, 12) the A fragments (row block,
-  // digit), [12, 16) the lowest-digit B fragments, [16, 24) the other B fragments; wavefront w takes
-  // u = q * kAllWaves + w, so each takes the same number (two thirds of its list) of the sixteen that the narrow form
-  // needs.  Copy p of a wavefront is fragment q = p % kPerTile of k tile p / kPerTile of the stage.
-  constexpr int kPerTile = kChunks / kAllWaves; // 6 or 3
-  // kOneA: the eight fragments f of a k tile that hold anything ([0, 4) A top digit, [4, 8) B lowest digit);
-  // wavefront w takes f = q * kAllWaves + w
-  constexpr int kOnePerTile = 2 * kSegs / kAllWaves; // 2 or 1
-  const uint4_t *cur[kPerWave], *cur_last[kPerWave];
-  int dest[kPerWave]; // byte offset inside a stage
+  // This wavefront's copies: of each part the fragments of k tile wave % 2 of the row blocks wave / 2 and wave / 2 + 2.
+  // A row block is a buffer resource that starts at the fragment's top digit in the first step of this block's share
+  // and ends with the last one: the copies run past the last step, where the range check (it covers the scalar offset
+  // too) turns them into zeros in LDS.  Row blocks past the end of the operand are clamped: those rows / columns are
+  // not stored.
+  constexpr int kStepAdvance = kGroups * 2 * kSegVec * 16; // bytes of a row block between a group's k steps
+  __amdgpu_buffer_rsrc_t rsrc[2][2];
 #pragma unroll
-  for (int p = 0; p < kPerWave; ++p) {
-    int sub, side, seg, d;
-    if (kOneA) {
-      sub = p / kOnePerTile;
-      const int f = (p - sub * kOnePerTile) * kAllWaves + wave_all;
-      side = f / kSegs, seg = f % kSegs, d = side ? kBDigit : 0;
-      if (p >= kOnePerTile * kGroups)
-        sub = 0, side = 0, seg = 0; // unused slot
-    } else {
-      sub = p / kPerTile;
-      const int q = p - sub * kPerTile;
-      const int u = q * kAllWaves + wave_all;
-      if (u < kSegs * kDigits)
-        side = 0, seg = u / kDigits, d = u - seg * kDigits;
-      else if (u < kSegs * kDigits + kSegs)
-        side = 1, seg = u - kSegs * kDigits, d = kBDigit;
-      else // the two digits of B that a narrow form leaves out
-        side = 1, seg = (u - kSegs * kDigits - kSegs) / (kDigits - 1),
-        d = (u - kSegs * kDigits - kSegs) % (kDigits - 1) + (kTopB ? 1 : 0);
+  for (int side = 0; side < 2; ++side)
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      int64_t rb = (side ? bn : bm) * kSegs + (wave >> 1) + 2 * q;
+      const int64_t limit = side ? a.b_row_blocks : a.a_row_blocks;
+      rb = rb < limit ? rb : limit - 1;
+      const int64_t tile = a.step_begin + group * 2 + (wave & 1);
+      const uint4_t *src = (side ? a.bd : a.ad) + (rb * a.k_tiles + tile) * kSegVec;
+      const int64_t span = (a.step_end - tile) * kSegVec * 16;
+      const uint64_t first = reinterpret_cast<uint64_t>(src);
+      const uint64_t base = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(first >> 32)) << 32) |
+                            (uint32_t)__builtin_amdgcn_readfirstlane((int)first);
+      rsrc[side][q] =
+          __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>(base), 0,
+                                            __builtin_amdgcn_readfirstlane(span > 0 ? (int)span : 0), 0x00020000);
     }
-    dest[p] = sub * kStageBytes + ((side * kSegs + seg) * kDigits + d) * kFragBytes;
-    int64_t rb = (side ? bn : bm) * kSegs + seg;
-    const int64_t limit = side ? a.b_row_blocks : a.a_row_blocks;
-    if (rb >= limit)
-      rb = limit - 1; // clamped: those rows / columns are not stored
-    const uint4_t *base = (side ? a.bd : a.ad) + (rb * a.k_tiles * kDigits + d) * 64;
-    cur[p] = base + (a.step_begin + sub) * kSegVec;
-    cur_last[p] = base + (a.step_end - kGroups + sub) * kSegVec;
-  }
   typedef __attribute__((address_space(3))) void lds_void_t;
-  // narrow: the first two thirds of each k tile's list (A fragments and lowest-digit B fragments)
-  constexpr int kNeeded = (kSegs * kDigits + kSegs) / kAllWaves; // 4 or 2 per k tile
-  constexpr int kCopies = kOneA ? kOnePerTile * kGroups : (kNarrow ? kNeeded * kGroups : kPerWave);
-  auto copy_next = [&](int buf) {
-#pragma unroll
-    for (int p = 0; p < kPerWave; ++p) {
-      if (!copy_slot_used(p, kOneA, kNarrow, kGroups))
-        continue;
-      __builtin_amdgcn_global_load_lds(cur[p] + lane, (lds_void_t *)(smem + buf * kGroupStageBytes + dest[p]), 16, 0,
-                                       0);
-      const uint4_t *next = cur[p] + kGroups * kSegVec;
-      cur[p] = next < cur_last[p] ? next : cur_last[p]; // the last calls copy the final tile again
-    }
+  unsigned char *ring = smem + group * kStages * kStageBytes;
+  const int a_lane = lane * 16;                                                            // rows as they are
+  const int b_lane = ((lane >> 5) * 32 + 2 * (lane & 15) + ((lane >> 4) & 1)) * 16;        // columns dealt out in pairs
+  // copy c (0..3) of the two parts of phase `ph` of the step at step_off into the buffer at byte offset `dest`
+  auto copy_one = [&](auto ph, int c, int step_off, int dest) __attribute__((always_inline)) {
+    constexpr int kPh = decltype(ph)::value;
+    const int part = c >> 1, q = c & 1;
+    const int side = kPh == 0 ? part : (kNarrow || kPh == 2 ? 0 : 1);
+    const int digit = kPh == 0 ? (part ? kBDigit : 0) : (side ? 2 - part : 1 + part);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        rsrc[side][q],
+        (lds_void_t *)(ring + dest + part * kPartBytes + (((wave >> 1) + 2 * q) * 2 + (wave & 1)) * kFragBytes), 16,
+        side ? b_lane : a_lane, step_off + digit * kFragBytes, 0, 0);
   };
 
-  i32x16_t acc[2][2][3];
+  i32x4_t acc[4][4][3];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < 4; ++j)
 #pragma unroll
       for (int t = 0; t < 3; ++t)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          acc[i][j][t][r] = 0;
+        acc[i][j][t] = i32x4_t{0, 0, 0, 0};
 
-  // The number of most recently issued k tiles the wait at the top of a tile may leave in flight, from the model of
+  // The number of most recently issued phases the wait at the top of a phase may leave in flight, from the model of
   // this loop's order of copies, waits, barriers and LDS reads (copy_pipeline.hpp)
   constexpr int kLoopWait = pipeline::one_tile_loop_wait(kStages, kStages - 1);
   static_assert(kLoopWait >= 0 && pipeline::one_tile_safe(kStages, kStages - 1, kLoopWait),
                 "the copy pipeline hands a buffer over too early");
-  static_assert(pipeline::counter_fits(kLoopWait, kPerWave), "vmcnt is a 6-bit counter");
+  static_assert(pipeline::counter_fits(kLoopWait, kCopies), "vmcnt is a 6-bit counter");
   static_assert(copies_per_call(kOneA, kNarrow, kGroups) == kCopies, "the wait counts the copies a call issues");
-#pragma unroll
-  for (int d = 0; d < kStages - 1; ++d)
-    copy_next(d);
-  int buf = 0;
-  for (int64_t kt = a.step_begin; kt < a.step_end; kt += kGroups) {
-    // tile kt has landed (the copies of the kStages - 2 tiles after it may still be in flight) and every wavefront
-    // is done with the buffer tile kt - 1 occupied, which tile kt + kStages - 1 takes over
+
+  // fragment f (0..3) of this wavefront's rows (part of side A) or columns (side B) in the part at `part`
+  const int a_frag = (wm * 2 * 2 + (lane >> 5)) * kFragBytes + (((lane >> 4) & 1) * 32 + (lane & 15)) * 16;
+  const int b_frag = a_frag + (wn - wm) * 4 * kFragBytes;
+  auto frag = [&](int lane_off, int part, int f) __attribute__((always_inline)) {
+    return __builtin_bit_cast(
+        i32x4_t, *reinterpret_cast<const uint4_t *>(ring + part + lane_off + (f >> 1) * 2 * kFragBytes + (f & 1) * 256));
+  };
+  int buf = 0; // byte offset of the phase's buffer
+  auto hand_over = [&]() __attribute__((always_inline)) {
+    // this phase's parts have landed (the copies of the two phases after it may still be in flight) and every
+    // wavefront is done with the buffer of the phase before it, which the copies issued next take over
     NBLA_WAIT_VMCNT(kLoopWait * kCopies);
     NBLA_BARRIER();
-    const uint4_t *sa = reinterpret_cast<const uint4_t *>(smem + buf * kGroupStageBytes + group * kStageBytes);
-    const uint4_t *sb = sa + kSideVec;
-    i32x4_t af[2][3], bf[2][3];
-    // digit by digit: the first products need the top digits' four fragments only
-    if (kNarrow) {
+  };
+  // Issue order, pinned (sched_barrier): the first two fragments of a phase, then its copies and its other reads dealt
+  // out between the MFMAs, each fragment read two fragments' MFMAs before it is used -- a wavefront cannot feed the
+  // matrix pipe while it issues a batch of other instructions or waits for LDS.
+  auto pin = []() __attribute__((always_inline)) { __builtin_amdgcn_sched_barrier(0); };
+  int ahead = 0; // byte offset of the step that the next copies belong to
+  // copy c of the phase three after phase kPh of the current step
+  auto copy_ahead = [&](auto ph, int c) __attribute__((always_inline)) {
+    constexpr int kPh = decltype(ph)::value, kTarget = kPh + kStages - 1;
+    copy_one(std::integral_constant<int, kTarget % kPhases>(), c, ahead + (kTarget / kPhases) * kStepAdvance,
+             (buf + (kStages - 1) * kStageBytes) & (kStages * kStageBytes - 1));
+  };
+  auto advance = [&]() __attribute__((always_inline)) { buf = (buf + kStageBytes) & (kStages * kStageBytes - 1); };
+  typedef std::integral_constant<int, 0> P0;
+  typedef std::integral_constant<int, 1> P1;
+  typedef std::integral_constant<int, 2> P2;
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
-        bf[i][kBDigit] = __builtin_bit_cast(i32x4_t, sb[((wn * 2 + i) * kDigits + kBDigit) * 64 + lane]);
-    }
+  for (int c = 0; c < kCopies; ++c)
+    copy_one(P0(), c, 0, 0);
 #pragma unroll
-    for (int d = 0; d < 3; ++d)
+  for (int c = 0; c < kCopies; ++c)
+    copy_one(std::integral_constant<int, 1 % kPhases>(), c, (1 / kPhases) * kStepAdvance, kStageBytes);
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        if (!kOneA || d == 0)
-          af[i][d] = __builtin_bit_cast(i32x4_t, sa[((wm * 2 + i) * kDigits + d) * 64 + lane]);
-        if (!kNarrow)
-          bf[i][d] = __builtin_bit_cast(i32x4_t, sb[((wn * 2 + i) * kDigits + d) * 64 + lane]);
+  for (int c = 0; c < kCopies; ++c)
+    copy_one(std::integral_constant<int, 2 % kPhases>(), c, (2 / kPhases) * kStepAdvance, 2 * kStageBytes);
+  auto mma = [&](i32x4_t &c, const i32x4_t &x, const i32x4_t &w) __attribute__((always_inline)) {
+    c = __builtin_amdgcn_mfma_i32_16x16x64_i8(x, w, c, 0, 0, 0);
+  };
+  const int steps = (int)((a.step_end - a.step_begin) / (2 * kGroups)); // k tiles come in multiples of eight
+  for (int left = steps; left > 0; --left) {
+    i32x4_t a0[4], b0[4];
+    hand_over();
+    a0[0] = frag(a_frag, buf, 0);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      b0[j] = frag(b_frag, buf + kPartBytes, j);
+    a0[1] = frag(a_frag, buf, 1);
+    pin();
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        mma(acc[i][j][0], a0[i], b0[j]);
+        if (i == 0 && (j & 1)) {
+          a0[2 + (j >> 1)] = frag(a_frag, buf, 2 + (j >> 1));
+          pin();
+        }
+        if (i == 1) {
+          copy_ahead(P0(), j);
+          pin();
+        }
       }
-    copy_next(buf == 0 ? kStages - 1 : buf - 1);
-    // Issue order (sched_group_barrier: 0x100 = LDS read, 0x008 = MFMA, 0x020 = the copies' loads): the fragments of
-    // the first products, then one further read per MFMA, then one copy per MFMA, instead of twelve reads and the
-    // copies in a row before the first MFMA -- a wavefront cannot feed the matrix pipe while it issues a batch of other
-    // instructions (the weight-gradient product of 4096 x 4096 x 11008: 1.14 -> 1.08 ms).
-    constexpr int kFirstReads = kOneA ? 4 : (kNarrow ? 4 : 4);
-    constexpr int kAllReads = kOneA ? 4 : (kNarrow ? 8 : 12);
-    constexpr int kAllMfmas = kOneA ? 4 : (kNarrow ? 12 : 24);
-    static_assert(kAllReads - kFirstReads + kCopies <= kAllMfmas, "more reads and copies than MFMAs to deal them out to");
-    if (kOneA) {
+    pin();
+    advance();
+    if (kNarrow && !kOneA) {
+      hand_over();
+      i32x4_t af[8];
+      af[0] = frag(a_frag, buf, 0);
+      af[1] = frag(a_frag, buf, 1);
+      pin();
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < 8; ++i) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-          acc[i][j][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i][0], bf[j][kBDigit], acc[i][j][0], 0, 0, 0);
-    } else if (kNarrow) {
-#pragma unroll
-      for (int t = 0; t < 3; ++t)
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j)
-            acc[i][j][t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i][t], bf[j][kBDigit], acc[i][j][t], 0, 0, 0);
-    } else {
-      // digit pairs (a digit, b digit) -> accumulator a + b
-      constexpr int da[6] = {0, 0, 1, 0, 1, 2};
-      constexpr int db[6] = {0, 1, 0, 2, 1, 0};
-#pragma unroll
-      for (int t = 0; t < 6; ++t)
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j)
-            acc[i][j][da[t] + db[t]] =
-                __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i][da[t]], bf[j][db[t]], acc[i][j][da[t] + db[t]], 0, 0, 0);
+        for (int j = 0; j < 4; ++j) {
+          mma(acc[i & 3][j][1 + (i >> 2)], af[i], b0[j]);
+          if (j == 0 && i + 2 < 8) {
+            af[i + 2] = frag(a_frag, buf + ((i + 2) >> 2) * kPartBytes, (i + 2) & 3);
+            pin();
+          }
+          if (i == 0) {
+            copy_ahead(P1(), j);
+            pin();
+          }
+        }
+        pin();
+      }
+      advance();
     }
-    __builtin_amdgcn_sched_group_barrier(0x100, kFirstReads, 0);
+    if (!kNarrow) {
+      i32x4_t b1[4];
+      {
+        hand_over();
+        i32x4_t bf[8]; // the third digit's, then the second's
+        bf[0] = frag(b_frag, buf, 0);
+        bf[1] = frag(b_frag, buf, 1);
+        pin();
 #pragma unroll
-    for (int q = 0; q < kAllReads - kFirstReads; ++q) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-    }
+        for (int j = 0; j < 8; ++j) {
 #pragma unroll
-    for (int q = 0; q < kCopies; ++q) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+          for (int i = 0; i < 4; ++i) {
+            mma(acc[i][j & 3][j < 4 ? 2 : 1], a0[i], bf[j]);
+            if (i == 0 && j + 2 < 8) {
+              bf[j + 2] = frag(b_frag, buf + ((j + 2) >> 2) * kPartBytes, (j + 2) & 3);
+              pin();
+            }
+            if (j == 0) {
+              copy_ahead(P1(), i);
+              pin();
+            }
+          }
+          pin();
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          b1[j] = bf[4 + j];
+        advance();
+      }
+      {
+        hand_over();
+        i32x4_t af[8]; // the second digit's, then the third's
+        af[0] = frag(a_frag, buf, 0);
+        af[1] = frag(a_frag, buf, 1);
+        pin();
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            mma(acc[i & 3][j][i < 4 ? 1 : 2], af[i], b0[j]);
+            if (j == 0 && i + 2 < 8) {
+              af[i + 2] = frag(a_frag, buf + ((i + 2) >> 2) * kPartBytes, (i + 2) & 3);
+              pin();
+            }
+            if (i == 0) {
+              copy_ahead(P2(), j);
+              pin();
+            }
+          }
+          if (i < 4) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              mma(acc[i & 3][j][2], af[i], b1[j]);
+          }
+          pin();
+        }
+        advance();
+      }
     }
-    __builtin_amdgcn_sched_group_barrier(0x008, kAllMfmas - (kAllReads - kFirstReads) - kCopies, 0);
-    __builtin_amdgcn_sched_barrier(0);
-    buf = (buf + 1 == kStages) ? 0 : buf + 1;
+    ahead += kStepAdvance;
   }
   NBLA_WAIT_VMCNT(0);
 
   if (kGroups == 2) {
-    // swap: every wavefront hands the row fragment it does not finish to its partner in the other group, one
-    // accumulator set at a time (8 wavefronts x 2 fragments x 16 registers x 64 lanes x 4 B = 64 KiB per round)
-    int *xs = reinterpret_cast<int *>(smem);
+    // swap: every wavefront hands the row block it does not finish to its partner in the other group, one accumulator
+    // set at a time (8 wavefronts x 2 x 4 tiles x 64 lanes x 16 B = 64 KiB per round)
+    i32x4_t *xs = reinterpret_cast<i32x4_t *>(smem);
     const int partner = wave_all ^ kWaves;
 #pragma unroll
     for (int t = 0; t < (kOneA ? 1 : 3); ++t) {
       __syncthreads(); // the stages (first round) or the previous round's values have been read
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
-        if (i != group) {
+      for (int i = 0; i < 4; ++i)
+        if ((i >> 1) != group) {
 #pragma unroll
-          for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-              xs[((wave_all * 2 + j) * 16 + r) * 64 + lane] = acc[i][j][t][r];
+          for (int j = 0; j < 4; ++j)
+            xs[((wave_all * 2 + (i & 1)) * 4 + j) * 64 + lane] = acc[i][j][t];
         }
       __syncthreads();
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
-        if (i == group) {
+      for (int i = 0; i < 4; ++i)
+        if ((i >> 1) == group) {
 #pragma unroll
-          for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-              acc[i][j][t][r] += xs[((partner * 2 + j) * 16 + r) * 64 + lane];
+          for (int j = 0; j < 4; ++j)
+            acc[i][j][t] += xs[((partner * 2 + (i & 1)) * 4 + j) * 64 + lane];
         }
     }
   }
 
   // y = (acc0 * 2^16 + acc1 * 2^8 + acc2) * 2^(16 - sa - sb); the narrow form has no factor 2^16 (b is its low digit)
   // unless b is the top digit of a row-scaled operand.
-  // Row by row: the row's offset (one 32-bit division when m is folded into two output indices) and shift are
-  // formed once and serve both column fragments.
-  const int col_in_frag = lane & 31, row_half = lane >> 5;
+  // Register r of lane l: row 4 (l / 16) + r of fragment i; columns 2 (l % 16) and the next of row block j / 2 (see the
+  // copy of B).  Row by row: the row's offset (one 32-bit division when m is folded into two output indices) and shift
+  // are formed once and serve all columns.
   const int32_t *bshift = (kNarrow && !kTopB) ? a.bshift_narrow : a.bshift;
-  int64_t n_col[2];
-  int32_t sb_n[2];
-  float bias_n[2];
+  int64_t n_col[2]; // the even one of a pair
+  int32_t sb_n[2][2];
+  float bias_n[2][2];
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    n_col[j] = bn * kBN + (wn * 2 + j) * 32 + col_in_frag;
-    const bool in = n_col[j] < a.N;
-    sb_n[j] = in ? plain_shift(bshift[n_col[j]]) : 0; // one-digit rows store their shift with a bias
-    bias_n[j] = (in && a.bias && a.finish) ? a.bias[n_col[j]] : 0.0f;
+  for (int jp = 0; jp < 2; ++jp) {
+    n_col[jp] = bn * kBN + (wn * 2 + jp) * 32 + 2 * (lane & 15);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const bool in = n_col[jp] + h < a.N;
+      sb_n[jp][h] = in ? plain_shift(bshift[n_col[jp] + h]) : 0; // one-digit rows store their shift with a bias
+      bias_n[jp][h] = (in && a.bias && a.finish) ? a.bias[n_col[jp] + h] : 0.0f;
+    }
   }
   const bool add_bias = a.bias && a.finish;
   const uint32_t inner = (uint32_t)a.inner;
-  // the 32 row shifts of each row fragment: one coalesced load up front (lane l holds row l % 32), handed out by
-  // shuffles, instead of a dependent global load per row inside the store loop
-  int32_t row_shift[2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    int64_t m = bm * kBM + (wm * 2 + i) * 32 + (lane & 31);
-    const int64_t last = a.a_row_blocks * kFragRows - 1;
-    row_shift[i] = plain_shift(a.ashift[m < last ? m : last]);
+  // the wavefront's 64 row shifts: one coalesced load up front (lane l holds row l), handed out by shuffles, instead of
+  // a dependent global load per row inside the store loop
+  int32_t row_shift;
+  {
+    const int64_t m = bm * kBM + wm * 64 + lane, last = a.a_row_blocks * kFragRows - 1;
+    row_shift = plain_shift(a.ashift[m < last ? m : last]);
   }
-  // Two copies of the stores, with and without reading y back first: with that load anywhere in the loop the
-  // compiler waits for all outstanding memory operations before every output, and the stores before it are
-  // outstanding memory operations -- each store would wait for the previous one.
-  auto store_rows = [&](auto accumulate_c) __attribute__((always_inline)) {
-    constexpr bool kAcc = decltype(accumulate_c)::value;
+  // Copies of the stores with and without reading y back first: with that load anywhere in the loop the compiler waits
+  // for all outstanding memory operations before every output, and the stores before it are outstanding memory
+  // operations -- each store would wait for the previous one.  Likewise with and without column bounds, for pairs of
+  // columns that are neighbours in memory (`pairs`).
+  auto store_rows = [&](auto accumulate_c, auto pairs_c) __attribute__((always_inline)) {
+    constexpr bool kAcc = decltype(accumulate_c)::value, kPairs = decltype(pairs_c)::value;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      if (kGroups == 2 && i != group)
+    for (int i = 0; i < 4; ++i) {
+      if (kGroups == 2 && (i >> 1) != group)
         continue;
-      const int64_t m0 = bm * kBM + (wm * 2 + i) * 32;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int row = 8 * (r >> 2) + 4 * row_half + (r & 3);
-        const int32_t sa_m = __shfl(row_shift[i], row);
-        const int64_t m = m0 + row;
+      for (int r = 0; r < 4; ++r) {
+        const int row = i * 16 + 4 * (lane >> 4) + r;
+        const int32_t sa_m = __shfl(row_shift, row);
+        const int64_t m = bm * kBM + wm * 64 + row;
         if (m >= a.M)
           continue;
         int64_t off;
@@ -344,40 +396,65 @@ __device__ __forceinline__ void gemm_digits_tile(const GemmDigitsArgs &a, unsign
           off = (int64_t)q * a.outer_stride + (mu - q * inner);
         }
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          if (n_col[j] >= a.N)
-            continue;
-          float v;
-          if (sa_m == kBadRow || sb_n[j] == kBadRow) {
-            v = __uint_as_float(0x7fc00000u);
-          } else {
-            // t = acc0 * 2^16 + acc1 * 2^8 + acc2 regrouped as hi * 2^16 + lo with 0 <= lo < 2^17 and |hi| < 2^30 (32-bit
-            // integer steps only), then one fused multiply-add: exact while |hi| < 2^24, else rounded twice (2^-24 of t)
-            const int a0 = acc[i][j][0][r], a1 = acc[i][j][1][r], a2 = acc[i][j][2][r];
-            const int hi = a0 + (a1 >> 8) + (a2 >> 16);
-            const int lo = ((a1 & 0xff) << 8) + (a2 & 0xffff);
-            const float t = fmaf((float)hi, 65536.0f, (float)lo);
-            // the two shifts are applied one after the other: each stays inside ldexpf's exponent range
-            v = ldexpf(ldexpf(t, ((kNarrow && !kTopB) ? 0 : 16) - sa_m), -sb_n[j]);
+        for (int jp = 0; jp < 2; ++jp) {
+          f32x2_t v;
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            if (sa_m == kBadRow || sb_n[jp][h] == kBadRow) {
+              v[h] = __uint_as_float(0x7fc00000u);
+            } else {
+              // t = acc0 * 2^16 + acc1 * 2^8 + acc2 regrouped as hi * 2^16 + lo with 0 <= lo < 2^17 and |hi| < 2^30
+              // (32-bit integer steps only), then one fused multiply-add: exact while |hi| < 2^24, else rounded twice
+              // (2^-24 of t)
+              const int a0 = acc[i][2 * jp + h][0][r], a1 = acc[i][2 * jp + h][1][r], a2 = acc[i][2 * jp + h][2][r];
+              const int hi = a0 + (a1 >> 8) + (a2 >> 16);
+              const int lo = ((a1 & 0xff) << 8) + (a2 & 0xffff);
+              const float t = fmaf((float)hi, 65536.0f, (float)lo);
+              // the two shifts are applied one after the other: each stays inside ldexpf's exponent range
+              v[h] = ldexpf(ldexpf(t, ((kNarrow && !kTopB) ? 0 : 16) - sa_m), -sb_n[jp][h]);
+            }
           }
-          float *dst = a.y + off + n_col[j] * a.n_stride;
-          if (kAcc)
-            v = *dst + v;
-          if (add_bias)
-            v = v + bias_n[j];
-          *dst = v;
+          if (kPairs) {
+            f32x2_u *dst = reinterpret_cast<f32x2_u *>(a.y + off + n_col[jp]);
+            if (kAcc)
+              v = *dst + v;
+            if (add_bias)
+              v[0] += bias_n[jp][0], v[1] += bias_n[jp][1];
+            *dst = v;
+          } else {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              if (n_col[jp] + h >= a.N)
+                continue;
+              float *dst = a.y + off + (n_col[jp] + h) * a.n_stride;
+              float w = v[h];
+              if (kAcc)
+                w = *dst + w;
+              if (add_bias)
+                w = w + bias_n[jp][h];
+              *dst = w;
+            }
+          }
         }
       }
     }
   };
-  if (a.accumulate)
-    store_rows(std::true_type());
-  else
-    store_rows(std::false_type());
+  const bool pairs = a.n_stride == 1 && (bn + 1) * kBN <= a.N;
+  if (a.accumulate) {
+    if (pairs)
+      store_rows(std::true_type(), std::true_type());
+    else
+      store_rows(std::true_type(), std::false_type());
+  } else {
+    if (pairs)
+      store_rows(std::false_type(), std::true_type());
+    else
+      store_rows(std::false_type(), std::false_type());
+  }
 #endif
 }
 
-template <int kStages, int kGroups>
+template <int kGroups>
 __global__ __launch_bounds__(kThreads * kGroups, kGroups == 1 ? 2 : 1) void gemm_digits_kernel(GemmDigitsArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   if (a.split_tiles > 0) {
@@ -397,9 +474,9 @@ __global__ __launch_bounds__(kThreads * kGroups, kGroups == 1 ? 2 : 1) void gemm
       one = one && one_digit_row(a.ashift[m < rows ? m : rows - 1]);
     }
     if (__syncthreads_and(one))
-      gemm_digits_tile<true, true, kStages, kGroups>(a, smem);
+      gemm_digits_tile<true, true, kGroups>(a, smem);
     else
-      gemm_digits_tile<true, false, kStages, kGroups>(a, smem);
+      gemm_digits_tile<true, false, kGroups>(a, smem);
   } else {
     // all rows of this tile's B row blocks one-digit rows (of a row-scaled operand; column-scaled ones never are)?
     int64_t bm, bn;
@@ -417,11 +494,11 @@ __global__ __launch_bounds__(kThreads * kGroups, kGroups == 1 ? 2 : 1) void gemm
     one_b = __syncthreads_and(one_b);
     one_a = __syncthreads_and(one_a);
     if (one_b && one_a)
-      gemm_digits_tile<true, true, kStages, kGroups, true>(a, smem);
+      gemm_digits_tile<true, true, kGroups, true>(a, smem);
     else if (one_b)
-      gemm_digits_tile<true, false, kStages, kGroups, true>(a, smem);
+      gemm_digits_tile<true, false, kGroups, true>(a, smem);
     else
-      gemm_digits_tile<false, false, kStages, kGroups>(a, smem);
+      gemm_digits_tile<false, false, kGroups>(a, smem);
   }
 }
 
@@ -507,15 +584,12 @@ int launch_gemm_digits(const void *adigits, const void *bdigits, const float *bi
   if (M >= ((int64_t)1 << 31) || N >= ((int64_t)1 << 31))
     return fail(NBLA_HIP_ERR_NOT_IMPLEMENTED, "digit product: more than 2^31 - 1 rows or columns.");
   const DigitOperand da = digit_operand(M, K), db = digit_operand(N, K);
-  static std::atomic<uint64_t> configured[3];
-  int rc = allow_dynamic_lds(reinterpret_cast<const void *>(gemm_digits_kernel<kStagesShared, 1>),
-                             kStagesShared * kStageBytes, configured[0], "hipFuncSetAttribute(gemm_digits LDS size)");
+  static std::atomic<uint64_t> configured[2];
+  int rc = allow_dynamic_lds(reinterpret_cast<const void *>(gemm_digits_kernel<1>), kStages * kStageBytes,
+                             configured[0], "hipFuncSetAttribute(gemm_digits LDS size)");
   if (!rc)
-    rc = allow_dynamic_lds(reinterpret_cast<const void *>(gemm_digits_kernel<kStagesAlone, 1>),
-                           kStagesAlone * kStageBytes, configured[1], "hipFuncSetAttribute(gemm_digits LDS size)");
-  if (!rc)
-    rc = allow_dynamic_lds(reinterpret_cast<const void *>(gemm_digits_kernel<kStagesShared, 2>),
-                           kStagesShared * 2 * kStageBytes, configured[2], "hipFuncSetAttribute(gemm_digits LDS size)");
+    rc = allow_dynamic_lds(reinterpret_cast<const void *>(gemm_digits_kernel<2>), 2 * kStages * kStageBytes,
+                           configured[1], "hipFuncSetAttribute(gemm_digits LDS size)");
   if (rc)
     return rc;
   GemmDigitsArgs a;
@@ -558,8 +632,8 @@ int launch_gemm_digits(const void *adigits, const void *bdigits, const float *bi
       part.y = static_cast<float *>(split_ws);
       part.inner = 1, part.outer_stride = N, part.n_stride = 1;
       part.accumulate = 0, part.bias = nullptr;
-      hipLaunchKernelGGL((gemm_digits_kernel<kStagesShared, 2>), dim3(blocks, (unsigned)splits), dim3(2 * kThreads),
-                         kStagesShared * 2 * kStageBytes, stream, part);
+      hipLaunchKernelGGL(gemm_digits_kernel<2>, dim3(blocks, (unsigned)splits), dim3(2 * kThreads),
+                         2 * kStages * kStageBytes, stream, part);
       NBLA_HIP_LAUNCH_CHECK("gemm_digits");
       if (n_stride != 1 && ceil_div(M, 32) <= 65535) {
         hipLaunchKernelGGL(gemm_digits_split_sum_rows, dim3((unsigned)ceil_div(N, 32), (unsigned)ceil_div(M, 32)),
@@ -576,16 +650,11 @@ int launch_gemm_digits(const void *adigits, const void *bdigits, const float *bi
       NBLA_HIP_LAUNCH_CHECK("gemm_digits_split_sum");
       continue;
     }
-    if (blocks <= 256 && chunk_tiles % 2 == 0) // at most one block per CU: eight wavefronts, two k groups (k tiles
-                                               // come in multiples of 8)
-      hipLaunchKernelGGL((gemm_digits_kernel<kStagesShared, 2>), dim3(blocks), dim3(2 * kThreads),
-                         kStagesShared * 2 * kStageBytes, stream, a);
-    else if (blocks <= 384) // fewer than 1.5 blocks per CU
-      hipLaunchKernelGGL((gemm_digits_kernel<kStagesAlone, 1>), dim3(blocks), dim3(kThreads),
-                         kStagesAlone * kStageBytes, stream, a);
+    if (blocks <= 256) // at most one block per CU: eight wavefronts, two k groups
+      hipLaunchKernelGGL(gemm_digits_kernel<2>, dim3(blocks), dim3(2 * kThreads), 2 * kStages * kStageBytes, stream,
+                         a);
     else
-      hipLaunchKernelGGL((gemm_digits_kernel<kStagesShared, 1>), dim3(blocks), dim3(kThreads),
-                         kStagesShared * kStageBytes, stream, a);
+      hipLaunchKernelGGL(gemm_digits_kernel<1>, dim3(blocks), dim3(kThreads), kStages * kStageBytes, stream, a);
     NBLA_HIP_LAUNCH_CHECK("gemm_digits");
   }
   return NBLA_HIP_OK;
