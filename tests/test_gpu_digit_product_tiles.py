@@ -1,0 +1,61 @@
+"""The digit x digit product (csrc/kernels/gemm_digits.hip) around its tiles: rows and columns at and one past 32, 64 and
+128, an odd number of columns (64-bit stores of column pairs), contractions of one to several k steps, split and in two
+k groups, outputs of one and of two blocks per CU, one-digit operands on either side, and sums added to what is there,
+against float64."""
+import numpy as np
+import pytest
+import torch
+
+from nnabla_amd import kernels
+from util import to_np
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(got, a, b, add=0.0):
+    """Operands are good to 2^-23 of their row's (column's) largest, the products left out below 2^-23 of both."""
+    a, b = a.double(), b.double()
+    k = a.shape[1]
+    big = a.abs().amax(1, keepdim=True) * b.abs().amax(0, keepdim=True)
+    ref = a @ b + add
+    bound = big * (k * 3 * 2.0 ** -23) + ref.abs() * 2.0 ** -22 + abs(add) * 2.0 ** -23
+    assert bool(((got.double() - ref).abs() <= bound).all())
+
+
+# samples (the contraction of dW), inputs, outputs: past the sizes that the one-launch product takes
+@pytest.mark.parametrize("M,K,N", [(4096, 33, 65), (3000, 129, 257), (2049, 1025, 1023), (300, 2049, 2175),
+                                   (1000, 2176, 2305), (257, 4097, 1100)])
+def test_weight_gradient(M, K, N):
+    kernels.init(0)
+    gen = torch.Generator(device="cuda").manual_seed(M + K + N)
+    x, dy = (torch.randn(M, n, generator=gen, device="cuda") for n in (K, N))
+    W = torch.randn(K, N, generator=gen, device="cuda")
+    old = torch.full((K, N), 2.0, device="cuda")
+    _check(kernels.affine_backward(dy, x, W, want=(False, True, False))[1], x.T, dy)
+    kernels.affine_backward(dy, x, W, dW=old, want=(False, True, False))
+    _check(old, x.T, dy, 2.0)
+
+
+@pytest.mark.parametrize("M,K,N", [(300, 4095, 1001), (1500, 2000, 2111)])
+@pytest.mark.parametrize("narrow_x", [False, True])
+@pytest.mark.parametrize("narrow_w", [False, True])
+def test_one_digit_operands(M, K, N, narrow_x, narrow_w):
+    kernels.init(0)
+    gen = torch.Generator(device="cuda").manual_seed(M + K + N)
+    x = torch.randn(M, K, generator=gen, device="cuda")
+    W = torch.randn(K, N, generator=gen, device="cuda")
+    b = torch.randn(N, generator=gen, device="cuda")
+    if narrow_x:
+        x = kernels.fixed_point_quantize(x, True, 8, 2.0 ** -4)
+    if narrow_w:
+        W = torch.sign(W) * torch.exp2(torch.randint(-5, 1, (K, N), generator=gen, device="cuda").float())
+    y = kernels.affine_digits(x, W, b)
+    _check(y - b, x, W) if not (narrow_x and narrow_w) else _exact(y, x, W, b)
+    dx = kernels.affine_backward(torch.randn(M, N, generator=gen, device="cuda"), x, W, want=(True, False, False))[0]
+    assert dx.shape == x.shape and bool(torch.isfinite(dx).all())
+
+
+def _exact(y, x, W, b):
+    """Small integers on both sides: the sum is exact, rounded once, and once more with the bias."""
+    ref = (x.double() @ W.double()).float() + b
+    assert np.array_equal(to_np(y), to_np(ref))
