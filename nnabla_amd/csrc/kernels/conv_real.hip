@@ -17,6 +17,10 @@
 // with all of the block's 2 x 2 fragments -- each weight operand, prepared once per call in the lanes' order, is read
 // from the L2 once per block and feeds twelve products -- and are added through LDS at the end.
 //
+// Geometries of at most one block per CU may take blocks of eight wavefronts and chunks of up to 64 channels instead (see
+// plan_real): [16,128,28,28] x [256,128,3,3] stride 2 forward 35 -> 30 us, dx of [8,256,14,14] x [256,256,3,3] 46.5 -> 42,
+// [4,512,7,7] x [512,512,1,1] 42 -> 34.
+//
 // What bounds it: a step of 24 MFMAs takes a wavefront 0.56 us (0.32 of the matrix cores alone), a chunk's barriers,
 // splitting and stores 0.8, and a block's start and end 7; with few blocks that chain is the time.  Digit operands of the
 // unfolded matrix -> this, dx: [16,128,28,28] x [256,128,3,3] stride 2 70 -> 47 us, [32,64,56,56] x [64,64,3,3] 319 -> 91,
@@ -44,11 +48,13 @@ constexpr int kThreads = 256, kWaves = 4;
 constexpr int kRows = 64, kPos = 64;
 constexpr uint32_t kOutside = 0x80000000u;     // a byte offset past the end of any tensor: such loads give zeros
 constexpr int kMaxTaps = 25, kMaxClasses = 9;
-constexpr int kLds = 78 * 1024;                // two blocks to a CU
-constexpr int kRedBytes = kWaves * kRows * kPos * 4;
+constexpr int kLds = 78 * 1024;                // two blocks of four wavefronts to a CU
+constexpr int kLdsWide = 150 * 1024;           // one block of eight
+constexpr int red_bytes(int waves) { return waves * kRows * kPos * 4; }
 constexpr int kMostItems = 5;                  // (position, eight channels) items a thread stages: registers
 constexpr uint32_t kLeast = (127u - 90u) << 23, kMost = (127u + 100u) << 23; // magnitudes, as bits
-static_assert(kMostItems * kThreads * 48 <= kLds && kRedBytes <= kLds, "");
+static_assert(kMostItems * kThreads * 48 <= kLds && red_bytes(kWaves) <= kLds, "");
+static_assert(4 * 2 * kThreads * 48 <= kLdsWide && red_bytes(2 * kWaves) <= kLdsWide, "");
 
 struct RealClass {
   int first, taps;  // of the taps' table
@@ -66,7 +72,7 @@ struct RealArgs {
   float *out;              // first channel of the group
   int64_t w_row, w_k;
   int N, CS, CD, Kc, R, IH, IW, OH, OW; // channels of the in- and output tensors, contraction channels and rows of the group
-  int ss, ds, row_tiles, ksteps, taps_all, chunk, slots, accumulate, signs, transposed;
+  int ss, ds, row_tiles, ksteps, taps_all, chunk, waves, slots, accumulate, signs, transposed;
   float zero_to;
   uint32_t in_bytes; // from `in` to the end of the tensor
   int classes;
@@ -161,10 +167,11 @@ __device__ __forceinline__ f32x16_t mma(const uint4_t &a, const uint4_t &b, f32x
 #endif
 }
 
-template <int kItems> __global__ __launch_bounds__(kThreads, 2) void conv_real_kernel(RealArgs a) {
+template <int kItems, int kW> __global__ __launch_bounds__(64 * kW, 2) void conv_real_kernel(RealArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)
+  constexpr int kT = 64 * kW;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[]; // [plane][octet][slots][16 bytes]; the exchange
-  __shared__ uint32_t s_max[2][kWaves];
+  __shared__ uint32_t s_max[2][kW];
   __shared__ int s_bad[kPos], s_shift[kRows];
   __shared__ float s_bias[kRows];
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, half = lane >> 5;
@@ -207,7 +214,7 @@ template <int kItems> __global__ __launch_bounds__(kThreads, 2) void conv_real_k
   int dst[kItems];      // LDS offset, a multiple of sixteen, plus the octet; negative: no such item
 #pragma unroll
   for (int i = 0; i < kItems; ++i) {
-    const int it = tid + kThreads * i;
+    const int it = tid + kT * i;
     const int o = run ? it / run : 0, s = it - o * run;
     const int f = min(run0 + s, a.N * in_plane - 1), n = f / in_plane;
     const bool is = it < items;
@@ -220,7 +227,7 @@ template <int kItems> __global__ __launch_bounds__(kThreads, 2) void conv_real_k
   auto load_x = [&](int c0) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < kItems; ++i) {
-      const int left = a.Kc - c0 - 8 * (dst[i] & 3);
+      const int left = a.Kc - c0 - 8 * (dst[i] & 15);
 #pragma unroll
       for (int j = 0; j < 8; ++j)
         xv[i][j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
@@ -241,7 +248,7 @@ template <int kItems> __global__ __launch_bounds__(kThreads, 2) void conv_real_k
       for (int q = 0; q < 16; ++q)
         acc[i][f][q] = 0.0f;
   uint32_t amax = 0u, amin = ~0u; // the largest magnitude of the run; the smallest one that is not zero, less one
-  const int row_frags = a.row_tiles * 2, sub_shift = a.chunk == 32 ? 1 : 0;
+  const int row_frags = a.row_tiles * 2, sub_shift = a.chunk >> 5, sub = (1 << sub_shift) - 1; // 16, 32 or 64 channels
   const int steps = C.taps << sub_shift;
   const uint4_t *wbase = reinterpret_cast<const uint4_t *>(a.w) + (int64_t)(row_tile * 2) * 64 + lane;
   const int64_t w_plane = (int64_t)row_frags * 64;
@@ -252,7 +259,7 @@ template <int kItems> __global__ __launch_bounds__(kThreads, 2) void conv_real_k
   auto load_w = [&](int kstep0, int s, uint4_t (&w)[2][3]) __attribute__((always_inline)) {
     const int sc = min(s, steps - 1);
     const int t = __builtin_amdgcn_readlane(taps_of_lanes, sc >> sub_shift) >> 16;
-    const int ks = min(kstep0, a.ksteps - 1 - sub_shift) + (sc & sub_shift);
+    const int ks = min(kstep0, a.ksteps - 1 - sub) + (sc & sub);
     const uint4_t *p = wbase + ((int64_t)t * a.ksteps + ks) * 3 * w_plane;
 #pragma unroll
     for (int d = 0; d < 3; ++d)
@@ -265,7 +272,7 @@ template <int kItems> __global__ __launch_bounds__(kThreads, 2) void conv_real_k
       return;
     const int tp = __builtin_amdgcn_readlane(taps_of_lanes, s >> sub_shift);
     const int dy = (signed char)(tp & 0xff), dx = (signed char)((tp >> 8) & 0xff);
-    const int o = ((s & sub_shift) * 2 + half) * a.slots;
+    const int o = ((s & sub) * 2 + half) * a.slots;
     uint4_t x[2][3];
 #pragma unroll
     for (int f = 0; f < 2; ++f) {
@@ -286,13 +293,13 @@ template <int kItems> __global__ __launch_bounds__(kThreads, 2) void conv_real_k
           acc[i][f] = mma(w[i][kPairs[p][0]], x[f][kPairs[p][1]], acc[i][f]);
   };
   uint4_t w0[2][3], w1[2][3], w2[2][3];
-  const int groups = (steps + 3 * kWaves - 1) / (3 * kWaves);
+  const int groups = (steps + 3 * kW - 1) / (3 * kW);
   __syncthreads();
   if (steps) {
     load_x(0);
     load_w(0, wave, w0);
-    load_w(0, wave + kWaves, w1);
-    load_w(0, wave + 2 * kWaves, w2);
+    load_w(0, wave + kW, w1);
+    load_w(0, wave + 2 * kW, w2);
   }
   for (int c0 = 0; c0 < a.Kc && steps; c0 += a.chunk) {
     __syncthreads(); // the steps of the chunk before have read their operands
@@ -316,21 +323,21 @@ template <int kItems> __global__ __launch_bounds__(kThreads, 2) void conv_real_k
     __syncthreads();
     const int kstep0 = c0 >> 4, next = (c0 + a.chunk) >> 4;
     int s = wave;
-    for (int grp = 1; grp < groups; ++grp, s += 3 * kWaves) {
+    for (int grp = 1; grp < groups; ++grp, s += 3 * kW) {
       step(s, w0);
-      load_w(kstep0, s + 3 * kWaves, w0);
-      step(s + kWaves, w1);
-      load_w(kstep0, s + 4 * kWaves, w1);
-      step(s + 2 * kWaves, w2);
-      load_w(kstep0, s + 5 * kWaves, w2);
+      load_w(kstep0, s + 3 * kW, w0);
+      step(s + kW, w1);
+      load_w(kstep0, s + 4 * kW, w1);
+      step(s + 2 * kW, w2);
+      load_w(kstep0, s + 5 * kW, w2);
     }
     load_x(c0 + a.chunk); // (past the last channel: zeros, without an access)
     step(s, w0);
     load_w(next, wave, w0);
-    step(s + kWaves, w1);
-    load_w(next, wave + kWaves, w1);
-    step(s + 2 * kWaves, w2);
-    load_w(next, wave + 2 * kWaves, w2);
+    step(s + kW, w1);
+    load_w(next, wave + kW, w1);
+    step(s + 2 * kW, w2);
+    load_w(next, wave + 2 * kW, w2);
   }
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) {
@@ -341,7 +348,7 @@ template <int kItems> __global__ __launch_bounds__(kThreads, 2) void conv_real_k
     s_max[0][wave] = amax, s_max[1][wave] = amin;
   __syncthreads();
 #pragma unroll
-  for (int w = 0; w < kWaves; ++w)
+  for (int w = 0; w < kW; ++w)
     amax = max(amax, s_max[0][w]), amin = min(amin, s_max[1][w]);
   // ---- the wavefronts' sums: each finishes sixteen of the rows
   float *s_red = reinterpret_cast<float *>(smem); // [wave][row][position]
@@ -365,7 +372,7 @@ template <int kItems> __global__ __launch_bounds__(kThreads, 2) void conv_real_k
   int any_bad = 0;
   if (suspect) {
     uint32_t big = 0u;
-    for (int k = wave; k < a.Kc; k += kWaves)
+    for (int k = wave; k < a.Kc; k += kW)
       for (int t = 0; t < C.taps; ++t) {
         const int iy = qy * a.ss + a.ty[C.first + t], ix = qx * a.ss + a.tx[C.first + t];
         if ((unsigned)iy < (unsigned)a.IH && (unsigned)ix < (unsigned)a.IW)
@@ -382,11 +389,11 @@ template <int kItems> __global__ __launch_bounds__(kThreads, 2) void conv_real_k
   }
   bool redo = false;
 #pragma unroll
-  for (int i = 0; i < kRows / kWaves; ++i) {
-    const int row = wave * (kRows / kWaves) + i, rr = row_tile * kRows + row, shift = s_shift[row];
+  for (int i = 0; i < kRows / kW; ++i) {
+    const int row = wave * (kRows / kW) + i, rr = row_tile * kRows + row, shift = s_shift[row];
     double sum = 0.0;
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w)
+    for (int w = 0; w < kW; ++w)
       sum += (double)s_red[(w * kRows + row) * kPos + lane];
     const float v = (float)ldexp(sum, -(shift == kBadRow ? 0 : shift)) + s_bias[row];
     float *o = out + (int64_t)rr * out_plane;
@@ -396,7 +403,7 @@ template <int kItems> __global__ __launch_bounds__(kThreads, 2) void conv_real_k
   }
   if (!redo)
     return;
-  for (int row = wave * (kRows / kWaves); row < (wave + 1) * (kRows / kWaves); ++row) {
+  for (int row = wave * (kRows / kW); row < (wave + 1) * (kRows / kW); ++row) {
     const int rr = row_tile * kRows + row;
     if (rr >= a.R || !(any_bad || s_shift[row] == kBadRow))
       continue;
@@ -431,6 +438,13 @@ int64_t class_slots(int64_t QH, int64_t QW, int64_t IH, int64_t IW, int64_t N, i
   if (vrows > N * IH)
     vrows = N * IH;
   return vrows * IW + 1;
+}
+
+// What a block's chunks take, in us: a chunk 0.8 and 0.56 for a step of each of four wavefronts, 1.05 of eight (what the
+// rounds of both say at [16,128,28,28] x [256,128,3,3] stride 2, 35 -> 30, and [4,96,27,27] x [48,96,5,5], 38 -> 44).
+double block_time(const RealArgs &a, int taps) {
+  const double rounds = (double)ceil_div(taps * (a.chunk / 16), a.waves);
+  return (double)ceil_div(a.Kc, a.chunk) * (0.8 + (a.waves == kWaves ? 0.56 : 1.05) * rounds);
 }
 
 // Fills everything but the pointers; false where the form does not cover the geometry.  Rows of positions that only the
@@ -486,21 +500,40 @@ bool plan_real(const ConvGeom &g, bool transposed, RealArgs &a) {
       const int64_t n = class_slots(c.QH, c.QW, a.IH, a.IW, a.N, a.ss, lo, hi);
       slots = n > slots ? n : slots;
     }
-  a.chunk = a.Kc > 16 && slots * 4 <= 4 * kThreads ? 32 : 16;
-  if (slots * (a.chunk / 8) > kMostItems * kThreads || (int64_t)tiles * a.row_tiles > 0x7fffffff)
+  if ((int64_t)tiles * a.row_tiles > 0x7fffffff)
     return false;
+  int most_taps = 0;
+  for (int c = 0; c < a.classes; ++c)
+    most_taps = a.cls[c].taps > most_taps ? a.cls[c].taps : most_taps;
+  a.waves = kWaves, a.chunk = a.Kc > 16 && slots * 4 <= 4 * kThreads ? 32 : 16;
+  if (slots * (a.chunk / 8) > kMostItems * kThreads)
+    return false;
+  // Where every CU gets one block at most, a block of eight wavefronts may take it: chunks of up to 64 channels leave
+  // fewer of a chunk's steps over after whole rounds of the wavefronts, and fewer barriers.
+  if ((int64_t)tiles * a.row_tiles <= 256) {
+    const int chunk = a.chunk;
+    double best = block_time(a, most_taps) - 1.5;
+    for (int c = 32; c <= 64; c *= 2) {
+      RealArgs wide = a;
+      wide.waves = 2 * kWaves, wide.chunk = c;
+      if (slots * (c / 8) > 4 * 2 * kThreads || (c > chunk && a.Kc <= c / 2) || block_time(wide, most_taps) >= best)
+        continue;
+      best = block_time(wide, most_taps), a.waves = 2 * kWaves, a.chunk = c;
+    }
+  }
   a.slots = (int)slots;
   a.ksteps = (int)ceil_div(a.Kc, a.chunk) * (a.chunk / 16);
   return (int64_t)a.Kc * a.taps_all * 4 <= 150 * 1024; // (a row of weights in LDS)
 }
 
-template <int kItems> int run_real(const RealArgs &a, int64_t blocks, size_t lds, hipStream_t stream) {
+template <int kItems, int kW> int run_real(const RealArgs &a, int64_t blocks, size_t lds, hipStream_t stream) {
   static std::atomic<uint64_t> configured{0};
-  const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(conv_real_kernel<kItems>), kLds, configured,
+  const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(conv_real_kernel<kItems, kW>),
+                                   kW == kWaves ? kLds : kLdsWide, configured,
                                    "hipFuncSetAttribute(conv_real_kernel LDS size)");
   if (rc)
     return rc;
-  hipLaunchKernelGGL(conv_real_kernel<kItems>, dim3((unsigned)blocks), dim3(kThreads), lds, stream, a);
+  hipLaunchKernelGGL((conv_real_kernel<kItems, kW>), dim3((unsigned)blocks), dim3(64 * kW), lds, stream, a);
   NBLA_HIP_LAUNCH_CHECK("conv_real_kernel");
   return NBLA_HIP_OK;
 }
@@ -512,9 +545,8 @@ size_t prepared_bytes(const RealArgs &a) {
 
 } // namespace
 
-// Where the geometry is covered, by an estimate of both forms in microseconds, from sizes measured on both: here, a
-// block's chunk takes 0.8 and 0.56 for each of a wavefront's steps, blocks that share a CU add up, launches and weights
-// come on top (dx, [1,512,7,7] x [512,512,3,3] 87 estimated 76, [64,512,7,7] 128 and 133, [32,256,14,14] x [256,256,3,3]
+// Where the geometry is covered, by an estimate of both forms in microseconds, from sizes measured on both: here, blocks
+// that share a CU add up, launches and weights come on top (dx, [1,512,7,7] x [512,512,3,3] 87 estimated 76, [64,512,7,7] 128 and 133, [32,256,14,14] x [256,256,3,3]
 // 71 and 73); on the digit path the unfolded matrix goes through memory (dx: written and gathered, 0.9 MB a microsecond
 // with the transposed gradient; forward: 1.8) and six digit products take 2.4 per 10^9 operations.  What the digits win
 // are few positions under many channels: [1,512,7,7] dx 44 against 87.
@@ -522,12 +554,11 @@ bool conv_real_applies(const ConvGeom &g, bool transposed, bool binary) {
   RealArgs a;
   if (!plan_real(g, transposed, a))
     return false;
-  const double chunks = (double)ceil_div(a.Kc, a.chunk);
   double total = 0.0, longest = 0.0;
   for (int c = 0; c < a.classes; ++c) {
     if (!a.cls[c].taps)
       continue;
-    const double block = chunks * (0.8 + 0.56 * (double)ceil_div(a.cls[c].taps * (a.chunk / 16), kWaves));
+    const double block = block_time(a, a.cls[c].taps);
     total += block * a.cls[c].tiles * a.row_tiles;
     longest = block > longest ? block : longest;
   }
@@ -570,12 +601,17 @@ int launch_conv_real(const float *in, const float *W, const float *bias, float *
   const RealClass &last = a.cls[a.classes - 1];
   const int64_t slab = (int64_t)a.slots * a.chunk * 6;
   const int64_t blocks = (int64_t)(last.tile0 + last.tiles) * a.row_tiles, items = a.slots * (a.chunk / 8);
-  const size_t lds = (size_t)(slab > kRedBytes ? slab : kRedBytes);
+  const size_t lds = (size_t)(slab > red_bytes(a.waves) ? slab : red_bytes(a.waves));
+  if (a.waves == 2 * kWaves) {
+    if (items <= 2 * 2 * kThreads)
+      return run_real<2, 2 * kWaves>(a, blocks, lds, stream);
+    return run_real<4, 2 * kWaves>(a, blocks, lds, stream);
+  }
   if (items <= 2 * kThreads)
-    return run_real<2>(a, blocks, lds, stream);
+    return run_real<2, kWaves>(a, blocks, lds, stream);
   if (items <= 4 * kThreads)
-    return run_real<4>(a, blocks, lds, stream);
-  return run_real<kMostItems>(a, blocks, lds, stream);
+    return run_real<4, kWaves>(a, blocks, lds, stream);
+  return run_real<kMostItems, kWaves>(a, blocks, lds, stream);
 }
 
 } // namespace nbla_hip
