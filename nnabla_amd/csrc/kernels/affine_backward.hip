@@ -84,15 +84,18 @@ BackwardPlan plan_backward(int64_t M, int64_t K, int64_t N) {
 }
 
 // dW[K, N] (+)= x^T . dy on the digit x digit product (both factors are real numbers): the operand rows are the
-// columns of x and of dy, the contraction runs over the M samples.
-int grad_weights(const float *x, const float *dy, float *dW, int64_t M, int64_t K, int64_t N, bool accumulate,
-                 char *base, const BackwardPlan &p, hipStream_t stream) {
+// columns of x and of dy, the contraction runs over the M samples.  *db (may be null): the bias gradient, taken along
+// where the operand of dy is made here; *db is then set to null.
+int grad_weights(const float *x, const float *dy, float *dW, float **db, bool accumulate_db, int64_t M, int64_t K,
+                 int64_t N, bool accumulate, char *base, const BackwardPlan &p, hipStream_t stream) {
   if (gemm_small_applies(K, M, N, kSmallGradWeights))
     return launch_gemm_small(x, true, dy, true, nullptr, dW, K, M, N, accumulate, stream);
+  float *sums = *db;
+  *db = nullptr;
   int rc = launch_split_digits_columns(x, K, base + p.a_planes_off, M, K, false, stream);
   if (rc)
     return rc;
-  rc = launch_split_digits_columns(dy, N, base + p.b_planes_off, M, N, false, stream);
+  rc = launch_split_digits_columns(dy, N, base + p.b_planes_off, M, N, false, stream, sums, accumulate_db);
   if (rc)
     return rc;
   return launch_gemm_digits(base + p.a_planes_off, base + p.b_planes_off, nullptr, dW, K, M, N, 1, N, 1, stream,
@@ -196,7 +199,7 @@ int nbla_hip_binary_affine_backward_f32(const float *dy, const float *x, const f
     }
   }
   if (dW) {
-    rc = grad_weights(x, dy, dW, M, K, N, accum_w != 0, base, p, stream);
+    rc = grad_weights(x, dy, dW, &db, accum_b != 0, M, K, N, accum_w != 0, base, p, stream);
     if (rc)
       return rc;
   }
@@ -220,7 +223,7 @@ int nbla_hip_affine_backward_f32(const float *dy, const float *x, const float *W
       return rc;
   }
   if (dW) {
-    rc = grad_weights(x, dy, dW, M, K, N, accum_w != 0, base, p, stream);
+    rc = grad_weights(x, dy, dW, &db, accum_b != 0, M, K, N, accum_w != 0, base, p, stream);
     if (rc)
       return rc;
   }

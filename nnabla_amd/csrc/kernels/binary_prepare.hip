@@ -888,53 +888,65 @@ void launch_split_digits_rows(const float *x, int64_t ldx, const float *cs, long
 // binades below its column's largest (INQ weights once they are fixed): then the scale is chosen so that each
 // value is an integer of magnitude <= 64 and sits in the lowest digit alone ("narrow" operand, flag word 0), and
 // the product needs three digit products instead of six and drops nothing.
-__global__ __launch_bounds__(kPrepBlock) void clear_column_scratch(uint32_t *__restrict__ cmax,
-                                                                   uint32_t *__restrict__ cmin, int64_t n,
-                                                                   int32_t *__restrict__ flag, int flag_value) {
-  const int64_t i = (int64_t)blockIdx.x * kPrepBlock + threadIdx.x;
-  if (i < n) {
-    cmax[i] = 0u;
-    cmin[i] = 0xffffffffu;
-  }
-  if (i == 0)
-    *flag = flag_value;
-}
-
-// Block = 64 column quads x 4 row groups over a slab of `slab` rows (a multiple of 4); 128-bit loads where the
-// layout allows, eight in flight per thread; the row groups are folded through LDS before the atomics.
-template <bool kVec, bool kDetect>
-__global__ __launch_bounds__(kPrepBlock) void column_absmax(const float *__restrict__ src, int64_t ld, int64_t R,
-                                                            int64_t C, uint32_t *__restrict__ cmax,
-                                                            uint32_t *__restrict__ cmin, int32_t *__restrict__ flag,
-                                                            int slab) {
+//
+// Statistics of a slab of rows per column: block = 64 column quads x 4 row groups over `slab` rows (a multiple of 4);
+// 128-bit loads at any alignment, eight in flight per thread; the row groups are folded through LDS.  The slabs' results
+// go to arrays of [slab][C] in the operand's own fragment area, which nothing holds yet, and column_stats_final folds
+// them: no atomics, so nothing has to be cleared first, and the columns' sums (a bias gradient that is wanted beside
+// the operand of dy) come along: [4096, 11008] with its sums 4.7 + 42 + 4.7 and 44 + 4.6 us in five launches -> 2.
+struct ColumnPartials {
+  uint32_t *max, *min, *other; // min: null without detect; other: one word per block
+  float *sum;                  // null: not wanted
+};
+template <bool kDetect, bool kSum>
+__global__ __launch_bounds__(kPrepBlock) void column_stats(const float *__restrict__ src, int64_t ld, int64_t R, int64_t C,
+                                                           ColumnPartials out, int32_t *__restrict__ flag, int slab) {
   __shared__ uint32_t part[4][256];
   __shared__ uint32_t part_min[kDetect ? 4 : 1][256];
+  __shared__ float part_sum[kSum ? 4 : 1][256];
   const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
   const int64_t c0 = ((int64_t)blockIdx.x * 64 + tx) * 4;
   const int64_t r0 = (int64_t)blockIdx.y * slab;
   const int64_t r_end = r0 + slab < R ? r0 + slab : R;
   uint32_t m[4] = {0u, 0u, 0u, 0u}, mn[4] = {0xffffffffu, 0xffffffffu, 0xffffffffu, 0xffffffffu};
+  float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
   bool other = false; // an element that is neither zero nor a normal power of two
   if (c0 < C) {
-#pragma unroll 8
-    for (int64_t r = r0 + ty; r < r_end; r += 4) {
-      float v[4];
-      if (kVec) {
-        const float4_t q = *reinterpret_cast<const float4_t *>(src + r * ld + c0);
-        v[0] = q.x, v[1] = q.y, v[2] = q.z, v[3] = q.w;
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          v[j] = (c0 + j < C) ? src[r * ld + c0 + j] : 0.0f;
-      }
+    // the last quad of a row that is no multiple of four: moved back onto the row, the columns before its own left out
+    const int64_t cl = c0 + 4 <= C ? c0 : (C >= 4 ? C - 4 : 0);
+    const int skip = (int)(c0 - cl);
+    auto take = [&](const float4_t &q) __attribute__((always_inline)) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const uint32_t u = __float_as_uint(v[j]) & 0x7fffffffu;
+        const uint32_t u = __float_as_uint(q[j]) & 0x7fffffffu;
         m[j] = u > m[j] ? u : m[j];
+        if (kSum)
+          sum[j] += q[j];
         if (kDetect && u) {
           mn[j] = u < mn[j] ? u : mn[j];
           other |= (u & 0x007fffffu) != 0u || (u >> 23) == 0u;
         }
+      }
+    };
+    if (C >= 4) {
+#pragma unroll 8
+      for (int64_t r = r0 + ty; r < r_end; r += 4)
+        take(*reinterpret_cast<const float4_u *>(src + r * ld + cl));
+    } else {
+      for (int64_t r = r0 + ty; r < r_end; r += 4) {
+        float4_t q = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (int j = 0; j < (int)C; ++j)
+          q[j] = src[r * ld + j];
+        take(q);
+      }
+    }
+    if (skip) { // column c0 + j is element skip + j of the quad read
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+#pragma unroll
+        for (int e = 1; e < 4; ++e)
+          if (e - skip == j)
+            m[j] = m[e], mn[j] = mn[e], sum[j] = sum[e];
       }
     }
   }
@@ -943,34 +955,44 @@ __global__ __launch_bounds__(kPrepBlock) void column_absmax(const float *__restr
     part[ty][tx * 4 + j] = m[j];
     if (kDetect)
       part_min[ty][tx * 4 + j] = mn[j];
+    if (kSum)
+      part_sum[ty][tx * 4 + j] = sum[j];
   }
-  if (kDetect && __any(other) && (threadIdx.x & 63) == 0 &&
-      __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
-    atomicOr(flag, 1);
-  __syncthreads();
-  const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (kDetect) {
+    const int any = __syncthreads_or(other);
+    if (threadIdx.x == 0)
+      out.other[(int64_t)blockIdx.y * gridDim.x + blockIdx.x] = any ? 1u : 0u;
+  } else {
+    __syncthreads();
+  }
+  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0)
+    *flag = kDetect ? 0 : 1;
+  const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x, at = (int64_t)blockIdx.y * C + c;
   if (c < C) {
-    uint32_t a = part[0][threadIdx.x], b = part[1][threadIdx.x], d = part[2][threadIdx.x], e = part[3][threadIdx.x];
-    a = a > b ? a : b;
-    d = d > e ? d : e;
-    a = a > d ? a : d;
-    if (a)
-      atomicMax(&cmax[c], a);
-    if (kDetect) {
-      a = part_min[0][threadIdx.x], b = part_min[1][threadIdx.x], d = part_min[2][threadIdx.x];
-      e = part_min[3][threadIdx.x];
-      a = a < b ? a : b;
-      d = d < e ? d : e;
-      a = a < d ? a : d;
-      if (a != 0xffffffffu)
-        atomicMin(&cmin[c], a);
-    }
+    const int t = threadIdx.x;
+    out.max[at] = max(max(part[0][t], part[1][t]), max(part[2][t], part[3][t]));
+    if (kDetect)
+      out.min[at] = min(min(part_min[0][t], part_min[1][t]), min(part_min[2][t], part_min[3][t]));
+    if (kSum)
+      out.sum[at] = ((part_sum[0][t] + part_sum[1][t]) + part_sum[2][t]) + part_sum[3][t];
   }
 }
 
-// Shift of every (padded) operand row from its column maximum; a NaN or an infinity marks the row.  The narrow
-// shift (largest element -> 64) replaces the maximum in `cmax`; a column spanning more than six binades raises the
-// flag.
+// The shift of one operand row from its column's largest magnitude; a NaN or an infinity marks the row.  With detect the
+// narrow shift (largest element -> 64) too; a column spanning more than six binades raises the flag.
+__device__ __forceinline__ int column_shifts(uint32_t m, uint32_t mn, bool detect, int32_t *flag, int32_t &narrow) {
+  const bool bad = m >= 0x7f800000u;
+  narrow = bad ? kBadRow : 0;
+  if (detect && !bad && m != 0u) {
+    const int e_max = (int)(m >> 23) - 127, e_min = (int)(mn >> 23) - 127;
+    narrow = 6 - e_max;
+    if (e_max - e_min > 6 && __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
+      atomicOr(flag, 1);
+  }
+  return bad ? kBadRow : (m == 0u ? 0 : digit_shift(m));
+}
+
+// Shift of every (padded) operand row from its column's statistics; the narrow shift replaces the maximum in `cmax`.
 __global__ __launch_bounds__(kPrepBlock) void column_shift(uint32_t *__restrict__ cmax,
                                                            const uint32_t *__restrict__ cmin,
                                                            int32_t *__restrict__ shift, int64_t C, int64_t rows,
@@ -978,20 +1000,56 @@ __global__ __launch_bounds__(kPrepBlock) void column_shift(uint32_t *__restrict_
   const int64_t c = (int64_t)blockIdx.x * kPrepBlock + threadIdx.x;
   if (c >= rows)
     return;
-  const uint32_t m = c < C ? cmax[c] : 0u;
-  const bool bad = m >= 0x7f800000u;
-  shift[c] = bad ? kBadRow : (m == 0u ? 0 : digit_shift(m));
-  if (detect) {
-    int narrow = 0;
-    if (bad) {
-      narrow = kBadRow;
-    } else if (m != 0u) {
-      const int e_max = (int)(m >> 23) - 127, e_min = (int)(cmin[c] >> 23) - 127;
-      narrow = 6 - e_max;
-      if (e_max - e_min > 6 && __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
-        atomicOr(flag, 1);
-    }
+  int32_t narrow;
+  shift[c] = column_shifts(c < C ? cmax[c] : 0u, detect && c < C ? cmin[c] : 0u, detect != 0, flag, narrow);
+  if (detect)
     cmax[c] = (uint32_t)narrow;
+}
+
+// The same from the slabs' statistics: block = 64 columns x 4 groups of slabs, folded through LDS in a fixed order; the
+// columns' sums go to db (added to it with `accumulate`).
+template <bool kDetect, bool kSum>
+__global__ __launch_bounds__(kPrepBlock) void column_stats_final(ColumnPartials in, int64_t slabs, int64_t blocks_x,
+                                                                 uint32_t *__restrict__ cmax, int32_t *__restrict__ shift,
+                                                                 int64_t C, int64_t rows, int32_t *__restrict__ flag,
+                                                                 float *__restrict__ db, int accumulate) {
+  __shared__ uint32_t part[4][64], part_min[kDetect ? 4 : 1][64];
+  __shared__ float part_sum[kSum ? 4 : 1][64];
+  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
+  const int64_t c = (int64_t)blockIdx.x * 64 + tx, cc = c < C ? c : C - 1;
+  uint32_t m = 0u, mn = 0xffffffffu, other = 0u;
+  float sum = 0.0f;
+#pragma unroll 4
+  for (int64_t s = ty; s < slabs; s += 4) {
+    m = max(m, in.max[s * C + cc]);
+    if (kDetect) {
+      mn = min(mn, in.min[s * C + cc]);
+      other |= in.other[s * blocks_x + (cc >> 8)];
+    }
+    if (kSum)
+      sum += in.sum[s * C + cc];
+  }
+  part[ty][tx] = m;
+  if (kDetect) {
+    part_min[ty][tx] = mn;
+    if (other && __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
+      atomicOr(flag, 1);
+  }
+  if (kSum)
+    part_sum[ty][tx] = sum;
+  __syncthreads();
+  if (ty != 0 || c >= rows)
+    return;
+  m = c < C ? max(max(m, part[1][tx]), max(part[2][tx], part[3][tx])) : 0u;
+  if (kDetect)
+    mn = min(min(mn, part_min[1][tx]), min(part_min[2][tx], part_min[3][tx]));
+  int32_t narrow;
+  shift[c] = column_shifts(m, mn, kDetect, flag, narrow);
+  if (kDetect)
+    cmax[c] = (uint32_t)narrow;
+  if (kSum && c < C) {
+    sum = ((sum + part_sum[1][tx]) + part_sum[2][tx]) + part_sum[3][tx];
+    db[c] = accumulate ? db[c] + sum : sum;
   }
 }
 
@@ -1052,48 +1110,65 @@ ColumnScratch column_scratch(void *digits, int64_t R, int64_t C) {
   return s;
 }
 
+namespace {
+
+int launch_split_columns(const float *src, int64_t ld, char *base, int64_t R, int64_t C, const DigitOperand &d,
+                         const ColumnScratch &cs, hipStream_t stream) {
+  const int64_t frags = d.k_tiles * d.row_blocks;
+  hipLaunchKernelGGL(split_digits_columns, dim3((unsigned)ceil_div(frags, kPrepBlock / 64)), dim3(kPrepBlock), 0,
+                     stream, src, ld, reinterpret_cast<const int32_t *>(base + d.shift_off),
+                     reinterpret_cast<const int32_t *>(cs.cmax), cs.flag, reinterpret_cast<uint4_t *>(base), R, C,
+                     d.k_tiles, d.row_blocks, frags);
+  NBLA_HIP_LAUNCH_CHECK("split_digits_columns");
+  return NBLA_HIP_OK;
+}
+
+} // namespace
+
 int launch_split_digits_columns_from_stats(const float *src, int64_t ld, void *digits, int64_t R, int64_t C,
                                            bool detect_narrow, hipStream_t stream) {
   const DigitOperand d = digit_operand(C, R);
   char *base = static_cast<char *>(digits);
   const ColumnScratch cs = column_scratch(digits, R, C);
-  int32_t *shift = reinterpret_cast<int32_t *>(base + d.shift_off);
   hipLaunchKernelGGL(column_shift, dim3((unsigned)ceil_div(d.rows, kPrepBlock)), dim3(kPrepBlock), 0, stream, cs.cmax,
-                     cs.cmin, shift, C, d.rows, cs.flag, detect_narrow ? 1 : 0);
+                     cs.cmin, reinterpret_cast<int32_t *>(base + d.shift_off), C, d.rows, cs.flag, detect_narrow ? 1 : 0);
   NBLA_HIP_LAUNCH_CHECK("column_shift");
-  const int64_t frags = d.k_tiles * d.row_blocks;
-  hipLaunchKernelGGL(split_digits_columns, dim3((unsigned)ceil_div(frags, kPrepBlock / 64)), dim3(kPrepBlock), 0,
-                     stream, src, ld, shift, reinterpret_cast<const int32_t *>(cs.cmax), cs.flag,
-                     reinterpret_cast<uint4_t *>(base), R, C, d.k_tiles, d.row_blocks, frags);
-  NBLA_HIP_LAUNCH_CHECK("split_digits_columns");
-  return NBLA_HIP_OK;
+  return launch_split_columns(src, ld, base, R, C, d, cs, stream);
 }
 
 int launch_split_digits_columns(const float *src, int64_t ld, void *digits, int64_t R, int64_t C, bool detect_narrow,
-                                hipStream_t stream) {
+                                hipStream_t stream, float *db, bool accumulate_db) {
+  const DigitOperand d = digit_operand(C, R);
+  char *base = static_cast<char *>(digits);
   const ColumnScratch cs = column_scratch(digits, R, C);
-  hipLaunchKernelGGL(clear_column_scratch, dim3((unsigned)ceil_div(cs.rows, kPrepBlock)), dim3(kPrepBlock), 0, stream,
-                     cs.cmax, cs.cmin, cs.rows, cs.flag, detect_narrow ? 0 : 1);
-  NBLA_HIP_LAUNCH_CHECK("clear_column_scratch");
-  int slab = 64; // taller slabs (fewer atomics per column) while a thousand blocks remain
+  int slab = 64; // taller slabs (fewer to fold) while a thousand blocks remain
   while (slab < 256 && ceil_div(C, 256) * ceil_div(R, 2 * slab) >= 1024)
     slab *= 2;
-  const dim3 grid((unsigned)ceil_div(C, 256), (unsigned)ceil_div(R, slab));
-  const bool vec = C % 4 == 0 && ld % 4 == 0 && aligned16(src);
-#define NBLA_LAUNCH_ABSMAX(V, D)                                                                                       \
-  hipLaunchKernelGGL((column_absmax<V, D>), grid, dim3(kPrepBlock), 0, stream, src, ld, R, C, cs.cmax, cs.cmin,       \
-                     cs.flag, slab)
-  if (vec && detect_narrow)
-    NBLA_LAUNCH_ABSMAX(true, true);
-  else if (vec)
-    NBLA_LAUNCH_ABSMAX(true, false);
-  else if (detect_narrow)
-    NBLA_LAUNCH_ABSMAX(false, true);
+  const int64_t blocks_x = ceil_div(C, 256), slabs = ceil_div(R, slab);
+  // (four words a column and slab of 64 rows or more, in an area of 96 bytes a column and k tile of 32 rows or less)
+  ColumnPartials parts;
+  parts.max = reinterpret_cast<uint32_t *>(base);
+  parts.min = parts.max + slabs * C;
+  parts.sum = reinterpret_cast<float *>(parts.min + slabs * C);
+  parts.other = reinterpret_cast<uint32_t *>(parts.sum + slabs * C);
+  const dim3 grid((unsigned)blocks_x, (unsigned)slabs), final_grid((unsigned)ceil_div(d.rows, 64));
+  int32_t *shift = reinterpret_cast<int32_t *>(base + d.shift_off);
+#define NBLA_LAUNCH_STATS(D, S)                                                                                        \
+  do {                                                                                                                 \
+    hipLaunchKernelGGL((column_stats<D, S>), grid, dim3(kPrepBlock), 0, stream, src, ld, R, C, parts, cs.flag, slab);  \
+    NBLA_HIP_LAUNCH_CHECK("column_stats");                                                                             \
+    hipLaunchKernelGGL((column_stats_final<D, S>), final_grid, dim3(kPrepBlock), 0, stream, parts, slabs, blocks_x,    \
+                       cs.cmax, shift, C, d.rows, cs.flag, db, accumulate_db ? 1 : 0);                                 \
+    NBLA_HIP_LAUNCH_CHECK("column_stats_final");                                                                       \
+  } while (0)
+  if (detect_narrow)
+    NBLA_LAUNCH_STATS(true, false);
+  else if (db)
+    NBLA_LAUNCH_STATS(false, true);
   else
-    NBLA_LAUNCH_ABSMAX(false, false);
-#undef NBLA_LAUNCH_ABSMAX
-  NBLA_HIP_LAUNCH_CHECK("column_absmax");
-  return launch_split_digits_columns_from_stats(src, ld, digits, R, C, detect_narrow, stream);
+    NBLA_LAUNCH_STATS(false, false);
+#undef NBLA_LAUNCH_STATS
+  return launch_split_columns(src, ld, base, R, C, d, cs, stream);
 }
 
 } // namespace nbla_hip

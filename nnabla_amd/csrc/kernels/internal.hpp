@@ -141,12 +141,13 @@ size_t gemm_bits_split_bytes(int64_t M, int64_t K, int64_t N);
 // Digit operand whose rows are the C columns of src [R, C] (row stride ld), contraction over src's rows.  With
 // detect_narrow the operand comes out in its one-digit form when every element is zero or a power of two within six
 // binades of its column's largest (its flag word tells the product which form it got).
+// db (may be null; not with detect_narrow): the columns' sums too, added to db with accumulate_db.
 int launch_split_digits_columns(const float *src, int64_t ld, void *digits, int64_t R, int64_t C, bool detect_narrow,
-                                hipStream_t stream);
+                                hipStream_t stream, float *db = nullptr, bool accumulate_db = false);
 // The statistics that pass gathers, kept in the operand's own row-sum area: per column the largest and the smallest
 // non-zero magnitude (bit patterns, by atomicMax / atomicMin from 0 / 0xffffffff) and a flag word raised when an
 // element is neither zero nor a normal power of two.  A kernel that touches every element of src anyway may fill them
-// itself (clearing them first) and call the second half of the pass.
+// itself (clearing them first) and call the second half of the pass; launch_split_digits_columns gathers them by slabs.
 struct ColumnScratch {
   uint32_t *cmax, *cmin;
   int32_t *flag;
