@@ -34,8 +34,8 @@ typedef int i32x4_t __attribute__((ext_vector_type(4)));
 typedef int i32x16_t __attribute__((ext_vector_type(16)));
 typedef uint32_t uint4_t __attribute__((ext_vector_type(4)));
 
-constexpr int kFusedRows = 32, kFusedCols = 64;
-constexpr int kFusedTiles = 4;                 // k tiles of x a wavefront keeps in registers
+constexpr int kFusedRows = 32;
+constexpr int kFusedTiles = 4;                 // k tiles of x a wavefront keeps in registers, at most
 constexpr uint32_t kOutside = 0x80000000u;     // a byte offset past the end of any buffer here
 
 struct FusedArgs {
@@ -62,9 +62,11 @@ __device__ __forceinline__ int fused_shift(uint32_t amax_bits) {
   return s;
 }
 
-template <int kWaves>
+// kTiles: k tiles of a wavefront (kWaves * kTiles of them cover K); kFrags: fragments of 32 columns of a block.
+template <int kWaves, int kTiles, int kFrags>
 __global__ __launch_bounds__(64 * kWaves, 2) void binary_affine_fused(FusedArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)
+  constexpr int kFusedCols = 32 * kFrags;
   extern __shared__ __attribute__((aligned(16))) int s_red[]; // [wave][32][lane]
   __shared__ uint32_t s_max[kWaves][kFusedRows], s_nonfinite[kWaves][kFusedRows];
   __shared__ float s_cs[kWaves][2][kFusedCols];
@@ -101,37 +103,37 @@ __global__ __launch_bounds__(64 * kWaves, 2) void binary_affine_fused(FusedArgs 
   const uint32_t col_off = (uint32_t)half * 16 * row_bytes + (uint32_t)(n0 + r) * 4;
 
   // sixteen rows of the lane's two columns in k tile t (t < k_tiles); rows past K repeat the last one or read as zero
-  auto load_w = [&](int t, float (&w)[2][16]) __attribute__((always_inline)) {
+  auto load_w = [&](int t, float (&w)[kFrags][16]) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
       const uint32_t soff = (uint32_t)min(t * kTileK + j, a.K - 1) * row_bytes;
 #pragma unroll
-      for (int f = 0; f < 2; ++f)
+      for (int f = 0; f < kFrags; ++f)
         w[f][j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(wr, (int)(col_off + 128 * f), (int)soff, 0));
     }
   };
   const int zero_byte = (int)a.zero_to;
-  float cs[2] = {0.0f, 0.0f};
-  i32x16_t acc[2][kDigits];
+  float cs[kFrags] = {};
+  i32x16_t acc[kFrags][kDigits];
 #pragma unroll
-  for (int f = 0; f < 2; ++f)
+  for (int f = 0; f < kFrags; ++f)
 #pragma unroll
     for (int d = 0; d < kDigits; ++d)
 #pragma unroll
       for (int q = 0; q < 16; ++q)
         acc[f][d][q] = 0;
   // the tile's bytes, and its magnitudes to the column sums
-  auto take_tile = [&](int t, float (&w)[2][16], uint4_t (&b)[2]) __attribute__((always_inline)) {
+  auto take_tile = [&](int t, float (&w)[kFrags][16], uint4_t (&b)[kFrags]) __attribute__((always_inline)) {
     const int k0 = t * kTileK + 16 * half;
     if (t * kTileK + kTileK > a.K) { // uniform: the last tile
 #pragma unroll
       for (int j = 0; j < 16; ++j)
 #pragma unroll
-        for (int f = 0; f < 2; ++f)
+        for (int f = 0; f < kFrags; ++f)
           w[f][j] = k0 + j < a.K ? w[f][j] : 0.0f;
     }
 #pragma unroll
-    for (int f = 0; f < 2; ++f)
+    for (int f = 0; f < kFrags; ++f)
 #pragma unroll
       for (int j4 = 0; j4 < 4; ++j4) {
         uint32_t byte[4];
@@ -147,9 +149,9 @@ __global__ __launch_bounds__(64 * kWaves, 2) void binary_affine_fused(FusedArgs 
         b[f][j4] = lo | hi;
       }
   };
-  auto multiply = [&](const uint4_t (&xd)[kDigits], const uint4_t (&b)[2]) __attribute__((always_inline)) {
+  auto multiply = [&](const uint4_t (&xd)[kDigits], const uint4_t (&b)[kFrags]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int f = 0; f < 2; ++f)
+    for (int f = 0; f < kFrags; ++f)
 #pragma unroll
       for (int d = 0; d < kDigits; ++d)
         acc[f][d] = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(i32x4_t, xd[d]),
@@ -157,10 +159,10 @@ __global__ __launch_bounds__(64 * kWaves, 2) void binary_affine_fused(FusedArgs 
   };
 
   // x: the row's values of the wavefront's k tiles, its largest finite magnitude over all wavefronts, the digits
-  f32x4_t xv[kFusedTiles][4];
+  f32x4_t xv[kTiles][4];
   const bool row_in = m0 + r < a.M;
 #pragma unroll
-  for (int i = 0; i < kFusedTiles; ++i) {
+  for (int i = 0; i < kTiles; ++i) {
     const int k0 = (wave + kWaves * i) * kTileK + 16 * half;
     const uint32_t off = (uint32_t)((m0 + r) * a.K + k0) * 4;
 #pragma unroll
@@ -169,12 +171,13 @@ __global__ __launch_bounds__(64 * kWaves, 2) void binary_affine_fused(FusedArgs 
           f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(xr, (int)(row_in && k0 + 4 * v < a.K ? off + 16 * v : kOutside),
                                                          0, 0));
   }
-  float w0[2][16], w1[2][16];
-  load_w(min(wave, k_tiles - 1), w0);
-  load_w(min(wave + kWaves, k_tiles - 1), w1);
+  float w[kTiles > 1 ? 2 : 1][kFrags][16];
+  load_w(min(wave, k_tiles - 1), w[0]);
+  if constexpr (kTiles > 1)
+    load_w(min(wave + kWaves, k_tiles - 1), w[1]);
   uint32_t amax = 0u, bad = 0u;
 #pragma unroll
-  for (int i = 0; i < kFusedTiles; ++i) {
+  for (int i = 0; i < kTiles; ++i) {
     const int k0 = (wave + kWaves * i) * kTileK + 16 * half;
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
@@ -197,9 +200,9 @@ __global__ __launch_bounds__(64 * kWaves, 2) void binary_affine_fused(FusedArgs 
   const int shift = amax ? fused_shift(amax) : 0;
   if (wave == 0 && half == 0)
     s_shift[r] = bad ? kBadRow : shift;
-  uint4_t xd[kFusedTiles][kDigits];
+  uint4_t xd[kTiles][kDigits];
 #pragma unroll
-  for (int i = 0; i < kFusedTiles; ++i) {
+  for (int i = 0; i < kTiles; ++i) {
     int q[16];
     uint32_t words[3][4];
 #pragma unroll
@@ -210,34 +213,23 @@ __global__ __launch_bounds__(64 * kWaves, 2) void binary_affine_fused(FusedArgs 
     for (int d = 0; d < kDigits; ++d)
       xd[i][d] = uint4_t{words[d][0], words[d][1], words[d][2], words[d][3]};
   }
-  static_assert(kFusedTiles == 4, "two pairs of tiles");
-  uint4_t b[2];
-  if (wave < k_tiles) {
-    take_tile(wave, w0, b);
-    load_w(min(wave + 2 * kWaves, k_tiles - 1), w0);
-    multiply(xd[0], b);
-  }
-  if (wave + kWaves < k_tiles) {
-    take_tile(wave + kWaves, w1, b);
-    load_w(min(wave + 3 * kWaves, k_tiles - 1), w1);
-    multiply(xd[1], b);
-  }
-  if (wave + 2 * kWaves < k_tiles) {
-    take_tile(wave + 2 * kWaves, w0, b);
-    multiply(xd[2], b);
-  }
-  if (wave + 3 * kWaves < k_tiles) {
-    take_tile(wave + 3 * kWaves, w1, b);
-    multiply(xd[3], b);
-  }
+  uint4_t b[kFrags];
+#pragma unroll
+  for (int i = 0; i < kTiles; ++i)
+    if (wave + i * kWaves < k_tiles) {
+      take_tile(wave + i * kWaves, w[i & (kTiles > 1 ? 1 : 0)], b);
+      if (i + 2 < kTiles)
+        load_w(min(wave + (i + 2) * kWaves, k_tiles - 1), w[i & (kTiles > 1 ? 1 : 0)]);
+      multiply(xd[i], b);
+    }
 
   // ---- the wavefronts' sums, one fragment of 32 columns at a time: each finishes 16 / kWaves accumulator registers
 #pragma unroll
-  for (int f = 0; f < 2; ++f)
+  for (int f = 0; f < kFrags; ++f)
     s_cs[wave][half][32 * f + r] = cs[f];
   int any_bad = 0;
 #pragma unroll
-  for (int f = 0; f < 2; ++f) {
+  for (int f = 0; f < kFrags; ++f) {
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
       s_red[(wave * 32 + 2 * q) * 64 + lane] = acc[f][0][q] * 256 + acc[f][1][q]; // below 2^30 for K up to 2^14
@@ -300,25 +292,29 @@ __global__ __launch_bounds__(64 * kWaves, 2) void binary_affine_fused(FusedArgs 
 #endif
 }
 
-template <int kWaves> int run_fused(const FusedArgs &a, hipStream_t stream) {
+template <int kWaves, int kTiles, int kFrags> int run_fused(FusedArgs &a, hipStream_t stream) {
   static std::atomic<uint64_t> configured{0};
   constexpr int lds = kWaves * 32 * 64 * 4;
-  const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(binary_affine_fused<kWaves>), lds, configured,
-                                   "hipFuncSetAttribute(binary_affine_fused LDS size)");
+  const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(binary_affine_fused<kWaves, kTiles, kFrags>), lds,
+                                   configured, "hipFuncSetAttribute(binary_affine_fused LDS size)");
   if (rc)
     return rc;
+  a.n_tiles = (int)ceil_div(a.N, 32 * kFrags), a.products = (int)(a.n_tiles * ceil_div(a.M, kFusedRows));
   int64_t writers = ceil_div((int64_t)a.K * a.N, (int64_t)64 * kWaves * 16);
   if (writers > 512)
     writers = 512;
   const dim3 grid((unsigned)(a.products + writers));
   hipEvent_t start, stop;
   if (product_timer_next(&start, &stop))
-    hipExtLaunchKernelGGL((binary_affine_fused<kWaves>), grid, dim3(64 * kWaves), lds, stream, start, stop, 0, a);
+    hipExtLaunchKernelGGL((binary_affine_fused<kWaves, kTiles, kFrags>), grid, dim3(64 * kWaves), lds, stream, start,
+                          stop, 0, a);
   else
-    hipLaunchKernelGGL((binary_affine_fused<kWaves>), grid, dim3(64 * kWaves), lds, stream, a);
+    hipLaunchKernelGGL((binary_affine_fused<kWaves, kTiles, kFrags>), grid, dim3(64 * kWaves), lds, stream, a);
   NBLA_HIP_LAUNCH_CHECK("binary_affine_fused");
   return NBLA_HIP_OK;
 }
+
+constexpr int kWideCols = 64; // columns of a block of two fragments
 
 } // namespace
 
@@ -332,7 +328,7 @@ bool fused_affine_applies(const float *W, const float *Wb, int64_t M, int64_t K,
       (K + 64) * N * 4 >= (1ll << 31) || (M + kFusedRows) * (K + 512) * 4 >= (1ll << 31))
     return false;
   // Two rounds of blocks at most: of 512 (four wavefronts, two blocks to a CU) or of 256.
-  const int64_t blocks = ceil_div(M, kFusedRows) * ceil_div(N, kFusedCols);
+  const int64_t blocks = ceil_div(M, kFusedRows) * ceil_div(N, kWideCols);
   return blocks <= (K <= 4 * kFusedTiles * kTileK ? 1024 : 512);
 }
 
@@ -343,8 +339,16 @@ int launch_fused_affine(const float *x, const float *W, float *Wb, float *alpha,
   a.M = (int)M, a.K = (int)K, a.N = (int)N;
   a.zero_to = zero_to, a.inv_k = (float)1 / K;
   a.x_bytes = (uint32_t)(M * K * 4), a.w_bytes = (uint32_t)(K * N * 4);
-  a.n_tiles = (int)ceil_div(N, kFusedCols), a.products = (int)(a.n_tiles * ceil_div(M, kFusedRows));
-  return K <= 4 * kFusedTiles * kTileK ? run_fused<4>(a, stream) : run_fused<8>(a, stream);
+  // Few blocks: the chain of one block is the time, so blocks of one fragment of columns, K over eight wavefronts and no
+  // more k tiles in a wavefront than there are (20 x 250 x 250: 9.1 -> 4.9 us).
+  if (ceil_div(M, kFusedRows) * ceil_div(N, kWideCols) <= 128) {
+    if (K <= 8 * kTileK)
+      return run_fused<8, 1, 1>(a, stream);
+    if (K <= 16 * kTileK)
+      return run_fused<8, 2, 1>(a, stream);
+    return run_fused<8, 4, 1>(a, stream);
+  }
+  return K <= 4 * kFusedTiles * kTileK ? run_fused<4, 4, 2>(a, stream) : run_fused<8, 4, 2>(a, stream);
 }
 
 } // namespace nbla_hip
