@@ -101,6 +101,11 @@ int binary_affine_forward(const float *x, const float *W, float *Wb, float *alph
     rc = ensure_init();
     return rc ? rc : launch_fused_affine(x, W, Wb, alpha, bias, y, M, K, N, zero_to, stream);
   }
+  // up to sixteen rows of x under a W whose rows are not 16-byte aligned and too many for one launch
+  if (!one_walk && small_m_affine_covers(Wb, M, K, N)) {
+    rc = ensure_init();
+    return rc ? rc : launch_small_m_affine(x, W, Wb, alpha, bias, y, M, K, N, zero_to, base, workspace_bytes, stream);
+  }
   if (one_walk || (rows_affine_covers(W, Wb, alpha, bias, y, M, K, N) && rows_affine_pays(M, K, N))) {
     // one walk over W: signs, column sums and the product together
     if (!representable && (rc = launch_clear_words(count, 1, stream)))

@@ -26,14 +26,15 @@ namespace nbla_hip {
 namespace {
 
 typedef float float4_t __attribute__((ext_vector_type(4)));
+typedef float float4_u __attribute__((ext_vector_type(4), aligned(4))); // one 128-bit access at any multiple of four bytes
 
 // Four wavefronts stacked in K over one 256-column strip; four such blocks per CU (128 registers per lane), so the
 // whole of a 4096 x 11008 weight matrix (688 blocks) is resident at once and no second round of blocks trails behind.
 constexpr int kWavesK = 4, kWavesN = 1;
 constexpr int kThreads = 64 * kWavesK * kWavesN;
-constexpr int blocks_per_cu(int MT) { return MT >= 16 ? 2 : 4; } // sixteen rows need more than 128 registers
-constexpr int kRowsPerWave = 64;                     // rows of W one wavefront walks
-constexpr int kSlabRows = kWavesK * kRowsPerWave;    // rows of W per block
+// sixteen rows, and eight with a row's end taken apart, need more than 128 registers
+constexpr int blocks_per_cu(int MT, bool aligned) { return MT >= (aligned ? 16 : 2) ? 2 : 4; }
+constexpr int kMostRowsPerWave = 64, kLeastRowsPerWave = 8; // rows of W one wavefront walks
 constexpr int kWaveCols = 256;                       // 64 lanes x float4
 constexpr int kStripCols = kWavesN * kWaveCols;      // columns per block
 
@@ -44,24 +45,38 @@ __device__ __forceinline__ float sign_of(float w, float zero_to) {
   return __builtin_islessgreater(w, 0.0f) ? one : zero_to;
 }
 
-__host__ __device__ inline int64_t small_m_slabs(int64_t K) { return ceil_div(K, kSlabRows); }
-__host__ __device__ inline int64_t small_m_padded_cols(int64_t N) { return ceil_div(N, kStripCols) * kStripCols; }
+inline int64_t small_m_padded_cols(int64_t N) { return ceil_div(N, kStripCols) * kStripCols; }
+inline int64_t small_m_slabs(int64_t K, int rows_per_wave) { return ceil_div(K, kWavesK * rows_per_wave); }
+// Rows of W per wavefront: 64 where that makes enough blocks to keep the memory busy, fewer where the walk of 64 rows, one
+// batch after the other, would be the launch's time on a few CUs (with the slabs limited, which the finishing launch
+// adds up).  One row of x: 100 x 1000 (K x N) 13.8 -> 4.2 us, 512 x 2048 9.0 -> 3.6; 4 rows: 1000 x 800 19.0 -> 5.0;
+// 12 rows: 300 x 3000 56 -> 12; from 256 blocks of 64 rows on fewer rows gain nothing (2 rows under 4096 x 4096: 22 -> 27).
+inline int small_m_rows_per_wave(int64_t K, int64_t N) {
+  int rows = kMostRowsPerWave;
+  while (rows > kLeastRowsPerWave && small_m_padded_cols(N) / kStripCols * small_m_slabs(K, rows) < 256 &&
+         small_m_slabs(K, rows / 2) <= 128)
+    rows /= 2;
+  return rows;
+}
 
 // partial[slab][r][Npad]: r < MT the dot products of input row r over the slab, r == MT the |W| column sums.
 //
 // The activations never enter vector registers: x[m, k] is the same for every lane, so it is read with scalar loads
 // and enters the multiply-add as a scalar operand.  kFull (decided per block) is the interior of W, where no row or
 // column test is needed; edge blocks run the same code with clamped loads and guarded stores.
-template <int MT, int kBatch, bool kFull>
+// kAligned: N a multiple of four (a lane's columns lie inside a row or past it).
+template <int MT, int kBatch, bool kFull, bool kAligned>
 __device__ __forceinline__ void small_m_walk(const float *__restrict__ W, float *__restrict__ Wb,
                                              const float *__restrict__ x, int64_t M, int64_t K, int64_t N,
-                                             int64_t k_wave, int64_t n0, float zero_to, float (&acc)[MT][4],
-                                             float (&cs)[4]) {
-  constexpr int kBatches = kRowsPerWave / kBatch;
-  static_assert(kBatches % 2 == 0, "the loop below consumes two batches per trip");
+                                             int64_t k_wave, int rows_per_wave, int64_t n0, float zero_to,
+                                             float (&acc)[MT][4], float (&cs)[4]) {
+  static_assert(kLeastRowsPerWave % (2 * kBatch) == 0, "the loop below consumes two batches per trip");
+  const int batches = rows_per_wave / kBatch;
   constexpr int kXRows = (32 / MT) < 1 ? 1 : ((32 / MT) > kBatch ? kBatch : (32 / MT)); // rows whose x is fetched at once
-  const bool col_ok = kFull || n0 < N;
-  const int64_t n_ld = col_ok ? n0 : N - 4; // loads are unconditional: a clamped address, masked afterwards
+  // Loads are unconditional: a clamped address, masked afterwards.  A lane whose four columns end past N loads the last
+  // four and takes its own from among them.
+  const int cols = kFull || n0 + 4 <= N ? 4 : (n0 < N ? (int)(N - n0) : 0); // columns of the lane
+  const int64_t n_ld = cols == 4 ? n0 : N - 4;
   const uint32_t lane_bytes = (uint32_t)(n_ld * 4);
   float4_t va[kBatch], vb[kBatch];
   auto load_batch = [&](int b, float4_t (&dst)[kBatch]) {
@@ -72,7 +87,7 @@ __device__ __forceinline__ void small_m_walk(const float *__restrict__ W, float 
         k = K - 1;
       const char *row = reinterpret_cast<const char *>(W + k * N); // uniform base + 32-bit lane offset
       // ordinary loads, nontemporal stores: the combination that streams fastest here (nontemporal loads cost a fifth)
-      dst[j] = *reinterpret_cast<const float4_t *>(row + lane_bytes);
+      dst[j] = *reinterpret_cast<const float4_u *>(row + lane_bytes);
     }
   };
   auto consume_batch = [&](int b, const float4_t (&src)[kBatch]) {
@@ -92,16 +107,29 @@ __device__ __forceinline__ void small_m_walk(const float *__restrict__ W, float 
         const int j = j0 + jj;
         const int64_t k = k_wave + b * kBatch + j;
         float4_t w = src[j];
+        if (!kFull && !kAligned && cols < 4) {
+#pragma unroll
+          for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int e = c + 1; e < 4; ++e)
+              w[c] = e - c == 4 - cols ? src[j][e] : w[c]; // (columns past N: whatever, not stored)
+        }
         if (!kFull && k >= K)
           w = float4_t{0.0f, 0.0f, 0.0f, 0.0f}; // |0| adds nothing, and the row's x reads as zero
         float s[4];
         s[0] = sign_of(w.x, zero_to), s[1] = sign_of(w.y, zero_to);
         s[2] = sign_of(w.z, zero_to), s[3] = sign_of(w.w, zero_to);
-        if (kFull || (col_ok && k < K)) {
+        if (kFull || (cols == 4 && k < K)) {
           float4_t o;
           o.x = s[0], o.y = s[1], o.z = s[2], o.w = s[3];
           char *row = reinterpret_cast<char *>(Wb + k * N);
-          __builtin_nontemporal_store(o, reinterpret_cast<float4_t *>(row + lane_bytes));
+          __builtin_nontemporal_store(o, reinterpret_cast<float4_u *>(row + lane_bytes));
+        }
+        if (!kFull && !kAligned && k < K && cols < 4) {
+#pragma unroll
+          for (int c = 0; c < 3; ++c)
+            if (c < cols)
+              Wb[k * N + n0 + c] = s[c];
         }
         cs[0] += fabsf(w.x), cs[1] += fabsf(w.y), cs[2] += fabsf(w.z), cs[3] += fabsf(w.w);
 #pragma unroll
@@ -116,20 +144,20 @@ __device__ __forceinline__ void small_m_walk(const float *__restrict__ W, float 
   // so that the compiler does not hoist further batches (their registers would spill).
   load_batch(0, va);
 #pragma clang loop unroll(disable)
-  for (int b = 0; b < kBatches; b += 2) {
+  for (int b = 0; b < batches; b += 2) {
     load_batch(b + 1, vb);
     consume_batch(b, va);
-    if (b + 2 < kBatches)
+    if (b + 2 < batches)
       load_batch(b + 2, va);
     consume_batch(b + 1, vb);
   }
 }
 
-template <int MT, int kBatch>
-__global__ __launch_bounds__(kThreads, blocks_per_cu(MT)) void binary_affine_small_m(const float *__restrict__ W, float *__restrict__ Wb,
+template <int MT, int kBatch, bool kAligned>
+__global__ __launch_bounds__(kThreads, blocks_per_cu(MT, kAligned)) void binary_affine_small_m(const float *__restrict__ W, float *__restrict__ Wb,
                                                                   const float *__restrict__ x,
                                                                   float *__restrict__ partial, int64_t M, int64_t K,
-                                                                  int64_t N, int64_t Npad, float zero_to) {
+                                                                  int64_t N, int64_t Npad, float zero_to, int rows_per_wave) {
   constexpr int kVals = (MT + 1) * 4; // accumulators per lane
   __shared__ __attribute__((aligned(16))) float red[2 * kWavesN * kVals * 64];
 
@@ -137,9 +165,9 @@ __global__ __launch_bounds__(kThreads, blocks_per_cu(MT)) void binary_affine_sma
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); // uniform: row indices stay in scalar registers
   const int wn = wave % kWavesN, wk = wave / kWavesN;
   const int64_t slab = blockIdx.y;
-  const int64_t k_slab = slab * kSlabRows;
+  const int64_t slab_rows = kWavesK * rows_per_wave, k_slab = slab * slab_rows;
   const int64_t n0 = (int64_t)blockIdx.x * kStripCols + wn * kWaveCols + 4 * lane;
-  const int64_t k_wave = k_slab + wk * kRowsPerWave;
+  const int64_t k_wave = k_slab + wk * rows_per_wave;
 
   float acc[MT][4];
   float cs[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -149,11 +177,11 @@ __global__ __launch_bounds__(kThreads, blocks_per_cu(MT)) void binary_affine_sma
     for (int c = 0; c < 4; ++c)
       acc[m][c] = 0.0f;
 
-  const bool full = k_slab + kSlabRows <= K && ((int64_t)blockIdx.x + 1) * kStripCols <= N && M == MT;
+  const bool full = k_slab + slab_rows <= K && ((int64_t)blockIdx.x + 1) * kStripCols <= N && M == MT;
   if (full)
-    small_m_walk<MT, kBatch, true>(W, Wb, x, M, K, N, k_wave, n0, zero_to, acc, cs);
+    small_m_walk<MT, kBatch, true, kAligned>(W, Wb, x, M, K, N, k_wave, rows_per_wave, n0, zero_to, acc, cs);
   else
-    small_m_walk<MT, kBatch, false>(W, Wb, x, M, K, N, k_wave, n0, zero_to, acc, cs);
+    small_m_walk<MT, kBatch, false, kAligned>(W, Wb, x, M, K, N, k_wave, rows_per_wave, n0, zero_to, acc, cs);
 
   // Fold over wk in a fixed order: (wk0 + wk2) + (wk1 + wk3), through LDS.
   auto slot = [&](int s) { return red + ((size_t)(s * kWavesN + wn) * kVals) * 64 + lane; };
@@ -201,27 +229,27 @@ __global__ __launch_bounds__(kThreads, blocks_per_cu(MT)) void binary_affine_sma
   *reinterpret_cast<float4_t *>(out + (size_t)MT * Npad) = o;
 }
 
-// Thread (m, four columns): the slabs in slab order, alpha (binary_weight_affine.cpp:68: the column sum times the
-// rounded reciprocal of K), scale, bias.
+// Thread (m, four columns, every fourth slab), folded through LDS in a fixed order: the slabs' sums, alpha
+// (binary_weight_affine.cpp:68: the column sum times the rounded reciprocal of K), scale, bias.
 template <int MT>
 __global__ __launch_bounds__(256) void binary_affine_small_m_finish(const float *__restrict__ partial,
                                                                     float *__restrict__ alpha,
                                                                     const float *__restrict__ bias,
                                                                     float *__restrict__ y, int64_t M, int64_t N,
                                                                     int64_t Npad, int64_t slabs, float inv_k) {
-  const int64_t n0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  __shared__ float4_t s_dot[3][64], s_cs[3][64];
+  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
+  const int64_t n0 = ((int64_t)blockIdx.x * 64 + tx) * 4; // below Npad, whose columns past N hold what nothing uses
   const int m = blockIdx.y;
-  if (n0 >= N)
-    return;
   float4_t dot = {0.0f, 0.0f, 0.0f, 0.0f}, cs = {0.0f, 0.0f, 0.0f, 0.0f};
-  // eight slabs' loads are issued before the first is added (the adds keep slab order)
+  // eight slabs' loads are issued before the first is added
   constexpr int kAhead = 8;
   const size_t slab_stride = (size_t)(MT + 1) * Npad;
-  for (int64_t s0 = 0; s0 < slabs; s0 += kAhead) {
+  for (int64_t s0 = ty; s0 < slabs; s0 += 4 * kAhead) {
     float4_t d[kAhead], c[kAhead];
 #pragma unroll
     for (int j = 0; j < kAhead; ++j) {
-      const int64_t s = (s0 + j < slabs) ? s0 + j : slabs - 1; // clamped loads, masked below
+      const int64_t s = (s0 + 4 * j < slabs) ? s0 + 4 * j : s0; // clamped loads, masked below
       const float *p = partial + (size_t)s * slab_stride + n0;
       d[j] = *reinterpret_cast<const float4_t *>(p + (size_t)m * Npad);
       if (alpha)
@@ -229,38 +257,74 @@ __global__ __launch_bounds__(256) void binary_affine_small_m_finish(const float 
     }
 #pragma unroll
     for (int j = 0; j < kAhead; ++j) {
-      if (s0 + j >= slabs)
+      if (s0 + 4 * j >= slabs)
         break;
-      dot.x += d[j].x, dot.y += d[j].y, dot.z += d[j].z, dot.w += d[j].w;
+      dot += d[j];
       if (alpha)
-        cs.x += c[j].x, cs.y += c[j].y, cs.z += c[j].z, cs.w += c[j].w;
+        cs += c[j];
     }
   }
+  if (ty) {
+    s_dot[ty - 1][tx] = dot;
+    s_cs[ty - 1][tx] = cs;
+  }
+  __syncthreads();
+  if (ty || n0 >= N)
+    return;
+#pragma unroll
+  for (int g = 0; g < 3; ++g) {
+    dot += s_dot[g][tx];
+    cs += s_cs[g][tx];
+  }
+  const int cols = n0 + 4 <= N ? 4 : (int)(N - n0);
+  auto store = [&](float *dst, const float4_t &v) __attribute__((always_inline)) {
+    if (cols == 4) {
+      *reinterpret_cast<float4_u *>(dst) = v;
+    } else {
+#pragma unroll
+      for (int c = 0; c < 3; ++c)
+        if (c < cols)
+          dst[c] = v[c];
+    }
+  };
   if (alpha) {
-    float4_t a;
-    a.x = cs.x * inv_k, a.y = cs.y * inv_k, a.z = cs.z * inv_k, a.w = cs.w * inv_k;
+    const float4_t a = cs * inv_k;
     if (m == 0)
-      *reinterpret_cast<float4_t *>(alpha + n0) = a;
-    dot.x = dot.x * a.x, dot.y = dot.y * a.y, dot.z = dot.z * a.z, dot.w = dot.w * a.w;
+      store(alpha + n0, a);
+    dot = dot * a;
   }
   if (bias) {
-    const float4_t b = *reinterpret_cast<const float4_t *>(bias + n0);
-    dot.x = dot.x + b.x, dot.y = dot.y + b.y, dot.z = dot.z + b.z, dot.w = dot.w + b.w;
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      if (c < cols)
+        dot[c] = dot[c] + bias[n0 + c];
   }
-  *reinterpret_cast<float4_t *>(y + (size_t)m * N + n0) = dot;
+  store(y + (size_t)m * N + n0, dot);
+}
+
+template <int MT>
+int launch_finish(const float *partial, float *alpha, const float *bias, float *y, int64_t M, int64_t K, int64_t N,
+                  int64_t slabs, hipStream_t stream) {
+  hipLaunchKernelGGL(binary_affine_small_m_finish<MT>, dim3((unsigned)ceil_div(N, 256), (unsigned)M), dim3(256), 0,
+                     stream, partial, alpha, bias, y, M, N, small_m_padded_cols(N), slabs, (float)1 / K);
+  NBLA_HIP_LAUNCH_CHECK("binary_affine_small_m_finish");
+  return NBLA_HIP_OK;
 }
 
 template <int MT, int kBatch>
 int launch_small_m(const float *x, const float *W, float *Wb, float *alpha, const float *bias, float *y, int64_t M,
                    int64_t K, int64_t N, float zero_to, float *partial, hipStream_t stream) {
-  const int64_t Npad = small_m_padded_cols(N), slabs = small_m_slabs(K);
-  hipLaunchKernelGGL((binary_affine_small_m<MT, kBatch>), dim3((unsigned)(Npad / kStripCols), (unsigned)slabs),
-                     dim3(kThreads), 0, stream, W, Wb, x, partial, M, K, N, Npad, zero_to);
+  const int rows_per_wave = small_m_rows_per_wave(K, N);
+  const int64_t Npad = small_m_padded_cols(N), slabs = small_m_slabs(K, rows_per_wave);
+  const dim3 grid((unsigned)(Npad / kStripCols), (unsigned)slabs);
+  if (N % 4 == 0)
+    hipLaunchKernelGGL((binary_affine_small_m<MT, kBatch, true>), grid, dim3(kThreads), 0, stream, W, Wb, x, partial, M, K,
+                       N, Npad, zero_to, rows_per_wave);
+  else
+    hipLaunchKernelGGL((binary_affine_small_m<MT, kBatch, false>), grid, dim3(kThreads), 0, stream, W, Wb, x, partial, M,
+                       K, N, Npad, zero_to, rows_per_wave);
   NBLA_HIP_LAUNCH_CHECK("binary_affine_small_m");
-  hipLaunchKernelGGL(binary_affine_small_m_finish<MT>, dim3((unsigned)ceil_div(N / 4, 256), (unsigned)M), dim3(256), 0,
-                     stream, partial, alpha, bias, y, M, N, Npad, slabs, (float)1 / K);
-  NBLA_HIP_LAUNCH_CHECK("binary_affine_small_m_finish");
-  return NBLA_HIP_OK;
+  return launch_finish<MT>(partial, alpha, bias, y, M, K, N, slabs, stream);
 }
 
 
@@ -549,10 +613,7 @@ int launch_few_rows_mma(const float *x, const float *W, float *Wb, float *alpha,
   hipLaunchKernelGGL((binary_affine_few_rows_mma<kMF>), dim3((unsigned)p.strips, (unsigned)p.slabs),
                      dim3(64 * kMmaWaves), 0, stream, W, Wb, x, partial, M, K, N, Npad, p.tiles_per_wave, zero_to);
   NBLA_HIP_LAUNCH_CHECK("binary_affine_few_rows_mma");
-  hipLaunchKernelGGL(binary_affine_small_m_finish<MT>, dim3((unsigned)ceil_div(N / 4, 256), (unsigned)M), dim3(256), 0,
-                     stream, partial, alpha, bias, y, M, N, Npad, p.slabs, (float)1 / K);
-  NBLA_HIP_LAUNCH_CHECK("binary_affine_small_m_finish");
-  return NBLA_HIP_OK;
+  return launch_finish<MT>(partial, alpha, bias, y, M, K, N, p.slabs, stream);
 }
 
 } // namespace
@@ -576,7 +637,14 @@ bool small_m_affine_applies(const float *x, const float *W, const float *Wb, con
   if (!(M >= 1 && K >= 1 && N % 4 == 0 && N < (1ll << 29) && Wb && aligned16(W) && aligned16(Wb) && aligned16(y) &&
         aligned16(alpha) && aligned16(bias)))
     return false;
-  return few_rows_mma_applies(x, M, K, N, zero_to) || (M <= kSmallMMaxRows && small_m_slabs(K) <= 65535);
+  return few_rows_mma_applies(x, M, K, N, zero_to) || (M <= kSmallMMaxRows && small_m_slabs(K, kMostRowsPerWave) <= 65535);
+}
+
+// Rows of W at any multiple of four bytes: the vector-ALU walk alone (5 rows under 1500 x 3001: 42 us as signs, digits and
+// product in five launches, 18 this way).
+bool small_m_affine_covers(const float *Wb, int64_t M, int64_t K, int64_t N) {
+  return M >= 1 && M <= kSmallMMaxRows && K >= 1 && N >= 4 && N < (1ll << 29) && Wb &&
+         small_m_slabs(K, kMostRowsPerWave) <= 65535;
 }
 
 // (sized without knowing x: the larger of the two forms where both may run)
@@ -590,7 +658,7 @@ size_t small_m_affine_workspace_bytes(int64_t M, int64_t K, int64_t N) {
   }
   if (M <= kSmallMMaxRows) {
     const int64_t mt = M <= 1 ? 1 : M <= 2 ? 2 : M <= 4 ? 4 : M <= 8 ? 8 : 16;
-    const size_t valu = (size_t)small_m_slabs(K) * (mt + 1) * small_m_padded_cols(N) * sizeof(float);
+    const size_t valu = (size_t)small_m_slabs(K, small_m_rows_per_wave(K, N)) * (mt + 1) * small_m_padded_cols(N) * sizeof(float);
     bytes = valu > bytes ? valu : bytes;
   }
   return bytes;
@@ -602,7 +670,7 @@ int launch_small_m_affine(const float *x, const float *W, float *Wb, float *alph
   if (workspace_bytes < small_m_affine_workspace_bytes(M, K, N) || !aligned16(workspace))
     return fail(NBLA_HIP_ERR_MEMORY, "small-M binary affine workspace too small or misaligned.");
   float *partial = static_cast<float *>(workspace);
-  if (few_rows_mma_applies(x, M, K, N, zero_to)) {
+  if (N % 4 == 0 && aligned16(W) && aligned16(Wb) && few_rows_mma_applies(x, M, K, N, zero_to)) {
     if (M <= 32)
       return launch_few_rows_mma<1>(x, W, Wb, alpha, bias, y, M, K, N, zero_to, partial, stream);
     return launch_few_rows_mma<2>(x, W, Wb, alpha, bias, y, M, K, N, zero_to, partial, stream);

@@ -172,6 +172,7 @@ constexpr int64_t kSmallMMaxRows = 16;  // rows the one-pass form multiplies on 
 constexpr int64_t kFewRowsMaxRows = 64; // rows the one-pass form multiplies on the matrix cores
 bool small_m_affine_applies(const float *x, const float *W, const float *Wb, const float *alpha, const float *bias,
                             const float *y, int64_t M, int64_t K, int64_t N, float zero_to);
+bool small_m_affine_covers(const float *Wb, int64_t M, int64_t K, int64_t N); // up to sixteen rows, any alignment
 size_t small_m_affine_workspace_bytes(int64_t M, int64_t K, int64_t N);
 int launch_small_m_affine(const float *x, const float *W, float *Wb, float *alpha, const float *bias, float *y,
                           int64_t M, int64_t K, int64_t N, float zero_to, void *workspace, size_t workspace_bytes,
