@@ -341,7 +341,9 @@ int launch_fused_affine(const float *x, const float *W, float *Wb, float *alpha,
   a.x_bytes = (uint32_t)(M * K * 4), a.w_bytes = (uint32_t)(K * N * 4);
   // Few blocks: the chain of one block is the time, so blocks of one fragment of columns, K over eight wavefronts and no
   // more k tiles in a wavefront than there are (20 x 250 x 250: 9.1 -> 4.9 us).
-  if (ceil_div(M, kFusedRows) * ceil_div(N, kWideCols) <= 128) {
+  // (Twice as many blocks with one k tile, where a block has little to do: 1000 x 120 x 500 8.5 -> 6.9; with more it is
+  // slower, 800 x 816 x 632 17 -> 22.)
+  if (ceil_div(M, kFusedRows) * ceil_div(N, kWideCols) <= (K <= 8 * kTileK ? 256 : 128)) {
     if (K <= 8 * kTileK)
       return run_fused<8, 1, 1>(a, stream);
     if (K <= 16 * kTileK)
