@@ -167,7 +167,14 @@ int nbla_hip_binary_affine_backward_f32(const float *dy, const float *x, const f
     return rc;
   hipStream_t stream = as_stream(stream_);
   char *base = static_cast<char *>(workspace);
-  if (dx) {
+  const bool one_part = quantize_zero_to == 1.0f || quantize_zero_to == -1.0f || quantize_zero_to == 0.0f;
+  if (dx && one_part && gemm_small_applies(M, N, K, kSmallGradInput)) {
+    // small layers: the signs straight from W, in one launch
+    rc = launch_gemm_small(dy, false, W, false, nullptr, dx, M, N, K, accum_x != 0, stream, true, alpha,
+                           quantize_zero_to);
+    if (rc)
+      return rc;
+  } else if (dx) {
     const bool representable = (quantize_zero_to == 1.0f || quantize_zero_to == -1.0f);
     uint32_t *bits = reinterpret_cast<uint32_t *>(base + p.bits_off);
     int *count = reinterpret_cast<int *>(base + p.count_off);

@@ -19,6 +19,11 @@
 // 35.2 -> 7.5 us, 512^3 40.6 -> 9.5, 200 x 1000 x 1000 43.7 -> 14.8, 1024^3 53 -> 29, 128 x 4096 x 4096 88 -> 45; weight
 // gradient at 200 x 1000 x 1000 36.4 -> 13.3, input gradient 31.9 -> 15.3.  Off float64 (relative, 2-norm): 3e-8 to 1.0e-7
 // where the digits are 1.6e-7 to 8.6e-7 off.
+//
+// With signs, Sign(B) stands for B, exact in one bf16 part: three products, no splitting of B.  The input gradient of a
+// small binary layer is dy alpha . Sign(W)^T this way, 29 us as packed signs, digits and product in four launches: 20 x
+// 250 x 250 5.0, 512^3 8.7, 200 x 368 x 257 6.4, 64 x 1000 x 1000 11.6, 600 x 700 x 800 (32) 16.2; off float64 3.6e-8, the
+// digits 1.5e-7.
 #include "bf16_parts.hpp"
 #include "common.hpp"
 #include "gemm_layout.hpp"
@@ -43,6 +48,8 @@ struct SmallArgs {
   float *y;          // [M, N], rows N apart
   int M, K, N, n_tiles, accumulate;
   uint32_t a_bytes, b_bytes;
+  const float *kscale; // may be null; with signs only: A(m, k) is multiplied by kscale[k] first, rounded once
+  float zero_to;       // with signs: what stands for a value of B that is neither negative nor positive (-1, 0 or 1)
 };
 
 // The sixteen values k = 32 t + 16 half .. of one row (column) of an operand with `count` of them, `f` the lane's own.
@@ -92,8 +99,14 @@ __device__ __forceinline__ f32x16_t mma(const uint4_t &a, const uint4_t &b, f32x
 #endif
 }
 
-// kFrags: fragments of 32 columns of a block
-template <int kWaves, int kFrags, bool kAAcross, bool kBAcross>
+// Sign(v), which bf16 holds in one part.
+__device__ __forceinline__ float small_sign(float v, float zero_to) {
+  const float one = __uint_as_float((__float_as_uint(v) & 0x80000000u) | 0x3f800000u);
+  return __builtin_islessgreater(v, 0.0f) ? one : zero_to;
+}
+
+// kFrags: fragments of 32 columns of a block.  kSigns: Sign(B) in the place of B, three products instead of six.
+template <int kWaves, int kFrags, bool kAAcross, bool kBAcross, bool kSigns>
 __global__ __launch_bounds__(64 * kWaves, 2) void gemm_small(SmallArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int kCols = 32 * kFrags;
@@ -120,15 +133,30 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_small(SmallArgs a) {
   uint32_t max_a = 0u, max_b[kFrags] = {};
 
   struct Tile {
-    float av[16], bv[kFrags][16];
+    float av[16], bv[kFrags][16], sc[kSigns ? 16 : 1];
   };
   auto load = [&](int t, Tile &w) __attribute__((always_inline)) {
     load_tile<kAAcross>(ar, t, half, m0 + r, a.M, a.K, w.av);
 #pragma unroll
     for (int f = 0; f < kFrags; ++f)
       load_tile<kBAcross>(br, t, half, n0 + 32 * f + r, a.N, a.K, w.bv[f]);
+    if (kSigns) {
+#pragma unroll
+      for (int j = 0; j < 16; ++j)
+        w.sc[j] = a.kscale ? a.kscale[min(t * kTile + 16 * half + j, a.K - 1)] : 1.0f;
+    }
   };
   auto take = [&](int t, Tile &w) __attribute__((always_inline)) {
+    if (kSigns) {
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        if (a.kscale)
+          w.av[j] = w.av[j] * w.sc[j];
+#pragma unroll
+        for (int f = 0; f < kFrags; ++f)
+          w.bv[f][j] = small_sign(w.bv[f][j], a.zero_to);
+      }
+    }
     if (t * kTile + kTile > a.K) { // uniform: the last tile
       const int k0 = t * kTile + 16 * half;
 #pragma unroll
@@ -145,7 +173,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_small(SmallArgs a) {
       max_a = max(max_a, __float_as_uint(w.av[j]) & 0x7fffffffu);
 #pragma unroll
       for (int f = 0; f < kFrags; ++f)
-        max_b[f] = max(max_b[f], __float_as_uint(w.bv[f][j]) & 0x7fffffffu);
+        if (!kSigns)
+          max_b[f] = max(max_b[f], __float_as_uint(w.bv[f][j]) & 0x7fffffffu);
     }
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
@@ -154,6 +183,16 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_small(SmallArgs a) {
 #pragma unroll
       for (int f = 0; f < kFrags; ++f) {
         uint4_t bh, bm, bl;
+        if (kSigns) {
+#pragma unroll
+          for (int p = 0; p < 4; ++p)
+            bh[p] = __builtin_amdgcn_perm(__float_as_uint(w.bv[f][8 * s + 2 * p + 1]), __float_as_uint(w.bv[f][8 * s + 2 * p]),
+                                          0x07060302u);
+          acc[f][0] = mma(ah, bh, acc[f][0]);
+          acc[f][1] = mma(al, bh, acc[f][1]);
+          acc[f][1] = mma(am, bh, acc[f][1]);
+          continue;
+        }
         split3(w.bv[f], s, bh, bm, bl);
         acc[f][0] = mma(ah, bh, acc[f][0]);
         acc[f][1] = mma(ah, bl, acc[f][1]);
@@ -242,8 +281,12 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_small(SmallArgs a) {
       continue;
     double sum = 0.0;
     for (int k = 0; k < a.K; ++k) {
-      const float av = kAAcross ? a.a[(int64_t)k * a.M + m] : a.a[(int64_t)m * a.K + k];
-      const float bv = kBAcross ? a.b[(int64_t)k * a.N + n] : a.b[(int64_t)n * a.K + k];
+      float av = kAAcross ? a.a[(int64_t)k * a.M + m] : a.a[(int64_t)m * a.K + k];
+      float bv = kBAcross ? a.b[(int64_t)k * a.N + n] : a.b[(int64_t)n * a.K + k];
+      if (kSigns) {
+        av = a.kscale ? av * a.kscale[k] : av;
+        bv = small_sign(bv, a.zero_to);
+      }
       sum = sum + (double)av * (double)bv;
     }
     const int64_t o = (int64_t)m * a.N + n;
@@ -253,17 +296,17 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_small(SmallArgs a) {
 #endif
 }
 
-template <int kFrags, bool kAAcross, bool kBAcross> int run_small(SmallArgs &a, hipStream_t stream) {
+template <int kFrags, bool kAAcross, bool kBAcross, bool kSigns = false> int run_small(SmallArgs &a, hipStream_t stream) {
   constexpr int kWaves = kWavesPerBlock;
   static std::atomic<uint64_t> configured{0};
   constexpr int lds = kWaves * 32 * 64 * 4;
-  const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(gemm_small<kWaves, kFrags, kAAcross, kBAcross>), lds,
+  const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(gemm_small<kWaves, kFrags, kAAcross, kBAcross, kSigns>), lds,
                                    configured, "hipFuncSetAttribute(gemm_small LDS size)");
   if (rc)
     return rc;
   a.n_tiles = (int)ceil_div(a.N, 32 * kFrags);
   const int64_t blocks = a.n_tiles * ceil_div(a.M, kRows);
-  hipLaunchKernelGGL((gemm_small<kWaves, kFrags, kAAcross, kBAcross>), dim3((unsigned)blocks), dim3(64 * kWaves), lds,
+  hipLaunchKernelGGL((gemm_small<kWaves, kFrags, kAAcross, kBAcross, kSigns>), dim3((unsigned)blocks), dim3(64 * kWaves), lds,
                      stream, a);
   NBLA_HIP_LAUNCH_CHECK("gemm_small");
   return NBLA_HIP_OK;
@@ -286,17 +329,21 @@ bool gemm_small_applies(int64_t M, int64_t K, int64_t N, int64_t limit) {
 }
 
 int launch_gemm_small(const float *A, bool a_across, const float *B, bool b_across, const float *bias, float *y,
-                      int64_t M, int64_t K, int64_t N, bool accumulate, hipStream_t stream) {
+                      int64_t M, int64_t K, int64_t N, bool accumulate, hipStream_t stream, bool signs,
+                      const float *kscale, float zero_to) {
   SmallArgs a;
   a.a = A, a.b = B, a.bias = bias, a.y = y;
   a.M = (int)M, a.K = (int)K, a.N = (int)N, a.accumulate = accumulate ? 1 : 0;
   a.a_bytes = (uint32_t)(M * K * 4), a.b_bytes = (uint32_t)(K * N * 4);
+  a.kscale = kscale, a.zero_to = zero_to;
   // few blocks: half as wide, so that a block's chain is shorter (20 x 250 x 250: 6.9 -> 4.9 us)
   const bool narrow = ceil_div(M, kRows) * ceil_div(N, kWideCols) <= 128;
   if (a_across)
     return narrow ? run_small<1, true, true>(a, stream) : run_small<2, true, true>(a, stream);
   if (b_across)
     return narrow ? run_small<1, false, true>(a, stream) : run_small<2, false, true>(a, stream);
+  if (signs)
+    return narrow ? run_small<1, false, false, true>(a, stream) : run_small<2, false, false, true>(a, stream);
   return narrow ? run_small<1, false, false>(a, stream) : run_small<2, false, false>(a, stream);
 }
 

@@ -20,14 +20,17 @@ int launch_gemm_f32(const float *x, const float *w, const float *colscale, const
 int launch_clear_words(void *dst, size_t count, hipStream_t stream);
 
 // y[M, N] = A . B (+ bias) of real-valued matrices in one launch, for small products (gemm_small.hip).  A is [M, K], or
-// [K, M] when a_across; B is [K, N] when b_across, else [N, K] (a_across without b_across is not there).
+// [K, M] when a_across; B is [K, N] when b_across, else [N, K] (a_across without b_across is not there).  signs (neither
+// across): Sign(B) in the place of B, with zero_to -1, 0 or 1 for what is neither negative nor positive, and A(m, k) times
+// kscale[k] (may be null).
 // `limit`: in units of about a microsecond, the time up to which it is the faster form, from measured sizes on both
 // sides: as x . W (the digit path 35 to 62 us there), as x^T . dy (36 to 48) and as dy . W^T (20 to 38: its operands
-// need no column statistics).
+// need no column statistics), as dy . Sign(W)^T (28 to 36, four launches).
 constexpr int64_t kSmallForward = 40, kSmallGradWeights = 40, kSmallGradInput = 24;
 bool gemm_small_applies(int64_t M, int64_t K, int64_t N, int64_t limit);
 int launch_gemm_small(const float *A, bool a_across, const float *B, bool b_across, const float *bias, float *y,
-                      int64_t M, int64_t K, int64_t N, bool accumulate, hipStream_t stream);
+                      int64_t M, int64_t K, int64_t N, bool accumulate, hipStream_t stream, bool signs = false,
+                      const float *kscale = nullptr, float zero_to = 1.0f);
 
 // Bit-weight product with the choice of store orientation: swap_out makes consecutive lanes write consecutive m
 // (for outputs whose m index is the contiguous one, e.g. convolution results [batch, O, Ho*Wo]).  keep_bad_rows: rows
