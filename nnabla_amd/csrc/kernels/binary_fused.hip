@@ -171,10 +171,10 @@ __global__ __launch_bounds__(64 * kWaves, 2) void binary_affine_fused(FusedArgs 
           f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(xr, (int)(row_in && k0 + 4 * v < a.K ? off + 16 * v : kOutside),
                                                          0, 0));
   }
-  float w[kTiles > 1 ? 2 : 1][kFrags][16];
-  load_w(min(wave, k_tiles - 1), w[0]);
+  float w0[kFrags][16], w1[kFrags][16];
+  load_w(min(wave, k_tiles - 1), w0);
   if constexpr (kTiles > 1)
-    load_w(min(wave + kWaves, k_tiles - 1), w[1]);
+    load_w(min(wave + kWaves, k_tiles - 1), w1);
   uint32_t amax = 0u, bad = 0u;
 #pragma unroll
   for (int i = 0; i < kTiles; ++i) {
@@ -213,15 +213,31 @@ __global__ __launch_bounds__(64 * kWaves, 2) void binary_affine_fused(FusedArgs 
     for (int d = 0; d < kDigits; ++d)
       xd[i][d] = uint4_t{words[d][0], words[d][1], words[d][2], words[d][3]};
   }
+  static_assert(kTiles == 1 || kTiles == 2 || kTiles == 4, "one tile, a pair or two pairs");
   uint4_t b[kFrags];
-#pragma unroll
-  for (int i = 0; i < kTiles; ++i)
-    if (wave + i * kWaves < k_tiles) {
-      take_tile(wave + i * kWaves, w[i & (kTiles > 1 ? 1 : 0)], b);
-      if (i + 2 < kTiles)
-        load_w(min(wave + (i + 2) * kWaves, k_tiles - 1), w[i & (kTiles > 1 ? 1 : 0)]);
-      multiply(xd[i], b);
+  if (wave < k_tiles) {
+    take_tile(wave, w0, b);
+    if constexpr (kTiles > 2)
+      load_w(min(wave + 2 * kWaves, k_tiles - 1), w0);
+    multiply(xd[0], b);
+  }
+  if constexpr (kTiles > 1)
+    if (wave + kWaves < k_tiles) {
+      take_tile(wave + kWaves, w1, b);
+      if constexpr (kTiles > 2)
+        load_w(min(wave + 3 * kWaves, k_tiles - 1), w1);
+      multiply(xd[1], b);
     }
+  if constexpr (kTiles > 2) {
+    if (wave + 2 * kWaves < k_tiles) {
+      take_tile(wave + 2 * kWaves, w0, b);
+      multiply(xd[2], b);
+    }
+    if (wave + 3 * kWaves < k_tiles) {
+      take_tile(wave + 3 * kWaves, w1, b);
+      multiply(xd[3], b);
+    }
+  }
 
   // ---- the wavefronts' sums, one fragment of 32 columns at a time: each finishes 16 / kWaves accumulator registers
 #pragma unroll
