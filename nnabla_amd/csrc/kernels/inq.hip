@@ -74,7 +74,17 @@ InqWorkspace plan_inq(int64_t size, int selection) {
 // Step A (inq_affine.cpp:95-102) fused with the max|w| scan of step C (:153-158).
 __global__ __launch_bounds__(kBlk) void inq_restore_absmax(float *__restrict__ W, const float *__restrict__ old_W,
                                                            const int *__restrict__ old_I, int64_t size, int vec,
-                                                           uint32_t *__restrict__ partial) {
+                                                           uint32_t *__restrict__ partial, ColumnScratch cols) {
+  // the column statistics that the quantize pass will gather (cols.cmax null: none wanted) start from their neutral
+  // values
+  if (cols.cmax) {
+    for (int64_t i = (int64_t)blockIdx.x * kBlk + threadIdx.x; i < cols.rows; i += (int64_t)gridDim.x * kBlk) {
+      cols.cmax[i] = 0u;
+      cols.cmin[i] = 0xffffffffu;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+      *cols.flag = 0;
+  }
   typedef float f4_t __attribute__((ext_vector_type(4)));
   typedef int i4_t __attribute__((ext_vector_type(4)));
   uint32_t mx = 0u; // bits of a non-negative float order like the float
@@ -158,44 +168,32 @@ __global__ __launch_bounds__(kBlk) void inq_restore_absmax(float *__restrict__ W
 }
 
 // n1, n2 and the pruning threshold (inq_affine.cpp:157-166).  `levels` is the
-// host's (int)pow(2, num_bits - 2).
-constexpr int kFinalizeThreads = 1024; // one round trip for the up to kMaxPartials partial maxima
-__global__ __launch_bounds__(kFinalizeThreads) void inq_finalize(const uint32_t *__restrict__ partial, int nparts, int levels,
-                                                   const uint32_t *__restrict__ n1_cuts, InqParams *__restrict__ params,
-                                                   ColumnScratch cols) {
-  // the column statistics that the quantize pass will gather (cols.cmax null: none wanted) start from their neutral
-  // values
-  if (cols.cmax) {
-    for (int64_t i = threadIdx.x; i < cols.rows; i += kFinalizeThreads) {
-      cols.cmax[i] = 0u;
-      cols.cmin[i] = 0xffffffffu;
-    }
-    if (threadIdx.x == 0)
-      *cols.flag = 0;
-  }
+// host's (int)pow(2, num_bits - 2).  Every block of the quantizing pass folds the partial maxima (4 KiB, in the L2) itself:
+// a launch of one block for it cost 4 to 5 us of the chain.  Block 0 leaves the result in `params` for the caller.
+__device__ __forceinline__ InqParams inq_fold_params(const uint32_t *__restrict__ partial, int nparts, int levels,
+                                                     const uint32_t *__restrict__ n1_cuts, InqParams *__restrict__ params) {
+  __shared__ uint32_t s_mx[kBlk / 64];
   uint32_t mx = 0u, unfixed = 0u; // (bit 31 of a partial result: the block met a weight that is not fixed)
-  for (int i = threadIdx.x; i < nparts; i += kFinalizeThreads) {
-    const uint32_t v = partial[i];
+  static_assert(kMaxPartials <= 4 * kBlk, "one round trip");
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int i = threadIdx.x + j * kBlk;
+    const uint32_t v = i < nparts ? partial[i] : 0u;
     unfixed |= v >> 31;
-    mx = (v & 0x7fffffffu) > mx ? (v & 0x7fffffffu) : mx;
+    mx = max(mx, v & 0x7fffffffu);
   }
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    const uint32_t o = __shfl_xor(mx, off);
-    mx = o > mx ? o : mx;
-  }
+  for (int off = 32; off >= 1; off >>= 1)
+    mx = max(mx, (uint32_t)__shfl_xor((int)mx, off));
   mx |= __any(unfixed != 0u) ? 0x80000000u : 0u;
-  __shared__ uint32_t s_mx[kFinalizeThreads / 64];
   if ((threadIdx.x & 63) == 0)
     s_mx[threadIdx.x >> 6] = mx;
   __syncthreads();
-  if (threadIdx.x != 0)
-    return;
-  unfixed = mx >> 31;
-  mx &= 0x7fffffffu;
-  for (int w = 1; w < kFinalizeThreads / 64; ++w) {
+  mx = 0u, unfixed = 0u;
+#pragma unroll
+  for (int w = 0; w < kBlk / 64; ++w) {
     unfixed |= s_mx[w] >> 31;
-    mx = (s_mx[w] & 0x7fffffffu) > mx ? (s_mx[w] & 0x7fffffffu) : mx;
+    mx = max(mx, s_mx[w] & 0x7fffffffu);
   }
   if (mx == 0u)
     mx = 0x3f800000u; // max_absval == 0 -> 1
@@ -220,7 +218,9 @@ __global__ __launch_bounds__(kFinalizeThreads) void inq_finalize(const uint32_t 
   p.n2 = n2;
   p.thr = thr;
   p.all_fixed = unfixed ? 0 : 1;
-  *params = p;
+  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0)
+    *params = p;
+  return p;
 }
 
 // Step C for one fixed weight (:168-190).
@@ -256,31 +256,61 @@ __device__ __forceinline__ float inq_quantize_value(float w, const InqParams &p,
   return w;
 }
 
-// Step C for the fixed weights (:168-190) and step F (:203-204).
+// What the quantizing pass folds its parameters from.
+struct InqFold {
+  const uint32_t *partial, *n1_cuts;
+  InqParams *params;
+  int nparts, levels;
+};
+
+// Step C for the fixed weights (:168-190) and step F (:203-204).  vec: 16-byte aligned arrays, four weights per lane and
+// access (1968 x 1968: 11.9 us with one, 8.2 with four and the parameters folded in).
 __global__ __launch_bounds__(kBlk) void inq_quantize(float *__restrict__ W, int *__restrict__ I, float *__restrict__ old_W,
-                                                     int *__restrict__ old_I, int64_t size, int fix_all,
-                                                     const InqParams *__restrict__ params,
-                                                     const uint32_t *__restrict__ e_cuts) {
+                                                     int *__restrict__ old_I, int64_t size, int vec, int fix_all,
+                                                     InqFold fold, const uint32_t *__restrict__ e_cuts) {
+  typedef float f4_t __attribute__((ext_vector_type(4)));
+  typedef int i4_t __attribute__((ext_vector_type(4)));
   __shared__ uint32_t s_cut[kNumBinades];
   for (int i = threadIdx.x; i < kNumBinades; i += kBlk)
     s_cut[i] = e_cuts[i];
-  __syncthreads();
-  const InqParams p = *params;
+  const InqParams p = inq_fold_params(fold.partial, fold.nparts, fold.levels, fold.n1_cuts, fold.params); // (a barrier)
+  // A fixed weight of a snapshot that held every weight as fixed was copied from that snapshot by this call's
+  // restoring pass; if quantizing leaves its bits alone, W, the snapshot and its indicator hold the values
+  // already and nothing is written (the steady state once every weight is fixed).
   const bool settled = p.all_fixed != 0 && !fix_all;
-  for (int64_t i = (int64_t)blockIdx.x * kBlk + threadIdx.x; i < size; i += (int64_t)gridDim.x * kBlk) {
+  const int64_t first = (int64_t)blockIdx.x * kBlk + threadIdx.x, stride = (int64_t)gridDim.x * kBlk;
+  const int64_t n4 = vec ? size / 4 : 0;
+  for (int64_t i = first; i < n4; i += stride) {
+    const f4_t w0 = reinterpret_cast<const f4_t *>(W)[i];
+    i4_t ind = {1, 1, 1, 1};
+    if (!fix_all)
+      ind = reinterpret_cast<const i4_t *>(I)[i];
+    f4_t w = w0;
+    bool same = settled;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      w[c] = ind[c] == 1 ? inq_quantize_value(w0[c], p, s_cut) : w0[c];
+      same = same && ind[c] == 1 && __float_as_uint(w[c]) == __float_as_uint(w0[c]);
+    }
+    if (same)
+      continue;
+    reinterpret_cast<f4_t *>(W)[i] = w;
+    if (fix_all)
+      reinterpret_cast<i4_t *>(I)[i] = ind; // otherwise unchanged
+    reinterpret_cast<f4_t *>(old_W)[i] = w;
+    reinterpret_cast<i4_t *>(old_I)[i] = ind;
+  }
+  for (int64_t i = 4 * n4 + first; i < size; i += stride) {
     const float w0 = W[i];
     float w = w0;
     const int ind = fix_all ? 1 : I[i];
     if (ind == 1)
       w = inq_quantize_value(w, p, s_cut);
-    // A fixed weight of a snapshot that held every weight as fixed was copied from that snapshot by this call's
-    // restoring pass; if quantizing leaves its bits alone, W, the snapshot and its indicator hold the values
-    // already and nothing is written (the steady state once every weight is fixed).
     if (settled && ind == 1 && __float_as_uint(w) == __float_as_uint(w0))
       continue;
     W[i] = w;
     if (fix_all)
-      I[i] = ind; // otherwise unchanged
+      I[i] = ind;
     old_W[i] = w;
     old_I[i] = ind;
   }
@@ -294,8 +324,8 @@ __global__ __launch_bounds__(kBlk) void inq_quantize(float *__restrict__ W, int 
 __global__ __launch_bounds__(kBlk) void inq_quantize_columns(float *__restrict__ W, int *__restrict__ I,
                                                              float *__restrict__ old_W, int *__restrict__ old_I,
                                                              int64_t R, int64_t C, int slab, int fix_all,
-                                                             const InqParams *__restrict__ params,
-                                                             const uint32_t *__restrict__ e_cuts, ColumnScratch cols) {
+                                                             InqFold fold, const uint32_t *__restrict__ e_cuts,
+                                                             ColumnScratch cols) {
   typedef float f4_t __attribute__((ext_vector_type(4)));
   typedef int i4_t __attribute__((ext_vector_type(4)));
   static_assert(kBlk == 256, "64 column quads x 4 row groups");
@@ -303,8 +333,7 @@ __global__ __launch_bounds__(kBlk) void inq_quantize_columns(float *__restrict__
   __shared__ uint32_t part[4][256], part_min[4][256];
   for (int i = threadIdx.x; i < kNumBinades; i += kBlk)
     s_cut[i] = e_cuts[i];
-  __syncthreads();
-  const InqParams p = *params;
+  const InqParams p = inq_fold_params(fold.partial, fold.nparts, fold.levels, fold.n1_cuts, fold.params); // (a barrier)
   const bool settled = p.all_fixed != 0 && !fix_all;
   const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
   const int64_t c0 = ((int64_t)blockIdx.x * 64 + tx) * 4;
@@ -615,8 +644,12 @@ int update_weights(float *W, int *I, float *old_W, int *old_I, int64_t size, int
   if (nparts > (unsigned)kMaxPartials)
     nparts = kMaxPartials;
 
+  const int vec = aligned16(W) && aligned16(I) && aligned16(old_W) && aligned16(old_I) ? 1 : 0;
+  const bool with_cols = cols && columns > 0 && columns % 4 == 0 && size % columns == 0 && vec;
+  ColumnScratch none;
+  none.cmax = none.cmin = nullptr, none.flag = nullptr, none.rows = 0;
   hipLaunchKernelGGL(inq_restore_absmax, dim3(nparts), dim3(kBlk), 0, stream, W, old_W, old_I, size,
-                     (aligned16(W) && aligned16(old_W) && aligned16(old_I)) ? 1 : 0, partial);
+                     (aligned16(W) && aligned16(old_W) && aligned16(old_I)) ? 1 : 0, partial, with_cols ? *cols : none);
   NBLA_HIP_LAUNCH_CHECK("inq_restore_absmax");
 
   const ChunkPlan cp = plan_chunks(size);
@@ -672,25 +705,21 @@ int update_weights(float *W, int *I, float *old_W, int *old_I, int64_t size, int
     }
   }
 
-  const int levels = (int)std::pow(2, num_bits - 2); // inq_affine.cpp:165
-  const bool with_cols = cols && columns > 0 && columns % 4 == 0 && size % columns == 0 && aligned16(W) &&
-                         aligned16(I) && aligned16(old_W) && aligned16(old_I);
-  ColumnScratch none;
-  none.cmax = none.cmin = nullptr, none.flag = nullptr, none.rows = 0;
-  hipLaunchKernelGGL(inq_finalize, dim3(1), dim3(kFinalizeThreads), 0, stream, partial, (int)nparts, levels,
-                     device_cut_table(kCutInqN1), params, with_cols ? *cols : none);
-  NBLA_HIP_LAUNCH_CHECK("inq_finalize");
+  const InqFold fold{partial, device_cut_table(kCutInqN1), params, (int)nparts,
+                     (int)std::pow(2, num_bits - 2)}; // inq_affine.cpp:165
   if (with_cols) {
     const int64_t R = size / columns;
     int slab = 64;
     while (slab < 256 && ceil_div(columns, 256) * ceil_div(R, 2 * slab) >= 1024)
       slab *= 2;
     hipLaunchKernelGGL(inq_quantize_columns, dim3((unsigned)ceil_div(columns, 256), (unsigned)ceil_div(R, slab)),
-                       dim3(kBlk), 0, stream, W, I, old_W, old_I, R, columns, slab, step == 1 ? 1 : 0, params,
+                       dim3(kBlk), 0, stream, W, I, old_W, old_I, R, columns, slab, step == 1 ? 1 : 0, fold,
                        device_cut_table(kCutInqExponent), *cols);
   } else {
-    hipLaunchKernelGGL(inq_quantize, dim3(grid_for(size)), dim3(kBlk), 0, stream, W, I, old_W, old_I, size,
-                       step == 1 ? 1 : 0, params, device_cut_table(kCutInqExponent));
+    int64_t blocks = ceil_div(vec ? size / 4 + 1 : size, kBlk);
+    blocks = blocks < 2048 ? blocks : 2048; // (every block folds the partial maxima)
+    hipLaunchKernelGGL(inq_quantize, dim3((unsigned)blocks), dim3(kBlk), 0, stream, W, I, old_W, old_I, size, vec,
+                       step == 1 ? 1 : 0, fold, device_cut_table(kCutInqExponent));
   }
   NBLA_HIP_LAUNCH_CHECK("inq_quantize");
   if (cols_done)
