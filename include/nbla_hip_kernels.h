@@ -713,6 +713,14 @@ int nbla_hip_copy_rows_f32(const float *src, int64_t src_stride, float *dst,
 /* y = max(0, x).  Replaces ReLU<float>::forward_impl,
  * src/nbla/function/generic/relu.cpp (std::max(T(0), x)). */
 int nbla_hip_relu_f32(const float *x, float *y, size_t size, void *stream);
+
+/* mid = max(0, x), y = FixedPointQuantize(mid; sign, n, delta): both functions'
+ * results, the bits of nbla_hip_relu_f32 followed by
+ * nbla_hip_fixed_point_quantize_f32, in one launch and without reading mid
+ * back.  mid and y may each be x or one another, not overlap otherwise. */
+int nbla_hip_relu_fixed_point_quantize_f32(const float *x, float *mid, float *y,
+                                           size_t size, int sign, int n,
+                                           float delta, void *stream);
 /* dx (+)= (y > 0 ? dy : 0) with y the forward output.  Replaces
  * ReLU<float>::backward_impl, src/nbla/function/generic/relu.cpp:41-66. */
 int nbla_hip_relu_backward_f32(const float *dy, const float *y, float *dx,

@@ -325,6 +325,27 @@ NBLA_API int nblac_function_forward(void *f, void **inputs, int ni, void **outpu
   return guarded(
       [&] { static_cast<FuncHandle *>(f)->func->forward(to_variables(inputs, ni), to_variables(outputs, no)); });
 }
+// The forward pass of `n` functions in order: function i takes the next num_inputs[i] of `inputs` and writes the next
+// num_outputs[i] of `outputs`.  A function and the one that follows it on its output may run as one launch.
+NBLA_API int nblac_functions_forward(int n, void **functions, const int *num_inputs, void **inputs, const int *num_outputs,
+                                     void **outputs) {
+  return guarded([&] {
+    for (int i = 0; i < n; ++i) {
+      Function *f = static_cast<FuncHandle *>(functions[i])->func.get();
+      const Variables in = to_variables(inputs, num_inputs[i]), out = to_variables(outputs, num_outputs[i]);
+      inputs += num_inputs[i], outputs += num_outputs[i];
+      if (i + 1 < n && in.size() == 1 && out.size() == 1 && num_inputs[i + 1] == 1 && num_outputs[i + 1] == 1) {
+        const Variables next_in = to_variables(inputs, 1), next_out = to_variables(outputs, 1);
+        Function *next = static_cast<FuncHandle *>(functions[i + 1])->func.get();
+        if (next_in[0] == out[0] && f->forward_with_next(in, out, *next, next_in, next_out)) {
+          ++inputs, ++outputs, ++i;
+          continue;
+        }
+      }
+      f->forward(in, out);
+    }
+  });
+}
 NBLA_API int nblac_function_recompute(void *f, void **inputs, int ni, void **outputs, int no) {
   return guarded(
       [&] { static_cast<FuncHandle *>(f)->func->recompute(to_variables(inputs, ni), to_variables(outputs, no)); });

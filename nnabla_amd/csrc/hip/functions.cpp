@@ -30,6 +30,18 @@ void FixedPointQuantizeHip<T>::forward_impl(const Variables &inputs, const Varia
                                                   nullptr));
 }
 
+template <typename T> bool FixedPointQuantizeHip<T>::forward_after_relu(Variable *x, Variable *mid, Variable *y) {
+  hip_set_device(this->ctx_);
+  const size_t size = (size_t)x->size();
+  if (mid == y || mid->data()->array() == y->data()->array()) // (the second result would take the first one's place)
+    return false;
+  const T *xp = x->get_data_pointer<T>(this->ctx_);
+  T *mp = mid->cast_data_and_get_pointer<T>(this->ctx_, true);
+  T *yp = y->cast_data_and_get_pointer<T>(this->ctx_, true);
+  NBLA_HIP_CALL(nbla_hip_relu_fixed_point_quantize_f32(xp, mp, yp, size, this->sign_, this->n_, this->delta_, nullptr));
+  return true;
+}
+
 template <typename T> void Pow2QuantizeHip<T>::forward_impl(const Variables &inputs, const Variables &outputs) {
   hip_set_device(this->ctx_);
   const T *x = inputs[0]->get_data_pointer<T>(this->ctx_);
@@ -624,6 +636,16 @@ template <typename T> void ReLUHip<T>::forward_impl(const Variables &inputs, con
   const T *x = inputs[0]->get_data_pointer<T>(this->ctx_);
   T *y = outputs[0]->cast_data_and_get_pointer<T>(this->ctx_, true);
   NBLA_HIP_CALL(nbla_hip_relu_f32(x, y, (size_t)inputs[0]->size(), nullptr));
+}
+
+template <typename T>
+bool ReLUHip<T>::forward_with_next_impl(const Variables &inputs, const Variables &outputs, Function &next,
+                                        const Variables &next_outputs) {
+  FixedPointQuantizeHip<T> *q = dynamic_cast<FixedPointQuantizeHip<T> *>(&next);
+  const Context a = this->ctx_, b = next.context();
+  if (!q || a.device_id != b.device_id || a.array_class != b.array_class)
+    return false;
+  return q->forward_after_relu(inputs[0], outputs[0], next_outputs[0]);
 }
 
 // ------------------------------------------------------------ Add2 and Concatenate

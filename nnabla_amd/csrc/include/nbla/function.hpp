@@ -32,6 +32,10 @@ public:
   void setup(const Variables &inputs, const Variables &outputs);
   // Re-runs setup when input shapes changed, then computes the outputs.
   void forward(const Variables &inputs, const Variables &outputs);
+  // Runs this function and `next`, whose only input is this one's only output, in one go where the pair has such a form;
+  // false (and nothing done) otherwise, or where either would have to be set up again first.
+  bool forward_with_next(const Variables &inputs, const Variables &outputs, Function &next, const Variables &next_inputs,
+                         const Variables &next_outputs);
   void backward(const Variables &inputs, const Variables &outputs, const vector<bool> &propagate_down,
                 const vector<bool> &accum);
   void setup_recompute(const Variables &inputs, const Variables &outputs);
@@ -66,6 +70,10 @@ public:
 protected:
   virtual void setup_impl(const Variables &inputs, const Variables &outputs) = 0;
   virtual void forward_impl(const Variables &inputs, const Variables &outputs) = 0;
+  virtual bool forward_with_next_impl(const Variables &inputs, const Variables &outputs, Function &next,
+                                      const Variables &next_outputs) {
+    return false;
+  }
   virtual void backward_impl(const Variables &inputs, const Variables &outputs, const vector<bool> &propagate_down,
                              const vector<bool> &accum) = 0;
   virtual void setup_recompute_impl(const Variables &inputs, const Variables &outputs) {}

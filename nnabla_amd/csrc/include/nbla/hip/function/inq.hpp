@@ -95,6 +95,8 @@ public:
 
 protected:
   virtual void forward_impl(const Variables &inputs, const Variables &outputs);
+  virtual bool forward_with_next_impl(const Variables &inputs, const Variables &outputs, Function &next,
+                                      const Variables &next_outputs);
   virtual void backward_impl(const Variables &inputs, const Variables &outputs, const vector<bool> &propagate_down,
                              const vector<bool> &accum);
 };

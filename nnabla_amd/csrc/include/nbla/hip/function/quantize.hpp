@@ -16,6 +16,8 @@ public:
   FixedPointQuantizeHip(const Context &ctx, bool sign, int n, float delta, bool ste_fine_grained)
       : FixedPointQuantize<T>(ctx, sign, n, delta, ste_fine_grained) {}
   virtual vector<string> allowed_array_classes() { return SingletonManager::get<Hip>()->array_classes(); }
+  // ReLU of x into `mid`, then this function of it into y, in one launch; false where the arrays' places do not allow it.
+  bool forward_after_relu(Variable *x, Variable *mid, Variable *y);
 
 protected:
   virtual void forward_impl(const Variables &inputs, const Variables &outputs);

@@ -76,6 +76,14 @@ void Function::forward(const Variables &inputs, const Variables &outputs) {
   this->forward_impl(inputs, outputs);
 }
 
+bool Function::forward_with_next(const Variables &inputs, const Variables &outputs, Function &next,
+                                 const Variables &next_inputs, const Variables &next_outputs) {
+  if (!called_setup_ || !next.called_setup_ || !shapes_match(in_shapes, inputs) || !shapes_match(out_shapes, outputs) ||
+      !shapes_match(next.in_shapes, next_inputs) || !shapes_match(next.out_shapes, next_outputs))
+    return false;
+  return this->forward_with_next_impl(inputs, outputs, next, next_outputs);
+}
+
 void Function::backward(const Variables &inputs, const Variables &outputs, const vector<bool> &propagate_down,
                         const vector<bool> &accum) {
   NBLA_CHECK(called_setup_, error_code::unclassified, "%s: setup() must be called before backward().",

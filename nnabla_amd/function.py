@@ -113,6 +113,22 @@ class Function(object):
         return outs[0] if len(outs) == 1 else tuple(outs)
 
 
+def forward_nodes(nodes):
+    """Runs the nodes in order, in one call of the host library: a graph of small functions is bound by what each of them
+    costs before its launch, and a function may run together with the one behind it (ReLU with FixedPointQuantize)."""
+    if not all(type(n) is FunctionNode and type(n.function) is Function for n in nodes):
+        for n in nodes:
+            n.forward()
+        return
+    count = len(nodes)
+    inputs = [v._h for n in nodes for v in n.inputs]
+    outputs = [v._h for n in nodes for v in n.outputs]
+    ints, handles = ctypes.c_int * count, ctypes.c_void_p
+    _capi.check(_capi.lib().nblac_functions_forward(
+        count, (handles * count)(*[n.function._h for n in nodes]), ints(*[len(n.inputs) for n in nodes]),
+        (handles * len(inputs))(*inputs), ints(*[len(n.outputs) for n in nodes]), (handles * len(outputs))(*outputs)))
+
+
 class FunctionNode(object):
     """A function bound to its input and output variables (CgFunction)."""
 

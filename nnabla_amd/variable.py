@@ -232,8 +232,8 @@ class Variable(object):
 
     def forward(self, clear_buffer=False, clear_no_need_grad=False):
         """Runs every function this variable depends on, in dependency order (CgVariable::forward)."""
-        for node in self._function_order():
-            node.forward()
+        from .function import forward_nodes
+        forward_nodes(self._function_order())
 
     def visit(self, f):
         """Calls ``f(function)`` for every function this variable depends on, in forward order
