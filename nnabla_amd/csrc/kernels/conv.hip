@@ -781,7 +781,7 @@ int binary_conv_forward(const float *x, const float *W, float *Wb, float *alpha,
   if (rc)
     return rc;
   hipStream_t stream = as_stream(stream_);
-  if (conv_direct_forward_applies(g)) { // many small groups: all of them in one launch each, over the materialised signs
+  if (conv_direct_forward_applies(g, true)) { // many small groups: all of them in one launch each, over the materialised signs
     rc = launch_conv_direct_binarize(W, Wb, alpha, g, zero_to, stream);
     if (rc)
       return rc;
@@ -893,7 +893,7 @@ int nbla_hip_binary_convolution_slab_plan(int64_t outer, int64_t C, int nd, cons
   if (rc)
     return rc;
   plan[0] = plan[1] = plan[2] = plan[3] = 0;
-  if (!conv_direct_forward_applies(g))
+  if (!conv_direct_forward_applies(g, true))
     conv_slab_plan_summary(g, plan);
   return NBLA_HIP_OK;
 }

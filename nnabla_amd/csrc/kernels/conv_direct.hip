@@ -718,7 +718,7 @@ static int direct_tile_width(const ConvGeom &g) {
 // The forward alone also for a single group of very few input channels under a kernel of many taps (the first layer
 // of an image network: 3 channels, 7 x 7): rows of the unfolded matrix that are mostly padding of the k tiles, which
 // the products on the matrix cores gather element by element.
-bool conv_direct_forward_applies(const ConvGeom &g) {
+bool conv_direct_forward_applies(const ConvGeom &g, bool binary) {
   if (conv_direct_applies(g))
     return true;
   if (g.group == 1 && g.Cg <= 4 && g.k_size >= 9 && g.O % 8 == 0 && g.O * g.Kg <= 0x7fffffffll &&
@@ -726,8 +726,15 @@ bool conv_direct_forward_applies(const ConvGeom &g) {
     return true;
   // ... and for at most 64 output channels over fewer than 24 input channels: the matrix-core products work on tiles
   // 256 channels wide and gather such inputs element by element, the tiled fp32 kernel is the faster one
-  // ([4,16,16,56,56] x [32,16,3,3,3]: 0.86 ms binary, 0.24 ms real-weight on the matrix cores)
-  return g.group == 1 && g.Cg < 24 && g.O <= 64 && direct_tile_width(g) != 0;
+  // ([4,16,16,56,56] x [32,16,3,3,3]: 0.86 ms binary, 0.24 ms real-weight on the matrix cores) -- unless the convolution
+  // over input positions in LDS (binary) or the bf16 one (real weights) covers the geometry, which read an input once for
+  // all taps: [8,18,14,14] x [16,18,3,3] 43 us here, 12.6 and (with the weights' quantization) 45 against 20 there,
+  // [32,16,56,56] x [64,16,3,3] 77 / 80 against 36 / 56, [16,16,28,28] x [32,16,5,5] 98 / 100 against 20 / 22, and a third of
+  // the distance from float64.  With a few taps there is little to save: [16,18,56,56] x [16,18,1,1] 15 / 17 against 17 / 30.
+  if (!(g.group == 1 && g.Cg < 24 && g.O <= 64 && direct_tile_width(g) != 0))
+    return false;
+  // Fewer than a thousand windows of a binary layer stay (its plan query promises so, [1,16,27,27] x [64,16,3,3] among them).
+  return g.k_size < 4 || !(binary ? g.M >= 1024 && conv_slab_applies(g) : conv_real_applies(g, false, false));
 }
 
 namespace {

@@ -877,7 +877,7 @@ int nbla_hip_inq_convolution_f32(const float *x, float *W, int32_t *I, float *ol
     if (rc)
       return rc;
   }
-  if (conv_direct_forward_applies(g)) // many small groups: all of them in one fp32 launch
+  if (conv_direct_forward_applies(g, false)) // many small groups: all of them in one fp32 launch
     return launch_conv_direct_forward(x, W, nullptr, bias, y, g, stream);
   if (conv_real_applies(g, false, false)) { // two dimensions, no dilation: no unfolded matrix
     for (int64_t grp = 0; grp < g.group; ++grp) {

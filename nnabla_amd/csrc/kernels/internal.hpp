@@ -63,7 +63,7 @@ int launch_affine_few_rows(const float *x, const float *W, const float *bias, fl
 // scale (may be null): alpha[o].  launch_conv_direct_binarize writes Wb = Sign(W) and alpha (may be null) for all
 // channels.  Backward: w as in the forward, or with take_sign the real-valued weights whose signs were used.
 bool conv_direct_applies(const ConvGeom &g);
-bool conv_direct_forward_applies(const ConvGeom &g); // (also a single group of very few input channels, many taps)
+bool conv_direct_forward_applies(const ConvGeom &g, bool binary); // (also a single group of very few input channels, many taps)
 // The weight gradient of few weights under many windows in fp32 (all groups); scratch: M * Kg floats are enough.
 bool conv_direct_dw_applies(const ConvGeom &g);
 // Whether it then keeps the sums of every (channel pair, tap) in threads, in this much scratch memory: short chains of
