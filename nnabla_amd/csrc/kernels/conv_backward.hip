@@ -287,8 +287,8 @@ int conv_backward(const float *dy, const float *x, const float *W, const float *
     dW = nullptr;
   }
   // the bias gradient straight from dy, every group at once (partial sums in the same buffer, after the weight
-  // gradient's in the stream)
-  if (db) {
+  // gradient's in the stream), where the weight gradient's product does not take it along
+  if (db && !(dW && p.product_dw)) {
     rc = launch_conv_direct_db(dy, db, g, accum_b, col, col_bytes, stream);
     if (rc)
       return rc;
@@ -296,7 +296,7 @@ int conv_backward(const float *dy, const float *x, const float *W, const float *
   }
   if (dW && p.product_dw) { // kernels of width 1, 3, 5 with half their width of padding: no unfolded matrix
     for (int64_t grp = 0; grp < g.group; ++grp) {
-      rc = launch_conv_dw(dy, x, dW, g, grp, accum_w, base, conv_dw_workspace_bytes(g), stream);
+      rc = launch_conv_dw(dy, x, dW, g, grp, accum_w, base, conv_dw_workspace_bytes(g), stream, db, accum_b);
       if (rc)
         return rc;
     }

@@ -102,7 +102,7 @@ struct DwPlan {
   int dy_off, tab_off, misc_off, lds;
   int slices;
   DwDivide by_xc, by_rows_x, by_q, by_g, by_r;
-  size_t max_off, shift_off, partial_off, total;
+  size_t max_off, shift_off, partial_off, sum_off, total;
 };
 
 struct DwArgs {
@@ -115,11 +115,14 @@ struct DwArgs {
   DwPlan p;
 };
 
-// Largest finite magnitude of every channel of x and dy over slices of the samples: block (slice, channel).
+// Largest finite magnitude of every channel of x and dy over slices of the samples: block (slice, channel).  kSum:
+// the sums of dy's channels too, for the bias gradient, which had read dy in a pass of its own (two launches, 8 to 12 us).
+template <bool kSum>
 __global__ __launch_bounds__(256) void conv_dw_maxima(const float *__restrict__ x, const float *__restrict__ dy,
-                                                      uint32_t *__restrict__ maxima, int N, int C, int O, int Cg, int Og,
-                                                      int xplane, int yplane) {
+                                                      uint32_t *__restrict__ maxima, float *__restrict__ sums, int N, int C,
+                                                      int O, int Cg, int Og, int xplane, int yplane) {
   __shared__ uint32_t s_max[4];
+  __shared__ float s_sum[4];
   const int ch = blockIdx.y, slice = blockIdx.x, tid = threadIdx.x;
   const bool is_x = ch < Cg;
   const int plane = is_x ? xplane : yplane;
@@ -127,9 +130,13 @@ __global__ __launch_bounds__(256) void conv_dw_maxima(const float *__restrict__ 
   const int64_t sample = is_x ? (int64_t)C * xplane : (int64_t)O * yplane;
   const int per = (N + (int)gridDim.x - 1) / (int)gridDim.x, n0 = slice * per, n1 = min(N, n0 + per);
   uint32_t amax = 0u;
-  auto take = [&](float v) __attribute__((always_inline)) {
+  float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  // (loads past the end repeat the last value)
+  auto take = [&](float v, int j, bool in) __attribute__((always_inline)) {
     const uint32_t m = __float_as_uint(v) & 0x7fffffffu;
     amax = max(amax, m < 0x7f800000u ? m : 0u);
+    if (kSum)
+      sum[j] += in ? v : 0.0f;
   };
   if (plane >= 256) {
     for (int n = n0; n < n1; ++n) {
@@ -141,7 +148,7 @@ __global__ __launch_bounds__(256) void conv_dw_maxima(const float *__restrict__ 
           v[j] = p[min(i + 256 * j, plane - 1)];
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          take(v[j]);
+          take(v[j], j, i + 256 * j < plane);
       }
     }
   } else { // several samples' planes side by side
@@ -155,18 +162,34 @@ __global__ __launch_bounds__(256) void conv_dw_maxima(const float *__restrict__ 
       }
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        take(v[j]);
+        take(v[j], j, i + 256 * j < total);
     }
   }
+  float all = (sum[0] + sum[1]) + (sum[2] + sum[3]);
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1)
     amax = max(amax, (uint32_t)__shfl_xor((int)amax, off));
+  if (kSum) {
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1)
+      all += __shfl_xor(all, off);
+  }
   if ((tid & 63) == 0)
-    s_max[tid >> 6] = amax;
+    s_max[tid >> 6] = amax, s_sum[tid >> 6] = all;
   __syncthreads();
-  if (tid == 0)
+  if (tid == 0) {
     maxima[slice * (Cg + Og) + ch] = max(max(s_max[0], s_max[1]), max(s_max[2], s_max[3]));
+    if (kSum && !is_x)
+      sums[slice * Og + (ch - Cg)] = (s_sum[0] + s_sum[1]) + (s_sum[2] + s_sum[3]);
+  }
 }
+
+// The bias gradient from the slices' sums of dy: further blocks of conv_dw_sum.
+struct DwBias {
+  const float *sums;
+  float *db; // null: not wanted
+  int slices, accumulate, first_block;
+};
 
 #if defined(__HIP_DEVICE_COMPILE__)
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t dw_rsrc(const float *p, uint32_t bytes) {
@@ -440,8 +463,18 @@ template <int kRuns>
 __global__ __launch_bounds__(256) void conv_dw_sum(const float *__restrict__ partial, const int32_t *__restrict__ shifts,
                                                    float *__restrict__ dW, int Og, int Cg, int taps, int splits,
                                                    int accumulate, const float *__restrict__ x,
-                                                   const float *__restrict__ dy, ConvGeom g, int64_t grp) {
+                                                   const float *__restrict__ dy, ConvGeom g, int64_t grp, DwBias bias) {
   constexpr int kOuts = 256 / kRuns;
+  if (bias.db && (int)blockIdx.x >= bias.first_block) {
+    const int o = ((int)blockIdx.x - bias.first_block) * 256 + threadIdx.x;
+    if (o < Og) {
+      double total = 0.0;
+      for (int s = 0; s < bias.slices; ++s)
+        total += (double)bias.sums[s * Og + o];
+      bias.db[o] = bias.accumulate ? bias.db[o] + (float)total : (float)total;
+    }
+    return;
+  }
   __shared__ double s_sum[kRuns][kOuts];
   const int col = threadIdx.x % kOuts, run = threadIdx.x / kOuts;
   const int64_t outs = (int64_t)taps * Og * Cg, at = (int64_t)blockIdx.x * kOuts + col;
@@ -591,7 +624,8 @@ bool make_dw_plan(const ConvGeom &g, DwPlan &p) {
   p.max_off = 0;
   p.shift_off = round_up((size_t)p.slices * channels * sizeof(uint32_t), 256);
   p.partial_off = p.shift_off + round_up((size_t)channels * sizeof(int32_t), 256);
-  p.total = p.partial_off + round_up((size_t)p.splits * g.Og * g.Kg * sizeof(float), 256);
+  p.sum_off = p.partial_off + round_up((size_t)p.splits * g.Og * g.Kg * sizeof(float), 256);
+  p.total = p.sum_off + round_up((size_t)p.slices * g.Og * sizeof(float), 256);
   return true;
 }
 
@@ -637,7 +671,7 @@ size_t conv_dw_workspace_bytes(const ConvGeom &g) {
 }
 
 int launch_conv_dw(const float *dy, const float *x, float *dW, const ConvGeom &g, int64_t grp, bool accumulate,
-                   void *workspace, size_t workspace_bytes, hipStream_t stream) {
+                   void *workspace, size_t workspace_bytes, hipStream_t stream, float *db, bool accumulate_db) {
   DwArgs a;
   if (!make_dw_plan(g, a.p))
     return fail(NBLA_HIP_ERR_NOT_IMPLEMENTED, "the weight gradient product does not cover this geometry.");
@@ -646,6 +680,7 @@ int launch_conv_dw(const float *dy, const float *x, float *dW, const ConvGeom &g
                 a.p.total);
   char *base = static_cast<char *>(workspace);
   uint32_t *maxima = reinterpret_cast<uint32_t *>(base + a.p.max_off);
+  float *sums = reinterpret_cast<float *>(base + a.p.sum_off);
   const int64_t x_first = grp * g.Cg * g.in_sp_size, dy_first = grp * g.Og * g.out_sp_size;
   a.x = x + x_first, a.dy = dy + dy_first;
   a.maxima = maxima;
@@ -657,8 +692,13 @@ int launch_conv_dw(const float *dy, const float *x, float *dW, const ConvGeom &g
   a.x_bytes = (uint32_t)((g.outer * g.C * g.in_sp_size - x_first) * 4);
   a.partial_bytes = (uint32_t)(a.p.splits * g.Og * g.Kg * 4);
   a.dy_bytes = (uint32_t)((g.outer * g.O * g.out_sp_size - dy_first) * 4);
-  hipLaunchKernelGGL(conv_dw_maxima, dim3((unsigned)a.p.slices, (unsigned)(g.Cg + g.Og)), dim3(256), 0, stream, a.x,
-                     a.dy, maxima, a.N, a.C, a.O, a.Cg, a.Og, (int)g.in_sp_size, (int)g.out_sp_size);
+  const dim3 max_grid((unsigned)a.p.slices, (unsigned)(g.Cg + g.Og));
+  if (db)
+    hipLaunchKernelGGL(conv_dw_maxima<true>, max_grid, dim3(256), 0, stream, a.x, a.dy, maxima, sums, a.N, a.C, a.O, a.Cg,
+                       a.Og, (int)g.in_sp_size, (int)g.out_sp_size);
+  else
+    hipLaunchKernelGGL(conv_dw_maxima<false>, max_grid, dim3(256), 0, stream, a.x, a.dy, maxima, sums, a.N, a.C, a.O, a.Cg,
+                       a.Og, (int)g.in_sp_size, (int)g.out_sp_size);
   NBLA_HIP_LAUNCH_CHECK("conv_dw_maxima");
   int rc;
   switch (a.p.KW * 4 + a.p.S) {
@@ -672,10 +712,15 @@ int launch_conv_dw(const float *dy, const float *x, float *dW, const ConvGeom &g
   if (rc)
     return rc;
   const int64_t outs = g.Og * g.Kg;
+  DwBias bias{sums, db ? db + grp * g.Og : nullptr, a.p.slices, accumulate_db ? 1 : 0, 0};
+  const int64_t bias_blocks = db ? ceil_div(g.Og, 256) : 0;
 #define NBLA_DW_SUM(RUNS)                                                                                              \
-  hipLaunchKernelGGL(conv_dw_sum<RUNS>, dim3((unsigned)ceil_div(outs * RUNS, 256)), dim3(256), 0, stream, a.partial,   \
-                     a.shifts, dW + grp * g.Og * g.Kg, a.Og, a.Cg, (int)g.k_size, a.p.splits, accumulate ? 1 : 0, x,   \
-                     dy, g, grp)
+  do {                                                                                                                 \
+    bias.first_block = (int)ceil_div(outs * RUNS, 256);                                                                \
+    hipLaunchKernelGGL(conv_dw_sum<RUNS>, dim3((unsigned)(bias.first_block + bias_blocks)), dim3(256), 0, stream,      \
+                       a.partial, a.shifts, dW + grp * g.Og * g.Kg, a.Og, a.Cg, (int)g.k_size, a.p.splits,             \
+                       accumulate ? 1 : 0, x, dy, g, grp, bias);                                                       \
+  } while (0)
   if (outs >= 2048 * 256)
     NBLA_DW_SUM(1);
   else if (outs >= 1024 * 256)

@@ -97,8 +97,10 @@ int launch_conv_real(const float *in, const float *W, const float *bias, float *
 // x, dy and dW are the whole tensors; workspace: conv_dw_workspace_bytes(g), 256-byte aligned.
 bool conv_dw_applies(const ConvGeom &g);
 size_t conv_dw_workspace_bytes(const ConvGeom &g);
+// db (may be null): the whole bias gradient, of which the group's part is written (added to with accumulate_db).
 int launch_conv_dw(const float *dy, const float *x, float *dW, const ConvGeom &g, int64_t grp, bool accumulate,
-                   void *workspace, size_t workspace_bytes, hipStream_t stream);
+                   void *workspace, size_t workspace_bytes, hipStream_t stream, float *db = nullptr,
+                   bool accumulate_db = false);
 // The binary convolution forward with the unfold done by LDS addressing (conv_slab.hip), two launches per group:
 // launch_conv_slab_prepare reads the group's weights [Og, Cg, taps] once and writes Wb = Sign(W) (may be null) and,
 // into `prepared` (conv_slab_prepared_bytes, 16-byte aligned), the packed bits in (tap, channel) order with the
