@@ -31,7 +31,7 @@
 // converted, 46 per MFMA of 32, 4 to 8 thousand for the epilogue); slab_form_cost weighs them.  Measured, whole forward
 // with the weights' pass, <4, 1, 2> -> the form taken: [32,64,56,56] x [64,64,3,3] 167 -> 44 us, [64,64,28,28] x
 // [64,64,1,1] 68 -> 18.5, [32,128,28,28] x [128,128,3,3] 71 -> 30, [32,96,27,27] x [48,96,5,5] 94 -> 33;
-// [32,256,14,14] x [256,256,3,3] keeps <4, 1, 2> (28.6 us, 31 in <4, 1, 1>).
+// [32,256,14,14] x [256,256,3,3] keeps <4, 1, 2> (27.4 us, 31 in <4, 1, 1>).
 //
 // Numerics: q = rint(x * 2^s) with s chosen so that the slab's largest finite magnitude lands in [2^29, 2^30); the
 // four digit products are accumulated exactly in int32, combined exactly in integers with the windows' sums of q
@@ -66,7 +66,7 @@ constexpr int kSlabMaxTaps = 64;
 constexpr int kSlabAhead = 8;        // k tiles of packed words a wavefront holds in registers ahead of its MFMAs
 constexpr int kSlabTopBit = 29;      // the slab's largest magnitude lands in [2^29, 2^30): two q add up in 32 bits
 constexpr int kSlabLevel = 3;        // windows smaller by more binades than this take a scale of their own
-constexpr int kSlabReduceBytes = 16 * 64 * 4; // per wavefront: one fragment of one digit's accumulators
+constexpr int kSlabReduceBytes = 2 * 16 * 64 * 4; // per wavefront: one fragment's accumulators, two integers each
 constexpr int kSlabHold = 4;         // work items of the set-up a wavefront keeps in registers between its two steps
 constexpr int kSlabLdsLimit = 156 * 1024;
 constexpr int kPrepThreads = 256;
@@ -580,31 +580,42 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
   }
 
   // ---- 3. (WK == 2) the two k groups' accumulators added exactly through LDS (the planes are free once every
-  // wavefront has left the loop), one digit at a time, in two alternating areas: a wavefront hands the fragment it does
-  // not finish (1 - wk) to its partner in the other k group and adds the partner's copy of fragment wk to its own.
-  i32x16_t fin[kSlabDigits];
+  // wavefront has left the loop): a wavefront hands the fragment it does not finish (1 - wk) to its partner in the other
+  // k group and adds the partner's copy of fragment wk to its own.  Two digits make one integer before they are handed
+  // over (hi = m_0 * 256 + m_1, lo = m_2 * 256 + m_3 as below, |m_d| <= 2^21: sums of both groups stay in 32 bits), so two
+  // registers of four cross the LDS, under one barrier instead of one per digit.  Digit by digit this took 4.4 of a block's
+  // 22.6 us and 27 registers were spilled; whole forward of [32,256,14,14] x [256,256,3,3] 29.35 -> 27.4 us.
+  i32x16_t fin[2]; // hi, lo of the fragment this wavefront finishes
   if constexpr (WK == 2) {
+    auto combine = [&](int j, i32x16_t (&out)[2]) __attribute__((always_inline)) {
+      const int F = frag0 + 2 * wn + j;
+#pragma unroll
+      for (int q = 0; q < 16; ++q) {
+        out[0][q] = ((acc[0][j][q] >> F) << 8) + (acc[1][j][q] >> F);
+        out[1][q] = ((acc[2][j][q] >> F) << 8) + (acc[3][j][q] >> F);
+      }
+    };
     uint4_t *red = reinterpret_cast<uint4_t *>(smem);
-    const int mine = wave * 4 * 64 + lane, theirs = (wave ^ (WN * WM)) * 4 * 64 + lane;
+    const int mine = wave * 8 * 64 + lane, theirs = (wave ^ (WN * WM)) * 8 * 64 + lane;
+    i32x16_t give[2];
+    if (wk) // uniform
+      combine(0, give), combine(1, fin);
+    else
+      combine(1, give), combine(0, fin);
     __syncthreads();
 #pragma unroll
-    for (int d = 0; d < kSlabDigits; ++d) {
-      uint4_t *area = red + (d & 1) * (kWaves * kSlabReduceBytes / 16);
-      const i32x16_t give = wk ? acc[d][0] : acc[d][1];
+    for (int q = 0; q < 8; ++q) {
+      uint4_t v;
+      v.x = give[q >> 2][4 * (q & 3) + 0], v.y = give[q >> 2][4 * (q & 3) + 1];
+      v.z = give[q >> 2][4 * (q & 3) + 2], v.w = give[q >> 2][4 * (q & 3) + 3];
+      red[mine + q * 64] = v;
+    }
+    __syncthreads();
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        uint4_t v;
-        v.x = give[4 * q + 0], v.y = give[4 * q + 1], v.z = give[4 * q + 2], v.w = give[4 * q + 3];
-        area[mine + q * 64] = v;
-      }
-      __syncthreads();
-      fin[d] = wk ? acc[d][1] : acc[d][0];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const uint4_t v = area[theirs + q * 64];
-        fin[d][4 * q + 0] += (int)v.x, fin[d][4 * q + 1] += (int)v.y;
-        fin[d][4 * q + 2] += (int)v.z, fin[d][4 * q + 3] += (int)v.w;
-      }
+    for (int q = 0; q < 8; ++q) {
+      const uint4_t v = red[theirs + q * 64];
+      fin[q >> 2][4 * (q & 3) + 0] += (int)v.x, fin[q >> 2][4 * (q & 3) + 1] += (int)v.y;
+      fin[q >> 2][4 * (q & 3) + 2] += (int)v.z, fin[q >> 2][4 * (q & 3) + 3] += (int)v.w;
     }
   }
 
@@ -620,11 +631,6 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
 #pragma unroll
   for (int jj = 0; jj < 3 - WK; ++jj) { // the fragments this wavefront finishes: both, or the one of its k group
   const int jf = WK == 2 ? wk : jj, fb = 2 * wn + jf;
-  if constexpr (WK == 1) {
-#pragma unroll
-    for (int d = 0; d < kSlabDigits; ++d)
-      fin[d] = acc[d][jj];
-  }
   const int F = frag0 + fb; // the fragment's place in its wide group: the scale of its accumulators
   const bool negate = F == 7;
   // channel of register q: c0 + 8 (q / 4) + q % 4; everything an output needs besides its accumulators is fetched
@@ -651,7 +657,11 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
 #pragma unroll
   for (int q = 0; q < 16; ++q) {
     const int cq = 8 * (q >> 2) + (q & 3);
-    const int hi = ((fin[0][q] >> F) << 8) + (fin[1][q] >> F), lo = ((fin[2][q] >> F) << 8) + (fin[3][q] >> F);
+    int hi, lo;
+    if constexpr (WK == 2)
+      hi = fin[0][q], lo = fin[1][q];
+    else
+      hi = ((acc[0][jj][q] >> F) << 8) + (acc[1][jj][q] >> F), lo = ((acc[2][jj][q] >> F) << 8) + (acc[3][jj][q] >> F);
     int A = negate ? s_hi + 2 * hi : s_hi - 2 * hi, B = negate ? s_lo + 2 * lo : s_lo - 2 * lo;
     A += B >> 16, B &= 0xffff; // the sum is A * 2^16 + B, 0 <= B < 2^16
     float v = ldexpf(fmaf((float)A, bad_scale, (float)B), -shift);
@@ -703,6 +713,7 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
     asm volatile("" : "+v"(tid), "+v"(row));
     tid &= kThreads - 1, row &= kRows - 1, lane = tid & 63, half = lane >> 5; // (the compiler knows their ranges again)
     limit = left;
+    __syncthreads(); // every wavefront has read its partner's sums
     shift = kSlabTopBit - binade_exponent(binade_of(left));
     for (int i = tid; i <= P.cap; i += kThreads)
       s_pixsum[i] = 0;
@@ -978,8 +989,8 @@ bool compute_slab_form(const ConvGeom &g, int form, int chunks, SlabRuns &runs, 
   p.slab_bytes = (int)slab_bytes;
   p.k_tiles = (int)(g.k_size * p.ct);
   int64_t off = slab_bytes;
-  if (f.wk == 2 && off < 2 * waves * kSlabReduceBytes) // two areas for the exchange between the k groups
-    off = 2 * waves * kSlabReduceBytes;
+  if (f.wk == 2 && off < waves * kSlabReduceBytes) // the exchange between the k groups
+    off = waves * kSlabReduceBytes;
   off = (int64_t)round_up((size_t)off, 16);
   p.pixsum_off = (int)off, off += 8 * (cap + 1);
   off = (int64_t)round_up((size_t)off, 16);
