@@ -31,7 +31,7 @@
 // converted, 46 per MFMA of 32, 4 to 8 thousand for the epilogue); slab_form_cost weighs them.  Measured, whole forward
 // with the weights' pass, <4, 1, 2> -> the form taken: [32,64,56,56] x [64,64,3,3] 167 -> 44 us, [64,64,28,28] x
 // [64,64,1,1] 68 -> 18.5, [32,128,28,28] x [128,128,3,3] 71 -> 30, [32,96,27,27] x [48,96,5,5] 94 -> 33;
-// [32,256,14,14] x [256,256,3,3] keeps <4, 1, 2> (27.4 us, 31 in <4, 1, 1>).
+// [32,256,14,14] x [256,256,3,3] keeps <4, 1, 2> (26.3 us).
 //
 // Numerics: q = rint(x * 2^s) with s chosen so that the slab's largest finite magnitude lands in [2^29, 2^30); the
 // four digit products are accumulated exactly in int32, combined exactly in integers with the windows' sums of q
@@ -137,11 +137,11 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // Blocks go to the eight XCDs round-robin: an XCD takes a contiguous run of tiles, so the tiles of one sample --
   // whose slabs overlap and whose outputs share cache lines -- meet in one L2.
-  const int64_t work = xcd_remap(blockIdx.x, gridDim.x);
-  const int cg = (int)(work % P.col_groups);
+  const uint32_t work = (uint32_t)xcd_remap(blockIdx.x, gridDim.x); // (below 2^31: checked by the host)
+  const int cg = (int)(work % (uint32_t)P.col_groups);
   const int wg = cg * kCols / kWideGroup, frag0 = (cg * kCols % kWideGroup) / 32; // first fragment in its wide group
-  const int tile_all = (int)(work / P.col_groups);
-  const int n = tile_all / P.tiles_per_sample, tile = tile_all - n * P.tiles_per_sample;
+  const int tile_all = (int)(work / (uint32_t)P.col_groups);
+  const int n = (int)((uint32_t)tile_all / (uint32_t)P.tiles_per_sample), tile = tile_all - n * P.tiles_per_sample;
   const int p0 = tile * P.tile_rows;
   const int rows = min(P.tile_rows, (int)g.out_sp_size - p0);
   const int taps = (int)g.k_size, plane = (int)g.in_sp_size, Cg = (int)g.Cg, CT = P.ct;
@@ -153,35 +153,54 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
   float *s_alpha = reinterpret_cast<float *>(smem + P.alpha_off), *s_bias = s_alpha + kCols;
   int *s_misc = reinterpret_cast<int *>(smem + P.misc_off); // the wavefronts' maxima, of the slab and of windows left
 
-  // ---- 0. the block's rows and the slab's extent.  Every wavefront walks all the rows (64 lanes at a time), so each
-  // finds the extent by itself and can start loading the slab before anything goes through LDS.
+  // ---- 0. the block's rows and the slab's extent, which every wavefront finds by itself: it can start loading the slab
+  // before anything goes through LDS.
   int half = lane >> 5;
   int row = (wave / WN) % WM * kSlabRows + (lane & 31); // the window of this lane in the product
   const bool row_in = row < rows;
+  // The block's first position is taken apart once, with whole divisions; a row adds at most 127 to it, so its own
+  // quotients are at most 129 larger and one product by the reciprocal is off by one at most.  (Divisions for every row
+  // and tap, 64-bit addresses for every load and every output, and the extent found by all lanes made a block's set-up and
+  // stores 1.5 to 2 us longer: [32,64,56,56] x [64,64,3,3] 17.8 -> 16.1 us per block, [32,256,14,14] x [256,256,3,3]
+  // 27.4 -> 26.3 us for the whole forward.)
+  const uint32_t line0 = (uint32_t)p0 / (uint32_t)g.out_sp[2], map0 = line0 / (uint32_t)g.out_sp[1];
+  const int first2 = p0 - (int)line0 * g.out_sp[2], first1 = (int)(line0 - map0 * (uint32_t)g.out_sp[1]);
+  auto carry = [](int v, int d, int &rest) __attribute__((always_inline)) { // v / d for v < d + 2^8, and v % d
+    int q = (int)((float)v * __builtin_amdgcn_rcpf((float)d));
+    rest = v - q * d;
+    if (rest < 0)
+      --q, rest += d;
+    else if (rest >= d)
+      ++q, rest -= d;
+    return q;
+  };
   auto decode = [&](int m, int &b0, int &b1, int &b2) __attribute__((always_inline)) {
-    int p = m < rows ? p0 + m : p0; // rows past the tile repeat its first row
-    const int o2 = p % g.out_sp[2];
-    p /= g.out_sp[2];
-    const int o1 = p % g.out_sp[1];
-    const int o0 = p / g.out_sp[1];
+    int o2, o1; // rows past the tile repeat its first row
+    const int line = first1 + carry(first2 + (m < rows ? m : 0), g.out_sp[2], o2);
+    const int o0 = (int)map0 + carry(line, g.out_sp[1], o1);
     b0 = o0 * g.stride[0] - g.pad[0], b1 = o1 * g.stride[1] - g.pad[1], b2 = o2 * g.stride[2] - g.pad[2];
     return (b0 * in1 + b1) * in2 + b2;
   };
   int lo, npix;
   {
-    int omin = 0x7fffffff, omax = -0x7fffffff;
-#pragma unroll
-    for (int m0 = 0; m0 < kRows; m0 += 64) {
-      int b0, b1, b2;
-      const int origin = decode(m0 + lane, b0, b1, b2);
-      omin = min(omin, origin), omax = max(omax, origin);
+    // Origins grow along a line, from line to line of a map at the same place in the line, and from map to map.  So the
+    // smallest is that of the first row, of the line after it or of the map after it, as far as the tile has them, and the
+    // largest that of the last row, or of the end of the line or of the map before it: scalars, no exchange of lanes.
+    auto origin_at = [&](int o0, int o1, int o2) __attribute__((always_inline)) {
+      return ((o0 * g.stride[0] - g.pad[0]) * in1 + o1 * g.stride[1] - g.pad[1]) * in2 + o2 * g.stride[2] - g.pad[2];
+    };
+    const int w = g.out_sp[2], h = g.out_sp[1], last = p0 + rows - 1;
+    const int line1 = (int)((uint32_t)last / (uint32_t)w), map1 = (int)((uint32_t)line1 / (uint32_t)h);
+    int omin = origin_at((int)map0, first1, first2), omax = origin_at(map1, line1 - map1 * h, last - line1 * w);
+    if (line1 > (int)line0) {
+      const int after = first1 + 1 < h ? first1 + 1 : 0, before = line1 - map1 * h;
+      omin = min(omin, origin_at((int)map0 + (after == 0), after, 0));
+      omax = max(omax, origin_at(before > 0 ? map1 : map1 - 1, before > 0 ? before - 1 : h - 1, w - 1));
     }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-      omin = min(omin, __shfl_xor(omin, off));
-      omax = max(omax, __shfl_xor(omax, off));
+    if (map1 > (int)map0) {
+      omin = min(omin, origin_at((int)map0 + 1, 0, 0));
+      omax = max(omax, origin_at(map1 - 1, h - 1, w - 1));
     }
-    omin = __builtin_amdgcn_readfirstlane(omin), omax = __builtin_amdgcn_readfirstlane(omax);
     lo = min(max(omin, 0), plane - 1);
     const int hi = min(max(omax + (int)slab_last_tap(g), 0), plane - 1);
     npix = min(hi - lo + 1, P.cap); // (the host sized the LDS for the exact maximum: the clamp never acts)
@@ -195,26 +214,34 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
   // staying in their registers; the scale is that of all channels, found before the first chunk is converted.
   const int pixel_runs = (npix + 63) >> 6;
   int groups16 = 2 * CT, ch_first = 0, items = pixel_runs * groups16; // the items that are walked: all channels, or a chunk
-  // item -> (first pixel, first channel)
+  float per_group = __builtin_amdgcn_rcpf((float)groups16);
+  // item -> (first pixel, first channel); fewer than 2^15 items: the quotient of the number plus one half keeps clear of
+  // whole numbers by more than the roundings
   auto item_of = [&](int item, int &pix0, int &ch0) __attribute__((always_inline)) {
-    const int pc = item / groups16;
+    const int pc = __builtin_amdgcn_readfirstlane((int)(((float)item + 0.5f) * per_group));
     pix0 = pc * 64, ch0 = ch_first + (item - pc * groups16) * 16;
   };
   auto take_chunk = [&](int chunk) __attribute__((always_inline)) {
     ch_first = chunk * P.ct_chunk * 32;
     groups16 = 2 * min(P.ct_chunk, CT - chunk * P.ct_chunk);
+    per_group = __builtin_amdgcn_rcpf((float)groups16);
     items = pixel_runs * groups16;
   };
   // Nothing but loads: a select or a branch on their results here would make a wavefront wait for one item's loads
-  // before it issues the next item's.  Channels past the last repeat it, pixels past the slab the first.
+  // before it issues the next item's.  Channels past the last repeat it, pixels past the slab the first.  The channel's
+  // address is a scalar that steps from load to load (a plane is below 2^32 bytes), the pixel's a 32-bit offset.
   auto load_item = [&](int item, float (&v)[16]) __attribute__((always_inline)) {
     int pix0, ch0;
     item_of(item, pix0, ch0);
     const int pix = pix0 + lane;
-    const float *src = xs + (pix < npix ? pix : 0);
+    const uint32_t off = (uint32_t)(pix < npix ? pix : 0) * 4u;
+    const char *src = reinterpret_cast<const char *>(xs + (int64_t)min(ch0, Cg - 1) * plane);
+    const int more = Cg - 1 - ch0; // channels after the item's first
 #pragma unroll
-    for (int c = 0; c < 16; ++c)
-      v[c] = src[(int64_t)min(ch0 + c, Cg - 1) * plane];
+    for (int c = 0; c < 16; ++c) {
+      v[c] = *reinterpret_cast<const float *>(src + off);
+      src += c < more ? (uint32_t)plane * 4u : 0u;
+    }
   };
   uint32_t amax = 0u;
   auto scan_item = [&](int item, float (&v)[16]) __attribute__((always_inline)) {
@@ -317,10 +344,8 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
   int b0, b1, b2;
   const int origin = decode(trow, b0, b1, b2);
   for (int t = tid / kRows; t < taps; t += kThreads / kRows) { // tap t of row trow: its pixel in the slab, if any
-    int q = t;
-    const int k2 = q % g.k[2];
-    q /= g.k[2];
-    const int k1 = q % g.k[1], k0 = q / g.k[1];
+    int k2, k1; // (fewer than kSlabMaxTaps taps)
+    const int k0 = carry(carry(t, g.k[2], k2), g.k[1], k1);
     const int e0 = k0 * g.dil[0], e1 = k1 * g.dil[1], e2 = k2 * g.dil[2];
     const int i0 = b0 + e0, i1 = b1 + e1, i2 = b2 + e2;
     const bool ok = trow < rows && (unsigned)i0 < (unsigned)in0 && (unsigned)i1 < (unsigned)in1 &&
@@ -626,13 +651,14 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
   // (s_hi -+ 2 hi) * 2^16 + (s_lo -+ 2 lo) = A * 2^16 + B with 0 <= B < 2^16: one fused multiply-add, rounded once
   // while |A| < 2^24 (sums below 2^40), else twice (2^-24 of the sum).
   if (finish) {
-  const int s_hi = (int)(rowsum >> 16), s_lo = (int)(rowsum & 0xffff);
   const int osz = (int)g.out_sp_size;
 #pragma unroll
   for (int jj = 0; jj < 3 - WK; ++jj) { // the fragments this wavefront finishes: both, or the one of its k group
   const int jf = WK == 2 ? wk : jj, fb = 2 * wn + jf;
   const int F = frag0 + fb; // the fragment's place in its wide group: the scale of its accumulators
-  const bool negate = F == 7;
+  // (-x - 1 = x ^ -1: for F = 7 the two that 2 * 1 makes go into the windows' sum)
+  const int flip = F == 7 ? -1 : 0;
+  const int s_hi = (int)(rowsum >> 16) + 2 * flip, s_lo = (int)(rowsum & 0xffff) + 2 * flip;
   // channel of register q: c0 + 8 (q / 4) + q % 4; everything an output needs besides its accumulators is fetched
   // before the stores (the compiler does not move a load across them)
   const int c0 = fb * 32 + 4 * half, og_left = (int)g.Og - cg * kCols - c0; // channels from c0 to the group's last
@@ -645,13 +671,21 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
     bi[q] = s_bias[c0 + 8 * (q >> 2) + (q & 3)];
   }
   float *ybase = a.y + (((int64_t)n * g.O + (int64_t)a.grp * g.Og + (int64_t)cg * kCols + c0) * g.out_sp_size + p0 + row);
+  // The fragment's outputs as a buffer that ends with the group's last channel: what lies past it is not stored, and an
+  // output's address is one 32-bit addition (32 channels are below 2^30 bytes: (Og + 256) * out_sp_size < 2^31).
+  const int frag_left = min(32, (int)g.Og - cg * kCols - fb * 32);
+  const uint64_t ystart = reinterpret_cast<uint64_t>(ybase - ((int64_t)4 * half * osz + row));
+  const __amdgpu_buffer_rsrc_t yrsrc = __builtin_amdgcn_make_buffer_rsrc(
+      reinterpret_cast<void *>(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(ystart >> 32)) << 32) |
+                               (uint32_t)__builtin_amdgcn_readfirstlane((int)ystart)),
+      0, __builtin_amdgcn_readfirstlane((frag_left * osz - p0) * 4), 0x00020000);
+  const int y_off = (4 * half * osz + row) * 4;
   float prev[16];
   if (a.accumulate) {
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const int cq = 8 * (q >> 2) + (q & 3);
-      prev[q] = cq < og_left ? ybase[cq * osz] : 0.0f;
-    }
+    for (int q = 0; q < 16; ++q)
+      prev[q] = __uint_as_float(
+          __builtin_amdgcn_raw_buffer_load_b32(yrsrc, y_off + (8 * (q >> 2) + (q & 3)) * osz * 4, 0, 0));
   }
   const float bad_scale = rowbad ? __uint_as_float(0x7fc00000u) : 65536.0f; // NaN through the multiply-add
 #pragma unroll
@@ -662,15 +696,14 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
       hi = fin[0][q], lo = fin[1][q];
     else
       hi = ((acc[0][jj][q] >> F) << 8) + (acc[1][jj][q] >> F), lo = ((acc[2][jj][q] >> F) << 8) + (acc[3][jj][q] >> F);
-    int A = negate ? s_hi + 2 * hi : s_hi - 2 * hi, B = negate ? s_lo + 2 * lo : s_lo - 2 * lo;
+    int A = s_hi - 2 * (hi ^ flip), B = s_lo - 2 * (lo ^ flip);
     A += B >> 16, B &= 0xffff; // the sum is A * 2^16 + B, 0 <= B < 2^16
     float v = ldexpf(fmaf((float)A, bad_scale, (float)B), -shift);
     if (a.accumulate)
       v = prev[q] + v;
     v = v * al[q];
     v = v + bi[q];
-    if (cq < og_left)
-      ybase[cq * osz] = v; // (Og * out_sp_size < 2^31: checked by the host)
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), yrsrc, y_off + cq * osz * 4, 0, 0);
   }
   // A window holding a NaN or an infinity (rare): the reference's product propagates such values output by output
   // (convolution.cpp:185-193: the row of the unfolded input, zeros where the window leaves the input, times
