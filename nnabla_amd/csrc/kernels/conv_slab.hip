@@ -31,7 +31,7 @@
 // converted, 46 per MFMA of 32, 4 to 8 thousand for the epilogue); slab_form_cost weighs them.  Measured, whole forward
 // with the weights' pass, <4, 1, 2> -> the form taken: [32,64,56,56] x [64,64,3,3] 167 -> 44 us, [64,64,28,28] x
 // [64,64,1,1] 68 -> 18.5, [32,128,28,28] x [128,128,3,3] 71 -> 30, [32,96,27,27] x [48,96,5,5] 94 -> 33;
-// [32,256,14,14] x [256,256,3,3] keeps <4, 1, 2> (26.3 us).
+// [32,256,14,14] x [256,256,3,3] keeps <4, 1, 2> (26.1 us).
 //
 // Numerics: q = rint(x * 2^s) with s chosen so that the slab's largest finite magnitude lands in [2^29, 2^30); the
 // four digit products are accumulated exactly in int32, combined exactly in integers with the windows' sums of q
@@ -162,16 +162,16 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
   // quotients are at most 129 larger and one product by the reciprocal is off by one at most.  (Divisions for every row
   // and tap, 64-bit addresses for every load and every output, and the extent found by all lanes made a block's set-up and
   // stores 1.5 to 2 us longer: [32,64,56,56] x [64,64,3,3] 17.8 -> 16.1 us per block, [32,256,14,14] x [256,256,3,3]
-  // 27.4 -> 26.3 us for the whole forward.)
+  // 27.4 -> 26.1 us for the whole forward.)
   const uint32_t line0 = (uint32_t)p0 / (uint32_t)g.out_sp[2], map0 = line0 / (uint32_t)g.out_sp[1];
   const int first2 = p0 - (int)line0 * g.out_sp[2], first1 = (int)(line0 - map0 * (uint32_t)g.out_sp[1]);
   auto carry = [](int v, int d, int &rest) __attribute__((always_inline)) { // v / d for v < d + 2^8, and v % d
     int q = (int)((float)v * __builtin_amdgcn_rcpf((float)d));
     rest = v - q * d;
-    if (rest < 0)
-      --q, rest += d;
-    else if (rest >= d)
-      ++q, rest -= d;
+    const int under = rest >> 31; // -1: one too many
+    q += under, rest += under & d;
+    const int over = (d - 1 - rest) >> 31; // -1: one too few
+    q -= over, rest -= over & d;
     return q;
   };
   auto decode = [&](int m, int &b0, int &b1, int &b2) __attribute__((always_inline)) {
