@@ -158,26 +158,16 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
   int half = lane >> 5;
   int row = (wave / WN) % WM * kSlabRows + (lane & 31); // the window of this lane in the product
   const bool row_in = row < rows;
-  // The block's first position is taken apart once, with whole divisions; a row adds at most 127 to it, so its own
-  // quotients are at most 129 larger and one product by the reciprocal is off by one at most.  (Divisions for every row
+  // The block's first position is taken apart once, with whole divisions; a row adds at most 127 to it.  (Divisions for every row
   // and tap, 64-bit addresses for every load and every output, and the extent found by all lanes made a block's set-up and
   // stores 1.5 to 2 us longer: [32,64,56,56] x [64,64,3,3] 17.8 -> 16.1 us per block, [32,256,14,14] x [256,256,3,3]
   // 27.4 -> 26.1 us for the whole forward.)
   const uint32_t line0 = (uint32_t)p0 / (uint32_t)g.out_sp[2], map0 = line0 / (uint32_t)g.out_sp[1];
   const int first2 = p0 - (int)line0 * g.out_sp[2], first1 = (int)(line0 - map0 * (uint32_t)g.out_sp[1]);
-  auto carry = [](int v, int d, int &rest) __attribute__((always_inline)) { // v / d for v < d + 2^8, and v % d
-    int q = (int)((float)v * __builtin_amdgcn_rcpf((float)d));
-    rest = v - q * d;
-    const int under = rest >> 31; // -1: one too many
-    q += under, rest += under & d;
-    const int over = (d - 1 - rest) >> 31; // -1: one too few
-    q -= over, rest -= over & d;
-    return q;
-  };
   auto decode = [&](int m, int &b0, int &b1, int &b2) __attribute__((always_inline)) {
     int o2, o1; // rows past the tile repeat its first row
-    const int line = first1 + carry(first2 + (m < rows ? m : 0), g.out_sp[2], o2);
-    const int o0 = (int)map0 + carry(line, g.out_sp[1], o1);
+    const int line = first1 + short_divide(first2 + (m < rows ? m : 0), g.out_sp[2], o2);
+    const int o0 = (int)map0 + short_divide(line, g.out_sp[1], o1);
     b0 = o0 * g.stride[0] - g.pad[0], b1 = o1 * g.stride[1] - g.pad[1], b2 = o2 * g.stride[2] - g.pad[2];
     return (b0 * in1 + b1) * in2 + b2;
   };
@@ -345,7 +335,7 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 2) void binary_conv_slab_kernel(
   const int origin = decode(trow, b0, b1, b2);
   for (int t = tid / kRows; t < taps; t += kThreads / kRows) { // tap t of row trow: its pixel in the slab, if any
     int k2, k1; // (fewer than kSlabMaxTaps taps)
-    const int k0 = carry(carry(t, g.k[2], k2), g.k[1], k1);
+    const int k0 = short_divide(short_divide(t, g.k[2], k2), g.k[1], k1);
     const int e0 = k0 * g.dil[0], e1 = k1 * g.dil[1], e2 = k2 * g.dil[2];
     const int i0 = b0 + e0, i1 = b1 + e1, i2 = b2 + e2;
     const bool ok = trow < rows && (unsigned)i0 < (unsigned)in0 && (unsigned)i1 < (unsigned)in1 &&
