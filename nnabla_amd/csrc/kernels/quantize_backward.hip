@@ -13,6 +13,9 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kUnroll = 4;
 
+// What an operation forms once per thread before its elements.
+template <typename Op> __device__ __forceinline__ void begin(Op &) {}
+
 // dx[i] = op(dy[i], x[i], i) (+ dx[i] when kAccum).  `op` returns the gradient contribution; kUseX tells whether x is
 // read at all.
 template <typename Op, bool kAccum, bool kUseX>
@@ -31,6 +34,7 @@ __global__ __launch_bounds__(kBlock) void grad_vec4(const float *__restrict__ dy
         o[j] = load4(dx + 4 * i);
     }
   }
+  begin(op); // under the loads
 #pragma unroll
   for (int j = 0; j < kUnroll; ++j) {
     const size_t i = base + (size_t)j * kBlock;
@@ -53,6 +57,7 @@ __global__ __launch_bounds__(kBlock) void grad_vec4(const float *__restrict__ dy
 template <typename Op, bool kAccum, bool kUseX>
 __global__ __launch_bounds__(kBlock) void grad_scalar(const float *__restrict__ dy, const float *__restrict__ x,
                                                       float *__restrict__ dx, size_t size, Op op) {
+  begin(op);
   for (size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x; i < size; i += (size_t)gridDim.x * kBlock)
     dx[i] = op.template apply<kAccum>(dy[i], kUseX ? x[i] : 0.0f, kAccum ? dx[i] : 0.0f, i);
 }
@@ -132,6 +137,32 @@ struct MinMaxGradOp {
     return kAccum ? mask + old : mask;
   }
 };
+
+// The range tensors of a call; bounds(k) = (m', M') of range k as minmax_bounds forms them, for kernels whose blocks
+// need one range each.
+struct RangeInputs {
+  const float *qr_min, *ql_min, *ql_max, *scale;
+  __device__ __forceinline__ float2 bounds(int64_t k) const {
+    float m_n, M_n;
+    nudge_qr_min_max(qr_min[k], ql_min[k], ql_max[k], scale[k], m_n, M_n);
+    return float2{m_n, M_n};
+  }
+};
+
+// The mask of one range for the whole tensor, its bounds formed by every thread from the range tensors: a launch of one
+// thread ahead of this one (minmax_bounds) is 4.8 us, and all of them wait for it.  Forward and gradient of
+// [64,256,56,56]: 193.7 -> 189.1 us.
+struct MinMaxGradOneOp {
+  RangeInputs ranges;
+  float2 b; // set by begin
+  template <bool kAccum> __device__ __forceinline__ float apply(float dy, float x, float old, size_t) const {
+    const float iv0 = (x >= b.x) ? 1.0f : 0.0f, iv1 = (x <= b.y) ? 1.0f : 0.0f;
+    float mask = iv0 * iv1;
+    mask = mask * dy;
+    return kAccum ? mask + old : mask;
+  }
+};
+__device__ __forceinline__ void begin(MinMaxGradOneOp &op) { op.b = op.ranges.bounds(0); }
 
 // The same mask for any pattern of kept and reduced axes: element i belongs to the kept index formed by its
 // coordinates along the kept axes.
@@ -311,17 +342,6 @@ __device__ __forceinline__ void block_sums(float lo, float hi, float2 *dst) {
     *dst = acc;
   }
 }
-// The range tensors of a call; bounds(k) = (m', M') of range k as minmax_bounds forms them, for kernels whose blocks
-// need one range each.
-struct RangeInputs {
-  const float *qr_min, *ql_min, *ql_max, *scale;
-  __device__ __forceinline__ float2 bounds(int64_t k) const {
-    float m_n, M_n;
-    nudge_qr_min_max(qr_min[k], ql_min[k], ql_max[k], scale[k], m_n, M_n);
-    return float2{m_n, M_n};
-  }
-};
-
 // kN float4s per thread, all loads issued before the first store (the compiler does not move a load across a store)
 // kAligned: 16-byte aligned addresses; otherwise 4-byte aligned ones (the same 128-bit accesses, which may straddle
 // cache lines)
@@ -817,7 +837,8 @@ int nbla_hip_min_max_quantize_backward_f32(const float *dy, const float *x, floa
   const bool wanted = range_grads || (mode.dx_mode == 2 && P.L.K > 1);
   const bool vec = aligned16(dy) && aligned16(x) && (!dx || aligned16(dx));
   const bool one_range_per_block = wanted && !P.inner && !P.rows && ((P.flat_chunks && vec) || P.row_parts);
-  if (((dx && ste_fine_grained) || range_grads) && !one_range_per_block) {
+  const bool one_mask = dx && ste_fine_grained && P.L.ok && P.L.K == 1 && !range_grads; // (not `wanted`)
+  if (((dx && ste_fine_grained) || range_grads) && !one_range_per_block && !one_mask) {
     hipLaunchKernelGGL(minmax_bounds, dim3((unsigned)((P.L.K + 63) / 64)), dim3(64), 0, stream, qr_min, ql_min, ql_max,
                        scale, bounds, P.L.K);
     NBLA_HIP_LAUNCH_CHECK("min_max_quantize backward bounds");
@@ -899,6 +920,9 @@ int nbla_hip_min_max_quantize_backward_f32(const float *dy, const float *x, floa
       MinMaxGradStridedOp op{bounds, axes};
       rc = launch_grad<MinMaxGradStridedOp, true>(dy, x, dx, (size_t)P.L.total, accum_x, op, stream,
                                                   "min_max_quantize backward");
+    } else if (one_mask) {
+      rc = launch_grad<MinMaxGradOneOp, true>(dy, x, dx, (size_t)P.L.total, accum_x, MinMaxGradOneOp{ranges, float2{}},
+                                              stream, "min_max_quantize backward");
     } else if (ste_fine_grained) {
       MinMaxGradOp op{bounds, P.L.K, P.L.R1};
       rc = launch_grad<MinMaxGradOp, true>(dy, x, dx, (size_t)P.L.total, accum_x, op, stream, "min_max_quantize backward");
