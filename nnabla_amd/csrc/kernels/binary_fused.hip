@@ -14,7 +14,8 @@
 // digit operand and the packed bits.  No alignment is asked for: rows of W and x start at any multiple of four bytes.
 //
 // What bounds it is latency: two round trips to memory (x and the first two k tiles of W, then the other two), the
-// exchanges and the launch.  Forward in a graph, the chain -> this: 20 x 250 x 250 (rows x inputs x outputs) 42 -> 9.8 us,
+// exchanges and the launch.  Forward in a graph, the chain -> this, blocks of 64 columns (the narrow ones below, where
+// they apply, take 60 to 85 % of it): 20 x 250 x 250 (rows x inputs x outputs) 42 -> 9.8 us,
 // 800 x 816 x 632 40 -> 16, 64 x 1001 x 1003 48 -> 14.6, 512^3 29 -> 12, 1024^3 43 -> 31 (two rounds of blocks; 4096 x
 // 512 x 512, two rounds as well, 34 -> 31; at three the chain is the faster one: 1000 x 300 x 3000 33 against 36).
 //
