@@ -280,7 +280,16 @@ __global__ __launch_bounds__(kPrepBlock, kBatch > 4 ? 1 : 4) void binarize_kn_wi
   __shared__ int s_zero[kPrepBlock / 64];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); // uniform: row indices stay in scalar registers
-  const int64_t wg = blockIdx.x, slab = blockIdx.y;
+  int64_t wg = blockIdx.x, slab = blockIdx.y;
+  // Neighbouring strips of unaligned rows share a cache line in every row: in one XCD's L2 it is read once.  With x's digits
+  // from 128-bit loads, forward of rows x inputs x outputs: 300 x 4095 x 11007 114 -> 109.5 us, 128 x 8191 x 5001
+  // 112 -> 103; four strips, 2000 x 1001 x 1003, 44.2 -> 44.7.  (Aligned rows share none, and their blocks are better spread as
+  // they come: 1024 x 4096 x 4096, four layers, 350 -> 352.  Stores through the cache, for their partial lines to meet
+  // there, are slower: 109.5 -> 129.6.)
+  if (!kAligned && gridDim.x >= 8) {
+    const uint32_t block = (uint32_t)xcd_remap(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
+    slab = block / gridDim.x, wg = block % gridDim.x;
+  }
   const int64_t k_wave = (slab * (kPrepBlock / 64) + wave) * kWideWaveRows;
   const int64_t n0 = wg * kWideGroup + 4 * lane;
   float cs[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -745,8 +754,8 @@ __device__ __noinline__ void redo_marked_row(const float *__restrict__ xrow, con
 // the 16 values of fragment half g of the tiles kSlots * t + ts, t < kPer.  Row maxima and row sums cross the
 // wavefronts through LDS; every store instruction then writes runs of kRows * 16 bytes of a fragment (the other rows
 // of the row block come from neighbouring blocks).  x is read once.
-// kAligned false: rows that do not start at multiples of 16 bytes or whose length is no multiple of four -- a lane's
-// four consecutive values come as four 32-bit loads, each checked against the row's end.
+// kAligned false: rows that do not start at multiples of 16 bytes or whose length is no multiple of four -- the same
+// 128-bit loads at multiples of four bytes, and single values where a row ends inside one.
 constexpr int kFusedWaves = 8;
 template <int kRows, int kPer, bool kAligned>
 __global__ __launch_bounds__(kFusedWaves * 64) void split_digits_rows(const float *__restrict__ x, int64_t ldx,
@@ -779,15 +788,21 @@ __global__ __launch_bounds__(kFusedWaves * 64) void split_digits_rows(const floa
         v[t][i] = (m < M && k < K) ? scaled4(*reinterpret_cast<const float4_t *>(row + k), cs, k)
                                    : float4_t{0.0f, 0.0f, 0.0f, 0.0f};
       } else {
-        float e[4];
+        float4_t e = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        if (m < M && k + 4 <= K) {
+          e = *reinterpret_cast<const float4_u *>(row + k);
+        } else if (m < M) {
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const bool in = m < M && k + c < K;
-          e[c] = in ? row[k + c] : 0.0f;
-          if (cs) // one rounded product per element, as scaled4
-            e[c] = e[c] * (in ? cs[k + c] : 0.0f);
+          for (int c = 0; c < 3; ++c)
+            if (k + c < K)
+              e[c] = row[k + c];
         }
-        v[t][i] = float4_t{e[0], e[1], e[2], e[3]};
+        if (cs) { // one rounded product per element, as scaled4
+#pragma unroll
+          for (int c = 0; c < 4; ++c)
+            e[c] = e[c] * (m < M && k + c < K ? cs[k + c] : 0.0f);
+        }
+        v[t][i] = e;
       }
     }
   }
