@@ -28,10 +28,12 @@
 // rows under 32 windows of a 3 x 3 kernel are converted for 32 windows, the four under 112 for 112).  Forms of four
 // wavefronts run two blocks to a CU, so one block's set-up and stores lie under the other's MFMAs.  What bounds the
 // kernel is those serial phases (a block: 5 to 8 thousand cycles until its loads are back, 450 per 64 x 16 values
-// converted, 46 per MFMA of 32, 4 to 8 thousand for the epilogue); slab_form_cost weighs them.  Measured, whole forward
+// converted, 46 per MFMA of 32 (the matrix clock under the power
+// limit), 3 to 7 thousand for the epilogue); slab_form_cost weighs them.  Measured, whole forward
 // with the weights' pass, <4, 1, 2> -> the form taken: [32,64,56,56] x [64,64,3,3] 167 -> 44 us, [64,64,28,28] x
 // [64,64,1,1] 68 -> 18.5, [32,128,28,28] x [128,128,3,3] 71 -> 30, [32,96,27,27] x [48,96,5,5] 94 -> 33;
-// [32,256,14,14] x [256,256,3,3] keeps <4, 1, 2> (26.1 us).
+// [32,256,14,14] x [256,256,3,3] keeps <4, 1, 2> (26.1 us).  Addresses and the extent as they are found now took these
+// from 44.3, 17.9, 30.3, 36.7 (of one day) to 41.2, 16.2, 28.1, 35.5.
 //
 // Numerics: q = rint(x * 2^s) with s chosen so that the slab's largest finite magnitude lands in [2^29, 2^30); the
 // four digit products are accumulated exactly in int32, combined exactly in integers with the windows' sums of q
