@@ -1,6 +1,7 @@
 """Function objects and graph nodes (the subset of python/src/nnabla/function.pyx.tmpl the path needs)."""
 import ctypes
 import weakref
+from array import array
 
 from . import _capi
 from .context import get_current_context
@@ -120,13 +121,15 @@ def forward_nodes(nodes):
         for n in nodes:
             n.forward()
         return
-    count = len(nodes)
-    inputs = [v._h for n in nodes for v in n.inputs]
-    outputs = [v._h for n in nodes for v in n.outputs]
-    ints, handles = ctypes.c_int * count, ctypes.c_void_p
-    _capi.check(_capi.lib().nblac_functions_forward(
-        count, (handles * count)(*[n.function._h for n in nodes]), ints(*[len(n.inputs) for n in nodes]),
-        (handles * len(inputs))(*inputs), ints(*[len(n.outputs) for n in nodes]), (handles * len(outputs))(*outputs)))
+    # Arrays of plain numbers and not of ctypes: a ctypes array has a type for every length, which lives until the next
+    # garbage collection and is made again ahead of a new graph's first launch (eleven functions after a collection: 130 to
+    # 185 us with ctypes arrays, 50 to 64 this way).
+    functions = array("Q", [n.function._h.value for n in nodes])
+    inputs = array("Q", [v._h.value for n in nodes for v in n.inputs])
+    outputs = array("Q", [v._h.value for n in nodes for v in n.outputs])
+    num_inputs, num_outputs = array("i", [len(n.inputs) for n in nodes]), array("i", [len(n.outputs) for n in nodes])
+    at = [ctypes.c_void_p(a.buffer_info()[0]) for a in (functions, num_inputs, inputs, num_outputs, outputs)]
+    _capi.check(_capi.lib().nblac_functions_forward(len(nodes), *at))
 
 
 class FunctionNode(object):

@@ -153,3 +153,42 @@ def test_caching_allocator_reuses_and_merges_host_blocks():
     big2 = nn.Variable((1 << 20,))
     big2.d = 0.0
     assert L.nblac_allocator_bytes(b"cpu", b"", 1) == level   # the freed block was reused, not re-allocated
+
+
+def test_a_graph_hands_its_functions_over_without_new_types(monkeypatch):
+    """Variable.forward gives the host library every function with its inputs and outputs in order, and makes no ctypes
+    array types for it: those are gone after a garbage collection, and a new graph's first launch waited for them to be made
+    again."""
+    import gc
+    with nn.context_scope(get_extension_context('hip')):
+        x, w = nn.Variable((3, 4)), nn.Variable((4, 4))
+        h = F.binary_connect_affine(F.relu(x), w, nn.Variable((4, 4)))
+        for _ in range(13):
+            h = F.relu(h)
+        h = F.add2(h, x)
+    seen = {}
+
+    class Host(object):
+        @staticmethod
+        def nblac_functions_forward(n, functions, num_inputs, inputs, num_outputs, outputs):
+            words = lambda p, count: list((ctypes.c_uint64 * count).from_address(p.value))
+            ints = lambda p: list((ctypes.c_int32 * n).from_address(p.value))
+            seen.update(functions=words(functions, n), num_inputs=ints(num_inputs), num_outputs=ints(num_outputs))
+            seen.update(inputs=words(inputs, sum(seen["num_inputs"])), outputs=words(outputs, sum(seen["num_outputs"])))
+            return 0
+
+    array_types = lambda: {id(o) for o in gc.get_objects() if type(o) is type(ctypes.Array)}
+    calls = []
+    monkeypatch.setattr(_capi, "lib", lambda: type("Counts", (), {
+        "nblac_functions_forward": staticmethod(lambda *a: calls.append(a) or 0)}))
+    gc.collect()
+    before = array_types()
+    h.forward()
+    assert array_types() <= before and len(calls) == 1
+    monkeypatch.setattr(_capi, "lib", lambda: Host)
+    h.forward()
+    nodes = h._function_order()
+    assert seen["functions"] == [n.function._h.value for n in nodes] and len(nodes) == 16
+    assert seen["num_inputs"] == [len(n.inputs) for n in nodes] and seen["num_outputs"] == [len(n.outputs) for n in nodes]
+    assert seen["inputs"] == [v._h.value for n in nodes for v in n.inputs]
+    assert seen["outputs"] == [v._h.value for n in nodes for v in n.outputs]
