@@ -283,15 +283,17 @@ size_t nbla_hip_affine_backward_workspace_bytes(int64_t M, int64_t K, int64_t N)
  * is the identity, sign.hpp:48-50).  Replaces
  * BinaryWeightAffine<float>::backward_impl, binary_weight_affine.cpp:124-146,
  * BinaryConnectAffine<float>::backward_impl, binary_connect_affine.cpp:73-92
- * and the Affine backward they call, affine.cpp:98-140.  dx runs on the
- * bit-weight product (W is binarised again into its transposed packing); Wb
- * (the forward's fp32 signs) is only needed when quantize_zero_to is neither +1
- * nor -1, and only read when W then holds weights that are neither negative nor
- * positive: they are counted on the device, the bit-weight product does
- * nothing when the count is non-zero and an fp32 product over Wb launched
- * behind it does nothing when it is zero (no synchronisation, the host never
- * reads the count).  dx, dW, db may be NULL (not propagated); accum_* != 0 adds
- * to the existing gradient. */
+ * and the Affine backward they call, affine.cpp:98-140.  Wb (the forward's fp32
+ * signs) is needed for dx when quantize_zero_to is neither +1 nor -1, at every
+ * size (NBLA_HIP_ERR_VALUE without it, before any launch).  Small layers take dx
+ * from the signs of W in one launch (bf16 parts of dy times alpha; for
+ * quantize_zero_to -1, 0 and 1); the others run it on the bit-weight product (W
+ * is binarised again into its transposed packing), where Wb is only read when W
+ * then holds weights that are neither negative nor positive: they are counted on
+ * the device, the bit-weight product does nothing when the count is non-zero and
+ * an fp32 product over Wb launched behind it does nothing when it is zero (no
+ * synchronisation, the host never reads the count).  dx, dW, db may be NULL (not
+ * propagated); accum_* != 0 adds to the existing gradient. */
 int nbla_hip_binary_affine_backward_f32(const float *dy, const float *x,
                                         const float *W, const float *Wb,
                                         const float *alpha, float *dx,

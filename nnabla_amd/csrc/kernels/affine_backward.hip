@@ -167,15 +167,16 @@ int nbla_hip_binary_affine_backward_f32(const float *dy, const float *x, const f
     return rc;
   hipStream_t stream = as_stream(stream_);
   char *base = static_cast<char *>(workspace);
-  const bool one_part = quantize_zero_to == 1.0f || quantize_zero_to == -1.0f || quantize_zero_to == 0.0f;
-  if (dx && one_part && gemm_small_applies(M, N, K, kSmallGradInput)) {
+  const bool representable = quantize_zero_to == 1.0f || quantize_zero_to == -1.0f;
+  if (dx && !representable && !Wb) // whichever form the size takes
+    return fail(NBLA_HIP_ERR_VALUE, "the binarised weights are needed when Sign(0) is neither +1 nor -1.");
+  if (dx && (representable || quantize_zero_to == 0.0f) && gemm_small_applies(M, N, K, kSmallGradInput)) {
     // small layers: the signs straight from W, in one launch
     rc = launch_gemm_small(dy, false, W, false, nullptr, dx, M, N, K, accum_x != 0, stream, true, alpha,
                            quantize_zero_to);
     if (rc)
       return rc;
   } else if (dx) {
-    const bool representable = (quantize_zero_to == 1.0f || quantize_zero_to == -1.0f);
     uint32_t *bits = reinterpret_cast<uint32_t *>(base + p.bits_off);
     int *count = reinterpret_cast<int *>(base + p.count_off);
     // Sign(W) packed for the contraction over n: W is stored [K, N] = [output column of dx][contraction]
@@ -196,8 +197,6 @@ int nbla_hip_binary_affine_backward_f32(const float *dy, const float *x, const f
     if (rc)
       return rc;
     if (!representable) {
-      if (!Wb)
-        return fail(NBLA_HIP_ERR_VALUE, "the binarised weights are needed when Sign(0) is neither +1 nor -1.");
       // dx[m, k] (+)= sum_n (dy[m, n] alpha[n]) Wb[k, n]
       rc = launch_gemm_f32_mapped(dy, Wb, true, nullptr, nullptr, dx, M, N, K, 1, K, 1, stream, count, alpha,
                                   accum_x != 0);

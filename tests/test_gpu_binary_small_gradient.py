@@ -63,3 +63,17 @@ def test_extreme_and_non_finite_values():
         assert np.array_equal(f(dx), f(ref))
     fin = np.isfinite(ref)
     assert (np.abs(dx - ref)[fin] <= (terms * 2.0 ** -21)[fin] + 2.0 ** -149).all()
+
+
+@pytest.mark.parametrize("M,K,N", [(20, 250, 250), (300, 3000, 2000)])  # in one launch, and by the bit-weight product
+@pytest.mark.parametrize("zero_to", [0.0, 0.5])
+def test_without_the_signs_it_is_refused_at_every_size(M, K, N, zero_to):
+    """Sign(0) that is neither +1 nor -1 needs the forward's signs for dx, whichever form the size takes, and dx is not
+    touched; the weights' gradient alone needs none."""
+    kernels.init(0)
+    dy, W, alpha = (torch.from_numpy(v).cuda() for v in _case(M, K, N))
+    x, dx = torch.zeros(M, K, device="cuda"), torch.full((M, K), 3.0, device="cuda")
+    with pytest.raises(kernels.KernelError):
+        kernels.binary_affine_backward(dy, x, W, None, alpha, zero_to, dx=dx, want=(True, False, False))
+    assert bool((dx == 3.0).all())
+    kernels.binary_affine_backward(dy, x, W, None, alpha, zero_to, want=(False, True, True))
