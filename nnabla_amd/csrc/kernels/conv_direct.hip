@@ -17,6 +17,8 @@
 #include "gemm_layout.hpp"
 #include "internal.hpp"
 
+#include <cmath>
+
 namespace nbla_hip {
 namespace {
 
@@ -715,6 +717,15 @@ static int direct_tile_width(const ConvGeom &g) {
   return 0;
 }
 
+// The tiled kernel's time in microseconds, from 1300 sizes measured of 1 to 23 channels, 8 to 64 maps, 4 to 25 taps and 64 to
+// 330000 windows (7 % off, 37 at the worst): a block's chain of loads, four taps of the innermost axis at a time, and its
+// products, or the CUs' share of all blocks.
+static double direct_tile_time(const ConvGeom &g, int width) {
+  const double loads = (double)(g.Cg * g.k[0] * g.k[1] * ceil_div(g.k[2], 4)), products = (double)(g.Kg * width) / 16.0;
+  const double blocks = (double)(g.outer * (g.O / width) * ceil_div(g.out_sp_size, (int64_t)kDirectBlock));
+  return 4.5 + std::hypot(0.28 * loads + 0.13 * products, blocks / 256.0 * (0.65 + 0.06 * loads + 0.036 * products));
+}
+
 // The forward alone also for a single group of very few input channels under a kernel of many taps (the first layer
 // of an image network: 3 channels, 7 x 7): rows of the unfolded matrix that are mostly padding of the k tiles, which
 // the products on the matrix cores gather element by element.
@@ -728,13 +739,22 @@ bool conv_direct_forward_applies(const ConvGeom &g, bool binary) {
   // 256 channels wide and gather such inputs element by element, the tiled fp32 kernel is the faster one
   // ([4,16,16,56,56] x [32,16,3,3,3]: 0.86 ms binary, 0.24 ms real-weight on the matrix cores) -- unless the convolution
   // over input positions in LDS (binary) or the bf16 one (real weights) covers the geometry, which read an input once for
-  // all taps: [8,18,14,14] x [16,18,3,3] 43 us here, 12.6 and (with the weights' quantization) 45 against 20 there,
-  // [32,16,56,56] x [64,16,3,3] 77 / 80 against 36 / 56, [16,16,28,28] x [32,16,5,5] 98 / 100 against 20 / 22, and a third of
-  // the distance from float64.  With a few taps there is little to save: [16,18,56,56] x [16,18,1,1] 15 / 17 against 17 / 30.
-  if (!(g.group == 1 && g.Cg < 24 && g.O <= 64 && direct_tile_width(g) != 0))
+  // all taps.  With a few taps there is little to save: [16,18,56,56] x [16,18,1,1] 15 us binary and 17 real here, 17 and 30
+  // there.
+  const int width = g.group == 1 && g.Cg < 24 && g.O <= 64 ? direct_tile_width(g) : 0;
+  if (width == 0)
     return false;
-  // Fewer than a thousand windows of a binary layer stay (its plan query promises so, [1,16,27,27] x [64,16,3,3] among them).
-  return g.k_size < 4 || !(binary ? g.M >= 1024 && conv_slab_applies(g) : conv_real_applies(g, false, false));
+  if (g.k_size < 4)
+    return true;
+  // Those forms spend their time on padding where channels or maps are very few and windows many, and on launches where all
+  // is little: an estimate of both sides, theirs 5 % up (what lies within is seldom 1.2 times off either way).  Device time
+  // here and there, binary (with the signs' pass): [1,16,8,8] x [8,16,2,2] 19.0 and 11.9 us, [1,23,28,28] x [16,23,3,5] 86
+  // and 15, [70,20,112,112] x [8,20,4,1] stride 2 49 and 99, [13,20,160,160] x [32,20,7,1] 171 and 742; real:
+  // [1,16,14,14] x [16,16,3,3] 28 and 13, [335,2,20,20] x [8,2,2,2] 7.0 and 44, [16,16,112,112] x [8,16,1,4] 19 and 56,
+  // [18,17,112,112] x [16,17,3,3] 56 and 112.  Off float64 the matrix-core forms are a third of this one.
+  const double here = direct_tile_time(g, width) + (binary ? 2.2 : 0.0);
+  const double there = binary ? conv_slab_time(g) : conv_real_applies(g, false, false) ? conv_real_forward_time(g) : 0.0;
+  return there <= 0.0 || here < 1.05 * there;
 }
 
 namespace {

@@ -88,6 +88,7 @@ int launch_conv_direct_backward(const float *dy, const float *x, const float *w,
 // tensors: the forward, or (transposed) the input gradient, dx (+)= from dy.  W: the group's weights, alpha (may be null)
 // scales them per output channel; signs: Sign(W) stands for them.  bias: the group's, forward only.
 bool conv_real_applies(const ConvGeom &g, bool transposed, bool binary); // and is the faster form
+double conv_real_forward_time(const ConvGeom &g); // estimated, in us, for few channels and maps; 0: not covered
 size_t conv_real_workspace_bytes(const ConvGeom &g, bool transposed);
 int launch_conv_real(const float *in, const float *W, const float *bias, float *out, const ConvGeom &g, bool transposed,
                      int64_t grp, bool accumulate, const float *alpha, bool signs, float zero_to, void *workspace,
@@ -108,6 +109,7 @@ int launch_conv_dw(const float *dy, const float *x, float *dW, const ConvGeom &g
 // alpha_out is not null (and writing it there), and writes the number of weights that are neither negative nor
 // positive to *zero_count when that is not null.  alpha_out and bias belong to the group; y is the whole output.
 bool conv_slab_applies(const ConvGeom &g);
+double conv_slab_time(const ConvGeom &g); // estimated, in us; 0: not covered
 size_t conv_slab_prepared_bytes(const ConvGeom &g);
 // The figures of the form that a geometry takes, where the kernel covers it: windows per block, blocks per sample (and
 // tile of channels), the input positions its LDS holds per block, LDS bytes.  Host only.

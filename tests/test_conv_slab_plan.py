@@ -98,7 +98,9 @@ def test_the_plan_holds_every_tap_and_is_tight():
 
 @pytest.mark.parametrize("C,in_sp,expected", [
     (8, (14, 14), False),      # too few input channels per group
-    (16, (27, 27), False),     # few channels to few maps: fp32 on the vector units
+    (12, (27, 27), False),     # the same: fp32 on the vector units
+    (16, (27, 27), True),      # as few as it takes, to few maps, however few the windows are
+    (16, (8, 8), True),
     (40, (14, 14), True),      # 40 channels padded to 64
     (256, (14, 14), True),
     (1024, (14, 14), True),    # the channels under a block do not fit the LDS: some after the other
@@ -106,6 +108,20 @@ def test_the_plan_holds_every_tap_and_is_tight():
 ])
 def test_which_geometries_take_the_form(C, in_sp, expected):
     plan = kernels.binary_convolution_slab_plan(1, C, in_sp, 64, (3, 3), (1, 1), (1, 1), (1, 1), 1)
+    assert (plan is not None) == expected
+
+
+@pytest.mark.parametrize("outer,C,in_sp,O,kernel,stride,expected", [
+    (1, 23, (28, 28), 16, (3, 5), 1, True),         # 15 us against 86 of the fp32 kernel
+    (1, 16, (8, 8), 8, (2, 2), 1, True),            # 12 against 19: the fewest windows
+    (16, 23, (56, 56), 64, (2, 2), 1, True),        # 19 against 47
+    (13, 20, (160, 160), 32, (7, 1), 1, False),     # 742 against 171: few channels and maps, many windows
+    (70, 20, (112, 112), 8, (4, 1), 2, False),      # 99 against 49
+    (134, 16, (80, 80), 16, (3, 2), 2, False),      # 92 against 48
+])
+def test_few_channels_to_few_maps_take_the_faster_form(outer, C, in_sp, O, kernel, stride, expected):
+    pad = tuple(k // 2 for k in kernel)
+    plan = kernels.binary_convolution_slab_plan(outer, C, in_sp, O, kernel, pad, (stride, stride), (1, 1), 1)
     assert (plan is not None) == expected
 
 

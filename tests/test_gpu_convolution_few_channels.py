@@ -1,5 +1,5 @@
-"""Convolutions of 16 to 23 channels to at most 64 maps, which the matrix-core forms take from four taps on (a thousand
-windows for binary weights) and the fp32 kernel otherwise: both sides of each line, against float64."""
+"""Convolutions of few channels to at most 64 maps, which the matrix-core forms take from four taps on where they are
+estimated the faster ones and the fp32 kernel otherwise: both sides of the line, few windows and many, against float64."""
 import numpy as np
 import pytest
 import torch
@@ -11,7 +11,8 @@ from util import to_np
 pytestmark = pytest.mark.gpu
 
 # batch, channels, height, width, maps, kernel, stride
-CASES = [(1, 16, 31, 33, 16, 3, 1), (1, 16, 32, 32, 16, 3, 1), (6, 23, 13, 14, 64, 3, 1), (5, 20, 28, 28, 33, 2, 2),
+CASES = [(1, 16, 8, 8, 16, 3, 1), (1, 23, 9, 9, 24, 2, 1), (2, 16, 27, 27, 64, 3, 1), (1, 16, 31, 33, 16, 3, 1),
+         (1, 16, 32, 32, 16, 3, 1), (6, 23, 13, 14, 64, 3, 1), (5, 20, 28, 28, 33, 2, 2),
          (4, 18, 27, 27, 24, 5, 2), (3, 17, 20, 21, 30, 1, 1), (2, 22, 40, 40, 64, (1, 3), 1)]
 
 
@@ -50,3 +51,25 @@ def test_both_weights_against_float64(case, zero_to):
     I = torch.zeros(w.shape, dtype=torch.int32, device="cuda")
     yr = kernels.inq_convolution(xd, wd.clone(), I, wd.clone(), I.clone(), bd, *geo, 1, 4, kernels.INQ_NO_SELECTION)
     check(to_np(yr), w.astype(np.float64))
+
+
+@pytest.mark.parametrize("B,C,sp,O,k", [(64, 16, (56, 56), 8, (1, 4)), (150, 2, (20, 20), 8, (2, 2)),
+                                        (16, 8, (112, 112), 16, (3, 3))])
+def test_real_weights_over_many_windows_stay_on_the_fp32_kernel(B, C, sp, O, k):
+    """Its products one after the other in fp32, bit for bit: on the matrix cores such layers take two to six times as long,
+    their rows of weights and channels being padding for the most part."""
+    kernels.init(0)
+    rng = np.random.RandomState(B + C + O)
+    x, w = rng.randn(B, C, *sp).astype(np.float32), rng.randn(O, C, *k).astype(np.float32)
+    pad = tuple(v // 2 for v in k)
+    I = torch.zeros(w.shape, dtype=torch.int32, device="cuda")
+    wd = torch.from_numpy(w).cuda()
+    y = to_np(kernels.inq_convolution(torch.from_numpy(x).cuda(), wd, I, wd.clone(), I.clone(), None, pad, (1, 1), (1, 1), 1,
+                                      4, kernels.INQ_NO_SELECTION))
+    xp = np.pad(x[-1], ((0, 0), (pad[0],) * 2, (pad[1],) * 2))
+    ref = np.zeros(y.shape[1:], np.float32)
+    for c in range(C):
+        for i in range(k[0]):
+            for j in range(k[1]):
+                ref = ref + xp[c, i:i + ref.shape[1], j:j + ref.shape[2]] * w[:, c, i, j, None, None]
+    assert np.array_equal(y[-1], ref)
