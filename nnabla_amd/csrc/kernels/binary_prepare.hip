@@ -947,12 +947,12 @@ __global__ __launch_bounds__(kPrepBlock) void column_stats(const float *__restri
 #pragma unroll 8
       for (int64_t r = r0 + ty; r < r_end; r += 4)
         take(*reinterpret_cast<const float4_u *>(src + r * ld + cl));
-    } else {
+    } else { // (several rows in flight here too: one at a time a layer of one or two outputs lost 4 to 5 us of 45 to 60)
+      const bool second = C > 1, third = C > 2;
+#pragma unroll 8
       for (int64_t r = r0 + ty; r < r_end; r += 4) {
-        float4_t q = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (int j = 0; j < (int)C; ++j)
-          q[j] = src[r * ld + j];
-        take(q);
+        const float *p = src + r * ld;
+        take(float4_t{p[0], second ? p[1] : 0.0f, third ? p[2] : 0.0f, 0.0f});
       }
     }
     if (skip) { // column c0 + j is element skip + j of the quad read
