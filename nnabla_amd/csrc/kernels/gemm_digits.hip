@@ -51,13 +51,16 @@ constexpr int kSegVec = kDigits * 64; // uint4 per fragment and k tile
 // CU).  64 KiB of LDS per block, two blocks per CU (or two k groups in one).
 constexpr int kStages = 4;
 constexpr int kPartBytes = kSegs * 2 * kFragBytes, kStageBytes = 2 * kPartBytes;
-constexpr int kCopies = kStageBytes / kFragBytes / kWaves; // 1 KiB copies per wavefront and phase
+constexpr int kCopies = kStageBytes / kFragBytes / kWaves; // 1 KiB copies per wavefront and phase, which the loop's wait counts
+static_assert(kCopies * kWaves * kFragBytes == kStageBytes, "a phase's copies fill its buffer");
+// MFMA tiles along either side of a wavefront's 64 x 64.  Every phase of every form deals its copies out behind the MFMAs
+// of one fragment, one copy behind each: as many as the wait counts.
+constexpr int kFrags = 4;
+static_assert(kFrags == kCopies, "a phase issues the copies that the wait counts");
 
 // Phases per k step: all nine digit pairs' leading six: {a0 b0} {a0 b2, a0 b1} {a1 b0, a1 b1, a2 b0}; one-digit B:
 // {a0 b} {a1 b, a2 b}; both one-digit: {a b}.
 constexpr int phases_per_step(bool one_a, bool narrow) { return one_a ? 1 : (narrow ? 2 : 3); }
-// Copies that a wavefront issues per phase, whatever the form: the unit in which the loop's wait counts.
-constexpr int copies_per_call(bool /*one_a*/, bool /*narrow*/, int /*groups*/) { return kCopies; }
 
 // Workgroup barrier without the memory fence of __syncthreads() (which would wait for every global -> LDS copy in
 // flight, including those of later k tiles); the waits that matter are explicit.
@@ -161,7 +164,6 @@ __device__ __forceinline__ void gemm_digits_tile(const GemmDigitsArgs &a, unsign
   static_assert(kLoopWait >= 0 && pipeline::one_tile_safe(kStages, kStages - 1, kLoopWait),
                 "the copy pipeline hands a buffer over too early");
   static_assert(pipeline::counter_fits(kLoopWait, kCopies), "vmcnt is a 6-bit counter");
-  static_assert(copies_per_call(kOneA, kNarrow, kGroups) == kCopies, "the wait counts the copies a call issues");
 
   // fragment f (0..3) of this wavefront's rows (part of side A) or columns (side B) in the part at `part`
   const int a_frag = (wm * 2 * 2 + (lane >> 5)) * kFragBytes + (((lane >> 4) & 1) * 32 + (lane & 15)) * 16;
@@ -217,7 +219,7 @@ __device__ __forceinline__ void gemm_digits_tile(const GemmDigitsArgs &a, unsign
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < kFrags; ++j) {
         mma(acc[i][j][0], a0[i], b0[j]);
         if (i == 0 && (j & 1)) {
           a0[2 + (j >> 1)] = frag(a_frag, buf, 2 + (j >> 1));
@@ -239,7 +241,7 @@ __device__ __forceinline__ void gemm_digits_tile(const GemmDigitsArgs &a, unsign
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < kFrags; ++j) {
           mma(acc[i & 3][j][1 + (i >> 2)], af[i], b0[j]);
           if (j == 0 && i + 2 < 8) {
             af[i + 2] = frag(a_frag, buf + ((i + 2) >> 2) * kPartBytes, (i + 2) & 3);
@@ -265,7 +267,7 @@ __device__ __forceinline__ void gemm_digits_tile(const GemmDigitsArgs &a, unsign
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
+          for (int i = 0; i < kFrags; ++i) {
             mma(acc[i][j & 3][j < 4 ? 2 : 1], a0[i], bf[j]);
             if (i == 0 && j + 2 < 8) {
               bf[j + 2] = frag(b_frag, buf + ((j + 2) >> 2) * kPartBytes, (j + 2) & 3);
@@ -292,7 +294,7 @@ __device__ __forceinline__ void gemm_digits_tile(const GemmDigitsArgs &a, unsign
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
+          for (int j = 0; j < kFrags; ++j) {
             mma(acc[i & 3][j][i < 4 ? 1 : 2], af[i], b0[j]);
             if (j == 0 && i + 2 < 8) {
               af[i + 2] = frag(a_frag, buf + ((i + 2) >> 2) * kPartBytes, (i + 2) & 3);

@@ -153,4 +153,23 @@ def test_kernels_take_their_waits_from_the_model():
     loop_waits = [w for w in re.findall(r"^ +NBLA_WAIT_VMCNT\(([^;\n]+)\);", digits, re.M) if w.strip() != "0"]
     assert loop_waits == ["kLoopWait * kCopies"], loop_waits
     assert "pipeline::one_tile_safe(kStages, kStages - 1, kLoopWait)" in digits
-    assert "copies_per_call(kOneA, kNarrow, kGroups) == kCopies" in digits
+
+
+def test_every_phase_of_the_digit_product_issues_the_copies_its_wait_counts():
+    """The wait at the top of a phase counts kCopies per phase: each phase deals out one copy per MFMA of one fragment (a
+    loop to kFrags, which the kernel asserts to be kCopies, at one value of the other loop's variable), and none elsewhere."""
+    digits = open(os.path.join(KERNELS, "gemm_digits.hip")).read()
+    assert "static_assert(kFrags == kCopies" in digits
+    loop = digits[digits.index("for (int left = steps; left > 0; --left) {"):]
+    loop = loop[:loop.index("NBLA_WAIT_VMCNT(0)")]
+    phases = re.findall(r"hand_over\(\);(.*?)advance\(\);", loop, re.S)
+    dealt = []
+    for phase in phases:
+        calls = re.findall(r"if \((\w) == \d\) \{\s*copy_ahead\((P\d)\(\), (\w)\);\s*pin\(\);\s*\}", phase)
+        assert len(calls) == 1 and phase.count("copy_ahead") == 1, phase
+        other, name, var = calls[0]
+        before = phase[:phase.index("copy_ahead")]
+        loops = re.findall(r"for \(int (\w) = 0; \w < (\w+); \+\+\w\)", before)
+        assert loops[-2:] and loops[-1] == (var, "kFrags") and loops[-2][0] == other != var, loops
+        dealt.append(name)
+    assert dealt == ["P0", "P1", "P1", "P2"] and loop.count("copy_ahead") == len(dealt)
