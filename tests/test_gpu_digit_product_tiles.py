@@ -36,23 +36,61 @@ def test_weight_gradient(M, K, N):
     _check(old, x.T, dy, 2.0)
 
 
-@pytest.mark.parametrize("M,K,N", [(300, 4095, 1001), (1500, 2000, 2111)])
+def _narrow_weights(K, N, gen):
+    return (torch.sign(torch.randn(K, N, generator=gen, device="cuda")) *
+            torch.exp2(torch.randint(-5, 1, (K, N), generator=gen, device="cuda").float()))
+
+
+# (past the one-launch product in both directions: split contractions, one block per CU, two blocks)
+ONE_DIGIT_SIZES = [(300, 4095, 1601), (1500, 2000, 2111), (2100, 2049, 1100)]
+
+
+@pytest.mark.parametrize("M,K,N", ONE_DIGIT_SIZES)
 @pytest.mark.parametrize("narrow_x", [False, True])
 @pytest.mark.parametrize("narrow_w", [False, True])
 def test_one_digit_operands(M, K, N, narrow_x, narrow_w):
     kernels.init(0)
     gen = torch.Generator(device="cuda").manual_seed(M + K + N)
     x = torch.randn(M, K, generator=gen, device="cuda")
-    W = torch.randn(K, N, generator=gen, device="cuda")
+    W = _narrow_weights(K, N, gen) if narrow_w else torch.randn(K, N, generator=gen, device="cuda")
     b = torch.randn(N, generator=gen, device="cuda")
     if narrow_x:
         x = kernels.fixed_point_quantize(x, True, 8, 2.0 ** -4)
-    if narrow_w:
-        W = torch.sign(W) * torch.exp2(torch.randint(-5, 1, (K, N), generator=gen, device="cuda").float())
     y = kernels.affine_digits(x, W, b)
     _check(y - b, x, W) if not (narrow_x and narrow_w) else _exact(y, x, W, b)
-    dx = kernels.affine_backward(torch.randn(M, N, generator=gen, device="cuda"), x, W, want=(True, False, False))[0]
-    assert dx.shape == x.shape and bool(torch.isfinite(dx).all())
+
+
+@pytest.mark.parametrize("M,K,N", ONE_DIGIT_SIZES)
+@pytest.mark.parametrize("narrow_dy", [False, True])
+@pytest.mark.parametrize("narrow_w", [False, True])
+def test_input_gradient_under_one_digit_rows(M, K, N, narrow_dy, narrow_w):
+    """dx = dy . W^T: both operands scaled by rows, so one-digit rows of W multiply their top digit, and those of dy with
+    them.  A tile that holds one other row takes the general form, which gives its remaining rows the same bits."""
+    kernels.init(0)
+    gen = torch.Generator(device="cuda").manual_seed(M + K + N + 1)
+    dy = torch.randn(M, N, generator=gen, device="cuda")
+    if narrow_dy:
+        dy = kernels.fixed_point_quantize(dy, True, 8, 2.0 ** -4)
+    W = _narrow_weights(K, N, gen) if narrow_w else torch.randn(K, N, generator=gen, device="cuda")
+    x = torch.zeros(M, K, device="cuda")
+    gradient = lambda g, w, out=None: kernels.affine_backward(g, x, w, dx=out, want=(True, False, False))[0]
+    dx = gradient(dy, W)
+    if narrow_dy and narrow_w:
+        assert torch.equal(dx, (dy.double() @ W.double().T).float())  # small integers on both sides
+    else:
+        _check(dx, dy, W.T)
+    old = torch.full((M, K), 2.0, device="cuda")
+    gradient(dy, W, old)
+    _check(old, dy, W.T, 2.0)
+    W2, dy2 = W.clone(), dy.clone()
+    for row in (5, K // 2, K - 1):
+        W2[row] = torch.randn(N, generator=gen, device="cuda")
+    kept = (W2 == W).all(1)
+    assert kept.sum() == K - 3 and torch.equal(gradient(dy, W2)[:, kept], dx[:, kept])
+    for row in (0, M // 2, M - 1):
+        dy2[row] = torch.randn(N, generator=gen, device="cuda")
+    kept = (dy2 == dy).all(1)
+    assert kept.sum() == M - 3 and torch.equal(gradient(dy2, W)[kept], dx[kept])
 
 
 def _exact(y, x, W, b):
