@@ -326,10 +326,12 @@ NBLA_API int nblac_function_forward(void *f, void **inputs, int ni, void **outpu
       [&] { static_cast<FuncHandle *>(f)->func->forward(to_variables(inputs, ni), to_variables(outputs, no)); });
 }
 // The forward pass of `n` functions in order: function i takes the next num_inputs[i] of `inputs` and writes the next
-// num_outputs[i] of `outputs`.  A function and the one that follows it on its output may run as one launch.
+// num_outputs[i] of `outputs`.  A function and the one that follows it on its output may run as one launch: *pairs is the
+// number of those.
 NBLA_API int nblac_functions_forward(int n, void **functions, const int *num_inputs, void **inputs, const int *num_outputs,
-                                     void **outputs) {
+                                     void **outputs, int *pairs) {
   return guarded([&] {
+    *pairs = 0;
     for (int i = 0; i < n; ++i) {
       Function *f = static_cast<FuncHandle *>(functions[i])->func.get();
       const Variables in = to_variables(inputs, num_inputs[i]), out = to_variables(outputs, num_outputs[i]);
@@ -338,7 +340,7 @@ NBLA_API int nblac_functions_forward(int n, void **functions, const int *num_inp
         const Variables next_in = to_variables(inputs, 1), next_out = to_variables(outputs, 1);
         Function *next = static_cast<FuncHandle *>(functions[i + 1])->func.get();
         if (next_in[0] == out[0] && f->forward_with_next(in, out, *next, next_in, next_out)) {
-          ++inputs, ++outputs, ++i;
+          ++inputs, ++outputs, ++i, ++*pairs;
           continue;
         }
       }

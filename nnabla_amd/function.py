@@ -116,11 +116,12 @@ class Function(object):
 
 def forward_nodes(nodes):
     """Runs the nodes in order, in one call of the host library: a graph of small functions is bound by what each of them
-    costs before its launch, and a function may run together with the one behind it (ReLU with FixedPointQuantize)."""
+    costs before its launch, and a function may run together with the one behind it (ReLU with FixedPointQuantize).
+    Returns how many pairs did."""
     if not all(type(n) is FunctionNode and type(n.function) is Function for n in nodes):
         for n in nodes:
             n.forward()
-        return
+        return 0
     # Arrays of plain numbers and not of ctypes: a ctypes array has a type for every length, which lives until the next
     # garbage collection and is made again ahead of a new graph's first launch (eleven functions after a collection: 130 to
     # 185 us with ctypes arrays, 50 to 64 this way).
@@ -129,7 +130,9 @@ def forward_nodes(nodes):
     outputs = array("Q", [v._h.value for n in nodes for v in n.outputs])
     num_inputs, num_outputs = array("i", [len(n.inputs) for n in nodes]), array("i", [len(n.outputs) for n in nodes])
     at = [ctypes.c_void_p(a.buffer_info()[0]) for a in (functions, num_inputs, inputs, num_outputs, outputs)]
-    _capi.check(_capi.lib().nblac_functions_forward(len(nodes), *at))
+    pairs = ctypes.c_int(0)
+    _capi.check(_capi.lib().nblac_functions_forward(len(nodes), *at, ctypes.byref(pairs)))
+    return pairs.value
 
 
 class FunctionNode(object):

@@ -10,6 +10,7 @@ import nnabla_amd as nn
 import nnabla_amd.functions as F
 from nnabla_amd import kernels
 from nnabla_amd.ext_utils import get_extension_context
+from nnabla_amd.function import forward_nodes
 from util import bits_equal, to_np
 
 pytestmark = pytest.mark.gpu
@@ -48,6 +49,12 @@ def test_the_bits_of_both_functions(size, sign, n, delta, shift):
     torch.cuda.synchronize()
     _pair(x2, mid, x2, sign, n, delta)  # the quantizer's result in the place of x
     assert bits_equal(to_np(mid), to_np(relu)) and bits_equal(to_np(x2), to_np(want))
+    _pair(x, y, y, sign, n, delta)  # both results in one place: the quantizer's stays
+    assert bits_equal(to_np(y), to_np(want))
+    x2 = x.clone()
+    torch.cuda.synchronize()
+    _pair(x2, x2, x2, sign, n, delta)  # and that the place of x
+    assert bits_equal(to_np(x2), to_np(want))
 
 
 def test_no_place_for_relu_is_refused():
@@ -70,7 +77,8 @@ def test_a_graph_gives_what_its_functions_give_one_by_one(shape):
         r2 = F.relu(q)                  # another pair, on the first one's result
         q2 = F.fixed_point_quantize(r2, False, 4, 0.25)
         z = F.add2(q2, r)               # ReLU's result is used elsewhere too
-    z.forward()
+    nodes = z._function_order()
+    assert forward_nodes(nodes) == 2  # both pairs ran as one launch each
     got = [v.d.copy() for v in (r, q, r2, q2, z)]
     for node in z._function_order():
         node.forward()
@@ -79,3 +87,22 @@ def test_a_graph_gives_what_its_functions_give_one_by_one(shape):
     x.d = -x.d  # new values through the same graph
     z.forward()
     assert np.array_equal(r.d, np.maximum(x.d, 0)) and not np.array_equal(r.d, got[0])
+
+
+def test_where_the_pair_does_not_hold_the_functions_run_one_by_one():
+    """A quantizer that writes into ReLU's own array, one that reads another variable than ReLU's result, one that comes
+    later in the order, and a ReLU that no quantizer follows."""
+    rng = np.random.RandomState(4)
+    with nn.context_scope(get_extension_context("hip")):
+        x = nn.Variable((33, 9))
+        x.d = rng.randn(33, 9).astype(np.float32) * 3
+        r = F.relu(x)
+        q = F.fixed_point_quantize(r, True, 8, 2 ** -4, outputs=[r.data])
+        assert forward_nodes(q._function_order()) == 0
+        assert bits_equal(q.d, np.minimum(np.round(np.maximum(x.d, 0) * 16) / 16, np.float32(127 / 16)))
+        a, b = F.relu(x), F.fixed_point_quantize(x, True, 8, 2 ** -4)
+        assert forward_nodes(F.add2(a, b)._function_order()) == 0
+        a = F.relu(x)
+        z = F.add2(F.relu(a), F.fixed_point_quantize(a, True, 8, 2 ** -4))
+        order = [n.name for n in z._function_order()]
+        assert order[1] == order[0] and forward_nodes(z._function_order()) == 0

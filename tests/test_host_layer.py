@@ -170,7 +170,7 @@ def test_a_graph_hands_its_functions_over_without_new_types(monkeypatch):
 
     class Host(object):
         @staticmethod
-        def nblac_functions_forward(n, functions, num_inputs, inputs, num_outputs, outputs):
+        def nblac_functions_forward(n, functions, num_inputs, inputs, num_outputs, outputs, pairs):
             words = lambda p, count: list((ctypes.c_uint64 * count).from_address(p.value))
             ints = lambda p: list((ctypes.c_int32 * n).from_address(p.value))
             seen.update(functions=words(functions, n), num_inputs=ints(num_inputs), num_outputs=ints(num_outputs))
