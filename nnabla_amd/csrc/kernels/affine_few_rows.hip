@@ -1,7 +1,7 @@
 // y = x . W (+ b) for a handful of rows of x and real-valued weights: with at most 16 rows the product is a single
 // pass over W, and turning W into digit operands for the matrix cores costs several such passes.  Plain fp32 on the
-// vector units, the contraction in ascending k inside a slab of K and the slabs added in order (affine.cpp:87-95 adds
-// in Eigen's order: equal to rounding; NaN and Inf propagate element by element as there).
+// vector units, the contraction in ascending k inside a slab of K and the slabs in four groups, in a fixed order
+// (affine.cpp:87-95 adds in Eigen's order: equal to rounding; NaN and Inf propagate element by element as there).
 //
 // Block (1024 columns, slab of K): a thread owns four consecutive columns (one 16-byte load per row of W, eight rows
 // in flight), the slab's rows of x sit in LDS and are read as broadcast 16-byte words (four k per read); a thread

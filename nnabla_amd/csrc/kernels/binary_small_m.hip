@@ -11,11 +11,15 @@
 //
 // The rows of x are the same for every lane: they are fetched with scalar loads and never occupy vector registers.
 //
-// Work decomposition: block = kWavesK wavefronts stacked in K; wavefront wk walks kRowsPerWave rows of the block's
-// 256-column strip.  The block's wavefronts fold their accumulators over wk through LDS (fixed order), and the block writes one
-// partial row per input row, plus the |W| column sums, for its slab of K.  A second, tiny launch adds the slabs in
-// slab order, forms alpha = colsum * ((float)1 / K) and scales: y = (sum_k s * x) * alpha + bias.  Every sum runs in a
-// fixed order, so results do not change from run to run.
+// Work decomposition: block = kWavesK wavefronts stacked in K; wavefront wk walks 8 to 64 rows (small_m_rows_per_wave)
+// of the block's 256-column strip.  The block's wavefronts fold their accumulators over wk through LDS (fixed order), and
+// the block writes one partial row per input row, plus the |W| column sums, for its slab of K.  A second, tiny launch adds
+// the slabs, every fourth one in each of four groups and then the groups, forms alpha = colsum * ((float)1 / K) and scales:
+// y = (sum_k s * x) * alpha + bias.  Every sum runs in a fixed order, so results do not change from run to run.
+//
+// Off float64 (relative, 2-norm; sums alone): 1.0e-7 to 2.2e-7 on N(0, 1), uniform, ReLU'd and outlier-ridden rows from 1 x
+// 1500 x 3001 to 16 x 60001 x 257, where the exact sums of 24-bit digits are 1.5e-7 to 7.5e-6 off (a digit counts from its
+// row's largest value); where all terms have one sign 4e-8 to 5e-8 against 2e-8, the rounding of the result itself.
 #include "common.hpp"
 #include "gemm_layout.hpp"
 #include "internal.hpp"
@@ -32,7 +36,8 @@ typedef float float4_u __attribute__((ext_vector_type(4), aligned(4))); // one 1
 // whole of a 4096 x 11008 weight matrix (688 blocks) is resident at once and no second round of blocks trails behind.
 constexpr int kWavesK = 4, kWavesN = 1;
 constexpr int kThreads = 64 * kWavesK * kWavesN;
-// sixteen rows, and eight with a row's end taken apart, need more than 128 registers
+// sixteen rows need more than 128 registers, and from two on the form that takes a row's end apart does (132 to 195; held to
+// 128 it spills 7 to 33)
 constexpr int blocks_per_cu(int MT, bool aligned) { return MT >= (aligned ? 16 : 2) ? 2 : 4; }
 constexpr int kMostRowsPerWave = 64, kLeastRowsPerWave = 8; // rows of W one wavefront walks
 constexpr int kWaveCols = 256;                       // 64 lanes x float4

@@ -359,7 +359,7 @@ template <int kItems, int kW> __global__ __launch_bounds__(64 * kW, 2) void conv
 #pragma unroll
   for (int w = 0; w < kW; ++w)
     amax = max(amax, s_max[0][w]), amin = min(amin, s_max[1][w]);
-  // ---- the wavefronts' sums: each finishes sixteen of the rows
+  // ---- the wavefronts' sums: each finishes its share of the rows, sixteen or (of eight wavefronts) eight
   float *s_red = reinterpret_cast<float *>(smem); // [wave][row][position]
 #pragma unroll
   for (int i = 0; i < 2; ++i)
