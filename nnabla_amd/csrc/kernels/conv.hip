@@ -227,7 +227,7 @@ __global__ __launch_bounds__(kShiftBlock) void conv_row_shift_windows(const floa
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
           const int c = c0 + kShiftWaves * j;
-          v[j] = src[(int64_t)(c < Cg ? c : wave) * plane];
+          v[j] = src[(int64_t)scan_channel(c, Cg) * plane];
         }
 #pragma unroll
         for (int j = 0; j < 16; ++j)

@@ -320,7 +320,7 @@ __device__ __forceinline__ void unfold_main_loop(const GemmBitsArgs &a, unsigned
 #pragma unroll
           for (int j = 0; j < 16; ++j) {
             const int c = c0 + 8 * j;
-            v[j] = src[(int64_t)(c < Cg ? c : wave) * plane];
+            v[j] = src[(int64_t)scan_channel(c, Cg) * plane];
           }
 #pragma unroll
           for (int j = 0; j < 16; ++j)
@@ -375,7 +375,7 @@ __device__ __forceinline__ void unfold_main_loop(const GemmBitsArgs &a, unsigned
   #pragma unroll
         for (int j = 0; j < 16; ++j) {
           const int c = c0 + 16 * j;
-          v[slot][j] = src[(int64_t)(c < Cg ? c : slice) * plane];
+          v[slot][j] = src[(int64_t)scan_channel(c, Cg) * plane];
         }
         okv[slot] = ok;
         c0v[slot] = c0;

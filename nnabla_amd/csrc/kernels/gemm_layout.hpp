@@ -91,6 +91,12 @@ __host__ __device__ inline DigitOperand digit_operand(int64_t M, int64_t K) {
   return d;
 }
 
+// Channel that a lane of a scan over Cg channels reads in its place for channel c: the loads of a round are issued
+// without a branch, and a round's last channels, or a lane's whole share when there are fewer channels than lanes,
+// lie past the group's.  They read its last channel again (a plane that other lanes read anyway) and the result is not
+// used; one past the last image's channels may lie past the tensor.
+__host__ __device__ constexpr int scan_channel(int c, int Cg) { return c < Cg ? c : Cg - 1; }
+
 #if defined(__HIPCC__)
 // Sixteen fixed-point values q (|q| <= kDigitMax) of one lane -> its four words of each digit fragment (digit 0 the
 // top one; value j in byte j % 4 of word j / 4).  The three balanced base-256 digits of q are the low three bytes of
