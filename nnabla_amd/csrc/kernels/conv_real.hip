@@ -239,8 +239,10 @@ template <int kItems, int kW> __global__ __launch_bounds__(64 * kW, 2) void conv
       const int left = a.Kc - c0 - 8 * (dst[i] & 15);
 #pragma unroll
       for (int j = 0; j < 8; ++j)
+        // (the range check takes the sum of both offsets; the scalar one stays inside the tensor, so that the sum with
+        // kOutside stays below 2^32)
         xv[i][j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-            xr, (int)(j < left ? src[i] : kOutside), min(c0 + j, a.Kc - 1) * in_plane * 4, 0)); // (the range check needs a scalar offset inside)
+            xr, (int)(j < left ? src[i] : kOutside), min(c0 + j, a.Kc - 1) * in_plane * 4, 0));
     }
   };
   const int plane_bytes = octets * a.slots * 16;
