@@ -1021,28 +1021,39 @@ __global__ __launch_bounds__(kPrepBlock) void column_shift(uint32_t *__restrict_
     cmax[c] = (uint32_t)narrow;
 }
 
-// The same from the slabs' statistics: block = 64 columns x 4 groups of slabs, folded through LDS in a fixed order; the
-// columns' sums go to db (added to it with `accumulate`).
-template <bool kDetect, bool kSum>
+// The same from the slabs' statistics: block = 256 / kGroups columns x kGroups groups of slabs, eight slabs in flight per
+// thread, folded through LDS in a fixed order; the columns' sums go to db (added to it with `accumulate`).
+template <bool kDetect, bool kSum, int kGroups>
 __global__ __launch_bounds__(kPrepBlock) void column_stats_final(ColumnPartials in, int64_t slabs, int64_t blocks_x,
                                                                  uint32_t *__restrict__ cmax, int32_t *__restrict__ shift,
                                                                  int64_t C, int64_t rows, int32_t *__restrict__ flag,
                                                                  float *__restrict__ db, int accumulate) {
-  __shared__ uint32_t part[4][64], part_min[kDetect ? 4 : 1][64];
-  __shared__ float part_sum[kSum ? 4 : 1][64];
-  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-  const int64_t c = (int64_t)blockIdx.x * 64 + tx, cc = c < C ? c : C - 1;
+  constexpr int kCols = kPrepBlock / kGroups, kBatch = 8;
+  __shared__ uint32_t part[kGroups][kCols], part_min[kDetect ? kGroups : 1][kCols];
+  __shared__ float part_sum[kSum ? kGroups : 1][kCols];
+  const int tx = threadIdx.x % kCols, ty = threadIdx.x / kCols;
+  const int64_t c = (int64_t)blockIdx.x * kCols + tx, cc = c < C ? c : C - 1;
   uint32_t m = 0u, mn = 0xffffffffu, other = 0u;
   float sum = 0.0f;
-#pragma unroll 4
-  for (int64_t s = ty; s < slabs; s += 4) {
-    m = max(m, in.max[s * C + cc]);
-    if (kDetect) {
-      mn = min(mn, in.min[s * C + cc]);
-      other |= in.other[s * blocks_x + (cc >> 8)];
+  for (int64_t s0 = ty; s0 < slabs; s0 += kBatch * kGroups) {
+    uint32_t vm[kBatch], vn[kBatch], vo[kBatch];
+    float vs[kBatch];
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) { // (past the end: the last slab again, its sum left out)
+      const int64_t s = s0 + j * kGroups < slabs ? s0 + j * kGroups : slabs - 1;
+      vm[j] = in.max[s * C + cc];
+      vn[j] = kDetect ? in.min[s * C + cc] : 0u;
+      vo[j] = kDetect ? in.other[s * blocks_x + (cc >> 8)] : 0u;
+      vs[j] = kSum ? in.sum[s * C + cc] : 0.0f;
     }
-    if (kSum)
-      sum += in.sum[s * C + cc];
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) {
+      m = max(m, vm[j]);
+      if (kDetect)
+        mn = min(mn, vn[j]), other |= vo[j];
+      if (kSum && s0 + j * kGroups < slabs)
+        sum += vs[j];
+    }
   }
   part[ty][tx] = m;
   if (kDetect) {
@@ -1055,17 +1066,20 @@ __global__ __launch_bounds__(kPrepBlock) void column_stats_final(ColumnPartials 
   __syncthreads();
   if (ty != 0 || c >= rows)
     return;
-  m = c < C ? max(max(m, part[1][tx]), max(part[2][tx], part[3][tx])) : 0u;
-  if (kDetect)
-    mn = min(min(mn, part_min[1][tx]), min(part_min[2][tx], part_min[3][tx]));
+#pragma unroll
+  for (int g = 1; g < kGroups; ++g) {
+    m = max(m, part[g][tx]);
+    if (kDetect)
+      mn = min(mn, part_min[g][tx]);
+    if (kSum)
+      sum += part_sum[g][tx];
+  }
   int32_t narrow;
-  shift[c] = column_shifts(m, mn, kDetect, flag, narrow);
+  shift[c] = column_shifts(c < C ? m : 0u, mn, kDetect, flag, narrow);
   if (kDetect)
     cmax[c] = (uint32_t)narrow;
-  if (kSum && c < C) {
-    sum = ((sum + part_sum[1][tx]) + part_sum[2][tx]) + part_sum[3][tx];
+  if (kSum && c < C)
     db[c] = accumulate ? db[c] + sum : sum;
-  }
 }
 
 // One wavefront per fragment (32 operand rows = columns of src, 32 contraction steps = rows of src); fragments are
@@ -1166,14 +1180,26 @@ int launch_split_digits_columns(const float *src, int64_t ld, void *digits, int6
   parts.min = parts.max + slabs * C;
   parts.sum = reinterpret_cast<float *>(parts.min + slabs * C);
   parts.other = reinterpret_cast<uint32_t *>(parts.sum + slabs * C);
-  const dim3 grid((unsigned)blocks_x, (unsigned)slabs), final_grid((unsigned)ceil_div(d.rows, 64));
+  const dim3 grid((unsigned)blocks_x, (unsigned)slabs);
+  // Many slabs under few columns: more groups of them, so that no thread walks through more of them than two rounds
+  // of eight (up to 1024 slabs).  Weight gradient of samples x inputs x outputs, four groups at any number of slabs
+  // -> this: 65536 x 256 x 256 231 -> 195 us, 200000 x 16 x 8 390 -> 350, 16384 x 512 x 512 91 -> 83; 4096 x 4096 x 11008 (32
+  // slabs) the same.
+  const int groups = slabs <= 64 ? 4 : (slabs <= 256 ? 16 : 64);
   int32_t *shift = reinterpret_cast<int32_t *>(base + d.shift_off);
+#define NBLA_LAUNCH_STATS_FINAL(D, S, G)                                                                               \
+  hipLaunchKernelGGL((column_stats_final<D, S, G>), dim3((unsigned)ceil_div(d.rows, kPrepBlock / G)), dim3(kPrepBlock),  \
+                     0, stream, parts, slabs, blocks_x, cs.cmax, shift, C, d.rows, cs.flag, db, accumulate_db ? 1 : 0)
 #define NBLA_LAUNCH_STATS(D, S)                                                                                        \
   do {                                                                                                                 \
     hipLaunchKernelGGL((column_stats<D, S>), grid, dim3(kPrepBlock), 0, stream, src, ld, R, C, parts, cs.flag, slab);  \
     NBLA_HIP_LAUNCH_CHECK("column_stats");                                                                             \
-    hipLaunchKernelGGL((column_stats_final<D, S>), final_grid, dim3(kPrepBlock), 0, stream, parts, slabs, blocks_x,    \
-                       cs.cmax, shift, C, d.rows, cs.flag, db, accumulate_db ? 1 : 0);                                 \
+    if (groups == 4)                                                                                                   \
+      NBLA_LAUNCH_STATS_FINAL(D, S, 4);                                                                                \
+    else if (groups == 16)                                                                                             \
+      NBLA_LAUNCH_STATS_FINAL(D, S, 16);                                                                               \
+    else                                                                                                               \
+      NBLA_LAUNCH_STATS_FINAL(D, S, 64);                                                                               \
     NBLA_HIP_LAUNCH_CHECK("column_stats_final");                                                                       \
   } while (0)
   if (detect_narrow)
@@ -1183,6 +1209,7 @@ int launch_split_digits_columns(const float *src, int64_t ld, void *digits, int6
   else
     NBLA_LAUNCH_STATS(false, false);
 #undef NBLA_LAUNCH_STATS
+#undef NBLA_LAUNCH_STATS_FINAL
   return launch_split_columns(src, ld, base, R, C, d, cs, stream);
 }
 

@@ -36,6 +36,43 @@ def test_weight_gradient(M, K, N):
     _check(old, x.T, dy, 2.0)
 
 
+# rows around the ends of slabs of 64, 128 and 256 rows and where the number of groups that fold their statistics changes; the
+# largest value of every column, and of dy's, lies in another slab: a slab left out gives digits that do not fit
+@pytest.mark.parametrize("M,K,N", [(4096, 40, 70), (4097, 1, 3), (16384, 33, 5), (16385, 7, 64), (16385, 300, 11),
+                                   (70001, 5, 66), (300000, 3, 2)])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_statistics_of_tall_columns(M, K, N, accumulate):
+    kernels.init(0)
+    gen = torch.Generator(device="cuda").manual_seed(M + K + N)
+    x, dy = (torch.randn(M, n, generator=gen, device="cuda") for n in (K, N))
+    x[torch.linspace(0, M - 1, K + 1, device="cuda").long()[1:], torch.arange(K, device="cuda")] = 300.0
+    dy[torch.linspace(0, M - 1, N, device="cuda").long().flip(0), torch.arange(N, device="cuda")] = -500.0
+    W = torch.randn(K, N, generator=gen, device="cuda")
+    given = dict(dW=torch.full((K, N), 2.0, device="cuda"), db=torch.full((N,), 3.0, device="cuda")) if accumulate else {}
+    _, dW, db = kernels.affine_backward(dy, x, W, want=(False, True, True), **given)
+    _check(dW, x.T, dy, 2.0 if accumulate else 0.0)
+    # chains: at most 64 rows of a slab and thread, four threads, 19 slabs a group (300000 rows), 64 groups, what was there
+    ref, bound = dy.double().sum(0) + (3.0 if accumulate else 0.0), dy.double().abs().sum(0) * (160 * 2.0 ** -24)
+    assert bool(((db.double() - ref).abs() <= bound + 1e-6).all())
+
+
+@pytest.mark.parametrize("K", [4097, 16384, 16385, 70001])
+@pytest.mark.parametrize("odd", ["none", "last", "first", "small"])
+def test_one_digit_weights_of_tall_columns(K, odd):
+    """Columns of powers of two are held in one digit unless a value in any slab is none, or is seven binades smaller."""
+    kernels.init(0)
+    gen = torch.Generator(device="cuda").manual_seed(K)
+    x, W = torch.randn(3, K, generator=gen, device="cuda"), _narrow_weights(K, 5, gen)
+    if odd != "none":
+        W[0 if odd == "first" else K - 1, 2] = 2.0 ** -9 if odd == "small" else 0.7
+        x[:, 0 if odd == "first" else K - 1] = 1000.0
+    _check(kernels.affine_digits(x, W), x, W)
+    if odd == "none": # (one-digit weights drop no product: what is left is x's rounding and the result's)
+        ref = x.double() @ W.double()
+        bound = x.abs().amax(1, keepdim=True).double() * W.double().abs().sum(0) * 2.0 ** -23 + ref.abs() * 2.0 ** -22
+        assert bool(((kernels.affine_digits(x, W).double() - ref).abs() <= bound).all())
+
+
 def _narrow_weights(K, N, gen):
     return (torch.sign(torch.randn(K, N, generator=gen, device="cuda")) *
             torch.exp2(torch.randint(-5, 1, (K, N), generator=gen, device="cuda").float()))
