@@ -563,15 +563,6 @@ __global__ __launch_bounds__(256) void gemm_digits_split_sum_rows(const float *_
   }
 }
 
-// Splits of the contraction for an output of `tiles` 128 x 128 tiles and `k_tiles` k tiles: as many as fill the CUs
-// with one block each, at least 16 k tiles per split; 1 = no split.
-inline int64_t digit_product_splits(int64_t tiles, int64_t k_tiles) {
-  if (tiles * 2 > 256 || k_tiles < 32)
-    return 1;
-  const int64_t by_cus = 256 / tiles, by_k = k_tiles / 16;
-  return by_cus < by_k ? by_cus : by_k;
-}
-
 } // namespace
 
 size_t gemm_digits_split_bytes(int64_t M, int64_t K, int64_t N) {
@@ -622,19 +613,18 @@ int launch_gemm_digits(const void *adigits, const void *bdigits, const float *bi
     a.finish = a.step_end == a.k_tiles ? 1 : 0;
     // the operands' last k tiles are padding to a multiple of eight: whole rounds of two k groups' steps are enough (20
     // samples, 3777 x 2246, with its operands: 62 -> 47 us)
-    const int64_t filled = ceil_div(ceil_div(K, kTileK), 4) * 4;
+    const int64_t filled = ceil_div(ceil_div(K, kTileK), 4) * 4, padded_tiles = a.step_end - a.step_begin;
     a.step_end = a.step_end < filled ? a.step_end : filled;
     a.split_tiles = 0;
     const unsigned blocks = (unsigned)(a.blocks_m * a.blocks_n);
     const int64_t chunk_tiles = a.step_end - a.step_begin;
-    int64_t splits = split_ws ? digit_product_splits(blocks, chunk_tiles) : 1;
-    while (splits > 1 && (size_t)splits * M * N * sizeof(float) > split_ws_bytes)
-      --splits;
+    const int64_t most = split_ws ? (int64_t)(split_ws_bytes / ((size_t)M * N * sizeof(float))) : 1;
+    const DigitSplit split = digit_split(blocks, padded_tiles, chunk_tiles, most);
+    const int64_t splits = split.count;
     if (splits > 1) {
       // few output tiles, long contraction: every split writes a dense partial result, summed in split order
       GemmDigitsArgs part = a;
-      part.split_tiles = ceil_div(ceil_div(chunk_tiles, splits), 8) * 8;
-      splits = ceil_div(chunk_tiles, part.split_tiles);
+      part.split_tiles = split.tiles;
       part.y = static_cast<float *>(split_ws);
       part.inner = 1, part.outer_stride = N, part.n_stride = 1;
       part.accumulate = 0, part.bias = nullptr;

@@ -91,6 +91,29 @@ __host__ __device__ inline DigitOperand digit_operand(int64_t M, int64_t K) {
   return d;
 }
 
+// Splits of the contraction of a digit x digit product for an output of `tiles` 128 x 128 tiles and `k_tiles` (padded) k
+// tiles: as many as fill the CUs with one block each, at least 16 k tiles per split; 1 = no split.
+__host__ __device__ inline int64_t digit_product_splits(int64_t tiles, int64_t k_tiles) {
+  if (tiles * 2 > 256 || k_tiles < 32)
+    return 1;
+  const int64_t by_cus = 256 / tiles, by_k = k_tiles / 16;
+  return by_cus < by_k ? by_cus : by_k;
+}
+// The same for the k tiles that hold something, `filled` of them, of which a split takes a multiple of eight; at most `most`
+// splits.  Counted from the padded tiles: 252 of 256 are sixteen splits of 16, where fifteen of 17 would be rounded up to
+// eleven of 24 (product of 3 rows and 8032 x 4 18.4 -> 15.4 us, of 562 and 7464 x 48 22.7 -> 19.7).
+struct DigitSplit {
+  int64_t count, tiles;
+};
+__host__ __device__ inline DigitSplit digit_split(int64_t tiles, int64_t padded, int64_t filled, int64_t most) {
+  DigitSplit s;
+  s.count = digit_product_splits(tiles, padded);
+  s.count = s.count < most ? s.count : (most > 1 ? most : 1);
+  s.tiles = ceil_div(ceil_div(filled, s.count), 8) * 8;
+  s.count = ceil_div(filled, s.tiles);
+  return s;
+}
+
 // Channel that a lane of a scan over Cg channels reads in its place for channel c: the loads of a round are issued
 // without a branch, and a round's last channels, or a lane's whole share when there are fewer channels than lanes,
 // lie past the group's.  They read its last channel again (a plane that other lanes read anyway) and the result is not
