@@ -14,7 +14,9 @@ pytestmark = pytest.mark.gpu
 
 # rows, inputs, outputs: W large enough that the one-launch form leaves it (more than 1024 inputs), or N a multiple of four
 SIZES = [(1, 1, 4), (1, 31, 8), (3, 33, 1000), (16, 100, 260), (1, 1025, 5), (2, 1030, 255), (5, 1500, 257), (9, 1027, 1023),
-         (16, 2049, 66), (12, 300, 3000), (7, 4099, 514), (4, 1100, 4099), (1, 4095, 11007), (1, 5000, 12)]
+         (16, 2049, 66), (12, 300, 3000), (7, 4099, 514), (4, 1100, 4099), (1, 4095, 11007), (1, 5000, 12),
+         # three, four and five slabs of 32 rows: the sums of up to four need no fold
+         (2, 96, 8), (4, 128, 300), (4, 129, 300), (8, 160, 261)]
 
 
 @pytest.mark.parametrize("M,K,N", SIZES)
@@ -40,6 +42,22 @@ def test_against_float64(M, K, N):
     y2, Wb2, _ = kernels.binary_weight_affine(xd, Wd, bd, Wb=Wd)  # in place: W is read before it is written
     assert Wb2.data_ptr() == Wd.data_ptr() and torch.equal(Wb2, Wb)
     assert torch.allclose(y2, y, rtol=0, atol=4e-6 * float(y.abs().max()) + 1e-6)
+
+
+# one to five and nine slabs of 64 rows on the matrix cores
+@pytest.mark.parametrize("M,K,N", [(9, 16, 8), (18, 64, 20), (33, 80, 260), (64, 192, 2608), (17, 256, 264), (64, 272, 300),
+                                   (40, 560, 12)])
+def test_few_slabs_on_the_matrix_cores(M, K, N):
+    kernels.init(0)
+    gen = torch.Generator(device="cuda").manual_seed(M + K + N)
+    x, W = torch.randn(M, K, generator=gen, device="cuda"), torch.randn(K, N, generator=gen, device="cuda")
+    b = torch.randn(N, generator=gen, device="cuda")
+    y, Wb, alpha = kernels.binary_weight_affine(x, W, b)
+    a64, terms = W.double().abs().mean(0), x.double().abs().sum(1, keepdim=True)
+    ref = (x.double() @ Wb.double()) * a64 + b
+    bound = terms * (K + 16) * 2.0 ** -24 * a64 + 4e-6 * ref.abs() + 2.0 ** -23 * b.abs()
+    assert torch.equal(Wb, torch.where(W < 0, -1.0, 1.0)) and bool((alpha.double() - a64).abs().le(2e-6 * a64).all())
+    assert bool(((y.double() - ref).abs() <= bound + 1e-7).all())
 
 
 @pytest.mark.parametrize("M,K,N", [(5, 1500, 3001), (16, 4099, 4099)])
